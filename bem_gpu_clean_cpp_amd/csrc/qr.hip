@@ -866,6 +866,11 @@ __global__ __launch_bounds__(NT) void qr_solve_small(const typename QT<T>::c2 *A
             }
             s_w[tid].x = wr;
             s_w[tid].y = wi;
+        } else if (tid < kNB) {
+            // a narrow last panel: these meet zeros below, which shared
+            // memory's old contents (infinities, NaNs) would not survive
+            s_w[tid].x = 0;
+            s_w[tid].y = 0;
         }
         __syncthreads();
         for (int i = j0 + tid; i < M; i += NT) {
@@ -998,6 +1003,11 @@ __global__ __launch_bounds__(NT) void qr_apply_step(const typename QT<T>::c2 *A,
             }
             s_w[tid].x = wr;
             s_w[tid].y = wi;
+        } else if (tid < kNB) {
+            // a narrow last panel: these meet zeros below, which shared
+            // memory's old contents (infinities, NaNs) would not survive
+            s_w[tid].x = 0;
+            s_w[tid].y = 0;
         }
         __syncthreads();
         T sr = 0, si = 0;
