@@ -17,7 +17,9 @@
 //                   of the reference (mesh.cu:253-595) in FP64;
 //   asm_tile        the regular 6x6 rule (mesh.cu:597-672) for every (row,
 //                   element) pair of a tile, FP32 (or FP64), with the singular
-//                   lanes taking the FP64 values;
+//                   lanes taking the FP64 values; asm_tile_fast is its FP32
+//                   form, with rules of 7, 12 or 16 points where every row of
+//                   the wave is far enough from the element (far_rules.hpp);
 //   asm_finalize    per row: 1 - sum c on the node diagonal
 //                   (atomicFuncs.cu:227-235, 99-102), and the boundary-condition
 //                   vector sum_e (cc/cb) sum_j g_j (atomicFuncs.cu:104-115);
@@ -27,11 +29,13 @@
 #include <algorithm>
 #include <cmath>
 #include <cstdio>
+#include <cstring>
 #include <map>
 #include <mutex>
 #include <vector>
 
 #include "bem_internal.hpp"
+#include "far_rules.hpp"
 #include "xcd.hpp"
 
 namespace bem {
@@ -77,6 +81,7 @@ template <typename R>
 struct AsmArgs {
     const float4 *__restrict__ pts;
     const ElemRec<R> *__restrict__ recs;
+    const FarRec *__restrict__ far;  // FP32 fast kernel: the far rules' element records
     const R *__restrict__ sing;  // (e*3+v)*16: p[0..5], c[6], bterm[7..8]
     const int *__restrict__ tile_ptr;
     const int *__restrict__ tile_entries;
@@ -90,6 +95,8 @@ struct AsmArgs {
     int M, N, nrbg, nwg;
     int r0;  // first row assembled (rows r0..M-1 land in A rows 0..M-r0-1)
     R k, kf, rw;  // k, k/(2 pi), rho*omega
+    double kf64;  // k/(2 pi)
+    int far_rho2, far7_rho2;  // (FP32 bits) rho^2 up to which the wavelength lets the far rules be used
     int impedance;  // any element with ca != 0
     QTab<R> q;
 };
@@ -155,6 +162,53 @@ __global__ void prep_elems(const double *__restrict__ pts64, const int *__restri
         r.vv[t] = (R)vv;
     }
     for (int i = 0; i < (int)(sizeof(r.pad) / sizeof(int)); i++) r.pad[i] = 0;
+    out[e] = r;
+}
+
+__global__ void prep_far(const double *__restrict__ pts64, const int *__restrict__ elems,
+                         const ElemRec<double> *__restrict__ recs, int E, FarRec *__restrict__ out) {
+    const int e = blockIdx.x * blockDim.x + threadIdx.x;
+    if (e >= E) return;
+    const ElemRec<double> &rec = recs[e];
+    FarRec r;
+    double u[3][3], uu[3] = {0, 0, 0};
+    for (int d = 0; d < 3; d++) {
+        double s = 0;
+        for (int j = 0; j < 3; j++) s += pts64[3 * elems[3 * e + j] + d];
+        r.c[d] = s / 3.0;
+        for (int j = 0; j < 3; j++) {
+            u[j][d] = pts64[3 * elems[3 * e + j] + d] - r.c[d];
+            uu[j] += u[j][d] * u[j][d];
+        }
+        r.u1[d] = (float)(2.0 * u[0][d]);
+        r.u2[d] = (float)(2.0 * u[1][d]);
+        r.n[d] = (float)rec.n[d];
+    }
+    r.sJ = (float)(rec.J / (4.0 * kPi));
+    for (int j = 0; j < 3; j++) r.uu[j] = (float)uu[j];
+    const double rho2 = fmax(uu[0], fmax(uu[1], uu[2]));
+    r.rho2 = (float)rho2;
+    r.far7 = (float)(kFar7D2 * rho2);
+    r.far12 = (float)(kFar12D2 * rho2);
+    r.far16 = (float)(kFar16D2 * rho2);
+    for (int j = 0; j < 3; j++) r.nodes[j] = rec.nodes[j];
+    for (int j = 0; j < 2; j++) {
+        r.beta[j] = (float)rec.beta[j];
+        r.gamma[j] = (float)rec.gamma[j];
+    }
+    auto dist2 = [&](double n1, double n2) {
+        double s = 0;
+        for (int d = 0; d < 3; d++) {
+            const double y = n1 * u[0][d] + n2 * u[1][d] + (1.0 - n1 - n2) * u[2][d];
+            s += y * y;
+        }
+        return (float)s;
+    };
+#pragma unroll
+    for (int q = 0; q < Far12::ng; q++) r.d12[q] = dist2(Far12::g1[q], Far12::g2[q]);
+#pragma unroll
+    for (int q = 0; q < Far16::ng; q++) r.d16[q] = dist2(Far16::g1[q], Far16::g2[q]);
+    r.pad[0] = r.pad[1] = 0;
     out[e] = r;
 }
 
@@ -444,7 +498,19 @@ __device__ __forceinline__ constexpr float gl_Wrho(int n, int m) {
     return (float)(0.25 * GL6::w[n] * GL6::w[m] * (0.5 + 0.5 * GL6::eta[m]) * (0.5 + 0.5 * GL6::eta[m]));
 }
 
-template <bool IMP, bool RAW, bool GH>
+typedef __attribute__((address_space(4))) const ElemRec<float> CElemRec;
+
+__device__ __forceinline__ bool wave_all(bool p) { return __builtin_amdgcn_ballot_w64(!p) == 0; }
+
+// The rule is chosen per (wave, element): the fewest points that every row of
+// the wave may take.  Element records and tile lists are read as scalar loads
+// (constant address space): as vector loads, which the compiler falls back to
+// because it cannot see that A is never the record array, a pair took 19 vector
+// memory instructions instead of 6 and a chain of waits (10242 nodes: 2.78 ms
+// against 2.12).
+// IMP: some element has ca != 0; SRC: some element has cc != 0 (without it
+// the boundary term is zero and no g is summed).
+template <bool IMP, bool RAW, bool GH, bool SRC>
 __global__ __launch_bounds__(256) void asm_tile_fast(AsmArgs<float> a) {
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
@@ -453,138 +519,227 @@ __global__ __launch_bounds__(256) void asm_tile_fast(AsmArgs<float> a) {
     const int rbg = L - tile * a.nrbg;
     const int row = a.r0 + (rbg * 4 + wave) * 64 + lane;
     const bool active = row < a.M;
+    if (wave_all(!active)) return;  // the workgroup's last waves may have no rows
+    const unsigned lrow = (unsigned)(row - a.r0);
     const float4 xp = a.pts[active ? row : 0];
+    const double xd = xp.x, yd = xp.y, zd = xp.z;
     const float k = a.k;
     const float krev = a.kf;  // k / (2 pi)
     const float inv4pi = (float)(1.0 / (4.0 * kPi));
     const float MAGIC = 12582912.0f;  // 1.5 * 2^23
     float c_acc = 0, br_acc = 0, bi_acc = 0;
-    const int it0 = a.tile_ptr[tile], it1 = a.tile_ptr[tile + 1];
+    CInt *entries = (CInt *)a.tile_entries, *slots = (CInt *)a.tile_slots;
+    const int it0 = ((CInt *)a.tile_ptr)[tile], it1 = ((CInt *)a.tile_ptr)[tile + 1];
+    // what an entry's first loads and branches need, asked for while the entry
+    // before is integrated: a wave that is alone on its SIMD (small meshes)
+    // then waits for fewer loads in turn
+    struct Next {
+        int ent, rho2, node[3], slot[3];
+        float far16;
+        double c[3];
+    } nx;
+    auto fetch = [&](int it) {
+        nx.ent = entries[it];
+        CFarRec &f = ((CFarRec *)a.far)[nx.ent >> 8];
+        nx.rho2 = __float_as_int(f.rho2);
+        nx.far16 = f.far16;
+#pragma unroll
+        for (int j = 0; j < 3; j++) {
+            nx.node[j] = f.nodes[j];
+            nx.slot[j] = GH ? slots[3 * it + j] : 0;
+            nx.c[j] = f.c[j];
+        }
+    };
+    if (it0 < it1) fetch(it0);
     for (int it = it0; it < it1; ++it) {
-        const int ent = a.tile_entries[it];
+        const Next cur = nx;
+        const int ent = cur.ent;
         const int e = ent >> 8;
-        const ElemRec<float> &rec = a.recs[e];
-        const float ax = rec.p3[0] - xp.x, ay = rec.p3[1] - xp.y, az = rec.p3[2] - xp.z;
-        const float dn = rec.n[0] * ax + rec.n[1] * ay + rec.n[2] * az;
-        const float aa = __builtin_fmaf(ax, ax, __builtin_fmaf(ay, ay, az * az));
-        // 2 a.v_n = 2 a.e1 + 2 theta_n a.f
-        const float ae1 = __builtin_fmaf(ax, rec.e1[0], __builtin_fmaf(ay, rec.e1[1], az * rec.e1[2]));
-        const float af = __builtin_fmaf(ax, rec.f[0], __builtin_fmaf(ay, rec.f[1], az * rec.f[2]));
-        const float ae1x2 = ae1 + ae1;
-        // S = sum W rho H~ and ht = sum W H~ over all 36 points; the theta
-        // moment h2 = sum_n theta_n A_n of the per-row sums A_n comes from the
-        // running totals S_n of S after each row,
-        //   h2 = sum_{n<5} (theta_n - theta_{n+1}) S_n + theta_5 S_5,
-        // and h1 = S - h2 (likewise g1, g2 from SC = sum W rho G~)
-        float Sr = 0, Si = 0, h2r = 0, h2i = 0, htr = 0, hti = 0, gr = 0, gi = 0, cc = 0;
-        float SCr = 0, SCi = 0, g2r = 0, g2i = 0;
+        if (it + 1 < it1) fetch(it + 1);
+        CFarRec &fr = ((CFarRec *)a.far)[e];
+        // the three columns this pair adds to: A's, or a ghost vertex's side
+        // column; their values so far are asked for before the quadrature
+        float2 *col[3];
+        float2 v[3];
 #pragma unroll
-        for (int n = 0; n < 6; n++) {
-            const float th = gl_theta(n);
-            const float tav = __builtin_fmaf(2.0f * th, af, ae1x2);
-            const float vv = rec.vv[n];
-#pragma unroll
-            for (int m = 0; m < 6; m++) {
-                const float rho = gl_rho(m), W = gl_W(n, m), Wr = gl_Wrho(n, m);
-                const float r2 = __builtin_fmaf(rho, __builtin_fmaf(rho, vv, tav), aa);
-                const float rinv = __builtin_amdgcn_rsqf(r2);
-                const float r = r2 * rinv;
-                float u;
-                if (RAW) {
-                    u = r * krev;
-                } else {
-                    const float t2 = __builtin_fmaf(r, krev, MAGIC);
-                    const float jf = t2 - MAGIC;
-                    u = __builtin_fmaf(r, krev, -jf);
-                }
-                const float sn = __builtin_amdgcn_sinf(u), cs = __builtin_amdgcn_cosf(u);
-                const float rinv2 = rinv * rinv;
-                const float q3 = rinv2 * rinv;  // 1/r^3
-                const float q2k = k * rinv2;    // k/r^2
-                // 4 pi r dG/dn / (-dn) = (cos kr - i sin kr)(1/r^3 + i k/r^2)
-                const float Hr = __builtin_fmaf(cs, q3, sn * q2k);
-                const float Hi = __builtin_fmaf(cs, q2k, -sn * q3);
-                Sr = __builtin_fmaf(Wr, Hr, Sr);
-                Si = __builtin_fmaf(Wr, Hi, Si);
-                htr = __builtin_fmaf(W, Hr, htr);
-                hti = __builtin_fmaf(W, Hi, hti);
-                // 4 pi G = (cos kr - i sin kr) / r
-                if (IMP) {
-                    const float Gr = cs * rinv, Gi = -sn * rinv;
-                    gr = __builtin_fmaf(W, Gr, gr);
-                    gi = __builtin_fmaf(W, Gi, gi);
-                    SCr = __builtin_fmaf(Wr, Gr, SCr);
-                    SCi = __builtin_fmaf(Wr, Gi, SCi);
-                } else {
-                    const float Wg = W * rinv;
-                    gr = __builtin_fmaf(Wg, cs, gr);
-                    gi = __builtin_fmaf(-Wg, sn, gi);
-                }
-                cc = __builtin_fmaf(W, q3, cc);
-            }
-            // theta moment of the rho-weighted sums from their running totals
-            const float dth = gl_dtheta(n);
-            h2r = __builtin_fmaf(dth, Sr, h2r);
-            h2i = __builtin_fmaf(dth, Si, h2i);
-            if (IMP) {
-                g2r = __builtin_fmaf(dth, SCr, g2r);
-                g2i = __builtin_fmaf(dth, SCi, g2i);
-            }
+        for (int j = 0; j < 3; j++) {
+            col[j] = nullptr;
+            if ((ent >> j) & 1) col[j] = a.A + (size_t)cur.node[j] * a.ldA;
+            else if (GH) col[j] = a.side + (size_t)cur.slot[j] * a.Mp;
+            v[j] = make_float2(0.f, 0.f);
+            if (col[j] && !((ent >> (3 + j)) & 1) && active) v[j] = col[j][lrow];
         }
-        const float h1r = Sr - h2r, h1i = Si - h2i;
-        const float g1r = SCr - g2r, g1i = SCi - g2i;
-        const float sJ = rec.J * inv4pi;
-        const float sh = -dn * sJ;
-        float p0r = sh * h1r, p0i = sh * h1i;
-        float p1r = sh * h2r, p1i = sh * h2i;
-        float p2r = sh * (htr - Sr), p2i = sh * (hti - Si);
-        const float sg = a.rw * sJ;
-        const float gsr = -sg * gi, gsi = sg * gr;
-        if (IMP) {
-            const float br = rec.beta[0], bi = rec.beta[1];
-            const float G0r = -sg * g1i, G0i = sg * g1r;
-            const float G1r = -sg * g2i, G1i = sg * g2r;
-            const float G2r = gsr - G0r - G1r, G2i = gsi - G0i - G1i;
-            p0r -= br * G0r - bi * G0i; p0i -= br * G0i + bi * G0r;
-            p1r -= br * G1r - bi * G1i; p1i -= br * G1i + bi * G1r;
-            p2r -= br * G2r - bi * G2i; p2i -= br * G2i + bi * G2r;
-        }
-        float cval = -dn * sJ * cc;
-        float btr = rec.gamma[0] * gsr - rec.gamma[1] * gsi;
-        float bti = rec.gamma[0] * gsi + rec.gamma[1] * gsr;
-        const int sv = (row == rec.nodes[0]) ? 0 : (row == rec.nodes[1]) ? 1 : (row == rec.nodes[2]) ? 2 : -1;
-        if (sv >= 0) {
-            const float *sg2 = a.sing + ((size_t)e * 3 + sv) * 16;
-            p0r = sg2[0]; p0i = sg2[1]; p1r = sg2[2]; p1i = sg2[3]; p2r = sg2[4]; p2i = sg2[5];
-            cval = sg2[6];
-            btr = sg2[7];
-            bti = sg2[8];
-        }
-        if (active) {
-            const float pr[3] = {p0r, p1r, p2r}, pi[3] = {p0i, p1i, p2i};
+        // centroid from the row, in FP64: the common phase k r0 is good to
+        // FP32 however many wavelengths the row is away
+        const double axd = cur.c[0] - xd, ayd = cur.c[1] - yd, azd = cur.c[2] - zd;
+        const double r02 = fma(axd, axd, fma(ayd, ayd, azd * azd));
+        const float r02f = (float)r02;
+        const int rho2 = cur.rho2;  // (positive floats compare as integers: scalar compares)
+        float pr[3], pi[3], cval, btr = 0, bti = 0;
+        if (rho2 <= a.far_rho2 && wave_all(!active || r02f >= cur.far16)) {
+            const float y = __builtin_amdgcn_rsqf(r02f);
+            const double ra = r02 * (double)y;
+            const double err = fma(-ra, ra, r02);  // r0^2 - ra^2
+            const double r0 = fma(err, 0.5 * (double)y, ra);
+            const float i0 = __builtin_fmaf(0.5f * y, (float)err * y * y, y);
+            const float u0 = (float)__builtin_amdgcn_fract(r0 * a.kf64);
+            const float s0 = __builtin_amdgcn_sinf(u0), c0 = __builtin_amdgcn_cosf(u0);
+            const float r0f = (float)r0;
+            const float kr0 = k * r0f, kr0rev = krev * r0f;
+            const float ax = (float)axd, ay = (float)ayd, az = (float)azd;
+            const float dn = fr.n[0] * ax + fr.n[1] * ay + fr.n[2] * az;
+            const float i02 = i0 * i0;
+            const float T1 = i02 * __builtin_fmaf(ax, fr.u1[0], __builtin_fmaf(ay, fr.u1[1], az * fr.u1[2]));
+            const float T2 = i02 * __builtin_fmaf(ax, fr.u2[0], __builtin_fmaf(ay, fr.u2[1], az * fr.u2[2]));
+            FarSums s;
+            if (rho2 <= a.far7_rho2 && wave_all(!active || r02f >= fr.far7))
+                far_sums<Far7, IMP, SRC>(fr.uu, nullptr, T1, T2, i02, kr0, kr0rev, s);
+            else if (wave_all(!active || r02f >= fr.far12))
+                far_sums<Far12, IMP, SRC>(fr.uu, fr.d12, T1, T2, i02, kr0, kr0rev, s);
+            else
+                far_sums<Far16, IMP, SRC>(fr.uu, fr.d16, T1, T2, i02, kr0, kr0rev, s);
+            // h_j = -dn sJ i0^3 e^{-i k r0} h_j', c = -dn sJ i0^3 c'
+            const float m = -dn * fr.sJ * (i02 * i0);
+            const float fx = m * c0, fy = -m * s0;
 #pragma unroll
             for (int j = 0; j < 3; j++) {
-                float2 *dst = nullptr;
-                if ((ent >> j) & 1) dst = a.A + (size_t)rec.nodes[j] * a.ldA + (row - a.r0);
-                else if (GH) dst = a.side + (size_t)a.tile_slots[3 * it + j] * a.Mp + (row - a.r0);
-                if (dst) {
-                    float2 v;
-                    if ((ent >> (3 + j)) & 1) {
-                        v.x = pr[j];
-                        v.y = pi[j];
-                    } else {
-                        v = *dst;
-                        v.x += pr[j];
-                        v.y += pi[j];
+                pr[j] = __builtin_fmaf(fx, s.hr[j], -fy * s.hi[j]);
+                pi[j] = __builtin_fmaf(fx, s.hi[j], fy * s.hr[j]);
+            }
+            cval = m * s.c;
+            if (IMP || SRC) {
+                // g_j = i rho omega sJ i0 e^{-i k r0} g_j'
+                const float sg = a.rw * fr.sJ * i0;
+                const float qx = sg * s0, qy = sg * c0;
+                float gsr = 0, gsi = 0;
+#pragma unroll
+                for (int j = 0; j < (IMP ? 3 : 1); j++) {
+                    const float Gr = __builtin_fmaf(qx, s.gr[j], -qy * s.gi[j]);
+                    const float Gi = __builtin_fmaf(qx, s.gi[j], qy * s.gr[j]);
+                    if (IMP) {
+                        pr[j] -= fr.beta[0] * Gr - fr.beta[1] * Gi;
+                        pi[j] -= fr.beta[0] * Gi + fr.beta[1] * Gr;
                     }
-                    *dst = v;
+                    gsr += Gr;
+                    gsi += Gi;
+                }
+                btr = fr.gamma[0] * gsr - fr.gamma[1] * gsi;
+                bti = fr.gamma[0] * gsi + fr.gamma[1] * gsr;
+            }
+        } else {
+            CElemRec &rec = ((CElemRec *)a.recs)[e];
+            const float ax = rec.p3[0] - xp.x, ay = rec.p3[1] - xp.y, az = rec.p3[2] - xp.z;
+            const float dn = rec.n[0] * ax + rec.n[1] * ay + rec.n[2] * az;
+            const float aa = __builtin_fmaf(ax, ax, __builtin_fmaf(ay, ay, az * az));
+            // 2 a.v_n = 2 a.e1 + 2 theta_n a.f
+            const float ae1 = __builtin_fmaf(ax, rec.e1[0], __builtin_fmaf(ay, rec.e1[1], az * rec.e1[2]));
+            const float af = __builtin_fmaf(ax, rec.f[0], __builtin_fmaf(ay, rec.f[1], az * rec.f[2]));
+            const float ae1x2 = ae1 + ae1;
+            // S = sum W rho H~ and ht = sum W H~ over all 36 points; the theta
+            // moment h2 = sum_n theta_n A_n of the per-row sums A_n comes from the
+            // running totals S_n of S after each row,
+            //   h2 = sum_{n<5} (theta_n - theta_{n+1}) S_n + theta_5 S_5,
+            // and h1 = S - h2 (likewise g1, g2 from SC = sum W rho G~)
+            float Sr = 0, Si = 0, h2r = 0, h2i = 0, htr = 0, hti = 0, gr = 0, gi = 0, cc = 0;
+            float SCr = 0, SCi = 0, g2r = 0, g2i = 0;
+    #pragma unroll
+            for (int n = 0; n < 6; n++) {
+                const float th = gl_theta(n);
+                const float tav = __builtin_fmaf(2.0f * th, af, ae1x2);
+                const float vv = rec.vv[n];
+    #pragma unroll
+                for (int m = 0; m < 6; m++) {
+                    const float rho = gl_rho(m), W = gl_W(n, m), Wr = gl_Wrho(n, m);
+                    const float r2 = __builtin_fmaf(rho, __builtin_fmaf(rho, vv, tav), aa);
+                    const float rinv = __builtin_amdgcn_rsqf(r2);
+                    const float r = r2 * rinv;
+                    float u;
+                    if (RAW) {
+                        u = r * krev;
+                    } else {
+                        const float t2 = __builtin_fmaf(r, krev, MAGIC);
+                        const float jf = t2 - MAGIC;
+                        u = __builtin_fmaf(r, krev, -jf);
+                    }
+                    const float sn = __builtin_amdgcn_sinf(u), cs = __builtin_amdgcn_cosf(u);
+                    const float rinv2 = rinv * rinv;
+                    const float q3 = rinv2 * rinv;  // 1/r^3
+                    const float q2k = k * rinv2;    // k/r^2
+                    // 4 pi r dG/dn / (-dn) = (cos kr - i sin kr)(1/r^3 + i k/r^2)
+                    const float Hr = __builtin_fmaf(cs, q3, sn * q2k);
+                    const float Hi = __builtin_fmaf(cs, q2k, -sn * q3);
+                    Sr = __builtin_fmaf(Wr, Hr, Sr);
+                    Si = __builtin_fmaf(Wr, Hi, Si);
+                    htr = __builtin_fmaf(W, Hr, htr);
+                    hti = __builtin_fmaf(W, Hi, hti);
+                    // 4 pi G = (cos kr - i sin kr) / r
+                    if (IMP) {
+                        const float Gr = cs * rinv, Gi = -sn * rinv;
+                        gr = __builtin_fmaf(W, Gr, gr);
+                        gi = __builtin_fmaf(W, Gi, gi);
+                        SCr = __builtin_fmaf(Wr, Gr, SCr);
+                        SCi = __builtin_fmaf(Wr, Gi, SCi);
+                    } else if (SRC) {
+                        const float Wg = W * rinv;
+                        gr = __builtin_fmaf(Wg, cs, gr);
+                        gi = __builtin_fmaf(-Wg, sn, gi);
+                    }
+                    cc = __builtin_fmaf(W, q3, cc);
+                }
+                // theta moment of the rho-weighted sums from their running totals
+                const float dth = gl_dtheta(n);
+                h2r = __builtin_fmaf(dth, Sr, h2r);
+                h2i = __builtin_fmaf(dth, Si, h2i);
+                if (IMP) {
+                    g2r = __builtin_fmaf(dth, SCr, g2r);
+                    g2i = __builtin_fmaf(dth, SCi, g2i);
                 }
             }
+            const float h1r = Sr - h2r, h1i = Si - h2i;
+            const float g1r = SCr - g2r, g1i = SCi - g2i;
+            const float sJ = rec.J * inv4pi;
+            const float sh = -dn * sJ;
+            float p0r = sh * h1r, p0i = sh * h1i;
+            float p1r = sh * h2r, p1i = sh * h2i;
+            float p2r = sh * (htr - Sr), p2i = sh * (hti - Si);
+            const float sg = a.rw * sJ;
+            const float gsr = -sg * gi, gsi = sg * gr;
+            if (IMP) {
+                const float br = rec.beta[0], bi = rec.beta[1];
+                const float G0r = -sg * g1i, G0i = sg * g1r;
+                const float G1r = -sg * g2i, G1i = sg * g2r;
+                const float G2r = gsr - G0r - G1r, G2i = gsi - G0i - G1i;
+                p0r -= br * G0r - bi * G0i; p0i -= br * G0i + bi * G0r;
+                p1r -= br * G1r - bi * G1i; p1i -= br * G1i + bi * G1r;
+                p2r -= br * G2r - bi * G2i; p2i -= br * G2i + bi * G2r;
+            }
+            cval = -dn * sJ * cc;
+            if (IMP || SRC) {
+                btr = rec.gamma[0] * gsr - rec.gamma[1] * gsi;
+                bti = rec.gamma[0] * gsi + rec.gamma[1] * gsr;
+            }
+            const int sv = (row == rec.nodes[0]) ? 0 : (row == rec.nodes[1]) ? 1 : (row == rec.nodes[2]) ? 2 : -1;
+            if (sv >= 0) {
+                const float *sg2 = a.sing + ((size_t)e * 3 + sv) * 16;
+                p0r = sg2[0]; p0i = sg2[1]; p1r = sg2[2]; p1i = sg2[3]; p2r = sg2[4]; p2i = sg2[5];
+                cval = sg2[6];
+                btr = sg2[7];
+                bti = sg2[8];
+            }
+            pr[0] = p0r; pr[1] = p1r; pr[2] = p2r;
+            pi[0] = p0i; pi[1] = p1i; pi[2] = p2i;
+        }
+        if (active) {
+#pragma unroll
+            for (int j = 0; j < 3; j++)
+                if (col[j]) col[j][lrow] = make_float2(v[j].x + pr[j], v[j].y + pi[j]);
         }
         if ((ent >> 6) & 1) {
             c_acc += cval;
-            br_acc += btr;
-            bi_acc += bti;
+            if (IMP || SRC) {
+                br_acc += btr;
+                bi_acc += bti;
+            }
         }
     }
     if (active) {
@@ -1435,7 +1590,7 @@ static long ghost_slot_bound(int N, int P) {
 }
 
 // wave_factor: the element-once plan has no halo to pay for more tiles, and
-// runs at twice the waves (icosphere s5: 5.56 ms with 102 tiles, 5.35 with 204)
+// runs at twice the waves (10242 nodes: 2.16 ms with 102 tiles, 1.90 with 204)
 static int choose_tiles(int M, int N, int E, int rows_per_wave, int wave_factor = 1) {
     const char *env = getenv("BEM_TILES");
     if (env && atoi(env) > 0) return std::min(atoi(env), N);
@@ -1565,7 +1720,7 @@ size_t device_problem_bytes(int M, int N, int E) {
     size_t b = 0;
     b += sizeof(float4) * M + sizeof(double) * 3 * M + sizeof(double2) * M;        // points, bterm
     b += (sizeof(int) + sizeof(float2)) * 3 * (size_t)E;                            // elements, bc
-    b += (sizeof(ElemRec<float>) + sizeof(ElemRec<double>)) * (size_t)E;            // element records
+    b += (sizeof(ElemRec<float>) + sizeof(ElemRec<double>) + sizeof(FarRec)) * (size_t)E;  // element records
     b += (sizeof(float) + sizeof(double)) * 48 * (size_t)E;                          // singular terms
     b += sizeof(int) * (P + 1 + 3 * (size_t)E + N);                                  // tile CSR, isolated
     b += (sizeof(float) + sizeof(float2) + sizeof(double) + sizeof(double2)) * P * Mp;  // tile partials
@@ -1626,6 +1781,7 @@ int device_problem_build(const Mesh &m, DeviceProblem &dp, hipStream_t s) {
     HOST_CALL(salloc(&dp.bc, 3 * (size_t)dp.E, s));
     HOST_CALL(salloc(&dp.rec32, dp.E, s));
     HOST_CALL(salloc(&dp.rec64, dp.E, s));
+    HOST_CALL(salloc(&dp.far32, dp.E, s));
     HOST_CALL(salloc(&dp.sing32, (size_t)dp.E * 48, s));
     HOST_CALL(salloc(&dp.sing64, (size_t)dp.E * 48, s));
     HOST_CALL(salloc(&dp.tile_ptr, plan.ptr.size(), s));
@@ -1656,10 +1812,8 @@ int device_problem_build(const Mesh &m, DeviceProblem &dp, hipStream_t s) {
     // runs at twice the waves as well, so it pays below 10 %: the 40962-node
     // ellipsoid (52 tiles, 7.9 % twice) assembles in 82.9 ms against 91.0 ms.
     dp.use_ghost = 0;
-    // Too many side columns for the bound: fewer tiles (two thirds each try;
-    // the 2562-node perturbed ellipsoid starts at 320 tiles of 8 nodes, and at
-    // 64 tiles assembles in 0.48 ms against 0.70 ms on the halo plan).  A halo
-    // under 5 % is left as it is.
+    // Too many side columns for the bound: fewer tiles (two thirds each try).
+    // A halo under 5 % is left as it is.
     GhostPlan gp;
     int gP = choose_tiles(dp.M, dp.N, dp.E, 64, 2);
     bool take = false;
@@ -1711,13 +1865,18 @@ int device_problem_build(const Mesh &m, DeviceProblem &dp, hipStream_t s) {
             HIP_CALL(hipStreamSynchronize(s));  // gp goes out of scope
         }
     }
-    dp.impedance = 0;
-    for (const auto &e : m.elems)
-        if (e.bc[0].x != 0.f || e.bc[0].y != 0.f) dp.impedance = 1;
+    dp.impedance = dp.source = 0;
+    for (const auto &e : m.elems) {
+        // (a NaN counts as set)
+        if (!(e.bc[0].x == 0.f && e.bc[0].y == 0.f)) dp.impedance = 1;
+        if (!(e.bc[2].x == 0.f && e.bc[2].y == 0.f)) dp.source = 1;
+    }
     const int bs = 256;
     prep_elems<float><<<(dp.E + bs - 1) / bs, bs, 0, s>>>(dp.pts64, dp.elems, dp.bc, dp.E, dp.rec32);
     HIP_CALL(hipGetLastError());
     prep_elems<double><<<(dp.E + bs - 1) / bs, bs, 0, s>>>(dp.pts64, dp.elems, dp.bc, dp.E, dp.rec64);
+    HIP_CALL(hipGetLastError());
+    prep_far<<<(dp.E + bs - 1) / bs, bs, 0, s>>>(dp.pts64, dp.elems, dp.rec64, dp.E, dp.far32);
     HIP_CALL(hipGetLastError());
     HIP_CALL(hipStreamSynchronize(s));  // host vectors above go out of scope
     dp.mesh_version = m.version;
@@ -1731,6 +1890,7 @@ void device_problem_free(DeviceProblem &dp) {
     sfree(dp.bc, dp.st);
     sfree(dp.rec32, dp.st);
     sfree(dp.rec64, dp.st);
+    sfree(dp.far32, dp.st);
     sfree(dp.sing32, dp.st);
     sfree(dp.sing64, dp.st);
     sfree(dp.tile_ptr, dp.st);
@@ -1811,6 +1971,7 @@ static int assemble_impl(DeviceProblem &dp, R k, C2 *A, long ldA, int r0, double
     AsmArgs<R> a;
     a.pts = dp.pts;
     a.recs = (const ElemRec<R> *)(sizeof(R) == 4 ? (void *)dp.rec32 : (void *)dp.rec64);
+    a.far = dp.far32;
     a.sing = sing;
     a.tile_ptr = dp.tile_ptr;
     a.tile_entries = dp.tile_entries;
@@ -1828,7 +1989,16 @@ static int assemble_impl(DeviceProblem &dp, R k, C2 *A, long ldA, int r0, double
     a.nwg = a.nrbg * dp.P;
     a.k = k;
     a.kf = (R)(kd / (2.0 * kPi));
+    a.kf64 = kd / (2.0 * kPi);
     a.rw = (R)rw;
+    {
+        // kappa^2 = k^2 rho^2 (a NaN k takes no far rule)
+        const float k2 = (float)(kd * kd);
+        const float f = kFarK2 / k2, f7 = kFar7K2 / k2;
+        a.far_rho2 = a.far7_rho2 = -1;
+        if (f >= 0.f) memcpy(&a.far_rho2, &f, sizeof f);
+        if (f7 >= 0.f) memcpy(&a.far7_rho2, &f7, sizeof f7);
+    }
     a.impedance = dp.impedance;
     for (int q = 0; q < kNQ; q++) {
         a.q.xi1[q] = sizeof(R) == 4 ? (R)qt.xi1[q] : (R)qt.dxi1[q];
@@ -1837,12 +2007,14 @@ static int assemble_impl(DeviceProblem &dp, R k, C2 *A, long ldA, int r0, double
     }
     a.tile_slots = nullptr;
     a.side = nullptr;
+    const int nrows = dp.M - r0;
     bool ghost = false;
     {
         TimedRegion tr;
         timing_begin(tr, sizeof(R) == 4 ? "asm_tile_f32" : "asm_tile_f64", s);
         dim3 grid(a.nwg), block(256);
-        if (dp.qg == 4) {
+        ghost = sizeof(R) == 4 && dp.use_ghost && !getenv("BEM_ASM_HALO") && !getenv("BEM_GENERIC_TILE");
+        if (dp.qg == 4 && !ghost) {
             if (dp.impedance) asm_tile<R, 4, true><<<grid, block, 0, s>>>(a);
             else asm_tile<R, 4, false><<<grid, block, 0, s>>>(a);
         } else if (sizeof(R) == 4 && !getenv("BEM_GENERIC_TILE")) {
@@ -1851,9 +2023,9 @@ static int assemble_impl(DeviceProblem &dp, R k, C2 *A, long ldA, int r0, double
             // distance (at most the bounding-box diagonal of the points) keeps
             // it below that
             const bool raw = kd / (2.0 * kPi) * dp.diam < 250.0;
-            ghost = dp.use_ghost && !getenv("BEM_ASM_HALO");
             AsmArgs<float> &af = *(AsmArgs<float> *)&a;
             if (ghost) {
+                af.nrbg = ((nrows + 63) / 64 + 3) / 4;
                 af.nwg = af.nrbg * dp.gP;
                 grid = dim3(af.nwg);
                 af.tile_ptr = dp.gtile_ptr;
@@ -1861,18 +2033,16 @@ static int assemble_impl(DeviceProblem &dp, R k, C2 *A, long ldA, int r0, double
                 af.tile_slots = dp.gtile_slots;
                 af.side = dp.side;
             }
-#define BEM_FAST(IMP_, RAW_)                                                          \
-    do {                                                                              \
-        if (ghost) asm_tile_fast<IMP_, RAW_, true><<<grid, block, 0, s>>>(af);       \
-        else asm_tile_fast<IMP_, RAW_, false><<<grid, block, 0, s>>>(af);            \
+#define BEM_FAST(IMP_, SRC_)                                                                     \
+    do {                                                                                         \
+        if (ghost && raw) asm_tile_fast<IMP_, true, true, SRC_><<<grid, block, 0, s>>>(af);      \
+        else if (ghost) asm_tile_fast<IMP_, false, true, SRC_><<<grid, block, 0, s>>>(af);       \
+        else if (raw) asm_tile_fast<IMP_, true, false, SRC_><<<grid, block, 0, s>>>(af);         \
+        else asm_tile_fast<IMP_, false, false, SRC_><<<grid, block, 0, s>>>(af);                 \
     } while (0)
-            if (dp.impedance) {
-                if (raw) BEM_FAST(true, true);
-                else BEM_FAST(true, false);
-            } else {
-                if (raw) BEM_FAST(false, true);
-                else BEM_FAST(false, false);
-            }
+            if (dp.impedance) BEM_FAST(true, true);
+            else if (dp.source) BEM_FAST(false, true);
+            else BEM_FAST(false, false);
 #undef BEM_FAST
         } else {
             if (dp.impedance) asm_tile<R, 1, true><<<grid, block, 0, s>>>(a);
@@ -1881,7 +2051,6 @@ static int assemble_impl(DeviceProblem &dp, R k, C2 *A, long ldA, int r0, double
         HIP_CALL(hipGetLastError());
         timing_end(tr, s);
     }
-    const int nrows = dp.M - r0;
     if (ghost && dp.ngnodes > 0) {
         if (ldA % 2 || dp.Mp % 2) BEM_FAIL("ghost_reduce needs even leading dimensions (ldA %ld, Mp %ld)", ldA, dp.Mp);
         TimedRegion tr;

@@ -153,6 +153,8 @@ struct alignas(16) ElemRec {
 };
 static_assert(sizeof(ElemRec<float>) == 128, "record size");
 
+struct FarRec;
+
 // ------------------------------------------------------------ assembly ---
 // Device-resident problem: mesh on the device and assembly scratch.
 struct DeviceProblem {
@@ -164,11 +166,13 @@ struct DeviceProblem {
     float2 *bc = nullptr;         // 3 * E (ca, cb, cc)
     ElemRec<float> *rec32 = nullptr;
     ElemRec<double> *rec64 = nullptr;
+    FarRec *far32 = nullptr;  // far-rule element records (far_rules.hpp)
     float *sing32 = nullptr;      // E * 3 * 16: singular contributions
     double *sing64 = nullptr;
     int P = 0;                    // column tiles
     int qg = 1;                   // lanes per row in the quadrature kernel
     int impedance = 0;            // some element has ca != 0
+    int source = 0;               // some element has cc != 0
     double diam = 0;              // bounding-box diagonal of the M points: bounds every |x - y|
     int *tile_ptr = nullptr;
     int *tile_entries = nullptr;
