@@ -1723,6 +1723,7 @@ size_t device_problem_bytes(int M, int N, int E) {
     b += (sizeof(ElemRec<float>) + sizeof(ElemRec<double>) + sizeof(FarRec)) * (size_t)E;  // element records
     b += (sizeof(float) + sizeof(double)) * 48 * (size_t)E;                          // singular terms
     b += sizeof(int) * (P + 1 + 3 * (size_t)E + N);                                  // tile CSR, isolated
+    b += 40 * 256;                                                                   // the packed arrays' alignment
     b += (sizeof(float) + sizeof(float2) + sizeof(double) + sizeof(double2)) * P * Mp;  // tile partials
     if (qg == 1) {
         // element-once plan: its side columns and index arrays
@@ -1734,6 +1735,96 @@ size_t device_problem_bytes(int M, int N, int E) {
     }
     return b;
 }
+
+namespace {
+// Arrays packed into one device allocation and, for those with host data, one
+// copy: 27 allocations and 14 pageable copies were most of the time it took
+// to set a small mesh up.  Every array starts at a multiple of 256 bytes;
+// the ones with host data come first.
+struct Pack {
+    struct Item {
+        void **dst;
+        const void *src;
+        size_t bytes;
+    };
+    std::vector<Item> items;
+    template <typename T>
+    void add(T **dst, const T *src, size_t n) {
+        items.push_back(Item{(void **)dst, src, n * sizeof(T)});
+    }
+    // (the stream is waited for: the packed copy and its sources may go)
+    int place(char **mem, hipStream_t s) {
+        std::stable_partition(items.begin(), items.end(), [](const Item &i) { return i.src != nullptr; });
+        size_t total = 0, up = 0;
+        for (const Item &i : items) {
+            total += (i.bytes + 255) / 256 * 256;
+            if (i.src) up = total;
+        }
+        HOST_CALL(salloc(mem, std::max<size_t>(total, 256), s));
+        std::vector<char> host(up);
+        size_t at = 0;
+        for (const Item &i : items) {
+            *i.dst = *mem + at;
+            if (i.src && i.bytes) memcpy(host.data() + at, i.src, i.bytes);
+            at += (i.bytes + 255) / 256 * 256;
+        }
+        if (up) {
+            HIP_CALL(hipMemcpyAsync(*mem, host.data(), up, hipMemcpyHostToDevice, s));
+            HIP_CALL(hipStreamSynchronize(s));
+        }
+        return EXIT_SUCCESS;
+    }
+};
+
+double diagonal(const double *lo, const double *hi) {
+    double s = 0;
+    for (int d = 0; d < 3; d++) s += (hi[d] - lo[d]) * (hi[d] - lo[d]);
+    return std::sqrt(s);
+}
+
+// the halo plan's tiles on the device (built when a kernel that walks them runs)
+int halo_plan(DeviceProblem &dp, hipStream_t s) {
+    if (dp.P > 0) return EXIT_SUCCESS;
+    Mesh m;
+    m.pnts.resize(3 * (size_t)dp.N);
+    for (size_t i = 0; i < m.pnts.size(); i++) m.pnts[i] = (float)dp.hpts[i];
+    m.elems.resize(dp.E);
+    for (int e = 0; e < dp.E; e++)
+        for (int j = 0; j < 3; j++) m.elems[e].nodes[j] = dp.helems[3 * e + j];
+    TilePlan plan;
+    build_tile_plan(m, choose_tiles(dp.M, dp.N, dp.E, 64 / dp.qg), plan);
+    Pack pk;
+    pk.add(&dp.tile_ptr, (const int *)plan.ptr.data(), plan.ptr.size());
+    pk.add(&dp.tile_entries, (const int *)plan.entries.data(), plan.entries.size());
+    HOST_CALL(pk.place(&dp.halo_mem, s));
+    dp.P = plan.P;
+    return EXIT_SUCCESS;
+}
+
+// The arrays an assembly in R writes besides the matrix, one allocation per
+// precision, grown when a plan of more tiles asks for it: the singular terms,
+// the tile partials of c and the BC sums (P tiles), the side columns.
+template <typename R>
+int asm_scratch(DeviceProblem &dp, int P, long nside, R **sing, R **cpart, R **bpart, R **side, hipStream_t s) {
+    const size_t pad = 256 / sizeof(R);
+    auto up = [&](size_t n) { return (n + pad - 1) / pad * pad; };
+    const size_t ns = up((size_t)dp.E * 48), nc = up((size_t)P * dp.Mp), nb = up((size_t)2 * P * dp.Mp);
+    const size_t n = ns + nc + nb + (size_t)2 * nside * dp.Mp;
+    char *&mem = sizeof(R) == 4 ? dp.scratch32 : dp.scratch64;
+    size_t &cap = sizeof(R) == 4 ? dp.cap32 : dp.cap64;
+    if (cap < n * sizeof(R)) {
+        sfree(mem, s);
+        cap = 0;
+        HOST_CALL(salloc(&mem, n * sizeof(R), s));
+        cap = n * sizeof(R);
+    }
+    *sing = (R *)mem;
+    *cpart = *sing + ns;
+    *bpart = *cpart + nc;
+    *side = *bpart + nb;
+    return EXIT_SUCCESS;
+}
+}  // namespace
 
 int device_problem_build(const Mesh &m, DeviceProblem &dp, hipStream_t s) {
     HOST_CALL(validate_mesh(m));
@@ -1747,130 +1838,81 @@ int device_problem_build(const Mesh &m, DeviceProblem &dp, hipStream_t s) {
     dp.ldA = ((long)dp.M + 63) / 64 * 64;
     dp.Mp = dp.ldA;
     std::vector<float4> p4(dp.M);
-    std::vector<double> p64(3 * (size_t)dp.M);
+    dp.hpts.resize(3 * (size_t)dp.M);
     for (int i = 0; i < dp.M; i++) {
         const float *src = i < dp.N ? &m.pnts[3 * i] : &m.chief[3 * (i - dp.N)];
         p4[i] = make_float4(src[0], src[1], src[2], 0.f);
-        for (int d = 0; d < 3; d++) p64[3 * i + d] = src[d];
+        for (int d = 0; d < 3; d++) {
+            dp.hpts[3 * i + d] = src[d];
+            dp.lo[d] = i ? std::min(dp.lo[d], (double)src[d]) : src[d];
+            dp.hi[d] = i ? std::max(dp.hi[d], (double)src[d]) : src[d];
+        }
     }
-    {
-        double lo[3], hi[3];
-        for (int d = 0; d < 3; d++) lo[d] = hi[d] = dp.M ? p64[d] : 0.0;
-        for (int i = 0; i < dp.M; i++)
-            for (int d = 0; d < 3; d++) {
-                lo[d] = std::min(lo[d], p64[3 * i + d]);
-                hi[d] = std::max(hi[d], p64[3 * i + d]);
-            }
-        dp.diam = std::sqrt((hi[0] - lo[0]) * (hi[0] - lo[0]) + (hi[1] - lo[1]) * (hi[1] - lo[1]) +
-                            (hi[2] - lo[2]) * (hi[2] - lo[2]));
-    }
-    std::vector<int> el(3 * (size_t)dp.E);
+    dp.diam = diagonal(dp.lo, dp.hi);
+    dp.helems.resize(3 * (size_t)dp.E);
     std::vector<float2> bc(3 * (size_t)dp.E);
-    for (int e = 0; e < dp.E; e++)
+    std::vector<char> used(dp.N, 0);
+    dp.impedance = dp.source = 0;
+    for (int e = 0; e < dp.E; e++) {
         for (int j = 0; j < 3; j++) {
-            el[3 * e + j] = m.elems[e].nodes[j];
+            dp.helems[3 * e + j] = m.elems[e].nodes[j];
+            used[m.elems[e].nodes[j]] = 1;
             bc[3 * e + j] = make_float2(m.elems[e].bc[j].x, m.elems[e].bc[j].y);
         }
-    TilePlan plan;
+        // (a NaN counts as set)
+        if (!(bc[3 * e].x == 0.f && bc[3 * e].y == 0.f)) dp.impedance = 1;
+        if (!(bc[3 * e + 2].x == 0.f && bc[3 * e + 2].y == 0.f)) dp.source = 1;
+    }
+    std::vector<int> isolated;  // nodes no element references
+    for (int i = 0; i < dp.N; i++)
+        if (!used[i]) isolated.push_back(i);
+    dp.n_isolated = (int)isolated.size();
     const int qg = choose_qg(dp.M, dp.E);
-    build_tile_plan(m, choose_tiles(dp.M, dp.N, dp.E, 64 / qg), plan);
-    dp.P = plan.P;
-    HOST_CALL(salloc(&dp.pts, dp.M, s));
-    HOST_CALL(salloc(&dp.pts64, 3 * (size_t)dp.M, s));
-    HOST_CALL(salloc(&dp.elems, 3 * (size_t)dp.E, s));
-    HOST_CALL(salloc(&dp.bc, 3 * (size_t)dp.E, s));
-    HOST_CALL(salloc(&dp.rec32, dp.E, s));
-    HOST_CALL(salloc(&dp.rec64, dp.E, s));
-    HOST_CALL(salloc(&dp.far32, dp.E, s));
-    HOST_CALL(salloc(&dp.sing32, (size_t)dp.E * 48, s));
-    HOST_CALL(salloc(&dp.sing64, (size_t)dp.E * 48, s));
-    HOST_CALL(salloc(&dp.tile_ptr, plan.ptr.size(), s));
-    HOST_CALL(salloc(&dp.tile_entries, plan.entries.size(), s));
-    dp.n_isolated = (int)plan.isolated.size();
-    HOST_CALL(salloc(&dp.isolated, std::max<size_t>(1, plan.isolated.size()), s));
-    HOST_CALL(salloc(&dp.cpart, (size_t)dp.P * dp.Mp, s));
-    HOST_CALL(salloc(&dp.bpart, (size_t)dp.P * dp.Mp, s));
-    HOST_CALL(salloc(&dp.cpart64, (size_t)dp.P * dp.Mp, s));
-    HOST_CALL(salloc(&dp.bpart64, (size_t)dp.P * dp.Mp, s));
-    HOST_CALL(salloc(&dp.bterm, (size_t)dp.M, s));
-    dp.hpts = p64;
-    dp.helems = el;
-    HIP_CALL(hipMemcpyAsync(dp.pts, p4.data(), p4.size() * sizeof(float4), hipMemcpyHostToDevice, s));
-    HIP_CALL(hipMemcpyAsync(dp.pts64, p64.data(), p64.size() * sizeof(double), hipMemcpyHostToDevice, s));
-    HIP_CALL(hipMemcpyAsync(dp.elems, el.data(), el.size() * sizeof(int), hipMemcpyHostToDevice, s));
-    HIP_CALL(hipMemcpyAsync(dp.bc, bc.data(), bc.size() * sizeof(float2), hipMemcpyHostToDevice, s));
-    HIP_CALL(hipMemcpyAsync(dp.tile_ptr, plan.ptr.data(), plan.ptr.size() * sizeof(int), hipMemcpyHostToDevice, s));
-    HIP_CALL(hipMemcpyAsync(dp.tile_entries, plan.entries.data(), plan.entries.size() * sizeof(int),
-                            hipMemcpyHostToDevice, s));
-    if (!plan.isolated.empty())
-        HIP_CALL(hipMemcpyAsync(dp.isolated, plan.isolated.data(), plan.isolated.size() * sizeof(int),
-                                hipMemcpyHostToDevice, s));
     dp.qg = qg;
     // element-once plan for the FP32 fast kernel: taken when the halo plan
     // integrates at least 5 % of the elements twice and the side columns stay
     // within ghost_slot_bound (device_problem_bytes counts that bound).  It
     // runs at twice the waves as well, so it pays below 10 %: the 40962-node
-    // ellipsoid (52 tiles, 7.9 % twice) assembles in 82.9 ms against 91.0 ms.
-    dp.use_ghost = 0;
+    // ellipsoid (52 tiles, 7.9 % twice) assembled in 82.9 ms against 91.0 ms
+    // (36 points everywhere).
     // Too many side columns for the bound: fewer tiles (two thirds each try).
     // A halo under 5 % is left as it is.
+    dp.use_ghost = 0;
     GhostPlan gp;
     int gP = choose_tiles(dp.M, dp.N, dp.E, 64, 2);
-    bool take = false;
     for (int tries = 0; qg == 1 && !getenv("BEM_NO_GHOST_PLAN") && tries < 8 && gP >= 4; tries++) {
         build_ghost_plan(m, gP, gp);
         if (gp.P != gP || gp.dup < kGhostMinDup || gp.nslots == 0) break;
         // (ghost_reduce puts the ghost nodes on grid.y: at most 65535)
         if (gp.nslots <= ghost_slot_bound(dp.N, gP) && gp.gnode.size() <= 65535) {
-            take = true;
+            dp.use_ghost = 1;
             break;
         }
         gP = gP * 2 / 3;
     }
-    {
-        if (take) {
-            dp.use_ghost = 1;
-            dp.gP = gP;
-            if (gP > dp.P) {
-                // the FP32 tile partials of c and the BC sums, one row per tile
-                sfree(dp.cpart, s);
-                sfree(dp.bpart, s);
-                HOST_CALL(salloc(&dp.cpart, (size_t)gP * dp.Mp, s));
-                HOST_CALL(salloc(&dp.bpart, (size_t)gP * dp.Mp, s));
-            }
-            dp.nslots = gp.nslots;
-            dp.ngnodes = (int)gp.gnode.size();
-            HOST_CALL(salloc(&dp.gtile_ptr, gp.ptr.size(), s));
-            HOST_CALL(salloc(&dp.gtile_entries, gp.entries.size(), s));
-            HOST_CALL(salloc(&dp.gtile_slots, gp.slots.size(), s));
-            HOST_CALL(salloc(&dp.gred_ptr, gp.gptr.size(), s));
-            HOST_CALL(salloc(&dp.gred_node, std::max<size_t>(1, gp.gnode.size()), s));
-            HOST_CALL(salloc(&dp.gred_own, std::max<size_t>(1, gp.gown.size()), s));
-            HOST_CALL(salloc(&dp.gred_slot, std::max<size_t>(1, gp.gslot.size()), s));
-            HOST_CALL(salloc(&dp.side, (size_t)dp.nslots * dp.Mp, s));
-            HIP_CALL(hipMemcpyAsync(dp.gtile_ptr, gp.ptr.data(), gp.ptr.size() * sizeof(int), hipMemcpyHostToDevice, s));
-            HIP_CALL(hipMemcpyAsync(dp.gtile_entries, gp.entries.data(), gp.entries.size() * sizeof(int),
-                                    hipMemcpyHostToDevice, s));
-            HIP_CALL(hipMemcpyAsync(dp.gtile_slots, gp.slots.data(), gp.slots.size() * sizeof(int),
-                                    hipMemcpyHostToDevice, s));
-            HIP_CALL(hipMemcpyAsync(dp.gred_ptr, gp.gptr.data(), gp.gptr.size() * sizeof(int), hipMemcpyHostToDevice, s));
-            if (!gp.gnode.empty()) {
-                HIP_CALL(hipMemcpyAsync(dp.gred_node, gp.gnode.data(), gp.gnode.size() * sizeof(int),
-                                        hipMemcpyHostToDevice, s));
-                HIP_CALL(hipMemcpyAsync(dp.gred_own, gp.gown.data(), gp.gown.size() * sizeof(int),
-                                        hipMemcpyHostToDevice, s));
-                HIP_CALL(hipMemcpyAsync(dp.gred_slot, gp.gslot.data(), gp.gslot.size() * sizeof(int),
-                                        hipMemcpyHostToDevice, s));
-            }
-            HIP_CALL(hipStreamSynchronize(s));  // gp goes out of scope
-        }
+    Pack pk;
+    pk.add(&dp.pts, (const float4 *)p4.data(), p4.size());
+    pk.add(&dp.pts64, (const double *)dp.hpts.data(), dp.hpts.size());
+    pk.add(&dp.elems, (const int *)dp.helems.data(), dp.helems.size());
+    pk.add(&dp.bc, (const float2 *)bc.data(), bc.size());
+    pk.add(&dp.isolated, (const int *)isolated.data(), isolated.size());
+    if (dp.use_ghost) {
+        dp.gP = gP;
+        dp.nslots = gp.nslots;
+        dp.ngnodes = (int)gp.gnode.size();
+        pk.add(&dp.gtile_ptr, (const int *)gp.ptr.data(), gp.ptr.size());
+        pk.add(&dp.gtile_entries, (const int *)gp.entries.data(), gp.entries.size());
+        pk.add(&dp.gtile_slots, (const int *)gp.slots.data(), gp.slots.size());
+        pk.add(&dp.gred_ptr, (const int *)gp.gptr.data(), gp.gptr.size());
+        pk.add(&dp.gred_node, (const int *)gp.gnode.data(), gp.gnode.size());
+        pk.add(&dp.gred_own, (const int *)gp.gown.data(), gp.gown.size());
+        pk.add(&dp.gred_slot, (const int *)gp.gslot.data(), gp.gslot.size());
     }
-    dp.impedance = dp.source = 0;
-    for (const auto &e : m.elems) {
-        // (a NaN counts as set)
-        if (!(e.bc[0].x == 0.f && e.bc[0].y == 0.f)) dp.impedance = 1;
-        if (!(e.bc[2].x == 0.f && e.bc[2].y == 0.f)) dp.source = 1;
-    }
+    pk.add(&dp.rec32, (const ElemRec<float> *)nullptr, dp.E);
+    pk.add(&dp.rec64, (const ElemRec<double> *)nullptr, dp.E);
+    pk.add(&dp.far32, (const FarRec *)nullptr, dp.E);
+    pk.add(&dp.bterm, (const double2 *)nullptr, dp.M);
+    HOST_CALL(pk.place(&dp.mem, s));
     const int bs = 256;
     prep_elems<float><<<(dp.E + bs - 1) / bs, bs, 0, s>>>(dp.pts64, dp.elems, dp.bc, dp.E, dp.rec32);
     HIP_CALL(hipGetLastError());
@@ -1878,50 +1920,67 @@ int device_problem_build(const Mesh &m, DeviceProblem &dp, hipStream_t s) {
     HIP_CALL(hipGetLastError());
     prep_far<<<(dp.E + bs - 1) / bs, bs, 0, s>>>(dp.pts64, dp.elems, dp.rec64, dp.E, dp.far32);
     HIP_CALL(hipGetLastError());
-    HIP_CALL(hipStreamSynchronize(s));  // host vectors above go out of scope
     dp.mesh_version = m.version;
     return EXIT_SUCCESS;
 }
 
-void device_problem_free(DeviceProblem &dp) {
-    sfree(dp.pts, dp.st);
-    sfree(dp.pts64, dp.st);
-    sfree(dp.elems, dp.st);
-    sfree(dp.bc, dp.st);
-    sfree(dp.rec32, dp.st);
-    sfree(dp.rec64, dp.st);
-    sfree(dp.far32, dp.st);
-    sfree(dp.sing32, dp.st);
-    sfree(dp.sing64, dp.st);
-    sfree(dp.tile_ptr, dp.st);
-    sfree(dp.tile_entries, dp.st);
-    sfree(dp.isolated, dp.st);
-    sfree(dp.gtile_ptr, dp.st);
-    sfree(dp.gtile_entries, dp.st);
-    sfree(dp.gtile_slots, dp.st);
-    sfree(dp.gred_ptr, dp.st);
-    sfree(dp.gred_node, dp.st);
-    sfree(dp.gred_own, dp.st);
-    sfree(dp.gred_slot, dp.st);
-    sfree(dp.side, dp.st);
-    dp.use_ghost = 0;
-    dp.nslots = dp.ngnodes = 0;
-    sfree(dp.cpart, dp.st);
-    sfree(dp.bpart, dp.st);
-    sfree(dp.cpart64, dp.st);
-    sfree(dp.bpart64, dp.st);
-    sfree(dp.bterm, dp.st);
-    sfree(dp.near_ptr, dp.st);
-    sfree(dp.near_row, dp.st);
-    sfree(dp.near_elem, dp.st);
-    sfree(dp.near_out, dp.st);
+// The problem of `base` with the P points `xs` in the place of its CHIEF
+// points, for rows N..N+P-1 (r0 = N) of an assembly: the element records and
+// the tiles are base's, which has to outlive dp; only the points, and the
+// arrays that the assembly writes, are dp's own.  Building it as a mesh of its
+// own took 2 ms of host time a call on 2562 nodes.
+int device_problem_rows(const DeviceProblem &base, const float *xs, int P, DeviceProblem &dp, hipStream_t s) {
+    device_problem_free(dp);
+    if (base.M == 0) BEM_FAIL("device problem not built");
+    dp = base;
+    dp.borrowed = true;
+    dp.mem = dp.halo_mem = dp.scratch32 = dp.scratch64 = nullptr;
+    dp.cap32 = dp.cap64 = 0;
+    dp.pts = nullptr;
+    dp.pts64 = nullptr;
+    dp.bterm = nullptr;
+    dp.near_ptr = dp.near_row = dp.near_elem = nullptr;
+    dp.near_out = nullptr;
     dp.near_factor = 0;
-    dp.near_levels = 0;
-    dp.near_npairs = 0;
+    dp.near_levels = dp.near_npairs = 0;
     dp.hnear_ptr.clear();
-    dp.hpts.clear();
-    dp.helems.clear();
-    dp.N = dp.C = dp.M = dp.E = dp.P = 0;
+    dp.st = s;
+    dp.C = P;
+    dp.M = dp.N + P;
+    dp.ldA = ((long)dp.M + 63) / 64 * 64;
+    dp.Mp = ((long)P + 63) / 64 * 64;
+    dp.hpts.resize(3 * (size_t)dp.N);
+    dp.hpts.insert(dp.hpts.end(), xs, xs + 3 * (size_t)P);
+    std::vector<float4> p4(dp.M);
+    for (int i = 0; i < dp.M; i++) {
+        const double *x = &dp.hpts[3 * (size_t)i];
+        p4[i] = make_float4((float)x[0], (float)x[1], (float)x[2], 0.f);
+        if (i >= dp.N)
+            for (int d = 0; d < 3; d++) {
+                dp.lo[d] = std::min(dp.lo[d], x[d]);
+                dp.hi[d] = std::max(dp.hi[d], x[d]);
+            }
+    }
+    dp.diam = diagonal(dp.lo, dp.hi);
+    Pack pk;
+    pk.add(&dp.pts, (const float4 *)p4.data(), p4.size());
+    pk.add(&dp.pts64, (const double *)dp.hpts.data(), dp.hpts.size());
+    pk.add(&dp.bterm, (const double2 *)nullptr, (size_t)P);
+    return pk.place(&dp.mem, s);
+}
+
+void device_problem_free(DeviceProblem &dp) {
+    hipStream_t st = dp.st;
+    sfree(dp.mem, st);
+    sfree(dp.halo_mem, st);
+    sfree(dp.scratch32, st);
+    sfree(dp.scratch64, st);
+    sfree(dp.near_ptr, st);
+    sfree(dp.near_row, st);
+    sfree(dp.near_elem, st);
+    sfree(dp.near_out, st);
+    dp = DeviceProblem{};
+    dp.st = st;
 }
 
 static void sing_tab(SingTab &t) {
@@ -1959,7 +2018,12 @@ static int assemble_impl(DeviceProblem &dp, R k, C2 *A, long ldA, int r0, double
     quad_tables(qt);
     SingTab st;
     sing_tab(st);
-    R *sing = sizeof(R) == 4 ? (R *)dp.sing32 : (R *)dp.sing64;
+    // the plan this call walks, and the arrays it writes
+    const bool ghost = sizeof(R) == 4 && dp.use_ghost && !getenv("BEM_ASM_HALO") && !getenv("BEM_GENERIC_TILE");
+    if (!ghost) HOST_CALL(halo_plan(dp, s));
+    const int P = ghost ? dp.gP : dp.P;
+    R *sing = nullptr, *cpart = nullptr, *bpart = nullptr, *side = nullptr;
+    HOST_CALL(asm_scratch<R>(dp, P, ghost ? dp.nslots : 0, &sing, &cpart, &bpart, &side, s));
     {
         TimedRegion tr;
         timing_begin(tr, "sing_elems", s);
@@ -1976,8 +2040,8 @@ static int assemble_impl(DeviceProblem &dp, R k, C2 *A, long ldA, int r0, double
     a.tile_ptr = dp.tile_ptr;
     a.tile_entries = dp.tile_entries;
     a.A = A;
-    a.cpart = sizeof(R) == 4 ? (R *)dp.cpart : (R *)dp.cpart64;
-    a.bpart = sizeof(R) == 4 ? (C2 *)dp.bpart : (C2 *)dp.bpart64;
+    a.cpart = cpart;
+    a.bpart = (C2 *)bpart;
     a.ldA = ldA;
     a.Mp = dp.Mp;
     a.M = dp.M;
@@ -1986,7 +2050,7 @@ static int assemble_impl(DeviceProblem &dp, R k, C2 *A, long ldA, int r0, double
     const int rpw = 64 / dp.qg;
     const int nrb = (dp.M - r0 + rpw - 1) / rpw;
     a.nrbg = (nrb + 3) / 4;
-    a.nwg = a.nrbg * dp.P;
+    a.nwg = a.nrbg * P;
     a.k = k;
     a.kf = (R)(kd / (2.0 * kPi));
     a.kf64 = kd / (2.0 * kPi);
@@ -2008,12 +2072,10 @@ static int assemble_impl(DeviceProblem &dp, R k, C2 *A, long ldA, int r0, double
     a.tile_slots = nullptr;
     a.side = nullptr;
     const int nrows = dp.M - r0;
-    bool ghost = false;
     {
         TimedRegion tr;
         timing_begin(tr, sizeof(R) == 4 ? "asm_tile_f32" : "asm_tile_f64", s);
         dim3 grid(a.nwg), block(256);
-        ghost = sizeof(R) == 4 && dp.use_ghost && !getenv("BEM_ASM_HALO") && !getenv("BEM_GENERIC_TILE");
         if (dp.qg == 4 && !ghost) {
             if (dp.impedance) asm_tile<R, 4, true><<<grid, block, 0, s>>>(a);
             else asm_tile<R, 4, false><<<grid, block, 0, s>>>(a);
@@ -2031,7 +2093,7 @@ static int assemble_impl(DeviceProblem &dp, R k, C2 *A, long ldA, int r0, double
                 af.tile_ptr = dp.gtile_ptr;
                 af.tile_entries = dp.gtile_entries;
                 af.tile_slots = dp.gtile_slots;
-                af.side = dp.side;
+                af.side = (float2 *)side;
             }
 #define BEM_FAST(IMP_, SRC_)                                                                     \
     do {                                                                                         \
@@ -2056,7 +2118,7 @@ static int assemble_impl(DeviceProblem &dp, R k, C2 *A, long ldA, int r0, double
         TimedRegion tr;
         timing_begin(tr, "ghost_reduce", s);
         dim3 grid((nrows + 511) / 512, dp.ngnodes);
-        ghost_reduce<<<grid, 256, 0, s>>>((float2 *)A, ldA, nrows, dp.side, dp.Mp, dp.gred_ptr, dp.gred_node,
+        ghost_reduce<<<grid, 256, 0, s>>>((float2 *)A, ldA, nrows, (const float2 *)side, dp.Mp, dp.gred_ptr, dp.gred_node,
                                           dp.gred_own, dp.gred_slot);
         HIP_CALL(hipGetLastError());
         timing_end(tr, s);
@@ -2069,8 +2131,7 @@ static int assemble_impl(DeviceProblem &dp, R k, C2 *A, long ldA, int r0, double
     {
         TimedRegion tr;
         timing_begin(tr, "asm_finalize", s);
-        asm_finalize<R, C2><<<(nrows + 255) / 256, 256, 0, s>>>(A, ldA, dp.M, dp.N, ghost ? dp.gP : dp.P, dp.Mp, r0,
-                                                             a.cpart,
+        asm_finalize<R, C2><<<(nrows + 255) / 256, 256, 0, s>>>(A, ldA, dp.M, dp.N, P, dp.Mp, r0, a.cpart,
                                                              a.bpart, bterm);
         HIP_CALL(hipGetLastError());
         timing_end(tr, s);

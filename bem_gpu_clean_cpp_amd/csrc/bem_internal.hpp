@@ -160,20 +160,27 @@ struct FarRec;
 struct DeviceProblem {
     int N = 0, C = 0, M = 0, E = 0;
     long ldA = 0;                 // leading dimension of the device A (M rounded up to 64)
+    long Mp = 0;                  // rows of a tile partial or side column
+    bool borrowed = false;        // the element and plan arrays are another problem's (device_problem_rows)
+    // one allocation each: the points, elements, records and element-once plan;
+    // the halo plan; what an assembly in FP32 / FP64 writes besides the matrix
+    char *mem = nullptr, *halo_mem = nullptr, *scratch32 = nullptr, *scratch64 = nullptr;
+    size_t cap32 = 0, cap64 = 0;  // bytes of scratch32 / scratch64
     float4 *pts = nullptr;        // M points (nodes then CHIEF), FP32
     double *pts64 = nullptr;      // 3 * M, FP64 copy
     int *elems = nullptr;         // 3 * E node indices
     float2 *bc = nullptr;         // 3 * E (ca, cb, cc)
     ElemRec<float> *rec32 = nullptr;
     ElemRec<double> *rec64 = nullptr;
-    FarRec *far32 = nullptr;  // far-rule element records (far_rules.hpp)
-    float *sing32 = nullptr;      // E * 3 * 16: singular contributions
-    double *sing64 = nullptr;
-    int P = 0;                    // column tiles
+    FarRec *far32 = nullptr;      // far-rule element records (far_rules.hpp)
+    double2 *bterm = nullptr;     // M: sum_e (cc/cb) sum_j g_j(x_i)
     int qg = 1;                   // lanes per row in the quadrature kernel
     int impedance = 0;            // some element has ca != 0
     int source = 0;               // some element has cc != 0
-    double diam = 0;              // bounding-box diagonal of the M points: bounds every |x - y|
+    double lo[3] = {0, 0, 0}, hi[3] = {0, 0, 0};  // bounding box of the M points
+    double diam = 0;              // its diagonal: bounds every |x - y|
+    // halo plan (TilePlan): P column tiles, 0 until a kernel that walks them runs
+    int P = 0;
     int *tile_ptr = nullptr;
     int *tile_entries = nullptr;
     int n_isolated = 0;
@@ -184,18 +191,13 @@ struct DeviceProblem {
     int *gtile_ptr = nullptr, *gtile_entries = nullptr, *gtile_slots = nullptr;
     int nslots = 0, ngnodes = 0;
     int *gred_ptr = nullptr, *gred_node = nullptr, *gred_own = nullptr, *gred_slot = nullptr;
-    float2 *side = nullptr;       // nslots * Mp side columns
-    float *cpart = nullptr;       // P * Mp  c partial sums
-    float2 *bpart = nullptr;      // P * Mp  boundary-condition partial sums
-    double *cpart64 = nullptr;
-    double2 *bpart64 = nullptr;
-    double2 *bterm = nullptr;     // M: sum_e (cc/cb) sum_j g_j(x_i)
-    long Mp = 0;
-    // near-singular FP64 correction (bem_set_near_field): host copies of the
-    // points and elements for the pair search, the (row, element) pairs in
-    // row order, and each pair's correction (13 doubles: g, h complex x 3, c)
+    // host copies of the points and elements, for the near-singular pair
+    // search and the halo plan
     std::vector<double> hpts;     // 3 * M
     std::vector<int> helems;      // 3 * E
+    // near-singular FP64 correction (bem_set_near_field): the (row, element)
+    // pairs in row order, and each pair's correction (13 doubles: g, h complex
+    // x 3, c)
     double near_factor = 0;       // factor the pairs were found with (0: none)
     int near_levels = 0;
     int near_npairs = 0;
@@ -207,6 +209,8 @@ struct DeviceProblem {
     hipStream_t st = nullptr;     // buffers are stream-ordered on this stream
 };
 int device_problem_build(const Mesh &m, DeviceProblem &dp, hipStream_t s);
+// rows for the P points xs over base's elements and tiles (base outlives dp)
+int device_problem_rows(const DeviceProblem &base, const float *xs, int P, DeviceProblem &dp, hipStream_t s);
 void device_problem_free(DeviceProblem &dp);
 size_t device_problem_bytes(int M, int N, int E);
 // assembly launch-shape tuning (assembly.hip)

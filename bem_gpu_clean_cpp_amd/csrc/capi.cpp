@@ -763,11 +763,8 @@ int bem_solver_field_matrix(bem_solver *sv, const bem_cart_coord *pts, int P) {
     if (!sv->prec) BEM_FAIL("solver not assembled");
     std::lock_guard<std::mutex> lk(sv->mu);
     hipStream_t s = sv->stream;
-    sv->fmesh = sv->mesh;
-    sv->fmesh.chief.assign((const float *)pts, (const float *)pts + 3 * (size_t)P);
-    sv->fmesh.version++;
     sv->fP = 0;
-    HOST_CALL(device_problem_build(sv->fmesh, sv->fdp, s));
+    HOST_CALL(device_problem_rows(sv->dp, (const float *)pts, P, sv->fdp, s));
     const long ldF = ((long)P + 63) / 64 * 64;
     const size_t need = (size_t)ldF * sv->dp.N;
     if (sv->f_cap < need) {

@@ -34,8 +34,7 @@ struct bem_solver {
     mutable bool asm_pending = false;
     hipEvent_t se0 = nullptr, se1 = nullptr;  // around the last solve
     bem::GmresCache *gcache = nullptr;         // GMRES workspace of the last solve's shape
-    // exterior field as a matrix: the mesh with the field points as extra rows
-    bem::Mesh fmesh;
+    // exterior field as a matrix: the field points as extra rows of the mesh
     bem::DeviceProblem fdp;
     float2 *F = nullptr;  // P x N radiation operator, ld ldF
     double2 *fbterm = nullptr;
