@@ -744,7 +744,7 @@ __global__ __launch_bounds__(256) void asm_tile_fast(AsmArgs<float> a) {
     }
     if (active) {
         a.cpart[(size_t)tile * a.Mp + (row - a.r0)] = c_acc;
-        a.bpart[(size_t)tile * a.Mp + (row - a.r0)] = make_float2(br_acc, bi_acc);
+        if (IMP || SRC) a.bpart[(size_t)tile * a.Mp + (row - a.r0)] = make_float2(br_acc, bi_acc);
     }
 }
 
@@ -793,37 +793,44 @@ __global__ void ghost_reduce(float2 *A, long ldA, int nrows, const float2 *__res
     }
 }
 
-// Per row: fixed-order sum of the tile partials in FP64.
+// Per row: sum of the tile partials in FP64 in a fixed order (16 runs of
+// consecutive tiles, one per wave of the workgroup, then the runs).  One wave
+// per 64 rows walked all tiles in turn before: 45 us for 4002 rows in 500
+// tiles, bound by the chain of loads.
 // Rows r0..M-1 (local index i = row - r0 in A, the partials and bterm).
+// src == 0: no element has a boundary term, its partials are not read.
+constexpr int kFinRuns = 16;
 template <typename R, typename C2>
-__global__ void asm_finalize(C2 *A, long ldA, int M, int N, int P, long Mp, int r0, const R *__restrict__ cpart,
-                             const C2 *__restrict__ bpart, double2 *__restrict__ bterm) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+__global__ __launch_bounds__(64 * kFinRuns) void asm_finalize(C2 *A, long ldA, int M, int N, int P, long Mp, int r0,
+                                                              const R *__restrict__ cpart,
+                                                              const C2 *__restrict__ bpart,
+                                                              double2 *__restrict__ bterm, int src) {
+    __shared__ double red[3][kFinRuns][64];
+    const int lane = threadIdx.x & 63, run = threadIdx.x >> 6;
+    const int i = blockIdx.x * 64 + lane;
     const int row = r0 + i;
-    if (row >= M) return;
     double cs = 0, br = 0, bi = 0;
-    // 8 tiles' partials in flight per step, added in tile order
-    int t = 0;
-    for (; t + 8 <= P; t += 8) {
-        R c[8];
-        C2 b[8];
-#pragma unroll
-        for (int u = 0; u < 8; u++) {
-            c[u] = cpart[(size_t)(t + u) * Mp + i];
-            b[u] = bpart[(size_t)(t + u) * Mp + i];
-        }
-#pragma unroll
-        for (int u = 0; u < 8; u++) {
-            cs += (double)c[u];
-            br += (double)b[u].x;
-            bi += (double)b[u].y;
+    if (row < M) {
+        const int per = (P + kFinRuns - 1) / kFinRuns;
+        const int t1 = min(P, (run + 1) * per);
+        for (int t = run * per; t < t1; t++) {
+            cs += (double)cpart[(size_t)t * Mp + i];
+            if (src) {
+                const C2 b = bpart[(size_t)t * Mp + i];
+                br += (double)b.x;
+                bi += (double)b.y;
+            }
         }
     }
-    for (; t < P; t++) {
-        cs += (double)cpart[(size_t)t * Mp + i];
-        const C2 b = bpart[(size_t)t * Mp + i];
-        br += (double)b.x;
-        bi += (double)b.y;
+    red[0][run][lane] = cs;
+    red[1][run][lane] = br;
+    red[2][run][lane] = bi;
+    __syncthreads();
+    if (run > 0 || row >= M) return;
+    for (int q = 1; q < kFinRuns; q++) {
+        cs += red[0][q][lane];
+        br += red[1][q][lane];
+        bi += red[2][q][lane];
     }
     if (row < N) {
         C2 *d = A + (size_t)row * ldA + i;
@@ -1584,13 +1591,17 @@ constexpr double kGhostMinDup = 1.05;
 
 // side columns the element-once plan may use: about the nodes on the tile
 // boundaries (4 sqrt(N P) + P; 4190 for N = 10242 in 102 tiles, which need
-// 3110), and never more than N / 2
+// 3110), and never more than 2 N.  (A bound of N / 2 kept meshes of a few
+// thousand nodes on fewer, longer tiles: 2562 nodes took 0.41 ms in 53 tiles,
+// 0.27 ms in 320; 642 nodes 0.23 ms in 35, 0.064 ms in 160.)
 static long ghost_slot_bound(int N, int P) {
-    return std::min((long)N / 2, (long)(4.0 * std::sqrt((double)N * P)) + P);
+    return std::min(2L * N, (long)(4.0 * std::sqrt((double)N * P)) + P);
 }
 
 // wave_factor: the element-once plan has no halo to pay for more tiles, and
-// runs at twice the waves (10242 nodes: 2.16 ms with 102 tiles, 1.90 with 204)
+// runs at twice the waves (10242 nodes: 2.16 ms with 102 tiles, 1.90 with
+// 204).  A wave walks its tile's list alone, so on a small mesh the longest
+// list is the assembly's time, and tiles go down to a few nodes.
 static int choose_tiles(int M, int N, int E, int rows_per_wave, int wave_factor = 1) {
     const char *env = getenv("BEM_TILES");
     if (env && atoi(env) > 0) return std::min(atoi(env), N);
@@ -1598,19 +1609,31 @@ static int choose_tiles(int M, int N, int E, int rows_per_wave, int wave_factor 
     const int target_waves = (tuned_shape(M, E, t) ? t.waves : kDefaultWaves) * wave_factor;
     const int nrb = (M + rows_per_wave - 1) / rows_per_wave;
     int P = (target_waves + nrb - 1) / nrb;
-    P = std::max(1, std::min(P, std::max(1, N / 8)));
+    // nodes per tile of the element-once plan: 4 below 1000 nodes, 8 up to 320
+    // tiles, then 16 (4002 nodes: 0.536 ms in 320 tiles, 0.556 in 640, with
+    // twice the side columns)
+    const int most = wave_factor == 1 ? N / 8 : N < 1000 ? N / 4 : std::min(N / 8, std::max(320, N / 16));
+    P = std::max(1, std::min(P, std::max(1, most)));
     return P;
 }
 
-static int choose_qg(int M, int E) {
+// lanes per row asked for by the environment or the tuner; 0: none
+static int asked_qg(int M, int E) {
     const char *env = getenv("BEM_QG");
     if (env) {
         int q = atoi(env);
         if (q == 1 || q == 4) return q;
     }
     TileShape t;
-    if (tuned_shape(M, E, t)) return t.qg;
-    return ((long)M * E < 4000000L) ? 4 : 1;
+    return tuned_shape(M, E, t) ? t.qg : 0;
+}
+
+// lanes per row of the halo plan's kernels.  (FP32 runs the element-once plan
+// with one lane a row at every size it can be built for: 642 nodes 0.064 ms
+// against 0.122 ms with four lanes, 162 nodes 0.05 against 0.066 ms.)
+static int choose_qg(int M, int E) {
+    const int q = asked_qg(M, E);
+    return q ? q : ((long)M * E < 4000000L) ? 4 : 1;
 }
 
 // Times the FP32 (or FP64) assembly of mesh m at wavenumber k for each
@@ -1622,7 +1645,7 @@ int autotune_assembly(const Mesh &m, double k, int precision, int *best_qg, int 
     std::vector<TileShape> cand;
     for (int qg : {1, 4})
         for (int w : {4096, 8192, 16384, 32768}) cand.push_back(TileShape{qg, w});
-    TileShape def{((long)M * E < 4000000L) ? 4 : 1, kDefaultWaves};
+    TileShape def{(precision == BEM_PREC_FP64 && (long)M * E < 4000000L) ? 4 : 1, kDefaultWaves};
     double bms = 1e300, dms = -1;
     TileShape best = def;
     hipEvent_t e0, e1;
@@ -1725,7 +1748,7 @@ size_t device_problem_bytes(int M, int N, int E) {
     b += sizeof(int) * (P + 1 + 3 * (size_t)E + N);                                  // tile CSR, isolated
     b += 40 * 256;                                                                   // the packed arrays' alignment
     b += (sizeof(float) + sizeof(float2) + sizeof(double) + sizeof(double2)) * P * Mp;  // tile partials
-    if (qg == 1) {
+    if (asked_qg(M, E) != 4) {
         // element-once plan: its side columns and index arrays
         const int gP = choose_tiles(M, N, E, 64, 2);
         const size_t gs = (size_t)ghost_slot_bound(N, gP);
@@ -1880,7 +1903,7 @@ int device_problem_build(const Mesh &m, DeviceProblem &dp, hipStream_t s) {
     dp.use_ghost = 0;
     GhostPlan gp;
     int gP = choose_tiles(dp.M, dp.N, dp.E, 64, 2);
-    for (int tries = 0; qg == 1 && !getenv("BEM_NO_GHOST_PLAN") && tries < 8 && gP >= 4; tries++) {
+    for (int tries = 0; asked_qg(dp.M, dp.E) != 4 && !getenv("BEM_NO_GHOST_PLAN") && tries < 8 && gP >= 4; tries++) {
         build_ghost_plan(m, gP, gp);
         if (gp.P != gP || gp.dup < kGhostMinDup || gp.nslots == 0) break;
         // (ghost_reduce puts the ghost nodes on grid.y: at most 65535)
@@ -2131,8 +2154,8 @@ static int assemble_impl(DeviceProblem &dp, R k, C2 *A, long ldA, int r0, double
     {
         TimedRegion tr;
         timing_begin(tr, "asm_finalize", s);
-        asm_finalize<R, C2><<<(nrows + 255) / 256, 256, 0, s>>>(A, ldA, dp.M, dp.N, P, dp.Mp, r0, a.cpart,
-                                                             a.bpart, bterm);
+        asm_finalize<R, C2><<<(nrows + 63) / 64, 64 * kFinRuns, 0, s>>>(
+            A, ldA, dp.M, dp.N, P, dp.Mp, r0, a.cpart, a.bpart, bterm, dp.impedance || dp.source);
         HIP_CALL(hipGetLastError());
         timing_end(tr, s);
     }
