@@ -625,9 +625,8 @@ int cgls_device(const float2 *A32, const double2 *A64, long lda, int M, int N, c
             if (R == 1) HOST_CALL(gemv_n_f32(A32, lda, M, N, w.p32, 0, w.q32, 0, 1, w.gws, s));
             else HOST_CALL(gemm_n_f32(A32, lda, M, N, w.p32, ld, w.q32, ld, R, w.gws, s, true));
         } else {
-            for (int q = 0; q < R; q++)
-                HOST_CALL(gemv_n_f64(A64, lda, M, N, w.p + (size_t)q * ld, 0, w.q64 + (size_t)q * ld, 0, 1, w.gws,
-                                     s));
+            if (R == 1) HOST_CALL(gemv_n_f64(A64, lda, M, N, w.p, 0, w.q64, 0, 1, w.gws, s));
+            else HOST_CALL(mres_f64(A64, lda, M, N, w.p, ld, nullptr, 0, w.q64, ld, R, w.gws, s));
         }
         return EXIT_SUCCESS;
     };
@@ -638,8 +637,8 @@ int cgls_device(const float2 *A32, const double2 *A64, long lda, int M, int N, c
             else if (w.AH) HOST_CALL(gemm_hc_f32(w.AH, M, N, w.q32, ld, w.w32, ld, R, w.gws, s));
             else HOST_CALL(gemm_h_f32(A32, lda, M, N, w.q32, ld, w.w32, ld, R, w.gws, s, true));
         } else {
-            for (int q = 0; q < R; q++)
-                HOST_CALL(gemv_h_f64(A64, lda, M, N, w.q64 + (size_t)q * ld, 0, w.w64 + (size_t)q * ld, 0, 1, s));
+            if (R == 1) HOST_CALL(gemv_h_f64(A64, lda, M, N, w.q64, 0, w.w64, 0, 1, s));
+            else HOST_CALL(mh_f64(A64, lda, M, N, w.q64, ld, w.w64, ld, R, s));
         }
         return EXIT_SUCCESS;
     };
@@ -760,11 +759,8 @@ int cgls_device(const float2 *A32, const double2 *A64, long lda, int M, int N, c
             if (w.AH) HOST_CALL(gemm_hc_f32z(w.AH, M, N, w.q32, ld, w.bW, ld, Rb, w.gws, s));
             else HOST_CALL(gemm_h_f32z(A32, lda, M, N, w.q32, ld, w.bW, ld, Rb, w.gws, s));
         } else {
-            for (int c = 0; c < Rb; c++) {
-                HOST_CALL(gemv_n_f64(A64, lda, M, N, w.bP + (size_t)c * ld, 0, w.q64 + (size_t)c * ld, 0, 1, w.gws,
-                                     s));
-                HOST_CALL(gemv_h_f64(A64, lda, M, N, w.q64 + (size_t)c * ld, 0, w.bW + (size_t)c * ld, 0, 1, s));
-            }
+            HOST_CALL(mres_f64(A64, lda, M, N, w.bP, ld, nullptr, 0, w.q64, ld, Rb, w.gws, s));
+            HOST_CALL(mh_f64(A64, lda, M, N, w.q64, ld, w.bW, ld, Rb, s));
         }
         return EXIT_SUCCESS;
     };

@@ -1618,54 +1618,54 @@ int rank_update_f32(const float2 *V, long ldv, int M, const float2 *W, int ldw, 
     return EXIT_SUCCESS;
 }
 
-// ------------------------------------------------- FP64-matrix residuals ---
-// Residuals and adjoint products for an FP64 matrix (the all-FP64 path) and
-// several right-hand sides: VALU FP64 kernels, 8 right-hand sides per pass.
-template <typename TA>
-struct A2T;
-template <>
-struct A2T<float> {
-    using c2 = float2;
-};
-template <>
-struct A2T<double> {
-    using c2 = double2;
-};
-
+// -------------------------------------------------- FP64-matrix products ---
+// Products, residuals and adjoint products of an FP64 matrix (the all-FP64
+// path) with several right-hand sides.  Bound by the read of A: 16 bytes an
+// element against 4 FMAs per right-hand side, so one pass over A serves 8
+// right-hand sides on the vector ALU (one GEMV each, as the solvers ran them
+// before, read A once per right-hand side: 5778 x 5762, 4 right-hand sides:
+// A X 4 x 106 us -> 96 us, A^H T 4 x 105 us -> 103 us).
 constexpr int kRG = 8;
 
-// part[(chunk * R + r) * ldp + i] = sum_{j in chunk} A[i, j] X[j, r] for r in [rg0, rg0 + 8)
-template <typename TA>
-__global__ __launch_bounds__(256) void mres_part(const typename A2T<TA>::c2 *__restrict__ A, long lda, int M, int N,
+// part[(chunk * R + r) * ldp + i] = sum_{j in chunk} A[i, j] X[j, r] for r in [rg0, rg0 + RG)
+// (r past the last: the last again, not stored)
+template <int RG>
+__global__ __launch_bounds__(256) void mres_part(const double2 *__restrict__ A, long lda, int M, int N,
                                                  const double2 *__restrict__ X, long ldx, int R, int rg0, int kc,
                                                  double2 *__restrict__ part, long ldp) {
     const int i = blockIdx.x * 256 + threadIdx.x;
     const int chunk = blockIdx.y;
     const int j0 = chunk * kc, j1 = min(N, j0 + kc);
-    const int nr = min(kRG, R - rg0);
-    double ar[kRG], ai[kRG];
+    if (i >= M) return;
+    const double2 *x[RG];
+    double ar[RG], ai[RG];
 #pragma unroll
-    for (int q = 0; q < kRG; q++) {
+    for (int q = 0; q < RG; q++) {
+        x[q] = X + (size_t)min(rg0 + q, R - 1) * ldx;
         ar[q] = 0;
         ai[q] = 0;
     }
-    if (i < M) {
-        for (int j = j0; j < j1; j++) {
-            const typename A2T<TA>::c2 a = A[(size_t)j * lda + i];
-            const double xr0 = (double)a.x, xi0 = (double)a.y;
+    auto add = [&](const double2 &a, int j) {
 #pragma unroll
-            for (int q = 0; q < kRG; q++) {
-                if (q < nr) {
-                    const double2 x = X[(size_t)(rg0 + q) * ldx + j];
-                    ar[q] = fma(xr0, x.x, fma(-xi0, x.y, ar[q]));
-                    ai[q] = fma(xr0, x.y, fma(xi0, x.x, ai[q]));
-                }
-            }
+        for (int q = 0; q < RG; q++) {
+            const double2 v = x[q][j];
+            ar[q] = fma(a.x, v.x, fma(-a.y, v.y, ar[q]));
+            ai[q] = fma(a.x, v.y, fma(a.y, v.x, ai[q]));
         }
+    };
+    const double2 *col = A + i;
+    int j = j0;
+    for (; j + 4 <= j1; j += 4) {
+        double2 a[4];
 #pragma unroll
-        for (int q = 0; q < kRG; q++)
-            if (q < nr) part[((size_t)chunk * R + rg0 + q) * ldp + i] = make_double2(ar[q], ai[q]);
+        for (int u = 0; u < 4; u++) a[u] = col[(size_t)(j + u) * lda];
+#pragma unroll
+        for (int u = 0; u < 4; u++) add(a[u], j + u);
     }
+    for (; j < j1; j++) add(col[(size_t)j * lda], j);
+#pragma unroll
+    for (int q = 0; q < RG; q++)
+        if (rg0 + q < R) part[((size_t)chunk * R + rg0 + q) * ldp + i] = make_double2(ar[q], ai[q]);
 }
 
 // out[r][i] = b[r][i] - sum_chunks part (b == nullptr: out = +sum)
@@ -1701,51 +1701,98 @@ __global__ __launch_bounds__(256) void mres_reduce(const double2 *__restrict__ p
     }
 }
 
-// Z[j][r] = sum_i conj(A[i, j]) T[i][r], one wave per column, 8 right-hand sides per pass
-template <typename TA>
-__global__ __launch_bounds__(256) void mh_kernel(const typename A2T<TA>::c2 *__restrict__ A, long lda, int M, int N,
-                                                 const double2 *__restrict__ T, long ldt, int R, int rg0,
-                                                 double2 *__restrict__ Z, long ldz) {
-    const int lane = threadIdx.x & 63;
-    const int j = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (j >= N) return;
-    const int nr = min(kRG, R - rg0);
-    double zr[kRG], zi[kRG];
+// Sums x[v] (V a power of two, at most 64) over the 64 lanes: afterwards lane
+// l holds the total of x[v(l)] in x[0], v(l) = the V-value index whose bits are
+// the high bits of l (bit H of the lane picks the upper half at each step).
+template <int V>
+__device__ __forceinline__ void reduce_scatter(double (&x)[V], int lane) {
+    int mask = 32;
 #pragma unroll
-    for (int q = 0; q < kRG; q++) {
-        zr[q] = 0;
-        zi[q] = 0;
+    for (int h = V / 2; h >= 1; h >>= 1) {
+        const bool up = (lane & mask) != 0;
+#pragma unroll
+        for (int i = 0; i < h; i++) {
+            // (selected as values: a select of the two addresses puts x in
+            // scratch memory)
+            const double lo = x[i], hi = x[i + h];
+            const double send = up ? lo : hi, keep = up ? hi : lo;
+            x[i] = keep + __shfl_xor(send, mask, 64);
+        }
+        mask >>= 1;
     }
-    const typename A2T<TA>::c2 *col = A + (size_t)j * lda;
-    for (int i = lane; i < M; i += 64) {
-        const double ar = (double)col[i].x, ai = (double)col[i].y;
+    for (; mask >= 1; mask >>= 1) x[0] += __shfl_xor(x[0], mask, 64);
+}
+
+// Z[j][r] = sum_i conj(A[i, j]) T[i][r] for the NC columns j of a workgroup of
+// NT threads and r in [rg0, rg0 + RG).  The waves split the rows, U steps of
+// loads in flight; the columns share each load of T (with one column a wave,
+// T comes from the L2 cache RG times as often as A from memory: 170 us for 4
+// right-hand sides on 5778 x 5762 against 103 us).
+template <int RG, int NC, int U, int NT>
+__global__ __launch_bounds__(NT) void mh_kernel(const double2 *__restrict__ A, long lda, int M, int N,
+                                                const double2 *__restrict__ T, long ldt, int R, int rg0,
+                                                double2 *__restrict__ Z, long ldz) {
+    constexpr int V = 2 * RG * NC;
+    __shared__ double red[NT / 64][V];
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    const int jb = blockIdx.x * NC;
+    const double2 *col[NC], *t[RG];
+    double z[V];
 #pragma unroll
-        for (int q = 0; q < kRG; q++) {
-            if (q < nr) {
-                const double2 t = T[(size_t)(rg0 + q) * ldt + i];
-                zr[q] = fma(ar, t.x, fma(ai, t.y, zr[q]));
-                zi[q] = fma(ar, t.y, fma(-ai, t.x, zi[q]));
+    for (int c = 0; c < NC; c++) col[c] = A + (size_t)min(jb + c, N - 1) * lda;
+#pragma unroll
+    for (int q = 0; q < RG; q++) t[q] = T + (size_t)min(rg0 + q, R - 1) * ldt;
+#pragma unroll
+    for (int v = 0; v < V; v++) z[v] = 0;
+    auto step = [&](const double2 (&a)[NC], const double2 (&tv)[RG]) {
+#pragma unroll
+        for (int c = 0; c < NC; c++)
+#pragma unroll
+            for (int q = 0; q < RG; q++) {
+                double &zr = z[2 * (c * RG + q)], &zi = z[2 * (c * RG + q) + 1];
+                zr = fma(a[c].x, tv[q].x, fma(a[c].y, tv[q].y, zr));
+                zi = fma(a[c].x, tv[q].y, fma(-a[c].y, tv[q].x, zi));
             }
+    };
+    int i = threadIdx.x;
+    for (; i + (U - 1) * NT < M; i += U * NT) {
+        double2 a[U][NC], tv[U][RG];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+#pragma unroll
+            for (int c = 0; c < NC; c++) a[u][c] = col[c][i + u * NT];
+#pragma unroll
+            for (int q = 0; q < RG; q++) tv[u][q] = t[q][i + u * NT];
         }
+#pragma unroll
+        for (int u = 0; u < U; u++) step(a[u], tv[u]);
     }
+    for (; i < M; i += NT) {
+        double2 a[NC], tv[RG];
 #pragma unroll
-    for (int q = 0; q < kRG; q++) {
+        for (int c = 0; c < NC; c++) a[c] = col[c][i];
 #pragma unroll
-        for (int m = 32; m >= 1; m >>= 1) {
-            zr[q] += __shfl_xor(zr[q], m, 64);
-            zi[q] += __shfl_xor(zi[q], m, 64);
-        }
+        for (int q = 0; q < RG; q++) tv[q] = t[q][i];
+        step(a, tv);
     }
-    if (lane == 0) {
+    reduce_scatter<V>(z, lane);
+    constexpr int kShare = 64 / V;  // lanes that hold the same value
+    if (lane % kShare == 0) red[wid][lane / kShare] = z[0];
+    __syncthreads();
+    if (threadIdx.x < V) {
+        const int v = threadIdx.x, cq = v >> 1, j = jb + cq / RG, r = rg0 + cq % RG;
+        double sum = red[0][v];
 #pragma unroll
-        for (int q = 0; q < kRG; q++)
-            if (q < nr) Z[(size_t)(rg0 + q) * ldz + j] = make_double2(zr[q], zi[q]);
+        for (int w = 1; w < NT / 64; w++) sum += red[w][v];
+        if (j < N && r < R) ((double *)(Z + (size_t)r * ldz + j))[v & 1] = sum;
     }
 }
 
+// about 768 workgroups of 256 rows (5778 x 5762, 4 right-hand sides: 110 us
+// with 2048, 93 us with 700, 111 us with 350)
 static void mres_shape(long M, long N, int &nch, int &kc) {
     const long tiles = (M + 255) / 256;
-    long target = std::max(1L, 2048 / std::max(1L, tiles));
+    long target = std::max(1L, 768 / std::max(1L, tiles));
     kc = (int)std::max(16L, (N + target - 1) / target);
     nch = (int)((N + kc - 1) / kc);
 }
@@ -1756,10 +1803,9 @@ size_t ws_mres(long M, long N, int R) {
     return (size_t)nch * (size_t)((M + 63) / 64 * 64) * (size_t)std::max(1, R) * sizeof(double2);
 }
 
-// out (M x R) = b - A X  (b == nullptr: out = A X), FP64 accumulation
-template <typename TA>
-static int mres_impl(const typename A2T<TA>::c2 *A, long lda, long M, long N, const double2 *X, long ldx,
-                     const double2 *b, long ldb, double2 *out, long ldo, int R, void *ws, hipStream_t s) {
+// out (M x R) = b - A X  (b == nullptr: out = A X); ws >= ws_mres(M, N, R)
+int mres_f64(const double2 *A, long lda, long M, long N, const double2 *X, long ldx, const double2 *b, long ldb,
+             double2 *out, long ldo, int R, void *ws, hipStream_t s) {
     if (M <= 0 || N <= 0 || R <= 0) return EXIT_SUCCESS;
     int nch, kc;
     mres_shape(M, N, nch, kc);
@@ -1768,8 +1814,13 @@ static int mres_impl(const typename A2T<TA>::c2 *A, long lda, long M, long N, co
     TimedRegion tr;
     timing_begin(tr, "mres_f64acc", s);
     for (int rg = 0; rg < R; rg += kRG) {
-        dim3 grid((unsigned)((M + 255) / 256), nch);
-        mres_part<TA><<<grid, 256, 0, s>>>(A, lda, (int)M, (int)N, X, ldx, R, rg, kc, part, ldp);
+        const dim3 grid((unsigned)((M + 255) / 256), nch);
+        const int nr = std::min(kRG, R - rg);
+#define BEM_MRES(RG_) mres_part<RG_><<<grid, 256, 0, s>>>(A, lda, (int)M, (int)N, X, ldx, R, rg, kc, part, ldp)
+        if (nr <= 2) BEM_MRES(2);
+        else if (nr <= 4) BEM_MRES(4);
+        else BEM_MRES(8);
+#undef BEM_MRES
         HIP_CALL(hipGetLastError());
     }
     timing_end(tr, s);
@@ -1779,28 +1830,25 @@ static int mres_impl(const typename A2T<TA>::c2 *A, long lda, long M, long N, co
     return EXIT_SUCCESS;
 }
 
-// Z (N x R) = A^H T, FP64 accumulation
-template <typename TA>
-static int mh_impl(const typename A2T<TA>::c2 *A, long lda, long M, long N, const double2 *T, long ldt, double2 *Z,
-                   long ldz, int R, hipStream_t s) {
+// Z (N x R) = A^H T
+int mh_f64(const double2 *A, long lda, long M, long N, const double2 *T, long ldt, double2 *Z, long ldz, int R,
+           hipStream_t s) {
     if (M <= 0 || N <= 0 || R <= 0) return EXIT_SUCCESS;
     TimedRegion tr;
     timing_begin(tr, "mh_f64acc", s);
     for (int rg = 0; rg < R; rg += kRG) {
-        mh_kernel<TA><<<(unsigned)((N + 3) / 4), 256, 0, s>>>(A, lda, (int)M, (int)N, T, ldt, R, rg, Z, ldz);
+        const int nr = std::min(kRG, R - rg);
+#define BEM_MH(RG_, U_, NT_)                                                                                    \
+    mh_kernel<RG_, 4, U_, NT_><<<(unsigned)((N + 3) / 4), NT_, 0, s>>>(A, lda, (int)M, (int)N, T, ldt, R, rg, \
+                                                                       Z, ldz)
+        if (nr <= 2) BEM_MH(2, 2, 256);
+        else if (nr <= 4) BEM_MH(4, 2, 128);
+        else BEM_MH(8, 1, 256);
+#undef BEM_MH
         HIP_CALL(hipGetLastError());
     }
     timing_end(tr, s);
     return EXIT_SUCCESS;
-}
-
-int mres_f64(const double2 *A, long lda, long M, long N, const double2 *X, long ldx, const double2 *b, long ldb,
-             double2 *out, long ldo, int R, void *ws, hipStream_t s) {
-    return mres_impl<double>(A, lda, M, N, X, ldx, b, ldb, out, ldo, R, ws, s);
-}
-int mh_f64(const double2 *A, long lda, long M, long N, const double2 *T, long ldt, double2 *Z, long ldz, int R,
-           hipStream_t s) {
-    return mh_impl<double>(A, lda, M, N, T, ldt, Z, ldz, R, s);
 }
 
 }  // namespace bem

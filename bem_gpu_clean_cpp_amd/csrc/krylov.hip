@@ -446,15 +446,16 @@ struct Operator {
                 }
             }
         } else {
-            for (int q = 0; q < R; q++) {
-                const double2 *vj = ws.V + (size_t)q * ws.vstride + (size_t)j * ws.ldv;
-                double2 *w = ws.w64 + (size_t)q * ws.ldv, *t = ws.t64 + (size_t)q * ws.ldv;
-                if (!normal()) {
-                    HOST_CALL(gemv_n_f64(A64, lda, M, N, vj, 0, w, 0, 1, ws.gws, s));
-                } else {
-                    HOST_CALL(gemv_n_f64(A64, lda, M, N, vj, 0, t, 0, 1, ws.gws, s));
-                    HOST_CALL(gemv_h_f64(A64, lda, M, N, t, 0, w, 0, 1, s));
-                }
+            // the systems' current basis vectors are vstride apart
+            const double2 *v = ws.V + (size_t)j * ws.ldv;
+            if (R == 1) {
+                double2 *t = normal() ? ws.t64 : ws.w64;
+                HOST_CALL(gemv_n_f64(A64, lda, M, N, v, 0, t, 0, 1, ws.gws, s));
+                if (normal()) HOST_CALL(gemv_h_f64(A64, lda, M, N, t, 0, ws.w64, 0, 1, s));
+            } else {
+                double2 *t = normal() ? ws.t64 : ws.w64;
+                HOST_CALL(mres_f64(A64, lda, M, N, v, ws.vstride, nullptr, 0, t, ws.ldv, R, ws.gws, s));
+                if (normal()) HOST_CALL(mh_f64(A64, lda, M, N, t, ws.ldv, ws.w64, ws.ldv, R, s));
             }
         }
         return EXIT_SUCCESS;
