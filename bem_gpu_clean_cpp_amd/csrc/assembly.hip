@@ -86,7 +86,7 @@ struct AsmArgs {
     const int *__restrict__ tile_ptr;
     const int *__restrict__ tile_entries;
     const int *__restrict__ tile_slots;  // element-once plan: side column of each ghost vertex
-    float2 *side;
+    typename std::conditional<sizeof(R) == 4, float2, double2>::type *side;
     typename std::conditional<sizeof(R) == 4, float2, double2>::type *A;
     R *cpart;
     typename std::conditional<sizeof(R) == 4, float2, double2>::type *bpart;
@@ -748,6 +748,239 @@ __global__ __launch_bounds__(256) void asm_tile_fast(AsmArgs<float> a) {
     }
 }
 
+// ------------------------------------------- FP64 fast path (one lane/row) ---
+// sin and cos for |x| <= 0.8: near-minimax polynomials (coefficients fitted in
+// 60 digits for this library; absolute error 1.5e-17 before rounding).
+__device__ __forceinline__ void sincos_small(double x, double &sn, double &cs) {
+    const double z = x * x;
+    double p = fma(z, 1.5909586259665044e-10, -2.5051009657015125e-08);
+    p = fma(z, p, 2.755731549825422e-06);
+    p = fma(z, p, -0.00019841269835557402);
+    p = fma(z, p, 0.00833333333333013);
+    p = fma(z, p, -0.16666666666666663);
+    sn = fma(z * x, p, x);
+    double q = fma(z, -1.137728782340167e-11, 2.0876069826994487e-09);
+    q = fma(z, q, -2.7557316893681153e-07);
+    q = fma(z, q, 2.4801587298014246e-05);
+    q = fma(z, q, -0.0013888888888886886);
+    q = fma(z, q, 0.041666666666666664);
+    cs = fma(z * z, q, fma(z, -0.5, 1.0));
+}
+// the same for |x| < 2^30: the quadrant is removed with pi/2 in three parts
+// (Cody and Waite 1980)
+__device__ __forceinline__ void sincos_wide(double x, double &sn, double &cs) {
+    const double n = rint(x * 0.6366197723675814);
+    double f = fma(-n, 1.5707963267948966, x);
+    f = fma(-n, 6.123233995736766e-17, f);
+    f = fma(-n, -1.4973849048591698e-33, f);
+    double s, c;
+    sincos_small(f, s, c);
+    const int q = (int)n;
+    const double a = (q & 1) ? c : s, b = (q & 1) ? s : c;
+    sn = (q & 2) ? -a : a;
+    cs = ((q + 1) & 2) ? -b : b;
+}
+// 1 / sqrt(x): v_rsq_f64 (relative error 2^-23) and one third-order step
+__device__ __forceinline__ double rsq_f64(double x) {
+    const double y = __builtin_amdgcn_rsq(x);
+    const double e = fma(-x * y, y, 1.0);
+    return fma(y * e, fma(0.375, e, 0.5), y);
+}
+
+// kappa^2 up to which an element's phases from its centroid's stay within 0.8
+constexpr float kSmallPhase64 = 0.63f;
+
+// rule constants of a theta row: 2 theta, 0.25 w, and 0.25 w (1 - theta), 0.25 w theta
+struct ThetaRow {
+    double th2, w, w1, w2;
+};
+__device__ constexpr ThetaRow kTheta[6] = {
+#define BEM_TH(n)                                                                            \
+    {                                                                                        \
+        1.0 + GL6::eta[n], 0.25 * GL6::w[n], 0.25 * GL6::w[n] * (0.5 - 0.5 * GL6::eta[n]),   \
+            0.25 * GL6::w[n] * (0.5 + 0.5 * GL6::eta[n])                                     \
+    }
+    BEM_TH(0), BEM_TH(1), BEM_TH(2), BEM_TH(3), BEM_TH(4), BEM_TH(5)
+#undef BEM_TH
+};
+
+// Sums of the 36 points relative to the phase k r0 of the element's centroid;
+// SMALL: |k (r - r0)| <= 0.8 on the element, so its sine and cosine need no
+// quadrant.
+struct FastSums64 {
+    double hr[3], hi[3], gr[3], gi[3], c;
+};
+template <bool IMP, bool SRC, bool SMALL>
+__device__ __forceinline__ void fast_sums64(double aa, double ae1x2, double af,
+                                            __attribute__((address_space(4))) const double *vv, double k, double kr0,
+                                            FastSums64 &s) {
+    double htr = 0, hti = 0, gtr = 0, gti = 0;
+    s.hr[0] = s.hr[1] = s.hi[0] = s.hi[1] = s.gr[0] = s.gr[1] = s.gi[0] = s.gi[1] = s.c = 0;
+#pragma unroll 1
+    for (int n = 0; n < 6; n++) {
+        const ThetaRow th = kTheta[n];
+        const double tav = fma(th.th2, af, ae1x2), v = vv[n];
+        // sums over m: B with w_m rho_m, A with w_m rho_m^2
+        double ar = 0, ai = 0, br = 0, bi = 0, gbr = 0, gbi = 0, gar = 0, gai = 0, c = 0;
+#pragma unroll
+        for (int m = 0; m < 6; m++) {
+            const double rho = 0.5 + 0.5 * GL6::eta[m], wr = GL6::w[m] * rho, wr2 = wr * rho;
+            const double r2 = fma(rho, fma(rho, v, tav), aa);
+            const double y = rsq_f64(r2);
+            const double d = fma(k, r2 * y, -kr0);
+            double sn, cs;
+            if (SMALL) sincos_small(d, sn, cs);
+            else sincos_wide(d, sn, cs);
+            const double y2 = y * y;
+            const double q3 = y2 * y, q2k = k * y2;
+            const double Hr = fma(cs, q3, sn * q2k), Hi = fma(cs, q2k, -sn * q3);
+            br = fma(wr, Hr, br);
+            bi = fma(wr, Hi, bi);
+            ar = fma(wr2, Hr, ar);
+            ai = fma(wr2, Hi, ai);
+            c = fma(wr, q3, c);
+            if (IMP || SRC) {
+                const double Gr = cs * y, Gi = -sn * y;
+                gbr = fma(wr, Gr, gbr);
+                gbi = fma(wr, Gi, gbi);
+                if (IMP) {
+                    gar = fma(wr2, Gr, gar);
+                    gai = fma(wr2, Gi, gai);
+                }
+            }
+        }
+        htr = fma(th.w, br, htr);
+        hti = fma(th.w, bi, hti);
+        s.hr[0] = fma(th.w1, ar, s.hr[0]);
+        s.hi[0] = fma(th.w1, ai, s.hi[0]);
+        s.hr[1] = fma(th.w2, ar, s.hr[1]);
+        s.hi[1] = fma(th.w2, ai, s.hi[1]);
+        s.c = fma(th.w, c, s.c);
+        if (IMP || SRC) {
+            gtr = fma(th.w, gbr, gtr);
+            gti = fma(th.w, gbi, gti);
+        }
+        if (IMP) {
+            s.gr[0] = fma(th.w1, gar, s.gr[0]);
+            s.gi[0] = fma(th.w1, gai, s.gi[0]);
+            s.gr[1] = fma(th.w2, gar, s.gr[1]);
+            s.gi[1] = fma(th.w2, gai, s.gi[1]);
+        }
+    }
+    s.hr[2] = htr - s.hr[0] - s.hr[1];
+    s.hi[2] = hti - s.hi[0] - s.hi[1];
+    s.gr[2] = gtr - s.gr[0] - s.gr[1];  // (without IMP: the whole sum)
+    s.gi[2] = gti - s.gi[0] - s.gi[1];
+}
+
+typedef __attribute__((address_space(4))) const ElemRec<double> CElemRec64;
+
+// The FP64 form of asm_tile_fast: the separable 36-point rule on every pair, on
+// the element-once plan.  Bound by the vector ALU: the generic kernel spent
+// about 290 issue slots a point on the library's sincos, square root and
+// division, at 396 registers (one wave per SIMD); here a point's phase is
+// taken from the centroid's, whose sine and cosine are computed once per pair,
+// so what is left is small and needs no reduction, and 1/r is one rsq step:
+// about 45 slots.  5762 nodes: 21.4 ms before.
+template <bool IMP, bool SRC>
+__global__ __launch_bounds__(256) void asm_tile_fast64(AsmArgs<double> a) {
+    const int lane = threadIdx.x & 63;
+    const int wave = threadIdx.x >> 6;
+    const int L = xcd_remap(blockIdx.x, a.nwg);
+    const int tile = L / a.nrbg;
+    const int rbg = L - tile * a.nrbg;
+    const int row = a.r0 + (rbg * 4 + wave) * 64 + lane;
+    const bool active = row < a.M;
+    if (wave_all(!active)) return;  // the workgroup's last waves may have no rows
+    const unsigned lrow = (unsigned)(row - a.r0);
+    const float4 xp = a.pts[active ? row : 0];
+    const double x0 = xp.x, x1 = xp.y, x2 = xp.z;
+    const double k = a.k, inv4pi = 1.0 / (4.0 * kPi);
+    double c_acc = 0, br_acc = 0, bi_acc = 0;
+    CInt *entries = (CInt *)a.tile_entries, *slots = (CInt *)a.tile_slots;
+    const int it0 = ((CInt *)a.tile_ptr)[tile], it1 = ((CInt *)a.tile_ptr)[tile + 1];
+    for (int it = it0; it < it1; ++it) {
+        const int ent = entries[it];
+        const int e = ent >> 8;
+        CFarRec &fr = ((CFarRec *)a.far)[e];
+        CElemRec64 &rec = ((CElemRec64 *)a.recs)[e];
+        const double cx = fr.c[0] - x0, cy = fr.c[1] - x1, cz = fr.c[2] - x2;
+        const double r02 = fma(cx, cx, fma(cy, cy, cz * cz));
+        const double kr0 = k * (r02 * rsq_f64(r02));
+        const double ax = rec.p3[0] - x0, ay = rec.p3[1] - x1, az = rec.p3[2] - x2;
+        const double dn = rec.n[0] * ax + rec.n[1] * ay + rec.n[2] * az;
+        const double aa = fma(ax, ax, fma(ay, ay, az * az));
+        const double ae1 = fma(ax, rec.e1[0], fma(ay, rec.e1[1], az * rec.e1[2]));
+        const double af = fma(ax, rec.f[0], fma(ay, rec.f[1], az * rec.f[2]));
+        FastSums64 s;
+        // (positive floats compare as integers)
+        if (__float_as_int(fr.rho2) <= a.far_rho2)
+            fast_sums64<IMP, SRC, true>(aa, ae1 + ae1, af, rec.vv, k, kr0, s);
+        else
+            fast_sums64<IMP, SRC, false>(aa, ae1 + ae1, af, rec.vv, k, kr0, s);
+        double s0, c0;
+        sincos_wide(kr0, s0, c0);
+        const double sJ = rec.J * inv4pi, m = -dn * sJ;
+        const double fx = m * c0, fy = -m * s0;
+        double pr[3], pi[3];
+#pragma unroll
+        for (int j = 0; j < 3; j++) {
+            pr[j] = fma(fx, s.hr[j], -fy * s.hi[j]);
+            pi[j] = fma(fx, s.hi[j], fy * s.hr[j]);
+        }
+        double cval = m * s.c, btr = 0, bti = 0;
+        if (IMP || SRC) {
+            const double sg = a.rw * sJ, qx = sg * s0, qy = sg * c0;
+            double gsr = 0, gsi = 0;
+#pragma unroll
+            for (int j = IMP ? 0 : 2; j < 3; j++) {
+                const double Gr = fma(qx, s.gr[j], -qy * s.gi[j]), Gi = fma(qx, s.gi[j], qy * s.gr[j]);
+                if (IMP) {
+                    pr[j] -= rec.beta[0] * Gr - rec.beta[1] * Gi;
+                    pi[j] -= rec.beta[0] * Gi + rec.beta[1] * Gr;
+                }
+                gsr += Gr;
+                gsi += Gi;
+            }
+            btr = rec.gamma[0] * gsr - rec.gamma[1] * gsi;
+            bti = rec.gamma[0] * gsi + rec.gamma[1] * gsr;
+        }
+        const int sv = (row == rec.nodes[0]) ? 0 : (row == rec.nodes[1]) ? 1 : (row == rec.nodes[2]) ? 2 : -1;
+        if (sv >= 0) {
+            const double *sg2 = a.sing + ((size_t)e * 3 + sv) * 16;
+#pragma unroll
+            for (int j = 0; j < 3; j++) {
+                pr[j] = sg2[2 * j];
+                pi[j] = sg2[2 * j + 1];
+            }
+            cval = sg2[6];
+            btr = sg2[7];
+            bti = sg2[8];
+        }
+        if (active) {
+#pragma unroll
+            for (int j = 0; j < 3; j++) {
+                double2 *col = (ent >> j) & 1 ? a.A + (size_t)rec.nodes[j] * a.ldA
+                                              : a.side + (size_t)slots[3 * it + j] * a.Mp;
+                double2 v = make_double2(0.0, 0.0);
+                if (!((ent >> (3 + j)) & 1)) v = col[lrow];
+                col[lrow] = make_double2(v.x + pr[j], v.y + pi[j]);
+            }
+        }
+        if ((ent >> 6) & 1) {
+            c_acc += cval;
+            if (IMP || SRC) {
+                br_acc += btr;
+                bi_acc += bti;
+            }
+        }
+    }
+    if (active) {
+        a.cpart[(size_t)tile * a.Mp + lrow] = c_acc;
+        if (IMP || SRC) a.bpart[(size_t)tile * a.Mp + lrow] = make_double2(br_acc, bi_acc);
+    }
+}
+
 // Columns of nodes no element references: only the diagonal survives.
 template <typename C2>
 __global__ void zero_columns(C2 *A, long ldA, int M, const int *__restrict__ cols, int ncols) {
@@ -762,35 +995,30 @@ __global__ void zero_columns(C2 *A, long ldA, int M, const int *__restrict__ col
 
 // Element-once plan: column of ghost node g += its side columns, in the order
 // they were made (the column is set when the node's own tile wrote nothing).
-__global__ void ghost_reduce(float2 *A, long ldA, int nrows, const float2 *__restrict__ side, long Mp,
+// W rows per thread, 16-byte accesses: two adjacent rows in FP32 (ldA and Mp
+// are even), one in FP64.
+template <typename V4, int W>
+__global__ void ghost_reduce(V4 *A, long ldA, int nrows, const V4 *__restrict__ side, long Mp,
                              const int *__restrict__ gptr, const int *__restrict__ gnode,
                              const int *__restrict__ gown, const int *__restrict__ gslot) {
-    // two adjacent rows per thread (16-byte accesses: ldA and Mp are even)
     const int g = blockIdx.y;
-    const int i = 2 * (blockIdx.x * blockDim.x + threadIdx.x);
-    if (i >= nrows) return;
-    float2 *col = A + (size_t)gnode[g] * ldA;
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= (nrows + W - 1) / W) return;
+    // (an odd last row of W = 2 takes the padding row with it: both are in bounds)
+    V4 *col = A + (size_t)gnode[g] * (ldA / W);
     const int s0 = gptr[g], s1 = gptr[g + 1];
-    const bool own = gown[g] != 0;
-    if (i + 1 < nrows) {
-        float4 acc = own ? *(const float4 *)(col + i) : make_float4(0.f, 0.f, 0.f, 0.f);
-        for (int t = s0; t < s1; t++) {
-            const float4 v = *(const float4 *)(side + (size_t)gslot[t] * Mp + i);
-            acc.x += v.x;
-            acc.y += v.y;
+    V4 acc{};
+    if (gown[g]) acc = col[i];
+    for (int t = s0; t < s1; t++) {
+        const V4 v = side[(size_t)gslot[t] * (Mp / W) + i];
+        acc.x += v.x;
+        acc.y += v.y;
+        if constexpr (W == 2) {
             acc.z += v.z;
             acc.w += v.w;
         }
-        *(float4 *)(col + i) = acc;
-    } else {
-        float2 acc = own ? col[i] : make_float2(0.f, 0.f);
-        for (int t = s0; t < s1; t++) {
-            const float2 v = side[(size_t)gslot[t] * Mp + i];
-            acc.x += v.x;
-            acc.y += v.y;
-        }
-        col[i] = acc;
     }
+    col[i] = acc;
 }
 
 // Per row: sum of the tile partials in FP64 in a fixed order (16 runs of
@@ -1752,8 +1980,9 @@ size_t device_problem_bytes(int M, int N, int E) {
         // element-once plan: its side columns and index arrays
         const int gP = choose_tiles(M, N, E, 64, 2);
         const size_t gs = (size_t)ghost_slot_bound(N, gP);
-        b += sizeof(float2) * gs * Mp;
-        if ((size_t)gP > P) b += (sizeof(float) + sizeof(float2)) * ((size_t)gP - P) * Mp;  // its tile partials
+        b += (sizeof(float2) + sizeof(double2)) * gs * Mp;
+        if ((size_t)gP > P)  // its tile partials
+            b += (sizeof(float) + sizeof(float2) + sizeof(double) + sizeof(double2)) * ((size_t)gP - P) * Mp;
         b += sizeof(int) * (gP + 1 + 4 * (size_t)E + 2 * (size_t)N + 2 * gs);
     }
     return b;
@@ -2042,7 +2271,9 @@ static int assemble_impl(DeviceProblem &dp, R k, C2 *A, long ldA, int r0, double
     SingTab st;
     sing_tab(st);
     // the plan this call walks, and the arrays it writes
-    const bool ghost = sizeof(R) == 4 && dp.use_ghost && !getenv("BEM_ASM_HALO") && !getenv("BEM_GENERIC_TILE");
+    // (FP64: the fast kernel's phases hold up to 2^30 quadrants)
+    const bool ghost = dp.use_ghost && !getenv("BEM_ASM_HALO") && !getenv("BEM_GENERIC_TILE") &&
+                       (sizeof(R) == 4 || std::fabs(kd) * dp.diam < 1e8);
     if (!ghost) HOST_CALL(halo_plan(dp, s));
     const int P = ghost ? dp.gP : dp.P;
     R *sing = nullptr, *cpart = nullptr, *bpart = nullptr, *side = nullptr;
@@ -2081,7 +2312,7 @@ static int assemble_impl(DeviceProblem &dp, R k, C2 *A, long ldA, int r0, double
     {
         // kappa^2 = k^2 rho^2 (a NaN k takes no far rule)
         const float k2 = (float)(kd * kd);
-        const float f = kFarK2 / k2, f7 = kFar7K2 / k2;
+        const float f = (sizeof(R) == 4 ? kFarK2 : kSmallPhase64) / k2, f7 = kFar7K2 / k2;
         a.far_rho2 = a.far7_rho2 = -1;
         if (f >= 0.f) memcpy(&a.far_rho2, &f, sizeof f);
         if (f7 >= 0.f) memcpy(&a.far7_rho2, &f7, sizeof f7);
@@ -2098,8 +2329,21 @@ static int assemble_impl(DeviceProblem &dp, R k, C2 *A, long ldA, int r0, double
     {
         TimedRegion tr;
         timing_begin(tr, sizeof(R) == 4 ? "asm_tile_f32" : "asm_tile_f64", s);
+        if (ghost) {
+            a.nrbg = ((nrows + 63) / 64 + 3) / 4;
+            a.nwg = a.nrbg * P;
+            a.tile_ptr = dp.gtile_ptr;
+            a.tile_entries = dp.gtile_entries;
+            a.tile_slots = dp.gtile_slots;
+            a.side = (C2 *)side;
+        }
         dim3 grid(a.nwg), block(256);
-        if (dp.qg == 4 && !ghost) {
+        if (sizeof(R) == 8 && ghost) {
+            AsmArgs<double> &ad = *(AsmArgs<double> *)&a;
+            if (dp.impedance) asm_tile_fast64<true, true><<<grid, block, 0, s>>>(ad);
+            else if (dp.source) asm_tile_fast64<false, true><<<grid, block, 0, s>>>(ad);
+            else asm_tile_fast64<false, false><<<grid, block, 0, s>>>(ad);
+        } else if (dp.qg == 4 && !ghost) {
             if (dp.impedance) asm_tile<R, 4, true><<<grid, block, 0, s>>>(a);
             else asm_tile<R, 4, false><<<grid, block, 0, s>>>(a);
         } else if (sizeof(R) == 4 && !getenv("BEM_GENERIC_TILE")) {
@@ -2109,15 +2353,6 @@ static int assemble_impl(DeviceProblem &dp, R k, C2 *A, long ldA, int r0, double
             // it below that
             const bool raw = kd / (2.0 * kPi) * dp.diam < 250.0;
             AsmArgs<float> &af = *(AsmArgs<float> *)&a;
-            if (ghost) {
-                af.nrbg = ((nrows + 63) / 64 + 3) / 4;
-                af.nwg = af.nrbg * dp.gP;
-                grid = dim3(af.nwg);
-                af.tile_ptr = dp.gtile_ptr;
-                af.tile_entries = dp.gtile_entries;
-                af.tile_slots = dp.gtile_slots;
-                af.side = (float2 *)side;
-            }
 #define BEM_FAST(IMP_, SRC_)                                                                     \
     do {                                                                                         \
         if (ghost && raw) asm_tile_fast<IMP_, true, true, SRC_><<<grid, block, 0, s>>>(af);      \
@@ -2140,9 +2375,11 @@ static int assemble_impl(DeviceProblem &dp, R k, C2 *A, long ldA, int r0, double
         if (ldA % 2 || dp.Mp % 2) BEM_FAIL("ghost_reduce needs even leading dimensions (ldA %ld, Mp %ld)", ldA, dp.Mp);
         TimedRegion tr;
         timing_begin(tr, "ghost_reduce", s);
-        dim3 grid((nrows + 511) / 512, dp.ngnodes);
-        ghost_reduce<<<grid, 256, 0, s>>>((float2 *)A, ldA, nrows, (const float2 *)side, dp.Mp, dp.gred_ptr, dp.gred_node,
-                                          dp.gred_own, dp.gred_slot);
+        constexpr int W = sizeof(R) == 4 ? 2 : 1;
+        using V4 = typename std::conditional<sizeof(R) == 4, float4, double2>::type;
+        dim3 grid(((nrows + W - 1) / W + 255) / 256, dp.ngnodes);
+        ghost_reduce<V4, W><<<grid, 256, 0, s>>>((V4 *)A, ldA, nrows, (const V4 *)side, dp.Mp, dp.gred_ptr,
+                                                 dp.gred_node, dp.gred_own, dp.gred_slot);
         HIP_CALL(hipGetLastError());
         timing_end(tr, s);
     }
