@@ -569,63 +569,20 @@ __global__ __launch_bounds__(256) void asm_tile_fast(AsmArgs<float> a) {
             v[j] = make_float2(0.f, 0.f);
             if (col[j] && !((ent >> (3 + j)) & 1) && active) v[j] = col[j][lrow];
         }
-        // centroid from the row, in FP64: the common phase k r0 is good to
-        // FP32 however many wavelengths the row is away
-        const double axd = cur.c[0] - xd, ayd = cur.c[1] - yd, azd = cur.c[2] - zd;
-        const double r02 = fma(axd, axd, fma(ayd, ayd, azd * azd));
-        const float r02f = (float)r02;
+        const FarDist fd = far_dist(cur.c, xd, yd, zd);
+        const float r02f = fd.r02f;
         const int rho2 = cur.rho2;  // (positive floats compare as integers: scalar compares)
         float pr[3], pi[3], cval, btr = 0, bti = 0;
         if (rho2 <= a.far_rho2 && wave_all(!active || r02f >= cur.far16)) {
-            const float y = __builtin_amdgcn_rsqf(r02f);
-            const double ra = r02 * (double)y;
-            const double err = fma(-ra, ra, r02);  // r0^2 - ra^2
-            const double r0 = fma(err, 0.5 * (double)y, ra);
-            const float i0 = __builtin_fmaf(0.5f * y, (float)err * y * y, y);
-            const float u0 = (float)__builtin_amdgcn_fract(r0 * a.kf64);
-            const float s0 = __builtin_amdgcn_sinf(u0), c0 = __builtin_amdgcn_cosf(u0);
-            const float r0f = (float)r0;
-            const float kr0 = k * r0f, kr0rev = krev * r0f;
-            const float ax = (float)axd, ay = (float)ayd, az = (float)azd;
-            const float dn = fr.n[0] * ax + fr.n[1] * ay + fr.n[2] * az;
-            const float i02 = i0 * i0;
-            const float T1 = i02 * __builtin_fmaf(ax, fr.u1[0], __builtin_fmaf(ay, fr.u1[1], az * fr.u1[2]));
-            const float T2 = i02 * __builtin_fmaf(ax, fr.u2[0], __builtin_fmaf(ay, fr.u2[1], az * fr.u2[2]));
+            const FarGeom g = far_geom(fr, fd, k, krev, a.kf64);
             FarSums s;
             if (rho2 <= a.far7_rho2 && wave_all(!active || r02f >= fr.far7))
-                far_sums<Far7, IMP, SRC>(fr.uu, nullptr, T1, T2, i02, kr0, kr0rev, s);
+                far_sums<Far7, IMP, SRC>(fr.uu, nullptr, g.T1, g.T2, g.i02, g.kr0, g.kr0rev, s);
             else if (wave_all(!active || r02f >= fr.far12))
-                far_sums<Far12, IMP, SRC>(fr.uu, fr.d12, T1, T2, i02, kr0, kr0rev, s);
+                far_sums<Far12, IMP, SRC>(fr.uu, fr.d12, g.T1, g.T2, g.i02, g.kr0, g.kr0rev, s);
             else
-                far_sums<Far16, IMP, SRC>(fr.uu, fr.d16, T1, T2, i02, kr0, kr0rev, s);
-            // h_j = -dn sJ i0^3 e^{-i k r0} h_j', c = -dn sJ i0^3 c'
-            const float m = -dn * fr.sJ * (i02 * i0);
-            const float fx = m * c0, fy = -m * s0;
-#pragma unroll
-            for (int j = 0; j < 3; j++) {
-                pr[j] = __builtin_fmaf(fx, s.hr[j], -fy * s.hi[j]);
-                pi[j] = __builtin_fmaf(fx, s.hi[j], fy * s.hr[j]);
-            }
-            cval = m * s.c;
-            if (IMP || SRC) {
-                // g_j = i rho omega sJ i0 e^{-i k r0} g_j'
-                const float sg = a.rw * fr.sJ * i0;
-                const float qx = sg * s0, qy = sg * c0;
-                float gsr = 0, gsi = 0;
-#pragma unroll
-                for (int j = 0; j < (IMP ? 3 : 1); j++) {
-                    const float Gr = __builtin_fmaf(qx, s.gr[j], -qy * s.gi[j]);
-                    const float Gi = __builtin_fmaf(qx, s.gi[j], qy * s.gr[j]);
-                    if (IMP) {
-                        pr[j] -= fr.beta[0] * Gr - fr.beta[1] * Gi;
-                        pi[j] -= fr.beta[0] * Gi + fr.beta[1] * Gr;
-                    }
-                    gsr += Gr;
-                    gsi += Gi;
-                }
-                btr = fr.gamma[0] * gsr - fr.gamma[1] * gsi;
-                bti = fr.gamma[0] * gsi + fr.gamma[1] * gsr;
-            }
+                far_sums<Far16, IMP, SRC>(fr.uu, fr.d16, g.T1, g.T2, g.i02, g.kr0, g.kr0rev, s);
+            far_terms<IMP, SRC>(fr, g, s, a.rw, pr, pi, cval, btr, bti);
         } else {
             CElemRec &rec = ((CElemRec *)a.recs)[e];
             const float ax = rec.p3[0] - xp.x, ay = rec.p3[1] - xp.y, az = rec.p3[2] - xp.z;
@@ -1103,118 +1060,208 @@ __global__ void rhs_fill(const double *__restrict__ pts64, int M, double k, int 
     B[(size_t)s * ldB + i] = v;
 }
 
+// rho^2 (as FP32 bits) up to which kappa^2 = k^2 rho^2 allows a rule (a NaN k: none)
+static void far_limits(double k, float kappa2, int &far_rho2, int &far7_rho2) {
+    const float k2 = (float)(k * k), f = kappa2 / k2, f7 = kFar7K2 / k2;
+    far_rho2 = far7_rho2 = -1;
+    if (f >= 0.f) memcpy(&far_rho2, &f, sizeof f);
+    if (f7 >= 0.f) memcpy(&far7_rho2, &f7, sizeof f7);
+}
+
 // ------------------------------------------------------------- field ---
 // Exterior pressure (genExtPressure / pntElemOffset, mesh.cu:1008-1073) at P
-// points for R nodal solutions.  Lane = field point; the wave walks a chunk of
-// elements (element data uniform, read with scalar loads) with the regular
-// 6x6 rule and accumulates sum_j (h_j - beta g_j) X[node_j] + gamma sum_j g_j;
-// chunk partials are summed in a fixed order by field_finalize.
+// points for R nodal solutions.  Lane = field point; a workgroup of 16 waves
+// walks a chunk of 64 elements, 4 per wave (element data and the solutions'
+// nodal values uniform, read with scalar loads), with the far rules
+// (far_rules.hpp) or the regular 6x6 rule as each point's distance asks, and
+// accumulates sum_j (h_j - beta g_j) X[node_j] + gamma sum_j g_j; the waves'
+// sums are added in LDS and the chunk partials by field_finalize, both in a
+// fixed order that does not depend on P: a point's value is the same bit for
+// bit alone and among others.
+//
+// What bounds it: with few points the chain of elements a wave walks alone,
+// since most lanes idle (64 elements a wave took 312 us for one point of a
+// 642-node body, and field_finalize's one thread per point 36 us for 8820
+// elements); with many, the vector ALU.
 constexpr int kFieldChunk = 64;
+constexpr int kFieldWaves = 16;
 constexpr int kFieldR = 16;
 
 struct FieldArgs {
     const float4 *__restrict__ xs;
-    const ElemRec<float> *__restrict__ recs;
+    const ElemRec<double> *__restrict__ recs;
+    const FarRec *__restrict__ far;
     const float2 *__restrict__ X;  // N x R, ldx
     long ldx;
     float2 *part;                  // [chunk][r][P]
     int P, E, R, r0;
     float k, kf, rw;
-    QTab<float> q;
+    double kf64;
+    int far_rho2, far7_rho2;
 };
 
-__global__ __launch_bounds__(64) void field_part(FieldArgs a) {
-    const int p = blockIdx.x * 64 + threadIdx.x;
+// p_j = h_j - beta g_j and the boundary term of one (point, element) pair by
+// the 36-point rule, the distances in FP64: in FP32 the error of r grows as
+// (size / distance)^2 next to the surface.
+__device__ __forceinline__ void field_pair_near(const FieldArgs &a, CElemRec64 &rec, const float4 xp, float *pr,
+                                                float *pi, float &btr, float &bti) {
+    const double ax = rec.p3[0] - (double)xp.x, ay = rec.p3[1] - (double)xp.y, az = rec.p3[2] - (double)xp.z;
+    const float dn = (float)(rec.n[0] * ax + rec.n[1] * ay + rec.n[2] * az);
+    const double aa = fma(ax, ax, fma(ay, ay, az * az));
+    const double ae1x2 = 2.0 * fma(ax, rec.e1[0], fma(ay, rec.e1[1], az * rec.e1[2]));
+    const double af = fma(ax, rec.f[0], fma(ay, rec.f[1], az * rec.f[2]));
+    float hr[3] = {0, 0, 0}, hi[3] = {0, 0, 0}, gr[3] = {0, 0, 0}, gi[3] = {0, 0, 0};
+#pragma unroll 1
+    for (int n = 0; n < 6; n++) {
+        const ThetaRow th = kTheta[n];
+        const double tav = fma(th.th2, af, ae1x2), vv = rec.vv[n];
+        // sums over m with w_m rho_m and w_m rho_m^2
+        float br = 0, bi = 0, ar = 0, ai = 0, gbr = 0, gbi = 0, gar = 0, gai = 0;
+#pragma unroll
+        for (int m = 0; m < 6; m++) {
+            const double rho = 0.5 + 0.5 * GL6::eta[m];
+            const float wr = (float)(GL6::w[m] * rho), wr2 = (float)(GL6::w[m] * rho * rho);
+            const float r2 = (float)fma(rho, fma(rho, vv, tav), aa);
+            const float rinv = rsq(r2);
+            float sn, cs;
+            sincos_rev(r2 * rinv * a.kf, sn, cs);
+            const float rinv2 = rinv * rinv, q3 = rinv2 * rinv, q2k = a.k * rinv2;
+            const float Hr = fmaf(cs, q3, sn * q2k), Hi = fmaf(cs, q2k, -sn * q3);
+            const float Gr = cs * rinv, Gi = -sn * rinv;
+            br = fmaf(wr, Hr, br);
+            bi = fmaf(wr, Hi, bi);
+            ar = fmaf(wr2, Hr, ar);
+            ai = fmaf(wr2, Hi, ai);
+            gbr = fmaf(wr, Gr, gbr);
+            gbi = fmaf(wr, Gi, gbi);
+            gar = fmaf(wr2, Gr, gar);
+            gai = fmaf(wr2, Gi, gai);
+        }
+        const float w = (float)th.w, w1 = (float)th.w1, w2 = (float)th.w2;
+        hr[0] = fmaf(w1, ar, hr[0]);
+        hi[0] = fmaf(w1, ai, hi[0]);
+        hr[1] = fmaf(w2, ar, hr[1]);
+        hi[1] = fmaf(w2, ai, hi[1]);
+        hr[2] = fmaf(w, br - ar, hr[2]);  // N_3 = 1 - rho
+        hi[2] = fmaf(w, bi - ai, hi[2]);
+        gr[0] = fmaf(w1, gar, gr[0]);
+        gi[0] = fmaf(w1, gai, gi[0]);
+        gr[1] = fmaf(w2, gar, gr[1]);
+        gi[1] = fmaf(w2, gai, gi[1]);
+        gr[2] = fmaf(w, gbr - gar, gr[2]);
+        gi[2] = fmaf(w, gbi - gai, gi[2]);
+    }
+    const float sJ = (float)(rec.J * (1.0 / (4.0 * kPi))), sh = -dn * sJ, sg = a.rw * sJ;
+    const float b0 = (float)rec.beta[0], b1 = (float)rec.beta[1];
+    float gsr = 0, gsi = 0;
+#pragma unroll
+    for (int j = 0; j < 3; j++) {
+        const float Gr = -sg * gi[j], Gi = sg * gr[j];
+        pr[j] = sh * hr[j] - (b0 * Gr - b1 * Gi);
+        pi[j] = sh * hi[j] - (b0 * Gi + b1 * Gr);
+        gsr += Gr;
+        gsi += Gi;
+    }
+    btr = (float)rec.gamma[0] * gsr - (float)rec.gamma[1] * gsi;
+    bti = (float)rec.gamma[0] * gsi + (float)rec.gamma[1] * gsr;
+}
+
+// RG: right-hand sides of a pass (the last ones of a.R may be fewer)
+template <int RG>
+__global__ __launch_bounds__(64 * kFieldWaves) void field_part(FieldArgs a) {
+    constexpr int kShare = RG < 4 ? RG : 4;  // right-hand sides summed over the waves together
+    __shared__ float2 red[kShare][kFieldWaves][64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int p = blockIdx.x * 64 + lane;
     const int chunk = blockIdx.y;
     const bool active = p < a.P;
     const float4 xp = a.xs[active ? p : 0];
-    const int e0 = chunk * kFieldChunk, e1 = min(a.E, e0 + kFieldChunk);
-    const int nr = min(kFieldR, a.R - a.r0);
-    float accr[kFieldR], acci[kFieldR];
+    constexpr int per = kFieldChunk / kFieldWaves;
+    const int e0 = __builtin_amdgcn_readfirstlane(chunk * kFieldChunk + wave * per), e1 = min(a.E, e0 + per);
+    const int nr = min(RG, a.R - a.r0);
+    float accr[RG], acci[RG];
 #pragma unroll
-    for (int r = 0; r < kFieldR; r++) {
+    for (int r = 0; r < RG; r++) {
         accr[r] = 0;
         acci[r] = 0;
     }
-    const float inv4pi = (float)(1.0 / (4.0 * kPi));
     for (int e = e0; e < e1; e++) {
-        const ElemRec<float> &rec = a.recs[e];
-        const float ax = rec.p3[0] - xp.x, ay = rec.p3[1] - xp.y, az = rec.p3[2] - xp.z;
-        const float dn = rec.n[0] * ax + rec.n[1] * ay + rec.n[2] * az;
-        float h1r = 0, h1i = 0, h2r = 0, h2i = 0, htr = 0, hti = 0, gr = 0, gi = 0;
-        float g1r = 0, g1i = 0, g2r = 0, g2i = 0;
-#pragma unroll 6
-        for (int i = 0; i < kNQ; i++) {
-            const float xi1 = a.q.xi1[i], xi2 = a.q.xi2[i], w = a.q.w[i];
-            const float dx = fmaf(xi1, rec.e1[0], fmaf(xi2, rec.e2[0], ax));
-            const float dy = fmaf(xi1, rec.e1[1], fmaf(xi2, rec.e2[1], ay));
-            const float dz = fmaf(xi1, rec.e1[2], fmaf(xi2, rec.e2[2], az));
-            const float r2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
-            const float rinv = rsq(r2);
-            const float r = r2 * rinv;
-            float sn, cs;
-            sincos_rev(r * a.kf, sn, cs);
-            const float Gr = cs * rinv, Gi = -sn * rinv;
-            const float w2 = w * rinv;
-            const float Hr = fmaf(Gr, rinv, -a.k * Gi) * w2;
-            const float Hi = fmaf(Gi, rinv, a.k * Gr) * w2;
-            htr += Hr; hti += Hi;
-            h1r = fmaf(xi1, Hr, h1r); h1i = fmaf(xi1, Hi, h1i);
-            h2r = fmaf(xi2, Hr, h2r); h2i = fmaf(xi2, Hi, h2i);
-            const float wGr = w * Gr, wGi = w * Gi;
-            gr += wGr; gi += wGi;
-            g1r = fmaf(xi1, wGr, g1r); g1i = fmaf(xi1, wGi, g1i);
-            g2r = fmaf(xi2, wGr, g2r); g2i = fmaf(xi2, wGi, g2i);
+        CFarRec &fr = ((CFarRec *)a.far)[e];
+        const FarGeom g = far_geom(fr, xp, a.k, a.kf, a.kf64);
+        float pr[3], pi[3], btr, bti;
+        const bool k16 = __float_as_int(fr.rho2) <= a.far_rho2, k7 = __float_as_int(fr.rho2) <= a.far7_rho2;
+        if (k16 && g.r02f >= fr.far16) {
+            FarSums s;
+            if (k7 && g.r02f >= fr.far7)
+                far_sums<Far7, true, true>(fr.uu, nullptr, g.T1, g.T2, g.i02, g.kr0, g.kr0rev, s);
+            else if (g.r02f >= fr.far12)
+                far_sums<Far12, true, true>(fr.uu, fr.d12, g.T1, g.T2, g.i02, g.kr0, g.kr0rev, s);
+            else
+                far_sums<Far16, true, true>(fr.uu, fr.d16, g.T1, g.T2, g.i02, g.kr0, g.kr0rev, s);
+            float cval;
+            far_terms<true, true>(fr, g, s, a.rw, pr, pi, cval, btr, bti);
+        } else {
+            field_pair_near(a, ((CElemRec64 *)a.recs)[e], xp, pr, pi, btr, bti);
         }
-        const float sJ = rec.J * inv4pi, sh = -dn * sJ, sg = a.rw * sJ;
-        float pr[3] = {sh * h1r, sh * h2r, sh * (htr - h1r - h2r)};
-        float pi[3] = {sh * h1i, sh * h2i, sh * (hti - h1i - h2i)};
-        const float gsr = -sg * gi, gsi = sg * gr;
-        const float G0r = -sg * g1i, G0i = sg * g1r, G1r = -sg * g2i, G1i = sg * g2r;
-        const float Gjr[3] = {G0r, G1r, gsr - G0r - G1r}, Gji[3] = {G0i, G1i, gsi - G0i - G1i};
-        const float br = rec.beta[0], bi = rec.beta[1];
 #pragma unroll
-        for (int j = 0; j < 3; j++) {
-            pr[j] -= br * Gjr[j] - bi * Gji[j];
-            pi[j] -= br * Gji[j] + bi * Gjr[j];
-        }
-        const float btr = rec.gamma[0] * gsr - rec.gamma[1] * gsi;
-        const float bti = rec.gamma[0] * gsi + rec.gamma[1] * gsr;
-#pragma unroll
-        for (int r = 0; r < kFieldR; r++) {
+        for (int r = 0; r < RG; r++) {
             if (r < nr) {
-                const float2 *xc = a.X + (size_t)(a.r0 + r) * a.ldx;
+                CFloat *xc = (CFloat *)(a.X + (size_t)(a.r0 + r) * a.ldx);
                 float sr = btr, si = bti;
 #pragma unroll
                 for (int j = 0; j < 3; j++) {
-                    const float2 xv = xc[rec.nodes[j]];
-                    sr += pr[j] * xv.x - pi[j] * xv.y;
-                    si += pr[j] * xv.y + pi[j] * xv.x;
+                    const float xr = xc[2 * (size_t)fr.nodes[j]], xi = xc[2 * (size_t)fr.nodes[j] + 1];
+                    sr += pr[j] * xr - pi[j] * xi;
+                    si += pr[j] * xi + pi[j] * xr;
                 }
                 accr[r] += sr;
                 acci[r] += si;
             }
         }
     }
-    if (active) {
 #pragma unroll
-        for (int r = 0; r < kFieldR; r++)
-            if (r < nr) a.part[((size_t)chunk * a.R + a.r0 + r) * a.P + p] = make_float2(accr[r], acci[r]);
+    for (int rb = 0; rb < RG; rb += kShare) {
+        if (rb >= nr) break;
+        if (rb > 0) __syncthreads();
+#pragma unroll
+        for (int r = 0; r < kShare; r++) red[r][wave][lane] = make_float2(accr[rb + r], acci[rb + r]);
+        __syncthreads();
+        if (wave < kShare && rb + wave < nr && active) {
+            float sr = 0, si = 0;
+#pragma unroll
+            for (int w = 0; w < kFieldWaves; w++) {
+                const float2 v = red[wave][w][lane];
+                sr += v.x;
+                si += v.y;
+            }
+            a.part[((size_t)chunk * a.R + a.r0 + rb + wave) * a.P + p] = make_float2(sr, si);
+        }
     }
 }
 
-// out[p, r] = inc_r(x_p) - sum_chunks part
-__global__ void field_finalize(const float4 *__restrict__ xs, int P, int R, int nchunks, const float2 *__restrict__ part,
-                               double k, int kind, double amp, const float *__restrict__ params, float2 *out,
-                               long ldo) {
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
+// out[p, r] = inc_r(x_p) - sum_chunks part, in FP64: 16 runs of every 16th
+// chunk per point, then the runs in order
+constexpr int kFieldRuns = 16;
+__global__ __launch_bounds__(256) void field_finalize(const float4 *__restrict__ xs, int P, int R, int nchunks,
+                                                      const float2 *__restrict__ part, double k, int kind, double amp,
+                                                      const float *__restrict__ params, float2 *out, long ldo) {
+    __shared__ double2 red[kFieldRuns][16];
+    const int lp = threadIdx.x & 15, run = threadIdx.x >> 4;
+    const int p = blockIdx.x * 16 + lp;
     const int r = blockIdx.y;
-    if (p >= P || r >= R) return;
     double sr = 0, si = 0;
-    for (int c = 0; c < nchunks; c++) {
-        const float2 v = part[((size_t)c * R + r) * P + p];
-        sr += v.x;
-        si += v.y;
+    if (p < P)
+        for (int c = run; c < nchunks; c += kFieldRuns) {
+            const float2 v = part[((size_t)c * R + r) * P + p];
+            sr += v.x;
+            si += v.y;
+        }
+    red[run][lp] = make_double2(sr, si);
+    __syncthreads();
+    if (run > 0 || p >= P) return;
+    for (int q = 1; q < kFieldRuns; q++) {
+        sr += red[q][lp].x;
+        si += red[q][lp].y;
     }
     const double x = xs[p].x, y = xs[p].y, z = xs[p].z;
     double ir = 0, ii = 0;
@@ -1236,23 +1283,20 @@ __global__ void field_finalize(const float4 *__restrict__ xs, int P, int R, int 
     out[(size_t)r * ldo + p] = make_float2((float)(ir - sr), (float)(ii - si));
 }
 
-int field_fp32(DeviceProblem &dp, float k, const float4 *xs, int P, const float2 *X, long ldx, int R,
-               const RhsSpec &rhs, float2 *out, long ldo, hipStream_t s) {
-    if (P <= 0 || R <= 0) return EXIT_SUCCESS;
+size_t field_part_bytes(int E, int P, int R) {
+    return sizeof(float2) * (size_t)((E + kFieldChunk - 1) / kFieldChunk) * R * P;
+}
+
+// Queues the field on s: params (3 R, or null: no incident field) and part
+// (field_part_bytes) on the device; nothing is allocated, no wait.
+int field_run(const DeviceProblem &dp, float k, const float4 *xs, int P, const float2 *X, long ldx, int R, int kind,
+              double amp, const float *params, float2 *part, float2 *out, long ldo, hipStream_t s) {
     const Config &cfg = config();
-    QuadTables qt;
-    quad_tables(qt);
     const int nch = (dp.E + kFieldChunk - 1) / kFieldChunk;
-    float2 *part = nullptr;
-    float *params = nullptr;
-    HOST_CALL(salloc(&part, (size_t)nch * R * P, s));
-    if (!rhs.params.empty()) {
-        HOST_CALL(salloc(&params, rhs.params.size(), s));
-        HIP_CALL(hipMemcpyAsync(params, rhs.params.data(), rhs.params.size() * sizeof(float), hipMemcpyHostToDevice, s));
-    }
     FieldArgs a;
     a.xs = xs;
-    a.recs = dp.rec32;
+    a.recs = dp.rec64;
+    a.far = dp.far32;
     a.X = X;
     a.ldx = ldx;
     a.part = part;
@@ -1261,30 +1305,41 @@ int field_fp32(DeviceProblem &dp, float k, const float4 *xs, int P, const float2
     a.R = R;
     a.k = k;
     a.kf = (float)((double)k / (2.0 * kPi));
+    a.kf64 = (double)k / (2.0 * kPi);
     a.rw = (float)((double)cfg.density * (double)(k * cfg.speed));
-    for (int q = 0; q < kNQ; q++) {
-        a.q.xi1[q] = qt.xi1[q];
-        a.q.xi2[q] = qt.xi2[q];
-        a.q.w[q] = qt.w[q];
-    }
+    far_limits((double)k, kFarK2, a.far_rho2, a.far7_rho2);
     TimedRegion tr;
     timing_begin(tr, "field_part", s);
     for (int r0 = 0; r0 < R; r0 += kFieldR) {
         a.r0 = r0;
-        dim3 grid((P + 63) / 64, nch);
-        field_part<<<grid, 64, 0, s>>>(a);
+        const dim3 grid((P + 63) / 64, nch), block(64 * kFieldWaves);
+        if (R - r0 == 1) field_part<1><<<grid, block, 0, s>>>(a);
+        else if (R - r0 <= 4) field_part<4><<<grid, block, 0, s>>>(a);
+        else field_part<kFieldR><<<grid, block, 0, s>>>(a);
         HIP_CALL(hipGetLastError());
     }
     timing_end(tr, s);
-    dim3 g2((P + 255) / 256, R);
-    field_finalize<<<g2, 256, 0, s>>>(xs, P, R, nch, part, (double)k, rhs.kind, (double)rhs.amp,
-                                      rhs.nrhs >= R ? params : nullptr, out, ldo);
-    hipError_t e = hipGetLastError();
+    field_finalize<<<dim3((P + 15) / 16, R), 256, 0, s>>>(xs, P, R, nch, part, (double)k, kind, amp, params, out, ldo);
+    HIP_CALL(hipGetLastError());
+    return EXIT_SUCCESS;
+}
+
+int field_fp32(DeviceProblem &dp, float k, const float4 *xs, int P, const float2 *X, long ldx, int R,
+               const RhsSpec &rhs, float2 *out, long ldo, hipStream_t s) {
+    if (P <= 0 || R <= 0) return EXIT_SUCCESS;
+    float2 *part = nullptr;
+    float *params = nullptr;
+    HOST_CALL(salloc(&part, field_part_bytes(dp.E, P, R) / sizeof(float2), s));
+    if (!rhs.params.empty()) {
+        HOST_CALL(salloc(&params, rhs.params.size(), s));
+        HIP_CALL(hipMemcpyAsync(params, rhs.params.data(), rhs.params.size() * sizeof(float), hipMemcpyHostToDevice, s));
+    }
+    const int rc = field_run(dp, k, xs, P, X, ldx, R, rhs.kind, (double)rhs.amp, rhs.nrhs >= R ? params : nullptr, part,
+                             out, ldo, s);
     (void)hipStreamSynchronize(s);
     sfree(part, s);
     sfree(params, s);
-    HIP_CALL(e);
-    return EXIT_SUCCESS;
+    return rc;
 }
 
 // ------------------------------------------- near-singular, FP64 ---
@@ -1750,34 +1805,7 @@ int field_fp32_noalloc(const DeviceProblem &dp, float k, const float *xs, int P,
     float2 *part = (float2 *)(b + round256(sizeof(float4) * (size_t)P) + 256);
     k_pack_field_points<<<(P + 255) / 256, 256, 0, s>>>(xs, P, xs4, src[0], src[1], src[2], params);
     HIP_CALL(hipGetLastError());
-    const Config &cfg = config();
-    QuadTables qt;
-    quad_tables(qt);
-    FieldArgs a;
-    a.xs = xs4;
-    a.recs = dp.rec32;
-    a.X = X;
-    a.ldx = dp.N;
-    a.part = part;
-    a.P = P;
-    a.E = dp.E;
-    a.R = 1;
-    a.r0 = 0;
-    a.k = k;
-    a.kf = (float)((double)k / (2.0 * kPi));
-    a.rw = (float)((double)cfg.density * (double)(k * cfg.speed));
-    for (int q = 0; q < kNQ; q++) {
-        a.q.xi1[q] = qt.xi1[q];
-        a.q.xi2[q] = qt.xi2[q];
-        a.q.w[q] = qt.w[q];
-    }
-    const int nch = (dp.E + kFieldChunk - 1) / kFieldChunk;
-    field_part<<<dim3((P + 63) / 64, nch), 64, 0, s>>>(a);
-    HIP_CALL(hipGetLastError());
-    field_finalize<<<dim3((P + 255) / 256, 1), 256, 0, s>>>(xs4, P, 1, nch, part, (double)k, BEM_RHS_POINT,
-                                                            (double)strength, params, out, P);
-    HIP_CALL(hipGetLastError());
-    return EXIT_SUCCESS;
+    return field_run(dp, k, xs4, P, X, dp.N, 1, BEM_RHS_POINT, (double)strength, params, part, out, P, s);
 }
 
 // --------------------------------------------------------------- host ---
@@ -2309,14 +2337,7 @@ static int assemble_impl(DeviceProblem &dp, R k, C2 *A, long ldA, int r0, double
     a.kf = (R)(kd / (2.0 * kPi));
     a.kf64 = kd / (2.0 * kPi);
     a.rw = (R)rw;
-    {
-        // kappa^2 = k^2 rho^2 (a NaN k takes no far rule)
-        const float k2 = (float)(kd * kd);
-        const float f = (sizeof(R) == 4 ? kFarK2 : kSmallPhase64) / k2, f7 = kFar7K2 / k2;
-        a.far_rho2 = a.far7_rho2 = -1;
-        if (f >= 0.f) memcpy(&a.far_rho2, &f, sizeof f);
-        if (f7 >= 0.f) memcpy(&a.far7_rho2, &f7, sizeof f7);
-    }
+    far_limits(kd, sizeof(R) == 4 ? kFarK2 : kSmallPhase64, a.far_rho2, a.far7_rho2);
     a.impedance = dp.impedance;
     for (int q = 0; q < kNQ; q++) {
         a.q.xi1[q] = sizeof(R) == 4 ? (R)qt.xi1[q] : (R)qt.dxi1[q];

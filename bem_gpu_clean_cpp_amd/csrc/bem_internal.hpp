@@ -242,6 +242,12 @@ int rhs_fp64(DeviceProblem &dp, double k, double2 *B, long ldB, const RhsSpec &r
 int field_fp32(DeviceProblem &dp, float k, const float4 *xs, int P, const float2 *X, long ldx, int R,
                const RhsSpec &rhs, float2 *out, long ldo, hipStream_t s);
 
+// queued on s without allocations: params (3 R or null) and part
+// (field_part_bytes) in device memory
+size_t field_part_bytes(int E, int P, int R);
+int field_run(const DeviceProblem &dp, float k, const float4 *xs, int P, const float2 *X, long ldx, int R, int kind,
+              double amp, const float *params, float2 *part, float2 *out, long ldo, hipStream_t s);
+
 // The same field for one right-hand side (an incident point source of the
 // given strength at src) with every temporary in the library's fixed-size
 // static device scratch: no allocation.  xs: P points of 3 floats, X: N nodal

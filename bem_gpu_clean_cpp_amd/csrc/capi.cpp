@@ -355,26 +355,29 @@ bem_complex bem_ext_pressure(float k, const bem_mesh *mc, bem_cart_coord src, be
     hipStream_t s;
     if (stream(&s) != EXIT_SUCCESS || validate_mesh(m->m) != EXIT_SUCCESS || mesh_device(m, s) != EXIT_SUCCESS)
         return fail();
+    // one copy in (the point, the source, the surface pressure), one out
     const int N = m->m.N();
+    std::vector<float> in(8 + 2 * (size_t)N);
+    memcpy(&in[0], x.coords, sizeof x.coords);
+    memcpy(&in[4], src.coords, sizeof src.coords);
+    memcpy(&in[8], surfPressure, sizeof(float2) * N);
     void *pa, *pb;
-    if (g_sa.get(sizeof(float2) * N + 64, &pa) || g_sb.get(sizeof(float4) + sizeof(float2) + 64, &pb)) return fail();
-    float2 *Xd = (float2 *)pa;
-    float4 *xd = (float4 *)pb;
-    float2 *od = (float2 *)((char *)pb + 32);
-    float4 xh = make_float4(x.coords[0], x.coords[1], x.coords[2], 0.f);
-    if (hipMemcpyAsync(Xd, surfPressure, sizeof(float2) * N, hipMemcpyHostToDevice, s) != hipSuccess ||
-        hipMemcpyAsync(xd, &xh, sizeof(float4), hipMemcpyHostToDevice, s) != hipSuccess) {
+    if (g_sa.get(in.size() * sizeof(float), &pa) ||
+        g_sb.get(field_part_bytes(m->dp.E, 1, 1) + sizeof(float2), &pb))
+        return fail();
+    const float *ind = (const float *)pa;
+    float2 *od = (float2 *)pb, o;
+    if (hipMemcpyAsync(pa, in.data(), in.size() * sizeof(float), hipMemcpyHostToDevice, s) != hipSuccess) {
         set_error(__FILE__, __LINE__, "copy failed");
         return fail();
     }
-    RhsSpec rhs;
-    rhs.kind = BEM_RHS_POINT;
-    rhs.nrhs = 1;
-    rhs.amp = config().strength;
-    rhs.params = {src.coords[0], src.coords[1], src.coords[2]};
-    if (field_fp32(m->dp, k, xd, 1, Xd, N, 1, rhs, od, 1, s) != EXIT_SUCCESS) return fail();
-    float2 o;
-    if (hipMemcpy(&o, od, sizeof(float2), hipMemcpyDeviceToHost) != hipSuccess) {
+    if (field_run(m->dp, k, (const float4 *)ind, 1, (const float2 *)(ind + 8), N, 1, BEM_RHS_POINT, config().strength,
+                  ind + 4, od + 1, od, 1, s) != EXIT_SUCCESS) {
+        (void)hipStreamSynchronize(s);  // `in` is still being read
+        return fail();
+    }
+    if (hipMemcpyAsync(&o, od, sizeof(float2), hipMemcpyDeviceToHost, s) != hipSuccess ||
+        hipStreamSynchronize(s) != hipSuccess) {
         set_error(__FILE__, __LINE__, "copy failed");
         return fail();
     }

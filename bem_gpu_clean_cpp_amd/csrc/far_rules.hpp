@@ -98,6 +98,53 @@ typedef __attribute__((address_space(4))) const FarRec CFarRec;
 typedef __attribute__((address_space(4))) const float CFloat;
 typedef __attribute__((address_space(4))) const int CInt;
 
+// The centroid from the row (point x), in FP64: the common phase k r0 is good
+// to FP32 however many wavelengths the row is away.
+struct FarDist {
+    double x, y, z, r02;
+    float r02f;
+};
+template <class C3>
+__device__ __forceinline__ FarDist far_dist(const C3 &c, double xd, double yd, double zd) {
+    FarDist d;
+    d.x = c[0] - xd;
+    d.y = c[1] - yd;
+    d.z = c[2] - zd;
+    d.r02 = fma(d.x, d.x, fma(d.y, d.y, d.z * d.z));
+    d.r02f = (float)d.r02;
+    return d;
+}
+
+// what the sums need of the pair (T_j = 2 (c - x).(p_j - c) / r0^2), and the
+// phase and normal distance of its terms
+struct FarGeom {
+    float r02f, i0, i02, kr0, kr0rev, s0, c0, dn, T1, T2;
+};
+__device__ __forceinline__ FarGeom far_geom(CFarRec &fr, const FarDist &d, float k, float krev, double kf64) {
+    FarGeom g;
+    const float y = __builtin_amdgcn_rsqf(d.r02f);
+    const double ra = d.r02 * (double)y;
+    const double err = fma(-ra, ra, d.r02);  // r0^2 - ra^2
+    const double r0 = fma(err, 0.5 * (double)y, ra);
+    g.r02f = d.r02f;
+    g.i0 = __builtin_fmaf(0.5f * y, (float)err * y * y, y);
+    const float u0 = (float)__builtin_amdgcn_fract(r0 * kf64);
+    g.s0 = __builtin_amdgcn_sinf(u0);
+    g.c0 = __builtin_amdgcn_cosf(u0);
+    const float r0f = (float)r0;
+    g.kr0 = k * r0f;
+    g.kr0rev = krev * r0f;
+    const float ax = (float)d.x, ay = (float)d.y, az = (float)d.z;
+    g.dn = fr.n[0] * ax + fr.n[1] * ay + fr.n[2] * az;
+    g.i02 = g.i0 * g.i0;
+    g.T1 = g.i02 * __builtin_fmaf(ax, fr.u1[0], __builtin_fmaf(ay, fr.u1[1], az * fr.u1[2]));
+    g.T2 = g.i02 * __builtin_fmaf(ax, fr.u2[0], __builtin_fmaf(ay, fr.u2[1], az * fr.u2[2]));
+    return g;
+}
+__device__ __forceinline__ FarGeom far_geom(CFarRec &fr, const float4 &x, float k, float krev, double kf64) {
+    return far_geom(fr, far_dist(fr.c, (double)x.x, (double)x.y, (double)x.z), k, krev, kf64);
+}
+
 // Sums over a far element, relative to the centroid's distance r0: with
 // i0 = 1 / r0, w = r0 / r and e^{-i phi}, phi = k (r - r0),
 //   h_j = sum W N_j w^2 (w + i k r0) e^{-i phi},  g_j = sum W N_j w e^{-i phi},
@@ -203,6 +250,40 @@ __device__ __forceinline__ void far_sums(CFloat *uu, CFloat *dd, float T1, float
             s.gr[0] = __builtin_fmaf((float)W, gr, s.gr[0]);
             s.gi[0] = __builtin_fmaf((float)W, gi, s.gi[0]);
         }
+    }
+}
+
+// The pair's terms from its sums: p_j = h_j - beta g_j with
+// h_j = -dn sJ i0^3 e^{-i k r0} h_j', g_j = i rho omega sJ i0 e^{-i k r0} g_j',
+// c = -dn sJ i0^3 c', and the boundary term gamma sum_j g_j.
+template <bool IMP, bool SRC>
+__device__ __forceinline__ void far_terms(CFarRec &fr, const FarGeom &g, const FarSums &s, float rw, float *pr,
+                                          float *pi, float &cval, float &btr, float &bti) {
+    const float m = -g.dn * fr.sJ * (g.i02 * g.i0);
+    const float fx = m * g.c0, fy = -m * g.s0;
+#pragma unroll
+    for (int j = 0; j < 3; j++) {
+        pr[j] = __builtin_fmaf(fx, s.hr[j], -fy * s.hi[j]);
+        pi[j] = __builtin_fmaf(fx, s.hi[j], fy * s.hr[j]);
+    }
+    cval = m * s.c;
+    if (IMP || SRC) {
+        const float sg = rw * fr.sJ * g.i0;
+        const float qx = sg * g.s0, qy = sg * g.c0;
+        float gsr = 0, gsi = 0;
+#pragma unroll
+        for (int j = 0; j < (IMP ? 3 : 1); j++) {
+            const float Gr = __builtin_fmaf(qx, s.gr[j], -qy * s.gi[j]);
+            const float Gi = __builtin_fmaf(qx, s.gi[j], qy * s.gr[j]);
+            if (IMP) {
+                pr[j] -= fr.beta[0] * Gr - fr.beta[1] * Gi;
+                pi[j] -= fr.beta[0] * Gi + fr.beta[1] * Gr;
+            }
+            gsr += Gr;
+            gsi += Gi;
+        }
+        btr = fr.gamma[0] * gsr - fr.gamma[1] * gsi;
+        bti = fr.gamma[0] * gsi + fr.gamma[1] * gsr;
     }
 }
 

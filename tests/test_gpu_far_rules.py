@@ -100,3 +100,40 @@ def test_small_tiles_match_oracle(tiles, monkeypatch):
     A, _ = s.system()
     s.close()
     assert np.linalg.norm(A - A0) <= (3e-7 + 6e-8 * k * 0.35) * np.linalg.norm(A0)
+
+
+# the direct field kernel: P around a wave, R around its passes of 1, 4 and 16,
+# points next to the surface (36 points) and far from it, against the oracle
+# with the same solutions.  The terms an FP32 sum over the elements adds, and
+# so its roundings, have the size int |dG/dn| |p| + rho omega int |G| (|beta| |p|
+# + |gamma|): up to 2 max|p| of the first (twice the solid angle of a closed
+# surface), the second from the elements' areas and distances.
+@pytest.mark.parametrize("bc", [(0, 1, 0), (0.5 + 0.25j, 1.0 - 0.5j, 0.3 + 0.1j)], ids=["rigid", "impedance"])
+@pytest.mark.parametrize("P,R", [(1, 1), (63, 2), (64, 4), (65, 5), (7, 16), (130, 17)])
+@pytest.mark.parametrize("dist", [1.03, 1.5, 8.0])
+def test_field_points_by_term_size(P, R, dist, bc):
+    m = bem.Mesh().icosphere(2, 0.1)
+    m.set_bc(*bc)
+    p, e, bcs = C.mesh_arrays(m)
+    k = 11.0
+    dirs = C.sphere_points(31, R, 1.0)
+    s = bem.Solver(m)
+    s.assemble(k, bem.PREC_FP32)
+    s.set_rhs(bem.RHS_PLANE, dirs, 1.0)
+    s.solve(bem.SOLVE_QR)
+    x = s.solution()
+    xs = C.sphere_points(32, P, 0.1 * dist)
+    out = s.field(xs)
+    one = s.field(xs[:1])
+    s.close()
+    x64 = xs.astype(np.float64)
+    inc = np.exp(-1j * k * x64 @ dirs.astype(np.float64).T)
+    f0 = orc.field(k, p.astype(np.float64), p.shape[0], e, bcs, x64, x, inc=inc, dtype=np.float64, **AIR)
+    f0 = np.asarray(f0).reshape(P, R)
+    tri = p[e].astype(np.float64)
+    area = np.linalg.norm(np.cross(tri[:, 1] - tri[:, 0], tri[:, 2] - tri[:, 0]), axis=1) / 2
+    G = (area / (4 * np.pi * np.linalg.norm(x64[:, None] - tri.mean(1)[None], axis=2))).sum(1)[:, None]
+    beta, gamma, rw = abs(bc[0] / bc[1]), abs(bc[2] / bc[1]), AIR["dens"] * k * AIR["speed"]
+    size = (2 + rw * G * beta) * np.abs(x).max(0)[None] + rw * G * gamma + np.abs(inc)
+    assert np.all(np.abs(out - f0) <= (3e-7 + 6e-8 * k * 0.1 * (dist + 1)) * size)
+    assert np.array_equal(out[:1], one)  # a point's value does not depend on the others
