@@ -225,6 +225,14 @@ def _c64(a):
     return np.ascontiguousarray(a, np.complex64)
 
 
+def _columns(a, own=False):
+    """The columns of a matrix as a C-ordered complex64 array, column after
+    column: what the C-ABI reads.  A matrix that lies so already (bem_system's)
+    is passed as it is; own: a copy the call may overwrite."""
+    at = np.asarray(a, np.complex64).T
+    return np.array(at, order="C", copy=True) if own else np.ascontiguousarray(at)
+
+
 # --------------------------------------------------------------- global ---
 def quad_init(order=6):
     """gaussQuad(order) + sendToDevice (numerical.cu:152-156, 227-231)."""
@@ -381,7 +389,7 @@ def qr_solve(A, B):
     """qrSolver (numerical.cu:580-644): least squares, returns X (N x nrhs) and Q^H B rows."""
     A = np.asarray(A)
     m, n = A.shape
-    a = np.array(_c64(A).T, order="C", copy=True)
+    a = _columns(A)  # bem_qr_solve does not modify it
     Bm = _c64(B)
     one = Bm.ndim == 1
     Bm = Bm.reshape(m, -1)
@@ -395,7 +403,7 @@ def lsq_solve(A, B, want_q=False):
     """lsqSolver (numerical.cu:506-554): returns (X, R, Q or None)."""
     A = np.asarray(A)
     m, n = A.shape
-    a = np.array(_c64(A).T, order="C", copy=True)  # overwritten with R
+    a = _columns(A, own=True)  # overwritten with R
     Bm = _c64(B).reshape(m, -1)
     b = np.array(Bm.T, order="C", copy=True)  # overwritten with the solution
     q = np.zeros((m, m), np.complex64) if want_q else None
@@ -407,7 +415,7 @@ def gmres(A, b, max_iter, threshold, x0=None):
     """GMRES (GMRES.cu:145-279) for a square system; returns x."""
     A = np.asarray(A)
     m = A.shape[0]
-    a = np.ascontiguousarray(_c64(A).T)
+    a = _columns(A)
     bb = _c64(b).reshape(m)
     x = np.zeros(m, np.complex64) if x0 is None else _c64(x0).reshape(m).copy()
     _check(lib().bem_gmres(_ptr(a), _ptr(bb), m, max_iter, threshold, _ptr(x)), "GMRES")

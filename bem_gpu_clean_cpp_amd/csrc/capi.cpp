@@ -50,6 +50,83 @@ Scratch g_sa, g_sb, g_sc;
 
 long round64(long m) { return (m + 63) / 64 * 64; }
 
+// ---- matrices between the caller's buffers and padded device matrices ----
+// Columns of n 8-byte units, ld on the device.  A pitched copy between host
+// and device (hipMemcpy2DAsync) goes column by column: 2562 columns of 20 kB
+// took 18 ms each way, where one contiguous copy takes 2-3 ms.  So contiguous
+// host columns are packed (unpacked) on the device, at most kPackBytes at a
+// time; host columns with gaps keep the pitched copy, which leaves the gaps
+// untouched.
+constexpr size_t kPackBytes = size_t(64) << 20;
+
+__global__ void k_copy_cols(const float2 *__restrict__ src, long lds, float2 *__restrict__ dst, long ldd, int n) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) dst[(size_t)blockIdx.y * ldd + i] = src[(size_t)blockIdx.y * lds + i];
+}
+__global__ void k_narrow_cols(const double2 *__restrict__ src, long lds, float2 *__restrict__ dst, long ldd, int n) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const double2 v = src[(size_t)blockIdx.y * lds + i];
+    dst[(size_t)blockIdx.y * ldd + i] = make_float2((float)v.x, (float)v.y);
+}
+
+// columns per packed copy (grid.y of the pack kernels)
+int pack_columns(int n, int cols) {
+    return (int)std::min<size_t>({(size_t)cols, std::max<size_t>(1, kPackBytes / (8 * (size_t)n)), 32768});
+}
+
+// host (ldh >= n units) <- device; the stream is waited for
+int copy_out(void *host, long ldh, const float2 *dev, long ldd, int n, int cols, hipStream_t s) {
+    if (n <= 0 || cols <= 0) return EXIT_SUCCESS;
+    hipError_t e = hipSuccess;
+    if (ldh != n || ldd == n || cols == 1) {
+        if (ldh == n && ldd == n)
+            e = hipMemcpyAsync(host, dev, (size_t)8 * n * cols, hipMemcpyDeviceToHost, s);
+        else
+            e = hipMemcpy2DAsync(host, 8 * ldh, dev, 8 * ldd, (size_t)8 * n, cols, hipMemcpyDeviceToHost, s);
+        (void)hipStreamSynchronize(s);
+        HIP_CALL(e);
+        return EXIT_SUCCESS;
+    }
+    const int per = pack_columns(n, cols);
+    float2 *pk = nullptr;
+    HOST_CALL(salloc(&pk, (size_t)n * per, s));
+    for (int c = 0; c < cols && e == hipSuccess; c += per) {
+        const int nc = std::min(per, cols - c);
+        k_copy_cols<<<dim3((n + 255) / 256, nc), 256, 0, s>>>(dev + (size_t)c * ldd, ldd, pk, n, n);
+        e = hipGetLastError();
+        if (e == hipSuccess)
+            e = hipMemcpyAsync((char *)host + (size_t)8 * n * c, pk, (size_t)8 * n * nc, hipMemcpyDeviceToHost, s);
+    }
+    (void)hipStreamSynchronize(s);
+    sfree(pk, s);
+    HIP_CALL(e);
+    return EXIT_SUCCESS;
+}
+
+// device <- host; the host buffer may go once the stream has been waited for
+int copy_in(float2 *dev, long ldd, const void *host, long ldh, int n, int cols, hipStream_t s) {
+    if (n <= 0 || cols <= 0) return EXIT_SUCCESS;
+    if (ldh != n || ldd == n || cols == 1) {
+        HIP_CALL(hipMemcpy2DAsync(dev, 8 * ldd, host, 8 * ldh, (size_t)8 * n, cols, hipMemcpyHostToDevice, s));
+        return EXIT_SUCCESS;
+    }
+    const int per = pack_columns(n, cols);
+    float2 *pk = nullptr;
+    HOST_CALL(salloc(&pk, (size_t)n * per, s));
+    hipError_t e = hipSuccess;
+    for (int c = 0; c < cols && e == hipSuccess; c += per) {
+        const int nc = std::min(per, cols - c);
+        e = hipMemcpyAsync(pk, (const char *)host + (size_t)8 * n * c, (size_t)8 * n * nc, hipMemcpyHostToDevice, s);
+        if (e != hipSuccess) break;
+        k_copy_cols<<<dim3((n + 255) / 256, nc), 256, 0, s>>>(pk, n, dev + (size_t)c * ldd, ldd, n);
+        e = hipGetLastError();
+    }
+    sfree(pk, s);
+    HIP_CALL(e);
+    return EXIT_SUCCESS;
+}
+
 template <typename C2>
 __global__ void k_gather_rows(const C2 *A, long lda, int N, const int *rows, int nr, double2 *out) {
     const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -224,13 +301,8 @@ static int system_impl(bem_mesh *mh, float k, const bem_cart_coord *srcs, int nu
     rhs.amp = config().strength;
     rhs.params.assign((const float *)srcs, (const float *)srcs + 3 * (size_t)numSrcs);
     HOST_CALL(rhs_fp32(dp, (double)k, Bd, dp.ldA, rhs, s));
-    HIP_CALL(hipMemcpy2DAsync(A, sizeof(bem_complex) * lda, Ad, sizeof(float2) * dp.ldA, sizeof(float2) * M, N,
-                              hipMemcpyDeviceToHost, s));
-    if (numSrcs > 0)
-        HIP_CALL(hipMemcpy2DAsync(B, sizeof(bem_complex) * ldb, Bd, sizeof(float2) * dp.ldA, sizeof(float2) * M,
-                                  numSrcs, hipMemcpyDeviceToHost, s));
-    HIP_CALL(hipStreamSynchronize(s));
-    return EXIT_SUCCESS;
+    HOST_CALL(copy_out(A, lda, Ad, dp.ldA, M, N, s));
+    return copy_out(B, ldb, Bd, dp.ldA, M, numSrcs, s);
 }
 
 int bem_system(const bem_mesh *m, float k, const bem_cart_coord *srcs, int numSrcs, bem_complex *A, int lda,
@@ -267,23 +339,15 @@ static int qr_host(bem_complex *A, int mA, int nA, int ldA, bem_complex *B, int 
     HOST_CALL(g_sb.get(sizeof(float2) * ld * std::max(1, nB), &pb));
     if (Q) HOST_CALL(g_sc.get(sizeof(float2) * (size_t)mA * mA, &pq));
     float2 *Ad = (float2 *)pa, *Bd = (float2 *)pb;
-    HIP_CALL(hipMemcpy2DAsync(Ad, sizeof(float2) * ld, A, sizeof(bem_complex) * ldA, sizeof(float2) * mA, nA,
-                              hipMemcpyHostToDevice, s));
-    if (nB > 0)
-        HIP_CALL(hipMemcpy2DAsync(Bd, sizeof(float2) * ld, B, sizeof(bem_complex) * ldB, sizeof(float2) * mA, nB,
-                                  hipMemcpyHostToDevice, s));
+    HOST_CALL(copy_in(Ad, ld, A, ldA, mA, nA, s));
+    HOST_CALL(copy_in(Bd, ld, B, ldB, mA, nB, s));
     if (Q || write_r) {
         HOST_CALL(qr_lsq_with_q_f32(Ad, ld, mA, nA, Bd, ld, nB, (float2 *)pq, mA, s));
     } else {
         HOST_CALL(qr_lsq_f32(Ad, ld, mA, nA, Bd, ld, nB, s));
     }
-    if (nB > 0)
-        HIP_CALL(hipMemcpy2DAsync(B, sizeof(bem_complex) * ldB, Bd, sizeof(float2) * ld, sizeof(float2) * mA, nB,
-                                  hipMemcpyDeviceToHost, s));
-    if (write_r) {
-        HIP_CALL(hipMemcpy2DAsync(A, sizeof(bem_complex) * ldA, Ad, sizeof(float2) * ld, sizeof(float2) * mA, nA,
-                                  hipMemcpyDeviceToHost, s));
-    }
+    HOST_CALL(copy_out(B, ldB, Bd, ld, mA, nB, s));
+    if (write_r) HOST_CALL(copy_out(A, ldA, Ad, ld, mA, nA, s));
     if (Q) HIP_CALL(hipMemcpyAsync(Q, pq, sizeof(float2) * (size_t)mA * mA, hipMemcpyDeviceToHost, s));
     HIP_CALL(hipStreamSynchronize(s));
     if (write_r) {
@@ -315,8 +379,7 @@ int bem_gmres(const bem_complex *A, const bem_complex *b, int m, int maxIter, fl
     HOST_CALL(g_sb.get(sizeof(double2) * ld * 2, &pb));
     float2 *Ad = (float2 *)pa;
     double2 *bd = (double2 *)pb, *xd = bd + ld;
-    HIP_CALL(hipMemcpy2DAsync(Ad, sizeof(float2) * ld, A, sizeof(bem_complex) * m, sizeof(float2) * m, m,
-                              hipMemcpyHostToDevice, s));
+    HOST_CALL(copy_in(Ad, ld, A, m, m, m, s));
     std::vector<double2> hb(m), hx(m);
     for (int i = 0; i < m; i++) {
         hb[i] = make_double2(b[i].x, b[i].y);
@@ -644,23 +707,25 @@ int bem_solver_get_solution_z(const bem_solver *sv, bem_zcomplex *x, int ldx) {
     if (ldx < sv->dp.N) BEM_FAIL("ldx must be >= N");
     std::lock_guard<std::mutex> lk(sv->mu);
     hipStream_t s = sv->stream;
-    HIP_CALL(hipMemcpy2DAsync(x, sizeof(bem_zcomplex) * ldx, sv->X64, sizeof(double2) * sv->dp.ldA,
-                              sizeof(double2) * sv->dp.N, sv->rhs.nrhs, hipMemcpyDeviceToHost, s));
-    HIP_CALL(hipStreamSynchronize(s));
-    return EXIT_SUCCESS;
+    return copy_out(x, 2L * ldx, (const float2 *)sv->X64, 2 * sv->dp.ldA, 2 * sv->dp.N, sv->rhs.nrhs, s);
 }
 
 int bem_solver_get_solution(const bem_solver *sv, bem_complex *x, int ldx) {
     if (!sv || !x) BEM_FAIL("null argument");
     if (ldx < sv->dp.N) BEM_FAIL("ldx must be >= N");
-    std::vector<bem_zcomplex> z((size_t)sv->dp.N * std::max(1, sv->rhs.nrhs));
-    HOST_CALL(bem_solver_get_solution_z(sv, z.data(), sv->dp.N));
-    for (int r = 0; r < sv->rhs.nrhs; r++)
-        for (int i = 0; i < sv->dp.N; i++) {
-            const bem_zcomplex v = z[(size_t)r * sv->dp.N + i];
-            x[(size_t)r * ldx + i] = {(float)v.x, (float)v.y};
-        }
-    return EXIT_SUCCESS;
+    if (sv->xr <= 0) BEM_FAIL("no solution");
+    std::lock_guard<std::mutex> lk(sv->mu);
+    hipStream_t s = sv->stream;
+    // narrowed on the device: half the bytes to copy, no pass over them here
+    const int N = sv->dp.N, R = sv->rhs.nrhs;
+    float2 *xd = nullptr;
+    HOST_CALL(salloc(&xd, (size_t)N * R, s));
+    k_narrow_cols<<<dim3((N + 255) / 256, R), 256, 0, s>>>(sv->X64, sv->dp.ldA, xd, N, N);
+    int rc = hipGetLastError() == hipSuccess ? EXIT_SUCCESS : EXIT_FAILURE;
+    if (rc != EXIT_SUCCESS) set_error(__FILE__, __LINE__, "launch failed");
+    else rc = copy_out(x, ldx, xd, N, N, R, s);
+    sfree(xd, s);
+    return rc;
 }
 
 __global__ void k_z2c_copy(const double2 *in, float2 *out, long n) {
@@ -686,11 +751,9 @@ int bem_solver_get_system(const bem_solver *sv, bem_complex *A, int lda, bem_com
             HIP_CALL(hipGetLastError());
             src = tmp;
         }
-        hipError_t e = hipMemcpy2DAsync(A, sizeof(bem_complex) * lda, src, sizeof(float2) * dp.ldA,
-                                        sizeof(float2) * dp.M, dp.N, hipMemcpyDeviceToHost, s);
-        (void)hipStreamSynchronize(s);
+        const int rc = copy_out(A, lda, src, dp.ldA, dp.M, dp.N, s);
         sfree(tmp, s);
-        HIP_CALL(e);
+        HOST_CALL(rc);
     }
     if (B && sv->rhs.nrhs > 0) {
         float2 *Bd = nullptr;
@@ -824,10 +887,7 @@ int bem_solver_get_field_matrix(const bem_solver *sv, bem_complex *F, int ldf) {
     if (ldf < sv->fP) BEM_FAIL("ldf must be >= P");
     std::lock_guard<std::mutex> lk(sv->mu);
     hipStream_t s = sv->stream;
-    HIP_CALL(hipMemcpy2DAsync(F, sizeof(bem_complex) * ldf, sv->F, sizeof(float2) * sv->ldF, sizeof(float2) * sv->fP,
-                              sv->dp.N, hipMemcpyDeviceToHost, s));
-    HIP_CALL(hipStreamSynchronize(s));
-    return EXIT_SUCCESS;
+    return copy_out(F, ldf, sv->F, sv->ldF, sv->fP, sv->dp.N, s);
 }
 
 int bem_solver_dims(const bem_solver *sv, int *M, int *N, int *nrhs) {
