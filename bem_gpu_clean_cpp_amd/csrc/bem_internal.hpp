@@ -292,18 +292,28 @@ int gemv_h_f64(const double2 *A, long lda, long M, long N, const double2 *x, lon
                hipStream_t s);
 
 // multi-right-hand-side products (gemm.hip)
+//
+// A product left as its chunk partials, for a consumer that sums them itself
+// (part[(chunk R + r) ldp + i] over chunk = 0 .. nch - 1, in that order) and so
+// saves the launch and the pass of the reduce; the partials lie in the
+// product's workspace until its next use.
+struct ProdParts {
+    const float2 *p = nullptr;
+    long ldp = 0;
+    int nch = 0;
+};
 size_t ws_gemm(long M, long N, int R);
 size_t ws_gemm_h_f32(long M, long N, int R);
 // long_chunks: fewer, longer FP32 column (row) chunks, faster for products a
 // refinement corrects; the default keeps the FP32 sums short (QR, field)
 int gemm_n_f32(const float2 *A, long lda, long M, long N, const float2 *X, long ldx, float2 *Y, long ldy, int R,
-               void *ws, hipStream_t s, bool long_chunks = false);
+               void *ws, hipStream_t s, bool long_chunks = false, ProdParts *parts = nullptr);
 int gemm_h_f32(const float2 *A, long lda, long M, long N, const float2 *T, long ldt, float2 *Z, long ldz, int R,
-               void *ws, hipStream_t s, bool long_chunks = false);
+               void *ws, hipStream_t s, bool long_chunks = false, ProdParts *parts = nullptr);
 int gemm_n_f32z(const float2 *A, long lda, long M, long N, const float2 *X, long ldx, double2 *Y, long ldy, int R,
-                void *ws, hipStream_t s);
+                void *ws, hipStream_t s, ProdParts *parts = nullptr);
 int gemm_h_f32z(const float2 *A, long lda, long M, long N, const float2 *T, long ldt, double2 *Z, long ldz, int R,
-                void *ws, hipStream_t s);
+                void *ws, hipStream_t s, ProdParts *parts = nullptr);
 // Adjoint products through a conjugate-transposed copy AH = A^H (N x M,
 // column-major, ldah = adjoint_copy_ld(N)): Z = A^H T then runs on the Y = A X
 // kernel, whose wave reads whole column segments of its operand.
@@ -319,9 +329,9 @@ int adjoint_copy_make(const float2 *A, long lda, long M, long N, int R, float2 *
                       float *bmax = nullptr, bool force = false);
 int adjoint_copy_fill(const float2 *A, long lda, long M, long N, float2 *AH, hipStream_t s, float *bmax = nullptr);
 int gemm_hc_f32(const float2 *AH, long M, long N, const float2 *T, long ldt, float2 *Z, long ldz, int R, void *ws,
-                hipStream_t s);
+                hipStream_t s, ProdParts *parts = nullptr);
 int gemm_hc_f32z(const float2 *AH, long M, long N, const float2 *T, long ldt, double2 *Z, long ldz, int R, void *ws,
-                 hipStream_t s);
+                 hipStream_t s, ProdParts *parts = nullptr);
 // FP16-split products (A and X read as FP16 hi/lo pairs on FP16 MFMA, FP32
 // accumulation): amax bounds |Re A|, |Im A| (adjoint_absmax_final after a
 // copy made with bmax); xs >= ws_split_x
@@ -337,7 +347,8 @@ size_t ws_mres(long M, long N, int R);
 // z R / nmat .. (z + 1) R / nmat - 1: the FP32 product with FP64 output and
 // the FP64-accumulated residual b - A X (ws >= ws_gemm(M, N, R))
 int gemm_n_f32z_batched(const float2 *A, long lda, long astride, int nmat, long M, long N, const float2 *X, long ldx,
-                        double2 *Y, long ldy, int R, void *ws, hipStream_t s);
+                        double2 *Y, long ldy, int R, void *ws, hipStream_t s,
+                        ProdParts *parts = nullptr);
 int mres_f32a_batched(const float2 *A, long lda, long astride, int nmat, long M, long N, const double2 *X, long ldx,
                       const double2 *b, long ldb, double2 *out, long ldo, int R, void *ws, hipStream_t s);
 // C -= V W (QR trailing update, V with 32 columns)

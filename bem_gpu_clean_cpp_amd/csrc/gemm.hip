@@ -32,6 +32,7 @@
 #include <type_traits>
 
 #include "bem_internal.hpp"
+#include "wave_sum.hpp"
 
 namespace bem {
 
@@ -835,7 +836,8 @@ static bool two_row_tiles(long M, int nch) {
 template <typename T, typename S = T, typename OC2 = typename MF<T>::c2>
 static int gemm_n_impl(const float2 *A, long lda, long M, long N, const typename MF<T>::c2 *X, long ldx,
                        const OC2 *b, long ldb, OC2 *Y, long ldy, int R, void *ws, const char *name, hipStream_t s,
-                       bool long_chunks, long astride = 0, int nmat = 1) {
+                       bool long_chunks, long astride = 0, int nmat = 1, ProdParts *parts = nullptr) {
+    if (parts) *parts = {};
     if (M <= 0 || N <= 0 || R <= 0) return EXIT_SUCCESS;
     if (lda % 2 || lda < (M + 31) / 32 * 32) BEM_FAIL("gemm_n needs an even lda >= roundup(M, 32)");
     if (nmat < 1 || R % nmat || (nmat > 1 && astride < lda * N) || nmat > 65535)
@@ -914,6 +916,12 @@ static int gemm_n_impl(const float2 *A, long lda, long M, long N, const typename
         HIP_CALL(hipGetLastError());
     }
     timing_end(tr, s);
+    if constexpr (sizeof(T) == 4) {
+        if (parts) {
+            *parts = {part, ldp, w32 ? nred : nch};
+            return EXIT_SUCCESS;
+        }
+    }
     dim3 g2((unsigned)((M + 255) / 256), R);
     gemm_reduce<T, S, OC2><<<g2, 256, 0, s>>>(part, ldp, w32 ? nred : nch, R, (int)M, b, ldb, Y, ldy);
     HIP_CALL(hipGetLastError());
@@ -922,7 +930,9 @@ static int gemm_n_impl(const float2 *A, long lda, long M, long N, const typename
 
 template <typename T, typename S = T, typename OC2 = typename MF<T>::c2>
 static int gemm_h_impl(const float2 *A, long lda, long M, long N, const typename MF<T>::c2 *Tv, long ldt, OC2 *Z,
-                       long ldz, int R, void *ws, const char *name, hipStream_t s, bool long_chunks) {
+                       long ldz, int R, void *ws, const char *name, hipStream_t s, bool long_chunks,
+                       ProdParts *parts = nullptr) {
+    if (parts) *parts = {};
     if (M <= 0 || N <= 0 || R <= 0) return EXIT_SUCCESS;
     if (lda % 2) BEM_FAIL("gemm_h needs an even lda");
     PShape ps;
@@ -961,6 +971,12 @@ static int gemm_h_impl(const float2 *A, long lda, long M, long N, const typename
         HIP_CALL(hipGetLastError());
     }
     timing_end(tr, s);
+    if constexpr (sizeof(T) == 4) {
+        if (parts) {
+            *parts = {part, ldp, nch};
+            return EXIT_SUCCESS;
+        }
+    }
     dim3 g2((unsigned)((N + 255) / 256), R);
     gemm_reduce<T, S, OC2><<<g2, 256, 0, s>>>(part, ldp, nch, R, (int)N, (const OC2 *)nullptr, 0, Z, ldz);
     HIP_CALL(hipGetLastError());
@@ -969,27 +985,27 @@ static int gemm_h_impl(const float2 *A, long lda, long M, long N, const typename
 
 // Y (M x R, ldy) = A X ; ws >= ws_gemm(M, N, R)
 int gemm_n_f32(const float2 *A, long lda, long M, long N, const float2 *X, long ldx, float2 *Y, long ldy, int R,
-               void *ws, hipStream_t s, bool long_chunks) {
+               void *ws, hipStream_t s, bool long_chunks, ProdParts *parts) {
     return gemm_n_impl<float>(A, lda, M, N, X, ldx, (const float2 *)nullptr, 0, Y, ldy, R, ws, "gemm_n_f32", s,
-                              long_chunks);
+                              long_chunks, 0, 1, parts);
 }
 
 // Z (N x R, ldz) = A^H T, T: M x R (ldt); ws >= ws_gemm(M, N, R)
 int gemm_h_f32(const float2 *A, long lda, long M, long N, const float2 *T, long ldt, float2 *Z, long ldz, int R,
-               void *ws, hipStream_t s, bool long_chunks) {
-    return gemm_h_impl<float>(A, lda, M, N, T, ldt, Z, ldz, R, ws, "gemm_h_f32", s, long_chunks);
+               void *ws, hipStream_t s, bool long_chunks, ProdParts *parts) {
+    return gemm_h_impl<float>(A, lda, M, N, T, ldt, Z, ldz, R, ws, "gemm_h_f32", s, long_chunks, parts);
 }
 
 // FP32 products whose fixed-order reduce writes FP64 vectors (the Krylov basis
 // input; refined, so long chunks)
 int gemm_n_f32z(const float2 *A, long lda, long M, long N, const float2 *X, long ldx, double2 *Y, long ldy, int R,
-                void *ws, hipStream_t s) {
+                void *ws, hipStream_t s, ProdParts *parts) {
     return gemm_n_impl<float, double, double2>(A, lda, M, N, X, ldx, (const double2 *)nullptr, 0, Y, ldy, R, ws,
-                                               "gemm_n_f32", s, true);
+                                               "gemm_n_f32", s, true, 0, 1, parts);
 }
 int gemm_h_f32z(const float2 *A, long lda, long M, long N, const float2 *T, long ldt, double2 *Z, long ldz, int R,
-                void *ws, hipStream_t s) {
-    return gemm_h_impl<float, double, double2>(A, lda, M, N, T, ldt, Z, ldz, R, ws, "gemm_h_f32", s, true);
+                void *ws, hipStream_t s, ProdParts *parts) {
+    return gemm_h_impl<float, double, double2>(A, lda, M, N, T, ldt, Z, ldz, R, ws, "gemm_h_f32", s, true, parts);
 }
 
 // ------------------------------------------ conjugate-transposed copy ---
@@ -1079,22 +1095,22 @@ int adjoint_copy_make(const float2 *A, long lda, long M, long N, int R, float2 *
 
 // Z (N x R) = A^H T through the copy: the Y = A X product of the N x M matrix AH
 int gemm_hc_f32(const float2 *AH, long M, long N, const float2 *T, long ldt, float2 *Z, long ldz, int R, void *ws,
-                hipStream_t s) {
+                hipStream_t s, ProdParts *parts) {
     return gemm_n_impl<float>(AH, adjoint_copy_ld(N), N, M, T, ldt, (const float2 *)nullptr, 0, Z, ldz, R, ws,
-                              "gemm_hc_f32", s, true);
+                              "gemm_hc_f32", s, true, 0, 1, parts);
 }
 int gemm_hc_f32z(const float2 *AH, long M, long N, const float2 *T, long ldt, double2 *Z, long ldz, int R, void *ws,
-                 hipStream_t s) {
+                 hipStream_t s, ProdParts *parts) {
     return gemm_n_impl<float, double, double2>(AH, adjoint_copy_ld(N), N, M, T, ldt, (const double2 *)nullptr, 0, Z,
-                                               ldz, R, ws, "gemm_hc_f32", s, true);
+                                               ldz, R, ws, "gemm_hc_f32", s, true, 0, 1, parts);
 }
 
 // several matrices at once (astride apart, R / nmat right-hand sides each):
 // the Krylov product with FP64 output and the FP64 residual b - A X
 int gemm_n_f32z_batched(const float2 *A, long lda, long astride, int nmat, long M, long N, const float2 *X, long ldx,
-                        double2 *Y, long ldy, int R, void *ws, hipStream_t s) {
+                        double2 *Y, long ldy, int R, void *ws, hipStream_t s, ProdParts *parts) {
     return gemm_n_impl<float, double, double2>(A, lda, M, N, X, ldx, (const double2 *)nullptr, 0, Y, ldy, R, ws,
-                                               "gemm_n_f32", s, true, astride, nmat);
+                                               "gemm_n_f32", s, true, astride, nmat, parts);
 }
 int mres_f32a_batched(const float2 *A, long lda, long astride, int nmat, long M, long N, const double2 *X, long ldx,
                       const double2 *b, long ldb, double2 *out, long ldo, int R, void *ws, hipStream_t s) {
@@ -1699,28 +1715,6 @@ __global__ __launch_bounds__(256) void mres_reduce(const double2 *__restrict__ p
     } else {
         out[(size_t)r * ldo + i] = make_double2(sr, si);
     }
-}
-
-// Sums x[v] (V a power of two, at most 64) over the 64 lanes: afterwards lane
-// l holds the total of x[v(l)] in x[0], v(l) = the V-value index whose bits are
-// the high bits of l (bit H of the lane picks the upper half at each step).
-template <int V>
-__device__ __forceinline__ void reduce_scatter(double (&x)[V], int lane) {
-    int mask = 32;
-#pragma unroll
-    for (int h = V / 2; h >= 1; h >>= 1) {
-        const bool up = (lane & mask) != 0;
-#pragma unroll
-        for (int i = 0; i < h; i++) {
-            // (selected as values: a select of the two addresses puts x in
-            // scratch memory)
-            const double lo = x[i], hi = x[i + h];
-            const double send = up ? lo : hi, keep = up ? hi : lo;
-            x[i] = keep + __shfl_xor(send, mask, 64);
-        }
-        mask >>= 1;
-    }
-    for (; mask >= 1; mask >>= 1) x[0] += __shfl_xor(x[0], mask, 64);
 }
 
 // Z[j][r] = sum_i conj(A[i, j]) T[i][r] for the NC columns j of a workgroup of

@@ -34,6 +34,7 @@
 
 #include "bem_internal.hpp"
 #include "hessenberg_ls.hpp"
+#include "wave_sum.hpp"
 
 namespace bem {
 
@@ -192,28 +193,174 @@ __global__ void kb_normalize(const double2 *__restrict__ w, long wstride, const 
     if (out32) out32[(size_t)r * o32stride + i] = make_float2((float)v.x, (float)v.y);
 }
 
-// One Gram-Schmidt pass after kb_mdot_part, in one launch: every workgroup
-// forms h_r[l] = sum_b part_r[b][l] (fixed order) in LDS; workgroup 0 stores
-// it to hout (and adds it to acc); then w_r += sign V_r h_r over the
-// workgroup's 256 rows, and the workgroup's partial of |w_r|^2 (fixed-order
-// tree) goes to npart_r[blockIdx.x].  Dynamic LDS: nv double2.
+// The newest basis vector of a chunk of Arnoldi steps is left unnormalised by
+// kb_final_maxpy; the next step's kb_mdot finishes it.  nb = 0: the vector is
+// normalised already.  Otherwise npart_r[0 .. nb - 1] are the partials of
+// |w_r|^2 (the value at K + 1 of its Hessenberg column, hslot), npart_r[nb]
+// the factor that undoes the scale of the FP32 copy.
+struct LazyNorm {
+    const double *npart = nullptr;
+    long nstride = 0;
+    int nb = 0;
+    double2 *hslot = nullptr;
+    long hsstride = 0;
+    bool scaled = false;  // the product was of the scaled FP32 copy
+};
+
+// basis vectors per wave of kb_mdot: 4 where the rows and systems alone give
+// enough workgroups (each group of 4 VQ vectors reads w again), else 1 (one
+// right-hand side of 10242 rows: 21 workgroups for up to 15 vectors leave most
+// of the chip idle; with one vector a wave the dots take 4.9 us)
+static int mdot_vecs(int nblk, int R) { return (long)nblk * R >= 64 ? 4 : 1; }
+
+// rows of a workgroup of kb_mdot: enough workgroups for small systems, few
+// partials for large ones (they are summed by every workgroup of the update)
+static int mdot_rows(int n) { return n <= 4096 ? 256 : n <= 16384 ? 512 : 1024; }
+
+// First half of a Gram-Schmidt pass for R systems (r = blockIdx.y), over the
+// rpb rows of the workgroup: w_r from the partials of the product (PARTS,
+// summed in chunk order as the product's own reduce does) or from win_r; the
+// rows of the unnormalised newest basis vector V_{nv-1} normalised in place and
+// w_r scaled alike (A v = (A w) / |w|); then part[blk (nv + 1) + l] = sum over
+// the rows of conj(V_l) w, and the rows' |w|^2 as entry nv.  blockIdx.z takes
+// 4 VQ of the nv + 1 sums; z = 0 stores w (wout, not win: the others may
+// still be reading).  Bound by latency for few basis vectors, by reading them
+// (from the 256 MB cache) for many.  16 systems of 2562 rows, restarts of 100:
+// 10.3 us a step, where the product's reduce (4.3), the dots (6.8) and the
+// normalisation (3.3) as launches of their own took 14.4 and two more gaps.
+// Dynamic LDS: rpb double2.
+template <bool PARTS, int VQ>
+__global__ __launch_bounds__(256) void kb_mdot(double2 *V, long ldv, long vstride, int nv, ProdParts pp, int R,
+                                               const double2 *__restrict__ win, double2 *__restrict__ wout,
+                                               long wstride, int n, int rpb, double2 *__restrict__ part, long pstride,
+                                               LazyNorm ln) {
+    extern __shared__ double2 s_w[];
+    __shared__ double s_sc[2];
+    const int r = blockIdx.y, lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int base = blockIdx.x * rpb;
+    double2 *Vr = V + (size_t)r * vstride;
+    const int l0 = blockIdx.z * 4 * VQ + wave;
+    // the basis rows of the first 256 go out before w is formed, so that their
+    // latency and that of w overlap; rows past n meet a w of zero and read the
+    // last row
+    double2 v[VQ][4];
+    auto load_v = [&](int i0) {
+#pragma unroll
+        for (int q = 0; q < VQ; q++) {
+            if (l0 + 4 * q >= nv) continue;
+            const double2 *vl = Vr + (size_t)(l0 + 4 * q) * ldv;
+#pragma unroll
+            for (int u = 0; u < 4; u++) v[q][u] = vl[min(base + i0 + lane + 64 * u, n - 1)];
+        }
+    };
+    load_v(0);
+    if (ln.nb && wave == 0) {
+        const double *np = ln.npart + (size_t)r * ln.nstride;
+        double q = 0;
+        for (int b = lane; b < ln.nb; b += 64) q += np[b];
+#pragma unroll
+        for (int m = 32; m >= 1; m >>= 1) q += __shfl_xor(q, m, 64);
+        if (lane == 0) {
+            const double sc = q > 0 ? 1.0 / sqrt(q) : 0.0;
+            s_sc[0] = sc;
+            s_sc[1] = ln.scaled ? sc * np[ln.nb] : sc;
+            if (blockIdx.x == 0 && blockIdx.z == 0) ln.hslot[(size_t)r * ln.hsstride] = make_double2(q, 0.0);
+        }
+    }
+    for (int i = threadIdx.x; i < rpb; i += 256) {
+        const int row = base + i;
+        double2 w = make_double2(0.0, 0.0);
+        if (row < n) {
+            if constexpr (PARTS) {
+                const float2 *p = pp.p + (size_t)r * pp.ldp + row;
+                const size_t cs = (size_t)R * pp.ldp;
+                int c = 0;
+                for (; c + 8 <= pp.nch; c += 8) {
+                    float2 q[8];
+#pragma unroll
+                    for (int u = 0; u < 8; u++) q[u] = p[(size_t)(c + u) * cs];
+#pragma unroll
+                    for (int u = 0; u < 8; u++) {
+                        w.x += (double)q[u].x;
+                        w.y += (double)q[u].y;
+                    }
+                }
+                for (; c < pp.nch; c++) {
+                    const float2 q = p[(size_t)c * cs];
+                    w.x += (double)q.x;
+                    w.y += (double)q.y;
+                }
+            } else {
+                w = win[(size_t)r * wstride + row];
+            }
+        }
+        s_w[i] = w;
+    }
+    __syncthreads();
+    const double vsc = ln.nb ? s_sc[0] : 1.0, wsc = ln.nb ? s_sc[1] : 1.0;
+    if (wout && blockIdx.z == 0)
+        for (int i = threadIdx.x; i < rpb && base + i < n; i += 256)
+            wout[(size_t)r * wstride + base + i] = make_double2(s_w[i].x * wsc, s_w[i].y * wsc);
+    double x[2 * VQ];
+#pragma unroll
+    for (int q = 0; q < 2 * VQ; q++) x[q] = 0.0;
+    for (int i0 = 0; i0 < rpb && base + i0 < n; i0 += 256) {
+        if (i0) load_v(i0);
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            double2 w = s_w[i0 + lane + 64 * u];
+            w.x *= wsc;
+            w.y *= wsc;
+            const int row = base + i0 + lane + 64 * u;
+#pragma unroll
+            for (int q = 0; q < VQ; q++) {
+                const int l = l0 + 4 * q;
+                if (l > nv) continue;
+                double2 vv = l < nv ? v[q][u] : w;
+                if (l == nv - 1 && ln.nb) {
+                    vv.x *= vsc;
+                    vv.y *= vsc;
+                    if (row < n) Vr[(size_t)l * ldv + row] = vv;
+                }
+                x[2 * q] = fma(vv.x, w.x, fma(vv.y, w.y, x[2 * q]));
+                x[2 * q + 1] = fma(vv.x, w.y, fma(-vv.y, w.x, x[2 * q + 1]));
+            }
+        }
+    }
+    reduce_scatter<2 * VQ>(x, lane);
+    constexpr int kShare = 32 / VQ;  // lanes that hold the same value
+    const int v2 = lane / kShare, l = l0 + 4 * (v2 >> 1);
+    if (lane % kShare == 0 && l <= nv)
+        ((double *)(part + (size_t)r * pstride + (size_t)blockIdx.x * (nv + 1) + l))[v2 & 1] = x[0];
+}
+
+// Second half of the pass: every workgroup forms h_r[l] = sum_b part_r[b][l]
+// (fixed order) and |w_r|^2 before the pass in LDS; workgroup 0 stores h to hout
+// (and adds it to acc); then w_r -= V_r h_r over the workgroup's 256 rows goes
+// to wout_r, and its partial of |w_r|^2 (fixed-order tree) to
+// npart_r[blockIdx.x].  With out32: the FP32 operand of the next product,
+// unnormalised but divided by |w_r| before the pass, so that it stays in the
+// range of FP32 whatever the scale of A; that factor goes to
+// npart_r[gridDim.x].  Dynamic LDS: nv + 1 double2.
 __global__ __launch_bounds__(256) void kb_final_maxpy(const double2 *__restrict__ part, long pstride, int nblk,
-                                                      const double2 *__restrict__ V, long ldv, long vstride, int nv,
+                                                      const double2 *V, long ldv, long vstride, int nv,
                                                       double2 *__restrict__ hout, long hstride,
-                                                      double2 *__restrict__ acc, long astride, double sign,
-                                                      double2 *__restrict__ w, long wstride, int n,
+                                                      double2 *__restrict__ acc, long astride, const double2 *w,
+                                                      long wstride, double2 *wout, long ostride,
+                                                      float2 *__restrict__ out32, long o32stride, int n,
                                                       double *__restrict__ npart, long nstride) {
     extern __shared__ double2 s_h[];
     __shared__ double s_n[4];
     const int r = blockIdx.y;
     const double2 *pr = part + (size_t)r * pstride;
-    for (int l = threadIdx.x; l < nv; l += 256) {
+    for (int l = threadIdx.x; l <= nv; l += 256) {
         double sr = 0, si = 0;
         int b = 0;
         for (; b + 8 <= nblk; b += 8) {
             double2 q[8];
 #pragma unroll
-            for (int u = 0; u < 8; u++) q[u] = pr[(size_t)(b + u) * nv + l];
+            for (int u = 0; u < 8; u++) q[u] = pr[(size_t)(b + u) * (nv + 1) + l];
 #pragma unroll
             for (int u = 0; u < 8; u++) {
                 sr += q[u].x;
@@ -221,12 +368,12 @@ __global__ __launch_bounds__(256) void kb_final_maxpy(const double2 *__restrict_
             }
         }
         for (; b < nblk; b++) {
-            const double2 q = pr[(size_t)b * nv + l];
+            const double2 q = pr[(size_t)b * (nv + 1) + l];
             sr += q.x;
             si += q.y;
         }
         s_h[l] = make_double2(sr, si);
-        if (blockIdx.x == 0) {
+        if (blockIdx.x == 0 && l < nv) {
             hout[(size_t)r * hstride + l] = make_double2(sr, si);
             if (acc) {
                 double2 a = acc[(size_t)r * astride + l];
@@ -238,6 +385,7 @@ __global__ __launch_bounds__(256) void kb_final_maxpy(const double2 *__restrict_
     }
     __syncthreads();
     const int i = blockIdx.x * 256 + threadIdx.x;
+    const double q0 = s_h[nv].x;
     double nrm = 0;
     if (i < n) {
         const double2 *Vr = V + (size_t)r * vstride;
@@ -261,24 +409,31 @@ __global__ __launch_bounds__(256) void kb_final_maxpy(const double2 *__restrict_
             si = fma(v.x, c.y, fma(v.y, c.x, si));
         }
         double2 o = w[(size_t)r * wstride + i];
-        o.x += sign * sr;
-        o.y += sign * si;
-        w[(size_t)r * wstride + i] = o;
+        o.x -= sr;
+        o.y -= si;
+        wout[(size_t)r * ostride + i] = o;
+        if (out32) {
+            const double sp = q0 > 0 ? 1.0 / sqrt(q0) : 0.0;
+            out32[(size_t)r * o32stride + i] = make_float2((float)(o.x * sp), (float)(o.y * sp));
+        }
         nrm = fma(o.x, o.x, o.y * o.y);
     }
 #pragma unroll
     for (int m = 32; m >= 1; m >>= 1) nrm += __shfl_xor(nrm, m, 64);
     if ((threadIdx.x & 63) == 0) s_n[threadIdx.x >> 6] = nrm;
     __syncthreads();
-    if (threadIdx.x == 0) npart[(size_t)r * nstride + blockIdx.x] = (s_n[0] + s_n[1]) + (s_n[2] + s_n[3]);
+    if (threadIdx.x == 0) {
+        npart[(size_t)r * nstride + blockIdx.x] = (s_n[0] + s_n[1]) + (s_n[2] + s_n[3]);
+        if (blockIdx.x == 0) npart[(size_t)r * nstride + gridDim.x] = sqrt(q0);
+    }
 }
 
-// |w_r|^2 = sum of the nb partials of kb_final_maxpy (one wave, fixed order);
-// workgroup 0 stores it to hslot_r; out_r = w_r / |w_r| (and its FP32 copy)
-__global__ __launch_bounds__(256) void kb_normalize_np(const double2 *__restrict__ w, long wstride,
+// The last step of a chunk: |w_r|^2 = sum of the nb partials of kb_final_maxpy
+// (one wave, fixed order); workgroup 0 stores it to hslot_r; w_r /= |w_r| in
+// place (and its FP32 copy)
+__global__ __launch_bounds__(256) void kb_normalize_np(double2 *__restrict__ w, long wstride,
                                                        const double *__restrict__ npart, long nstride, int nb,
                                                        double2 *__restrict__ hslot, long hsstride,
-                                                       double2 *__restrict__ out, long ostride,
                                                        float2 *__restrict__ out32, long o32stride, int n) {
     __shared__ double s_q;
     const int r = blockIdx.y;
@@ -300,7 +455,7 @@ __global__ __launch_bounds__(256) void kb_normalize_np(const double2 *__restrict
     const double sc = q > 0 ? 1.0 / sqrt(q) : 0.0;
     const double2 x = w[(size_t)r * wstride + i];
     const double2 v = make_double2(x.x * sc, x.y * sc);
-    out[(size_t)r * ostride + i] = v;
+    w[(size_t)r * wstride + i] = v;
     if (out32) out32[(size_t)r * o32stride + i] = make_float2((float)v.x, (float)v.y);
 }
 
@@ -319,7 +474,7 @@ constexpr size_t kMaxGraphs = 512;  // captured Arnoldi chunks kept per workspac
 constexpr int kGraphAfter = 2;       // eager launches of a chunk before it is captured
 
 struct KrylovWS {
-    int n = 0, m = 0, R = 0, restart = 0, nblk = 0;
+    int n = 0, m = 0, R = 0, restart = 0, nblk = 0, rpb = 0;
     long ldv = 0, vstride = 0, hstride = 0, pstride = 0;
     double2 *V = nullptr, *w64 = nullptr, *t64 = nullptr, *r = nullptr, *h = nullptr, *part = nullptr;
     float2 *v32 = nullptr, *w32 = nullptr, *t32 = nullptr;
@@ -333,7 +488,7 @@ struct KrylovWS {
     // normal equations (several right-hand sides); refreshed every solve
     float2 *AH = nullptr;
     double2 *hch = nullptr;  // Hessenberg columns of an Arnoldi chunk
-    double *npart = nullptr;  // per system: |w|^2 partials of the 256-row workgroups
+    double *npart = nullptr;  // per system: |w|^2 partials of the 256-row workgroups, and |w| before the pass
     long nstride = 0;
     hipStream_t st = nullptr;
     ~KrylovWS() {
@@ -350,7 +505,8 @@ struct KrylovWS {
         ldv = ((long)std::max(n, m) + 63) / 64 * 64;
         vstride = ldv * (restart + 1);
         hstride = 2L * (restart + 2);
-        nblk = (int)((std::max(n, m) + 1023) / 1024);
+        rpb = mdot_rows(n);
+        nblk = std::max((n + rpb - 1) / rpb, (n + 1023) / 1024);
         pstride = (long)nblk * (restart + 2);
         HOST_CALL(salloc(&V, (size_t)vstride * R, s));
         HOST_CALL(salloc(&w64, (size_t)ldv * R, s));
@@ -363,7 +519,7 @@ struct KrylovWS {
         HOST_CALL(salloc(&t32, (size_t)ldv * R, s));
         const size_t g = std::max(std::max(ws_gemv_n(m, n, 1), ws_gemm(m, n, R)), ws_mres(m, n, R));
         HOST_CALL(salloc(&gws, g, s));
-        nstride = (n + 255) / 256;
+        nstride = (n + 255) / 256 + 1;
         HOST_CALL(salloc(&npart, (size_t)nstride * R, s));
         return EXIT_SUCCESS;
     }
@@ -381,16 +537,6 @@ static int bdot(KrylovWS &ws, const double2 *V, long vstride, int nv, const doub
     const int bt = std::min(256, 64 * ((nv + 63) / 64));
     dim3 g2((nv + bt - 1) / bt, ws.R);
     kb_mdot_final<<<g2, bt, 0, s>>>(ws.part, ws.pstride, nblk, nv, out, ostride, acc, astride ? astride : ostride);
-    HIP_CALL(hipGetLastError());
-    return EXIT_SUCCESS;
-}
-
-// the partials of V_r^H w_r alone (kb_final_maxpy sums them)
-static int bdot_part(KrylovWS &ws, const double2 *V, long vstride, int nv, const double2 *w, long wstride, int n,
-                     hipStream_t s) {
-    const int nblk = (n + 1023) / 1024;
-    dim3 g1(nblk, ws.R, (nv + 3) / 4);
-    kb_mdot_part<<<g1, 256, 0, s>>>(V, ws.ldv, vstride, nv, w, wstride, n, ws.part, ws.pstride);
     HIP_CALL(hipGetLastError());
     return EXIT_SUCCESS;
 }
@@ -414,7 +560,8 @@ struct Operator {
     int nmat = 1;
     bool normal() const { return M > N; }
     // w64_r <- op(V_r[:, j]) for every system (FP32 A reads v32)
-    int apply(KrylovWS &ws, int j, hipStream_t s) const {
+    // (with pp: a multi-RHS FP32 product may be left as its partials, pp->p set)
+    int apply(KrylovWS &ws, int j, hipStream_t s, ProdParts *pp = nullptr) const {
         const int bs = 256;
         const int R = ws.R;
         if (A32) {
@@ -436,13 +583,13 @@ struct Operator {
                 // the products' fixed-order reduce writes the FP64 vector directly
                 if (nmat > 1) {
                     HOST_CALL(gemm_n_f32z_batched(A32, lda, astride, nmat, M, N, ws.v32, ws.ldv, ws.w64, ws.ldv, R,
-                                                  ws.gws, s));
+                                                  ws.gws, s, pp));
                 } else if (!normal()) {
-                    HOST_CALL(gemm_n_f32z(A32, lda, M, N, ws.v32, ws.ldv, ws.w64, ws.ldv, R, ws.gws, s));
+                    HOST_CALL(gemm_n_f32z(A32, lda, M, N, ws.v32, ws.ldv, ws.w64, ws.ldv, R, ws.gws, s, pp));
                 } else {
                     HOST_CALL(gemm_n_f32(A32, lda, M, N, ws.v32, ws.ldv, ws.t32, ws.ldv, R, ws.gws, s, true));
-                    if (AH) HOST_CALL(gemm_hc_f32z(AH, M, N, ws.t32, ws.ldv, ws.w64, ws.ldv, R, ws.gws, s));
-                    else HOST_CALL(gemm_h_f32z(A32, lda, M, N, ws.t32, ws.ldv, ws.w64, ws.ldv, R, ws.gws, s));
+                    if (AH) HOST_CALL(gemm_hc_f32z(AH, M, N, ws.t32, ws.ldv, ws.w64, ws.ldv, R, ws.gws, s, pp));
+                    else HOST_CALL(gemm_h_f32z(A32, lda, M, N, ws.t32, ws.ldv, ws.w64, ws.ldv, R, ws.gws, s, pp));
                 }
             }
         } else {
@@ -758,30 +905,57 @@ int gmres_device(const float2 *A32, const double2 *A64, long lda, int M, int N, 
             auto launch_chunk = [&](int j, int c) -> int {
             for (int t = 0; t < c; t++) {
                 const int jj = j + t;
-                HOST_CALL(op.apply(ws, jj, s));
                 double2 *h1 = ws.hch + (size_t)t * hs, *h2 = ws.h + (K + 2);
                 dim3 gg((N + bs - 1) / bs, R);
                 if (fused) {
-                    // per pass: partial dots, then sums + update + |w|^2 partials
-                    // in one launch; the normalisation sums the partials
-                    const int nblk = (N + 1023) / 1024;
-                    const size_t lds = sizeof(double2) * (jj + 1);
-                    HOST_CALL(bdot_part(ws, ws.V, ws.vstride, jj + 1, ws.w64, ldv, N, s));
-                    kb_final_maxpy<<<gg, bs, lds, s>>>(ws.part, ws.pstride, nblk, ws.V, ldv, ws.vstride, jj + 1, h1,
-                                                       hcs, nullptr, 0, -1.0, ws.w64, ldv, N, ws.npart, ws.nstride);
+                    // one product and two launches a step: w from the product's
+                    // partials, the previous vector normalised, the dots; then
+                    // sums, update, |w|^2 partials.  The second pass runs on w
+                    // alone; the last vector of the chunk is normalised by
+                    // itself, since the host reads its norm.
+                    ProdParts pp;
+                    HOST_CALL(op.apply(ws, jj, s, &pp));
+                    const int nblk = (N + ws.rpb - 1) / ws.rpb, vq = mdot_vecs(nblk, R);
+                    const dim3 gd(nblk, R, (jj + 2 + 4 * vq - 1) / (4 * vq));
+                    const size_t ldsw = sizeof(double2) * ws.rpb, ldsh = sizeof(double2) * (jj + 2);
+                    const int nv = jj + 1;
+                    LazyNorm ln;
+                    if (t > 0) {
+                        ln.npart = ws.npart;
+                        ln.nstride = ws.nstride;
+                        ln.nb = (int)gg.x;
+                        ln.hslot = h1 - hs + (K + 1);
+                        ln.hsstride = hcs;
+                        ln.scaled = op.A32 != nullptr;
+                    }
+                    double2 *vnext = ws.V + (size_t)(jj + 1) * ldv;
+                    float2 *v32 = op.A32 ? ws.v32 : nullptr;
+                    // (w64 is what the product wrote: the scaled w goes to t64)
+                    auto *dots = pp.p ? (vq == 4 ? kb_mdot<true, 4> : kb_mdot<true, 1>)
+                                      : (vq == 4 ? kb_mdot<false, 4> : kb_mdot<false, 1>);
+                    dots<<<gd, 256, ldsw, s>>>(ws.V, ldv, ws.vstride, nv, pp, R, ws.w64, ws.t64, ldv, N, ws.rpb,
+                                               ws.part, ws.pstride, ln);
+                    kb_final_maxpy<<<gg, bs, ldsh, s>>>(ws.part, ws.pstride, (int)gd.x, ws.V, ldv, ws.vstride, nv, h1,
+                                                        hcs, nullptr, 0, ws.t64, ldv, cgs2 ? ws.t64 : vnext,
+                                                        cgs2 ? ldv : ws.vstride, cgs2 ? nullptr : v32, ldv, N,
+                                                        ws.npart, ws.nstride);
                     HIP_CALL(hipGetLastError());
                     if (cgs2) {
-                        HOST_CALL(bdot_part(ws, ws.V, ws.vstride, jj + 1, ws.w64, ldv, N, s));
-                        kb_final_maxpy<<<gg, bs, lds, s>>>(ws.part, ws.pstride, nblk, ws.V, ldv, ws.vstride, jj + 1,
-                                                           h2, ws.hstride, h1, hcs, -1.0, ws.w64, ldv, N, ws.npart,
-                                                           ws.nstride);  // h1 += h2
+                        auto *dots2 = vq == 4 ? kb_mdot<false, 4> : kb_mdot<false, 1>;
+                        dots2<<<gd, 256, ldsw, s>>>(ws.V, ldv, ws.vstride, nv, pp, R, ws.t64, nullptr, ldv, N, ws.rpb,
+                                                    ws.part, ws.pstride, LazyNorm{});
+                        kb_final_maxpy<<<gg, bs, ldsh, s>>>(ws.part, ws.pstride, (int)gd.x, ws.V, ldv, ws.vstride, nv,
+                                                            h2, ws.hstride, h1, hcs, ws.t64, ldv, vnext, ws.vstride,
+                                                            v32, ldv, N, ws.npart, ws.nstride);  // h1 += h2
                         HIP_CALL(hipGetLastError());
                     }
-                    kb_normalize_np<<<gg, bs, 0, s>>>(ws.w64, ldv, ws.npart, ws.nstride, (int)gg.x, h1 + (K + 1), hcs,
-                                                      ws.V + (size_t)(jj + 1) * ldv, ws.vstride,
-                                                      op.A32 ? ws.v32 : nullptr, ldv, N);
-                    HIP_CALL(hipGetLastError());
+                    if (t == c - 1) {
+                        kb_normalize_np<<<gg, bs, 0, s>>>(vnext, ws.vstride, ws.npart, ws.nstride, (int)gg.x,
+                                                          h1 + (K + 1), hcs, v32, ldv, N);
+                        HIP_CALL(hipGetLastError());
+                    }
                 } else {
+                HOST_CALL(op.apply(ws, jj, s));
                 HOST_CALL(bdot(ws, ws.V, ws.vstride, jj + 1, ws.w64, ldv, N, h1, hcs, s));
                 kb_maxpy<<<gg, bs, 0, s>>>(ws.V, ldv, ws.vstride, jj + 1, h1, hcs, -1.0, ws.w64, ldv, N);
                 HIP_CALL(hipGetLastError());
