@@ -67,17 +67,15 @@ int gemv_n_f32a(const float2 *A, long lda, long M, long N, const double2 *x, lon
 int resid_n_f64(const double2 *A, long lda, long M, long N, const double2 *x, long ldx, const double2 *b, long ldb,
                 double2 *r, long ldr, int R, void *ws, hipStream_t s);
 
-// out[r] = sum_i |v_r[i]|^2 (FP64, fixed-order tree); with act: the system
-// stays active while out[r] > thr[r]
-template <typename C2>
-__global__ __launch_bounds__(1024) void kc_norm2(const C2 *__restrict__ v, long ld, int n, double *__restrict__ out,
-                                                 const double *__restrict__ thr, int *__restrict__ act) {
+// out[r] = sum_i |v_r[i]|^2 (FP64, fixed-order tree)
+__global__ __launch_bounds__(1024) void kc_norm2(const double2 *__restrict__ v, long ld, int n,
+                                                 double *__restrict__ out) {
     __shared__ double red[1024];
     const int r = blockIdx.x;
-    const C2 *vr = v + (size_t)r * ld;
+    const double2 *vr = v + (size_t)r * ld;
     double sum = 0;
     for (int i = threadIdx.x; i < n; i += 1024) {
-        const double x = (double)vr[i].x, y = (double)vr[i].y;
+        const double x = vr[i].x, y = vr[i].y;
         sum = fma(x, x, fma(y, y, sum));
     }
     red[threadIdx.x] = sum;
@@ -86,50 +84,146 @@ __global__ __launch_bounds__(1024) void kc_norm2(const C2 *__restrict__ v, long 
         if (threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
         __syncthreads();
     }
-    if (threadIdx.x == 0) {
-        out[r] = red[0];
-        if (act) act[r] = act[r] && red[0] > thr[r];
+    if (threadIdx.x == 0) out[r] = red[0];
+}
+
+// The vector work of a CG step in three launches (a kernel of a few 100 kB
+// takes about 4.7 us from start to end whatever it does, so their number is
+// what counts): kc_q after A p, kc_xs after A^H q, then kc_p.  Norms travel as one
+// partial per workgroup of 256 rows, summed in a fixed order by every workgroup
+// of the kernel that needs them.  PARTS: the product's chunk partials are
+// summed here, in chunk order and in FP32 as its own reduce does; otherwise the
+// product is read from memory.  5 systems of 4412 rows: a step takes 75.5 us, 57
+// of them the products; with reduces, norms and updates as six launches of
+// their own (28 us of kernels) it took 83.
+
+// sum of the nb partials, in every lane of the workgroup (one barrier)
+__device__ __forceinline__ double sum_partials(const double *__restrict__ p, int nb, double *s_sum) {
+    if (threadIdx.x < 64) {
+        double v = 0;
+        for (int b = threadIdx.x; b < nb; b += 64) v += p[b];
+#pragma unroll
+        for (int m = 32; m >= 1; m >>= 1) v += __shfl_xor(v, m, 64);
+        if (threadIdx.x == 0) *s_sum = v;
     }
+    __syncthreads();
+    return *s_sum;
 }
 
-// alpha = gamma / delta: x += alpha p, s -= alpha w (w = A^H q)
-template <typename W2>
-__global__ void kc_upd_xs(int N, const double *__restrict__ gam, const double *__restrict__ del,
-                          const int *__restrict__ act, const double2 *__restrict__ p, double2 *__restrict__ x,
-                          const W2 *__restrict__ w, double2 *__restrict__ sv, long ld) {
-    const int r = blockIdx.y;
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= N) return;
-    const double d = del[r];
+// the workgroup's sum of v to *out (one barrier)
+__device__ __forceinline__ void store_partial(double v, double *s_n, double *out) {
+#pragma unroll
+    for (int m = 32; m >= 1; m >>= 1) v += __shfl_xor(v, m, 64);
+    if ((threadIdx.x & 63) == 0) s_n[threadIdx.x >> 6] = v;
+    __syncthreads();
+    if (threadIdx.x == 0) *out = (s_n[0] + s_n[1]) + (s_n[2] + s_n[3]);
+}
+
+__device__ __forceinline__ float2 sum_parts(const ProdParts &pp, int R, int r, int i) {
+    const float2 *p = pp.p + (size_t)r * pp.ldp + i;
+    const size_t cs = (size_t)R * pp.ldp;
+    float2 w = make_float2(0.f, 0.f);
+    int c = 0;
+    for (; c + 8 <= pp.nch; c += 8) {
+        float2 q[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++) q[u] = p[(size_t)(c + u) * cs];
+#pragma unroll
+        for (int u = 0; u < 8; u++) {
+            w.x += q[u].x;
+            w.y += q[u].y;
+        }
+    }
+    for (; c < pp.nch; c++) {
+        const float2 q = p[(size_t)c * cs];
+        w.x += q.x;
+        w.y += q.y;
+    }
+    return w;
+}
+
+// q = A p (PARTS: formed and stored here), dpart = partials of |q|^2
+template <typename C2, bool PARTS>
+__global__ __launch_bounds__(256) void kc_q(int M, ProdParts pp, C2 *__restrict__ q, long ld,
+                                            double *__restrict__ dpart) {
+    __shared__ double s_n[4];
+    const int r = blockIdx.y, i = blockIdx.x * 256 + threadIdx.x;
+    double nrm = 0;
+    if (i < M) {
+        C2 v;
+        if constexpr (PARTS) {
+            v = sum_parts(pp, gridDim.y, r, i);
+            q[(size_t)r * ld + i] = v;
+        } else {
+            v = q[(size_t)r * ld + i];
+        }
+        nrm = fma((double)v.x, (double)v.x, (double)v.y * (double)v.y);
+    }
+    store_partial(nrm, s_n, dpart + (size_t)r * gridDim.x + blockIdx.x);
+}
+
+// alpha = gamma / |q|^2: x += alpha p, s -= alpha w (w = A^H q), spart = partials
+// of |s|^2
+template <typename C2, bool PARTS>
+__global__ __launch_bounds__(256) void kc_xs(int N, const double *__restrict__ gam, const double *__restrict__ dpart,
+                                             int nbq, const int *__restrict__ act, const double2 *__restrict__ p,
+                                             double2 *__restrict__ x, ProdParts pp, const C2 *__restrict__ w,
+                                             double2 *__restrict__ sv, long ld, double *__restrict__ spart) {
+    __shared__ double s_d, s_n[4];
+    const int r = blockIdx.y, i = blockIdx.x * 256 + threadIdx.x;
+    const size_t o = (size_t)r * ld + i;
+    // loads go out before the sum of the partials is waited for
+    C2 wv = {};
+    double2 pv = make_double2(0, 0), xv = pv, ss = pv;
+    if (i < N) {
+        pv = p[o];
+        xv = x[o];
+        ss = sv[o];
+        if constexpr (PARTS) wv = sum_parts(pp, gridDim.y, r, i);
+        else wv = w[o];
+    }
+    const double d = sum_partials(dpart + (size_t)r * nbq, nbq, &s_d);
     const double a = (act[r] && d > 0) ? gam[r] / d : 0.0;
-    const size_t o = (size_t)r * ld + i;
-    const double2 pv = p[o];
-    double2 xv = x[o];
-    xv.x = fma(a, pv.x, xv.x);
-    xv.y = fma(a, pv.y, xv.y);
-    x[o] = xv;
-    const W2 wv = w[o];
-    double2 ss = sv[o];
-    ss.x = fma(-a, (double)wv.x, ss.x);
-    ss.y = fma(-a, (double)wv.y, ss.y);
-    sv[o] = ss;
+    double nrm = 0;
+    if (i < N) {
+        xv.x = fma(a, pv.x, xv.x);
+        xv.y = fma(a, pv.y, xv.y);
+        x[o] = xv;
+        ss.x = fma(-a, (double)wv.x, ss.x);
+        ss.y = fma(-a, (double)wv.y, ss.y);
+        sv[o] = ss;
+        nrm = fma(ss.x, ss.x, ss.y * ss.y);
+    }
+    store_partial(nrm, s_n, spart + (size_t)r * gridDim.x + blockIdx.x);
 }
 
-// beta = gamma' / gamma: p = s + beta p, p32 = p
-template <typename S2>
-__global__ void kc_upd_p(int N, const double *__restrict__ gnew, const double *__restrict__ gold,
-                         const int *__restrict__ act, const S2 *__restrict__ sv, double2 *__restrict__ p,
-                         float2 *__restrict__ p32, long ld) {
-    const int r = blockIdx.y;
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= N) return;
-    const double go = gold[r];
-    const double b = (act[r] && go > 0) ? gnew[r] / go : 0.0;
+// gamma' = |s|^2, beta = gamma' / gamma: p = s + beta p, p32 = p; the system
+// stays active while gamma' > thr.  gamma and the flag of the next step go to
+// slots of their own: other workgroups still read this step's.
+__global__ __launch_bounds__(256) void kc_p(int N, const double *__restrict__ spart, const double *__restrict__ gold,
+                                            double *__restrict__ gnew, const double *__restrict__ thr,
+                                            const int *__restrict__ act, int *__restrict__ act_new,
+                                            const double2 *__restrict__ sv, double2 *__restrict__ p,
+                                            float2 *__restrict__ p32, long ld) {
+    __shared__ double s_g;
+    const int r = blockIdx.y, i = blockIdx.x * 256 + threadIdx.x;
     const size_t o = (size_t)r * ld + i;
-    const S2 s = sv[o];
-    double2 pv = p[o];
-    pv.x = fma(b, pv.x, (double)s.x);
-    pv.y = fma(b, pv.y, (double)s.y);
+    double2 s = make_double2(0, 0), pv = s;
+    if (i < N) {
+        s = sv[o];
+        pv = p[o];
+    }
+    const double gn = sum_partials(spart + (size_t)r * gridDim.x, gridDim.x, &s_g);
+    const double go = gold[r];
+    const int on = act[r] && gn > thr[r];
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        gnew[r] = gn;
+        act_new[r] = on;
+    }
+    if (i >= N) return;
+    const double b = (on && go > 0) ? gn / go : 0.0;
+    pv.x = fma(b, pv.x, s.x);
+    pv.y = fma(b, pv.y, s.y);
     p[o] = pv;
     if (p32) p32[o] = make_float2((float)pv.x, (float)pv.y);
 }
@@ -474,7 +568,7 @@ struct CglsWS {
     float2 *AH = nullptr;  // conjugate-transposed copy of an FP32 A (null: adjoint products read A)
     char *xsplit = nullptr;   // FP16-split products: planes of the right-hand sides
     float *amaxws = nullptr;  // and the bound on |A|
-    double *gam = nullptr, *del = nullptr, *g0 = nullptr, *thr = nullptr;
+    double *gam = nullptr, *dpart = nullptr, *spart = nullptr, *g0 = nullptr, *thr = nullptr;
     int *act = nullptr, *done = nullptr;
     char *gws = nullptr;
     // block CG: Q, S (QR input / scratch), P, P (next), W = A^H A P, the
@@ -488,7 +582,8 @@ struct CglsWS {
     ~CglsWS() {
         sfree(rr, st); sfree(s64, st); sfree(d, st); sfree(p, st); sfree(q64, st); sfree(w64, st);
         sfree(p32, st); sfree(q32, st); sfree(w32, st); sfree(AH, st); sfree(xsplit, st); sfree(amaxws, st);
-        sfree(gam, st); sfree(del, st); sfree(g0, st); sfree(thr, st); sfree(act, st); sfree(done, st); sfree(gws, st);
+        sfree(gam, st); sfree(dpart, st); sfree(spart, st); sfree(g0, st); sfree(thr, st); sfree(act, st);
+        sfree(done, st); sfree(gws, st);
         sfree(bQ, st); sfree(bS, st); sfree(bP, st); sfree(bP2, st); sfree(bW, st); sfree(bX, st); sfree(bP32, st);
         sfree(gpart, st); sfree(gseg, st); sfree(gsum, st); sfree(dcm, st); sfree(bidx, st);
         if (hgram) {
@@ -530,10 +625,12 @@ int cgls_device(const float2 *A32, const double2 *A64, long lda, int M, int N, c
         HOST_CALL(salloc(&w.w64, nv, s));
     }
     HOST_CALL(salloc(&w.gam, 2 * (size_t)R, s));
-    HOST_CALL(salloc(&w.del, R, s));
+    const int nbq = (M + 255) / 256, nbn = (N + 255) / 256;
+    HOST_CALL(salloc(&w.dpart, (size_t)nbq * R, s));
+    HOST_CALL(salloc(&w.spart, (size_t)nbn * R, s));
     HOST_CALL(salloc(&w.g0, R, s));
     HOST_CALL(salloc(&w.thr, R, s));
-    HOST_CALL(salloc(&w.act, R, s));
+    HOST_CALL(salloc(&w.act, 2 * (size_t)R, s));
     HOST_CALL(salloc(&w.done, R, s));
     HOST_CALL(salloc(&w.gws, std::max(std::max(ws_gemv_n(M, N, 1), ws_gemm(M, N, R)), ws_mres(M, N, R)), s));
     // Block steps pay three dozen small launches, a host wait and the R x R
@@ -612,30 +709,30 @@ int cgls_device(const float2 *A32, const double2 *A64, long lda, int M, int N, c
     };
     std::vector<double> hg(R);
     auto norms = [&](std::vector<double> &out) -> int {
-        kc_norm2<double2><<<R, 1024, 0, s>>>(w.s64, ld, N, w.g0, nullptr, nullptr);
+        kc_norm2<<<R, 1024, 0, s>>>(w.s64, ld, N, w.g0);
         HIP_CALL(hipGetLastError());
         HIP_CALL(hipMemcpyAsync(hg.data(), w.g0, sizeof(double) * R, hipMemcpyDeviceToHost, s));
         HIP_CALL(hipStreamSynchronize(s));
         for (int q = 0; q < R; q++) out[q] = std::sqrt(std::max(0.0, hg[q]));
         return EXIT_SUCCESS;
     };
-    // one operator step of every system: q = A p, s = A^H r
-    auto prod_n = [&]() -> int {
+    // q = A p and w = A^H q of a step; an FP32 product of several systems may be
+    // left as its partials (pp->p set), in w.gws until the next product
+    auto prod_n = [&](ProdParts *pp) -> int {
         if (f32) {
             if (R == 1) HOST_CALL(gemv_n_f32(A32, lda, M, N, w.p32, 0, w.q32, 0, 1, w.gws, s));
-            else HOST_CALL(gemm_n_f32(A32, lda, M, N, w.p32, ld, w.q32, ld, R, w.gws, s, true));
+            else HOST_CALL(gemm_n_f32(A32, lda, M, N, w.p32, ld, w.q32, ld, R, w.gws, s, true, pp));
         } else {
             if (R == 1) HOST_CALL(gemv_n_f64(A64, lda, M, N, w.p, 0, w.q64, 0, 1, w.gws, s));
             else HOST_CALL(mres_f64(A64, lda, M, N, w.p, ld, nullptr, 0, w.q64, ld, R, w.gws, s));
         }
         return EXIT_SUCCESS;
     };
-    // w = A^H q
-    auto prod_h = [&]() -> int {
+    auto prod_h = [&](ProdParts *pp) -> int {
         if (f32) {
             if (R == 1) HOST_CALL(gemv_h_f32(A32, lda, M, N, w.q32, 0, w.w32, 0, 1, s));
-            else if (w.AH) HOST_CALL(gemm_hc_f32(w.AH, M, N, w.q32, ld, w.w32, ld, R, w.gws, s));
-            else HOST_CALL(gemm_h_f32(A32, lda, M, N, w.q32, ld, w.w32, ld, R, w.gws, s, true));
+            else if (w.AH) HOST_CALL(gemm_hc_f32(w.AH, M, N, w.q32, ld, w.w32, ld, R, w.gws, s, pp));
+            else HOST_CALL(gemm_h_f32(A32, lda, M, N, w.q32, ld, w.w32, ld, R, w.gws, s, true, pp));
         } else {
             if (R == 1) HOST_CALL(gemv_h_f64(A64, lda, M, N, w.q64, 0, w.w64, 0, 1, s));
             else HOST_CALL(mh_f64(A64, lda, M, N, w.q64, ld, w.w64, ld, R, s));
@@ -648,15 +745,25 @@ int cgls_device(const float2 *A32, const double2 *A64, long lda, int M, int N, c
         for (int it = 0; it < n; it++) {
             const int cur = it & 1;
             double *gc = w.gam + (size_t)cur * R, *gn = w.gam + (size_t)(1 - cur) * R;
-            HOST_CALL(prod_n());
-            if (f32) kc_norm2<float2><<<R, 1024, 0, s>>>(w.q32, ld, M, w.del, nullptr, nullptr);
-            else kc_norm2<double2><<<R, 1024, 0, s>>>(w.q64, ld, M, w.del, nullptr, nullptr);
+            int *ac = w.act + (size_t)cur * R, *an = w.act + (size_t)(1 - cur) * R;
+            const dim3 gq(nbq, R), gx(nbn, R);
+            ProdParts pq, pw;
+            HOST_CALL(prod_n(&pq));
+            if (pq.p) kc_q<float2, true><<<gq, bs, 0, s>>>(M, pq, w.q32, ld, w.dpart);
+            else if (f32) kc_q<float2, false><<<gq, bs, 0, s>>>(M, pq, w.q32, ld, w.dpart);
+            else kc_q<double2, false><<<gq, bs, 0, s>>>(M, pq, w.q64, ld, w.dpart);
             HIP_CALL(hipGetLastError());
-            HOST_CALL(prod_h());
-            if (f32) kc_upd_xs<float2><<<gN, bs, 0, s>>>(N, gc, w.del, w.act, w.p, w.d, w.w32, w.s64, ld);
-            else kc_upd_xs<double2><<<gN, bs, 0, s>>>(N, gc, w.del, w.act, w.p, w.d, w.w64, w.s64, ld);
-            kc_norm2<double2><<<R, 1024, 0, s>>>(w.s64, ld, N, gn, w.thr, w.act);
-            kc_upd_p<double2><<<gN, bs, 0, s>>>(N, gn, gc, w.act, w.s64, w.p, f32 ? w.p32 : nullptr, ld);
+            HOST_CALL(prod_h(&pw));
+            if (pw.p)
+                kc_xs<float2, true><<<gx, bs, 0, s>>>(N, gc, w.dpart, nbq, ac, w.p, w.d, pw, nullptr, w.s64, ld,
+                                                      w.spart);
+            else if (f32)
+                kc_xs<float2, false><<<gx, bs, 0, s>>>(N, gc, w.dpart, nbq, ac, w.p, w.d, pw, w.w32, w.s64, ld,
+                                                       w.spart);
+            else
+                kc_xs<double2, false><<<gx, bs, 0, s>>>(N, gc, w.dpart, nbq, ac, w.p, w.d, pw, w.w64, w.s64, ld,
+                                                        w.spart);
+            kc_p<<<gx, bs, 0, s>>>(N, w.spart, gc, gn, w.thr, ac, an, w.s64, w.p, f32 ? w.p32 : nullptr, ld);
             HIP_CALL(hipGetLastError());
         }
         return EXIT_SUCCESS;
