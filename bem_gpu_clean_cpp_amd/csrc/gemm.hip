@@ -1555,81 +1555,118 @@ void product_tune_clear() {
 }
 
 // ------------------------------------------------ QR rank-nb update ---
-// C (M x nc, ldc) -= V (M x 32, ldv) W, W stored per column of C (W[c * ldw + l],
-// l < 32; columns l >= nb of V and rows l >= nb of W are zero).  The
-// trailing update of the blocked Householder QR: wave tile 32 complex rows x
-// (16 G) columns of C, K = 32; no split-K (K is one panel), C updated in place.
-template <int G>
-__global__ __launch_bounds__(256) void rank_update_mfma(const float2 *__restrict__ V, long ldv, int M,
-                                                        const float2 *__restrict__ W, int ldw, int nc,
-                                                        float2 *__restrict__ Cm, long ldc) {
+// C (M x nc, ldc) -= V (M x 32, ldv) W with W = T^H (V^H C), from the chunk
+// partials of Z = C^H V (the adjoint product, 32 right-hand sides) and the upper
+// triangular T (row-major 32 x 32, zero past nb; columns l >= nb of V are zero).
+// A workgroup takes 128 rows x 32 columns: it sums Z of its columns and forms
+// their W in shared memory while its C and V are on their way, then the product
+// on MFMA (wave: 32 rows, K = 32).  W is the operand of the result's rows, so
+// that 16 lanes hold 16 consecutive rows of a column of C and loads and stores
+// are 128-byte segments.  Bound by latency: 11 us at 642 nodes, where reduce,
+// W and the update as launches of their own took 25.
+__global__ __launch_bounds__(256) void qr_trail(const float2 *__restrict__ V, long ldv, int M,
+                                                const float2 *__restrict__ T, int nb, ProdParts zp, int nc,
+                                                float2 *__restrict__ C, long ldc) {
     typedef MF<float>::v4 v4;
+    __shared__ float2 s_z[32][33], s_t[32][33], s_w[32][33];  // Z[q][c], T[q][l], W[c][l]
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int row0 = (blockIdx.x * 4 + wave) * 32;
-    if (row0 >= M) return;
-    const int c0 = blockIdx.y * 16 * G;
     const int m = lane & 15, kk = lane >> 4;
-    v4 acc[G][2][4];
+    const int row0 = (blockIdx.x * 4 + wave) * 32, c0 = blockIdx.y * 32;
+    // rows past M and columns past nc read the last ones and are not stored
+    float2 v[8][2], cv[2][2][4];
 #pragma unroll
-    for (int g = 0; g < G; g++)
+    for (int h = 0; h < 2; h++) {
+        const int i = min(row0 + 16 * h + m, M - 1);
 #pragma unroll
-        for (int p = 0; p < 2; p++)
+        for (int u = 0; u < 8; u++) v[u][h] = V[(size_t)(4 * u + kk) * ldv + i];
 #pragma unroll
-            for (int t = 0; t < 4; t++) acc[g][p][t] = (v4){0, 0, 0, 0};
-    const float4 *Vb = reinterpret_cast<const float4 *>(V + row0 + 2 * m);
-    const long ldv4 = ldv / 2;
-    const float2 *Wg[G];
+        for (int g = 0; g < 2; g++)
 #pragma unroll
-    for (int g = 0; g < G; g++) Wg[g] = W + (size_t)min(c0 + g * 16 + m, nc - 1) * ldw;
-    float4 a[8];
-    float2 w[8][G];
+            for (int q = 0; q < 4; q++)
+                cv[h][g][q] = C[(size_t)min(c0 + 16 * g + MF<float>::drow(kk, q), nc - 1) * ldc + i];
+    }
+    const int tc = threadIdx.x & 31, tq = threadIdx.x >> 5;
+    const int cc = min(c0 + tc, nc - 1);
 #pragma unroll
-    for (int u = 0; u < 8; u++) {
-        const int L = 4 * u + kk;
-        a[u] = Vb[(size_t)L * ldv4];
+    for (int u = 0; u < 4; u++) s_t[tq + 8 * u][tc] = T[(tq + 8 * u) * 32 + tc];
+    float zr[4] = {0, 0, 0, 0}, zi[4] = {0, 0, 0, 0};
+    // 8 chunks in flight, added in chunk order
+    for (int k0 = 0; k0 < zp.nch; k0 += 8) {
+        float2 z[8][4];
 #pragma unroll
-        for (int g = 0; g < G; g++) w[u][g] = Wg[g][L];
+        for (int h = 0; h < 8; h++)
+#pragma unroll
+            for (int u = 0; u < 4; u++)
+                z[h][u] = zp.p[((size_t)min(k0 + h, zp.nch - 1) * 32 + tq + 8 * u) * zp.ldp + cc];
+#pragma unroll
+        for (int h = 0; h < 8; h++)
+            if (k0 + h < zp.nch)
+#pragma unroll
+                for (int u = 0; u < 4; u++) {
+                    zr[u] += z[h][u].x;
+                    zi[u] += z[h][u].y;
+                }
     }
 #pragma unroll
-    for (int u = 0; u < 8; u++) {
-        const float av[4] = {a[u].x, a[u].y, a[u].z, a[u].w};
+    for (int u = 0; u < 4; u++) s_z[tq + 8 * u][tc] = make_float2(zr[u], zi[u]);
+    __syncthreads();
+    // W[c][l] = conj(sum_{q <= l} T[q][l] Z[q][c])
 #pragma unroll
-        for (int g = 0; g < G; g++)
-#pragma unroll
-            for (int t = 0; t < 4; t++) {
-                acc[g][0][t] = MF<float>::mma(av[t], w[u][g].x, acc[g][0][t]);
-                acc[g][1][t] = MF<float>::mma(av[t], w[u][g].y, acc[g][1][t]);
-            }
+    for (int u = 0; u < 4; u++) {
+        const int l = tq + 8 * u;
+        float sr = 0, si = 0;
+        for (int q = 0; q <= l; q++) {
+            const float2 t = s_t[q][l], z = s_z[q][tc];
+            sr = fmaf(t.x, z.x, fmaf(-t.y, z.y, sr));
+            si = fmaf(t.x, z.y, fmaf(t.y, z.x, si));
+        }
+        s_w[tc][l] = l < nb ? make_float2(sr, -si) : make_float2(0.f, 0.f);
     }
+    __syncthreads();
+    v4 ar[2][2], ai[2][2];
 #pragma unroll
-    for (int g = 0; g < G; g++) {
-        const int n = c0 + g * 16 + m;
-        if (n >= nc) continue;
-        float2 *cc = Cm + (size_t)n * ldc;
+    for (int h = 0; h < 2; h++)
 #pragma unroll
-        for (int v = 0; v < 4; v++) {
-            const int mp = MF<float>::drow(kk, v);
+        for (int g = 0; g < 2; g++) {
+            ar[h][g] = (v4){0, 0, 0, 0};
+            ai[h][g] = (v4){0, 0, 0, 0};
+        }
+#pragma unroll
+    for (int u = 0; u < 8; u++)
+#pragma unroll
+        for (int g = 0; g < 2; g++) {
+            const float2 w = s_w[16 * g + m][4 * u + kk];
 #pragma unroll
             for (int h = 0; h < 2; h++) {
-                const int i = row0 + 2 * mp + h;
-                if (i < M) {
-                    float2 o = cc[i];
-                    o.x -= acc[g][0][2 * h][v] - acc[g][1][2 * h + 1][v];
-                    o.y -= acc[g][0][2 * h + 1][v] + acc[g][1][2 * h][v];
-                    cc[i] = o;
-                }
+                ar[h][g] = MF<float>::mma(w.x, v[u][h].x, ar[h][g]);
+                ar[h][g] = MF<float>::mma(-w.y, v[u][h].y, ar[h][g]);
+                ai[h][g] = MF<float>::mma(w.x, v[u][h].y, ai[h][g]);
+                ai[h][g] = MF<float>::mma(w.y, v[u][h].x, ai[h][g]);
             }
         }
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+        const int i = row0 + 16 * h + m;
+        if (i >= M) continue;
+#pragma unroll
+        for (int g = 0; g < 2; g++)
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const int n = c0 + 16 * g + MF<float>::drow(kk, q);
+                if (n < nc)
+                    C[(size_t)n * ldc + i] =
+                        make_float2(cv[h][g][q].x - ar[h][g][q], cv[h][g][q].y - ai[h][g][q]);
+            }
     }
 }
 
-// C -= V W as above; V needs 32 columns and ldv >= roundup(M, 32), even
-int rank_update_f32(const float2 *V, long ldv, int M, const float2 *W, int ldw, int nc, float2 *C, long ldc,
-                    hipStream_t s) {
+int qr_trail_f32(const float2 *V, long ldv, int M, const float2 *T, int nb, const ProdParts &zp, int nc, float2 *C,
+                 long ldc, hipStream_t s) {
     if (M <= 0 || nc <= 0) return EXIT_SUCCESS;
-    if (ldv % 2 || ldv < (M + 31) / 32 * 32) BEM_FAIL("rank_update needs an even ldv >= roundup(M, 32)");
-    dim3 grid((unsigned)((M + 127) / 128), (unsigned)((nc + 31) / 32));
-    rank_update_mfma<2><<<grid, 256, 0, s>>>(V, ldv, M, W, ldw, nc, C, ldc);
+    if (ldv < M || ldc < M || !zp.p || zp.ldp < nc) BEM_FAIL("qr_trail: leading dimensions below the sizes");
+    const dim3 grid((unsigned)((M + 127) / 128), (unsigned)((nc + 31) / 32));
+    if (grid.y > 65535) BEM_FAIL("qr_trail: %d columns are too many", nc);
+    qr_trail<<<grid, 256, 0, s>>>(V, ldv, M, T, nb, zp, nc, C, ldc);
     HIP_CALL(hipGetLastError());
     return EXIT_SUCCESS;
 }

@@ -11,9 +11,10 @@
 //   qr_vhc      W = T^H (V^H C) for the trailing columns C (one workgroup per
 //               column, the nb dot products in one pass over the column);
 //   qr_update   C -= V W (the rank-nb trailing update, GEMM-shaped);
-//   FP32 trailing updates run on MFMA instead: V^H C as the adjoint product
-//               (C^H V, gemm.hip) against an explicit copy of the panel's V,
-//               W = T^H (V^H C), then C -= V W with the rank-32 MFMA update;
+//   FP32 panels are formed from their Gram matrix instead (qr_gram, qr_recon,
+//               qr_form_v), and FP32 trailing updates run on MFMA: V^H C as the
+//               adjoint product (C^H V, gemm.hip) against an explicit copy of
+//               the panel's V, then W = T^H (V^H C) and C -= V W in one launch;
 //   trsv_upper  R x = (Q^H b)[0:N] by column-oriented back substitution.
 #include <hip/hip_runtime.h>
 
@@ -38,7 +39,6 @@ struct QT<double> {
 
 constexpr int kNB = 32;  // panel width
 constexpr int kCG = 8;   // panel columns updated together
-constexpr int kColThreads = 256;  // rows per workgroup of the tall-panel column launches
 
 template <typename T>
 __device__ __forceinline__ T wsum(T v) {
@@ -63,14 +63,15 @@ __device__ __forceinline__ C2 vget(const C2 *A, long lda, int j0, int l, int i) 
     return z;
 }
 
+// (at most 1024 threads, all of the workgroup; shared arrays of the caller)
 template <typename T>
-__global__ __launch_bounds__(1024) void qr_panel(typename QT<T>::c2 *A, long lda, int M, int j0, int nb,
-                                                 typename QT<T>::c2 *Tout /* nb x nb, ld kNB */, int make_t) {
+__device__ __forceinline__ void panel_one_wg(typename QT<T>::c2 *A, long lda, int M, int j0, int nb,
+                             typename QT<T>::c2 *Tout /* nb x nb, ld kNB */, int make_t,
+                             typename QT<T>::c2 (*s_Y)[kNB] /* v_l^H v_m for l < m */,
+                             typename QT<T>::c2 (*s_T)[kNB]) {
     using C2 = typename QT<T>::c2;
     __shared__ T red[2][16];
     __shared__ T s_tau[kNB];
-    __shared__ C2 s_Y[kNB][kNB];  // v_l^H v_m for l < m
-    __shared__ C2 s_T[kNB][kNB];
     __shared__ T s_red[16][2 * kCG];
     __shared__ T s_d[2 * kCG];
     const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6, nw = blockDim.x >> 6;
@@ -234,6 +235,13 @@ __global__ __launch_bounds__(1024) void qr_panel(typename QT<T>::c2 *A, long lda
     for (int p = tid; p < kNB * kNB; p += blockDim.x) Tout[p] = s_T[p / kNB][p % kNB];
 }
 
+template <typename T>
+__global__ __launch_bounds__(1024) void qr_panel(typename QT<T>::c2 *A, long lda, int M, int j0, int nb,
+                                                 typename QT<T>::c2 *Tout, int make_t) {
+    __shared__ typename QT<T>::c2 s_Y[kNB][kNB], s_T[kNB][kNB];
+    panel_one_wg<T>(A, lda, M, j0, nb, Tout, make_t, s_Y, s_T);
+}
+
 // Sum of 2 kNB = 64 per-lane values over the wave, scattered: on return lane
 // l holds the wave total of slot l in x[0].  Each halving step sends one half
 // of the live slots to the partner lane and keeps the other half (the half
@@ -302,307 +310,373 @@ __device__ __forceinline__ void wave_reduce_scatter64<float>(float (&x)[2 * kNB]
     reduce_scatter_dpp<1, 0xB1>(x, lane);   // quad_perm [1,0,3,2]
 }
 
-// Panel of exactly kNB columns and at most NT * RPT rows (rows j0..M-1) with
-// the panel in registers: thread t holds rows j0 + t + NT q (q < RPT) of all
-// kNB columns, so a column step costs three barriers and no memory traffic.
-// The column loop is unrolled so every register index is static.
+// FP32 panels in three launches instead of one step per column.  The panel P
+// (rows j0..M-1, nb <= 32 columns) gets the same compact WY form as from
+// reflectors, by way of its Gram matrix:
+//   qr_gram    partials of G = P^H P in FP64 (exact products of FP32 numbers);
+//   qr_recon   one workgroup: Cholesky G = R^H R, then the reflectors from R
+//              and the top rows P_1 alone (Householder reconstruction: Ballard,
+//              Demmel, Grigori, Jacquelin, Nguyen & Solomonik 2014): P_1 - S R =
+//              L U with unit diagonal phases S chosen against cancellation as
+//              the elimination goes, s_k = -phase(pivot), so |U_kk| >= R_kk and
+//              no pivoting is needed.  Then V = [L; P_2 U^-1], R_h = S R and
+//              T = -U R_h^-1 L^-H, with Q^H P = [R_h; 0] for
+//              Q = I - V T V^H: the phases and tau of the column-wise algorithm;
+//   qr_form_v  the rows P_2 U^-1 of V, and V with its unit diagonal and zeros.
+// All in FP64, with V, R and T rounded to FP32 once.  The loss of orthogonality
+// is about 1e-18 kappa^2 (kappa: condition number of the panel with columns
+// scaled to norm 1), so panels of kappa^2 > 1e9, those whose Gram matrix is not
+// numerically positive definite (dependent or zero columns, numbers that are
+// not finite) and those with a column that needs no reflection take the
+// column-wise algorithm inside qr_recon instead.
 //
-// Column step jj (j = j0 + jj): the norm below the diagonal (wave sums ->
-// s_nrm) gives the reflector; then one scattered wave reduction forms
-// sum_r conj(v(r)) a_c(r) for every other column c (-> s_red, summed over the
-// waves by 2 kNB threads -> s_fin).  For c > jj that is v^H a_c, which with
-// tau updates a_c.  For c < jj the column holds v_c, exact on every row where
-// v is nonzero (r >= j > j0 + c), so the sum is conj(v_c^H v); those give
-// column jj of U = diag(1/tau) + the strictly upper part of V^H V, and after
-// the last column T = U^-1 (H_1 ... H_kNB = I - V T V^H; Schreiber & Van Loan
-// 1989, Joffrain et al. 2006).  Each shared array is written only after a
-// barrier that follows its last read, so three barriers per column suffice.
-//
-// Writes the Householder vectors and R back in place, T to Tout (kNB x kNB,
-// row-major, zero below the diagonal) and the explicit V (unit diagonal, zero
-// above it) to Vd[l * ldv + (i - j0)] for rows i = j0..M-1.
-template <int NT, int RPT>
-__global__ __launch_bounds__(NT) void qr_panel_reg(float2 *A, long lda, int M, int j0, float2 *Tout, float2 *Vd,
-                                                   long ldv) {
-    constexpr int NW = NT / 64;
-    __shared__ float s_nrm[NW];
-    __shared__ float s_red[NW][2 * kNB];
-    __shared__ float2 s_fin[kNB];
-    __shared__ float2 s_U[kNB][kNB];  // strictly upper part of V^H V (row q, column m)
-    __shared__ float s_tau[kNB];
-    __shared__ float s_bc[2];
-    const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
-    float2 a[RPT][kNB];
+// 5 + 36 + 5 us a panel of up to 2000 rows.  The column-wise panels that this
+// replaces were bound by their 32 serial steps: 69 us (256 rows), 98 (512) and
+// 135 (1024) with the panel in one workgroup's registers, 330 + 40 us with a
+// launch per column above.  With qr_trail, a QR solve of 642 nodes went from
+// 4.1 to 2.8 ms, 1962: 22.1 to 9.1, 10242: 317 to 150.
+constexpr int kNN = kNB * kNB;
+// rows up to which the trailing update sums the partials of C^H V itself (each
+// 128 rows of it sum them again): QR solve of 4002 nodes 23.9-24.3 ms for 0 to
+// 2048, 26.4 always; 10242 nodes 150 ms, 175 always; below 2000 nodes within 2 %
+constexpr int kTrailRows = 1024;
+constexpr int kGramChunk = 64;      // rows of a panel staged at a time
+constexpr int kGramParts = 16;      // at most this many partials (one workgroup sums them)
+constexpr double kPanelCond2 = 1e9;
+
+// part[blk][i][j] = sum over the block's rpb rows (a multiple of kGramChunk) of
+// conj(P_i) P_j, zero past nb, on FP64 MFMA in the three-product form; wave w
+// takes the 16 x 16 tile (w % 2, w / 2).  Pc receives a copy of the panel
+// (qr_form_v writes V over the panel while it reads P).
+__global__ __launch_bounds__(256) void qr_gram(const float2 *__restrict__ A, long lda, int M, int j0, int nb, int rpb,
+                                               double2 *__restrict__ part, float2 *__restrict__ Pc, long ldv) {
+    typedef double v4d __attribute__((ext_vector_type(4)));
+    __shared__ float2 s_p[kNB][kGramChunk + 1];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int m = lane & 15, kk = lane >> 4;
+    const int a0 = 16 * (wave & 1), b0 = 16 * (wave >> 1);
+    v4d acc[3];
 #pragma unroll
-    for (int q = 0; q < RPT; q++) {
-        const int r = j0 + tid + NT * q;
+    for (int q = 0; q < 3; q++) acc[q] = (v4d){0, 0, 0, 0};
+    for (int r0 = 0; r0 < rpb; r0 += kGramChunk) {
+        const int i = blockIdx.x * rpb + r0 + lane;  // row of the panel
+        float2 v[kNB / 4];
 #pragma unroll
-        for (int c = 0; c < kNB; c++) a[q][c] = r < M ? A[(size_t)(j0 + c) * lda + r] : make_float2(0.f, 0.f);
-    }
-#pragma clang loop unroll(full)
-    for (int jj = 0; jj < kNB; jj++) {
-        const int j = j0 + jj;
-        // |x|^2 over rows > j, and alpha = A[j, j] to everyone
-        float sq = 0.f;
-#pragma unroll
-        for (int q = 0; q < RPT; q++) {
-            const int r = j0 + tid + NT * q;
-            if (r > j && r < M) sq += a[q][jj].x * a[q][jj].x + a[q][jj].y * a[q][jj].y;
-            if (r == j) {
-                s_bc[0] = a[q][jj].x;
-                s_bc[1] = a[q][jj].y;
-            }
+        for (int u = 0; u < kNB / 4; u++) {
+            const int c = wave + 4 * u;
+            v[u] = make_float2(0.f, 0.f);
+            if (j0 + i < M && c < nb) v[u] = A[(size_t)(j0 + c) * lda + j0 + i];
         }
-        sq = wsum(sq);
-        if (lane == 0) s_nrm[wid] = sq;
+        __syncthreads();  // the previous rows are read
+#pragma unroll
+        for (int u = 0; u < kNB / 4; u++) {
+            const int c = wave + 4 * u;
+            s_p[c][lane] = v[u];
+            if (j0 + i < M) Pc[(size_t)c * ldv + i] = v[u];
+        }
         __syncthreads();
-        float tot = 0.f;
-#pragma unroll
-        for (int w = 0; w < NW; w++) tot += s_nrm[w];
-        const float2 alpha = make_float2(s_bc[0], s_bc[1]);
-        const float aa = sqrtf(alpha.x * alpha.x + alpha.y * alpha.y);
-        const float xnorm = sqrtf(aa * aa + tot);
-        float tau = 0.f;
-        float2 scale = make_float2(0.f, 0.f), beta = alpha;
-        if (tot > 0 || (xnorm > 0 && alpha.y != 0)) {
-            const float phr = aa > 0 ? alpha.x / aa : 1.f, phi = aa > 0 ? alpha.y / aa : 0.f;
-            beta = make_float2(-phr * xnorm, -phi * xnorm);
-            const float dr = alpha.x - beta.x, di = alpha.y - beta.y;
-            const float dd = dr * dr + di * di;
-            scale = make_float2(dr / dd, -di / dd);
-            tau = 2.f / (1.f + tot / dd);
-        }
-        // v = x / (alpha - beta) below the diagonal (v_j = 1, zero above);
-        // R[j, j] = beta
-        float2 v[RPT];
-#pragma unroll
-        for (int q = 0; q < RPT; q++) {
-            const int r = j0 + tid + NT * q;
-            if (r > j && r < M) {
-                const float2 x = a[q][jj];
-                a[q][jj] = make_float2(x.x * scale.x - x.y * scale.y, x.x * scale.y + x.y * scale.x);
-                v[q] = a[q][jj];
-            } else {
-                if (r == j) a[q][jj] = beta;
-                v[q] = make_float2(r == j ? 1.f : 0.f, 0.f);
-            }
-        }
-        {
-            // slots 2c, 2c + 1: sum_r conj(v(r)) a_c(r) for c != jj (slot pair
-            // jj zero), one scattered wave reduction for all of them
-            float x[2 * kNB];
-#pragma unroll
-            for (int c = 0; c < kNB; c++) {
-                float pr = 0.f, pi = 0.f;
-                if (c != jj) {
-#pragma unroll
-                    for (int q = 0; q < RPT; q++) {
-                        pr += v[q].x * a[q][c].x + v[q].y * a[q][c].y;
-                        pi += v[q].x * a[q][c].y - v[q].y * a[q][c].x;
-                    }
-                }
-                x[2 * c] = pr;
-                x[2 * c + 1] = pi;
-            }
-            wave_reduce_scatter64(x, lane);
-            s_red[wid][lane] = x[0];
-            __syncthreads();
-            if (tid < 2 * kNB) {
-                float t = 0.f;
-#pragma unroll
-                for (int w = 0; w < NW; w++) t += s_red[w][tid];
-                ((float *)s_fin)[tid] = (tid >> 1) > jj ? t * tau : t;
-            }
-            __syncthreads();
-#pragma unroll
-            for (int c = jj + 1; c < kNB; c++) {
-                const float2 e = s_fin[c];
-#pragma unroll
-                for (int q = 0; q < RPT; q++) {
-                    a[q][c].x -= e.x * v[q].x - e.y * v[q].y;
-                    a[q][c].y -= e.x * v[q].y + e.y * v[q].x;
-                }
-                if ((c & 3) == 3) __builtin_amdgcn_sched_barrier(0);
-            }
-            // column jj of U: v_q^H v = conj(s_fin[q]) for q < jj
-            if (tid < jj) {
-                s_U[tid][jj] = make_float2(s_fin[tid].x, -s_fin[tid].y);
-            } else if (tid == jj) {
-                s_tau[jj] = tau;
-            }
+#pragma unroll 4
+        for (int r = 0; r < kGramChunk; r += 4) {
+            const float2 x = s_p[a0 + m][r + kk], y = s_p[b0 + m][r + kk];
+            const double ur = x.x, ui = -(double)x.y, vr = y.x, vi = y.y;
+            acc[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(ur, vr + vi, acc[0], 0, 0, 0);
+            acc[1] = __builtin_amdgcn_mfma_f64_16x16x4f64(ur + ui, vi, acc[1], 0, 0, 0);
+            acc[2] = __builtin_amdgcn_mfma_f64_16x16x4f64(ui - ur, vr, acc[2], 0, 0, 0);
         }
     }
+    double2 *pb = part + (size_t)blockIdx.x * kNN;
 #pragma unroll
-    for (int q = 0; q < RPT; q++) {
-        const int r = j0 + tid + NT * q;
-        if (r < M) {
+    for (int v = 0; v < 4; v++)
+        pb[(a0 + kk + 4 * v) * kNB + b0 + m] = make_double2(acc[0][v] - acc[1][v], acc[0][v] + acc[2][v]);
+}
+
+// 1 / x and 1 / sqrt(x): the hardware's estimates (relative error 2^-23) and one
+// third-order step
+__device__ __forceinline__ double rcp_step(double x) {
+    const double y = __builtin_amdgcn_rcp(x), e = fma(-x, y, 1.0);
+    return fma(y, fma(e, e, e), y);
+}
+__device__ __forceinline__ double rsq_step(double x) {
+    const double y = __builtin_amdgcn_rsq(x), e = fma(-x * y, y, 1.0);
+    return fma(y * e, fma(0.375, e, 0.5), y);
+}
+__device__ __forceinline__ double2 zmul(double2 a, double2 b) {
+    return make_double2(fma(a.x, b.x, -a.y * b.y), fma(a.x, b.y, a.y * b.x));
+}
+__device__ __forceinline__ double2 zfms(double2 c, double2 a, double2 b) {  // c - a b
+    return make_double2(fma(-a.x, b.x, fma(a.y, b.y, c.x)), fma(-a.x, b.y, fma(-a.y, b.x, c.y)));
+}
+
+// The reflectors of a panel from the partials of its Gram matrix: R (above and
+// on the diagonal) and L (below it) to the top rows of the panel, T to Tout,
+// the top rows of V to Vd, U^-1 to Y (row-major), *bad = 0.  Panels that the
+// reconstruction does not take (above) are factored column by column instead,
+// with T, and *bad = 1.
+//
+// One workgroup; thread t holds the entries (i, j), i = t / 32 + kRowStep e,
+// j = t % 32, of two matrices that are eliminated in place and in step: G and
+// P_1 - S R.  Step k needs row k of R only, which is row k of G's elimination
+// scaled, so both take one barrier a step: the rows and columns k of both as
+// they stand go through shared memory, and every thread finishes the pivots for
+// itself.  The update is one multiply-add per entry without a condition: the
+// pivot entry of a published row is 1 and that of a column -1, and the
+// publishing threads clear the entries that start anew (inverse of row and
+// column k).  Afterwards G holds U0^-1 (j >= i), and P_1 - S R holds U^-1
+// (j >= i) and L^-1 (j < i); U0, U and L follow from the published rows and
+// columns.  36 us, bound by the 32 steps (0.8 us each: the FP64 chain of the
+// pivots, two rounds through shared memory, a barrier); 256 threads 41 us, 1024
+// 37; the two eliminations one after the other 45.  (Entries are separate
+// doubles: branches on whole entries, or a select of their addresses, put them
+// in scratch memory: 93 us.)
+// R_kk = d rd from the pivot d of G, and for the pivot p of the top rows
+// s = -phase(p) and 1 / (p - s R_kk) = -conj(s) / (|p| + R_kk)
+struct PanelPivot {
+    double rd;
+    double2 s, inv;
+    __device__ __forceinline__ PanelPivot(double d, double2 p) {
+        rd = rsq_step(d);
+        const double aa = fma(p.x, p.x, p.y * p.y), y = rsq_step(aa);
+        s = make_double2(aa > 0 ? -p.x * y : -1.0, aa > 0 ? -p.y * y : 0.0);
+        const double q = rcp_step(fma(d, rd, aa > 0 ? aa * y : 0.0));
+        inv = make_double2(-s.x * q, s.y * q);
+    }
+};
+constexpr int kRecThreads = 512;
+constexpr int kRowStep = kRecThreads / kNB, kEnt = kNN / kRecThreads;
+__global__ __launch_bounds__(kRecThreads) void qr_recon(const double2 *__restrict__ part, int nblk, float2 *A, long lda,
+                                                        int M, int j0, int nb, float2 *__restrict__ Tout,
+                                                        float2 *__restrict__ Vd, long ldv, double2 *__restrict__ Y,
+                                                        int *__restrict__ bad) {
+    __shared__ double2 s_ra[kNB][kNB + 1], s_rb[kNB][kNB + 1], s_cb[kNB][kNB + 1];  // published rows, columns
+    __shared__ double2 s_ca[2][kNB];
+    __shared__ double2 s_pb[kNB], s_sign[kNB], s_u[kNB], s_inv[kNB];
+    __shared__ double s_pa[kNB], s_g[kNB], s_w[kRecThreads / 64];
+    __shared__ int s_flat;
+    const int tid = threadIdx.x, i0 = tid >> 5, j = tid & 31;
+    const int Mp = M - j0;
+    double gx[kEnt], gy[kEnt], wx[kEnt], wy[kEnt];  // entries of G and of P_1 - S R
+    {
+        double2 v[kEnt][kGramParts];
 #pragma unroll
-            for (int c = 0; c < kNB; c++) {
-                A[(size_t)(j0 + c) * lda + r] = a[q][c];
-                const int d = j0 + c;
-                Vd[(size_t)c * ldv + (r - j0)] = r > d ? a[q][c] : make_float2(r == d ? 1.f : 0.f, 0.f);
+        for (int e = 0; e < kEnt; e++)
+#pragma unroll
+            for (int b = 0; b < kGramParts; b++)
+                v[e][b] = part[(size_t)min(b, nblk - 1) * kNN + tid + kRecThreads * e];
+#pragma unroll
+        for (int e = 0; e < kEnt; e++) {
+            const int i = i0 + kRowStep * e;
+            float2 top = make_float2(0.f, 0.f);
+            if (i < Mp && j < nb) top = A[(size_t)(j0 + j) * lda + j0 + i];
+            wx[e] = top.x;
+            wy[e] = top.y;
+            double x = 0, y = 0;
+#pragma unroll
+            for (int b = 0; b < kGramParts; b++) {
+                x += b < nblk ? v[e][b].x : 0.0;
+                y += b < nblk ? v[e][b].y : 0.0;
             }
+            const bool in = i < nb && j < nb;
+            gx[e] = in ? x : i == j ? 1.0 : 0.0;
+            gy[e] = in ? y : 0.0;
+            if (i == j) s_g[i] = gx[e];  // |P_i|^2
+        }
+    }
+    if (tid == 0) s_flat = 0;
+    for (int k = 0; k < kNB; k++) {
+        const int b = k & 1;
+#pragma unroll
+        for (int e = 0; e < kEnt; e++) {
+            const int i = i0 + kRowStep * e;
+            const bool at = j == k;
+            if (i == k) {
+                s_ra[k][j] = make_double2(at ? 1.0 : j > k ? gx[e] : 0.0, j > k ? gy[e] : 0.0);
+                s_rb[k][j] = make_double2(at ? 1.0 : wx[e], at ? 0.0 : wy[e]);
+            }
+            if (at) {
+                s_ca[b][i] = make_double2(i == k ? -1.0 : gx[e], i == k ? 0.0 : gy[e]);
+                s_cb[k][i] = make_double2(i == k ? -1.0 : wx[e], i == k ? 0.0 : wy[e]);
+                if (i == k) {
+                    s_pa[k] = gx[e];
+                    s_pb[k] = make_double2(wx[e], wy[e]);
+                }
+            }
+            const bool fresh = at || (i == k && j > k);
+            gx[e] = fresh ? 0.0 : gx[e];
+            gy[e] = fresh ? 0.0 : gy[e];
+            wx[e] = fresh ? 0.0 : wx[e];
+            wy[e] = fresh ? 0.0 : wy[e];
+        }
+        __syncthreads();
+        const double d = s_pa[k];
+        const double2 p = s_pb[k], ra = s_ra[k][j], rw = s_rb[k][j];
+        double2 ca[kEnt], cb[kEnt];
+#pragma unroll
+        for (int e = 0; e < kEnt; e++) {
+            ca[e] = s_ca[b][i0 + kRowStep * e];
+            cb[e] = s_cb[k][i0 + kRowStep * e];
+        }
+        const PanelPivot pv(d, p);
+        const double di = pv.rd * pv.rd;
+        const double tx = j > k ? ra.x * pv.rd : 0.0, ty = j > k ? ra.y * pv.rd : 0.0;  // R_kj
+        const double2 rb = zfms(rw, pv.s, make_double2(tx, ty));
+#pragma unroll
+        for (int e = 0; e < kEnt; e++) {
+            const double ax = ca[e].x * di, ay = ca[e].y * di;
+            gx[e] = fma(-ax, ra.x, fma(ay, ra.y, gx[e]));
+            gy[e] = fma(-ax, ra.y, fma(-ay, ra.x, gy[e]));
+            // rows up to k keep their entries left of column k
+            const bool old = j < k && i0 + kRowStep * e <= k;
+            const double2 f = zmul(cb[e], pv.inv);
+            const double bx = old ? 0.0 : f.x, by = old ? 0.0 : f.y;
+            wx[e] = fma(-bx, rb.x, fma(by, rb.y, wx[e]));
+            wy[e] = fma(-bx, rb.y, fma(-by, rb.x, wy[e]));
         }
     }
     __syncthreads();
-    // T = U^-1 with U = diag(1/tau) + the strictly upper part of V^H V (the
-    // inverse of larft's T; Joffrain et al. 2006).  Lane j of wave 0 back-
-    // substitutes column j: t_j = tau_j, t_i = -tau_i sum_{k=i+1..j} U[i][k] t_k,
-    // written with tau_i rather than 1 / U[i][i], so a tau of zero gives the zero
-    // row and column larft gives.  The per-column recurrence of larft inside the
-    // column loop was a serial chain of up to 31 dependent shared-memory reads
-    // per column; this is one triangular solve per panel.
-    // t_k is zero above row j until written, so the sums need no bound on k,
-    // the loads of a row of U need no condition, and only t_j is kept by a
-    // select
     if (tid < kNB) {
-        const int j = tid;
-        float2 t[kNB];
+        const double d = s_pa[tid];
+        const double2 p = s_pb[tid];
+        const PanelPivot pv(d, p);
+        s_sign[tid] = pv.s;
+        s_inv[tid] = pv.inv;
+        s_u[tid] = make_double2(fma(-pv.s.x, d * pv.rd, p.x), fma(-pv.s.y, d * pv.rd, p.y));
+        // a real pivot with no weight left below it needs no reflection
+        if (tid < nb && p.y == 0 && d - p.x * p.x <= 1e-12 * (p.x * p.x)) s_flat = 1;
+    }
+    __syncthreads();
+    // G = U0^H D^-1 U0, D = diag(U0): R = D^-1/2 U0, R^-1 = U0^-1 D^1/2; the
+    // condition number of the panel with its columns scaled to norm 1
+    double2 R[kEnt], U[kEnt], L[kEnt], Ri[kEnt];
+    const double2 sgn = s_sign[j], inv = s_inv[j];
+    double k2 = 0;
+    const double dj = s_pa[j], rj = dj * rsq_step(dj);
 #pragma unroll
-        for (int i = 0; i < kNB; i++) t[i] = make_float2(i == j ? s_tau[i] : 0.f, 0.f);
+    for (int e = 0; e < kEnt; e++) {
+        const int i = i0 + kRowStep * e;
+        const bool up = j >= i, off = j > i;
+        const double ri = rsq_step(s_pa[i]);
+        const double2 ra = s_ra[i][j], rb = s_rb[i][j], cb = s_cb[j][i], ui = s_u[i];
+        const double2 r = make_double2(off ? ra.x * ri : 0.0, off ? ra.y * ri : 0.0);
+        const double2 u = zfms(rb, s_sign[i], r), l = zmul(cb, inv);
+        R[e] = make_double2(j == i ? rj : r.x, r.y);
+        U[e] = make_double2(off ? u.x : j == i ? ui.x : 0.0, off ? u.y : j == i ? ui.y : 0.0);
+        L[e] = make_double2(up ? (j == i ? 1.0 : 0.0) : l.x, up ? 0.0 : l.y);
+        Ri[e] = make_double2(up ? gx[e] * rj : 0.0, up ? gy[e] * rj : 0.0);
+        k2 = fma(kNB * s_g[i], fma(Ri[e].x, Ri[e].x, Ri[e].y * Ri[e].y), k2);
+    }
 #pragma unroll
-        for (int i = kNB - 2; i >= 0; i--) {
-            float2 u[kNB];
+    for (int m = 32; m >= 1; m >>= 1) k2 += __shfl_xor(k2, m, 64);
+    if ((tid & 63) == 0) s_w[tid >> 6] = k2;
+    __syncthreads();
+    k2 = 0;
 #pragma unroll
-            for (int k = i + 1; k < kNB; k++) u[k] = s_U[i][k];
-            float sr = 0.f, si = 0.f;
+    for (int w = 0; w < kRecThreads / 64; w++) k2 += s_w[w];
+    if (!(k2 <= kPanelCond2) || s_flat) {  // (also NaN)
+        __syncthreads();
+        panel_one_wg<float>(A, lda, M, j0, nb, Tout, 1, (float2(*)[kNB])&s_ra[0][0], (float2(*)[kNB])&s_rb[0][0]);
+        if (tid == 0) *bad = 1;
+        return;
+    }
+    if (tid == 0) *bad = 0;
+    // T = -U (R^-1 S^H) L^-H
+    double2 t[kEnt];
 #pragma unroll
-            for (int k = i + 1; k < kNB; k++) {
-                sr += u[k].x * t[k].x - u[k].y * t[k].y;
-                si += u[k].x * t[k].y + u[k].y * t[k].x;
-            }
-            const float ti = s_tau[i];
-            if (i != j) t[i] = make_float2(-ti * sr, -ti * si);
+    for (int e = 0; e < kEnt; e++) {
+        const int i = i0 + kRowStep * e;
+        s_ra[i][j] = zmul(Ri[e], make_double2(sgn.x, -sgn.y));
+        s_rb[j][i] = make_double2(i == j ? 1.0 : j > i ? 0.0 : wx[e], j >= i ? 0.0 : -wy[e]);  // L^-H
+        s_cb[i][j] = make_double2(-U[e].x, -U[e].y);
+        t[e] = make_double2(0.0, 0.0);
+    }
+    __syncthreads();
+#pragma unroll 4
+    for (int k = 0; k < kNB; k++) {
+        const double2 y = s_rb[k][j];
+#pragma unroll
+        for (int e = 0; e < kEnt; e++) t[e] = zfms(t[e], s_ra[i0 + kRowStep * e][k], y);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < kEnt; e++) {
+        s_rb[i0 + kRowStep * e][j] = t[e];
+        t[e] = make_double2(0.0, 0.0);
+    }
+    __syncthreads();
+#pragma unroll 4
+    for (int k = 0; k < kNB; k++) {
+        const double2 y = s_rb[k][j];
+#pragma unroll
+        for (int e = 0; e < kEnt; e++) t[e] = zfms(t[e], s_cb[i0 + kRowStep * e][k], y);
+    }
+#pragma unroll
+    for (int e = 0; e < kEnt; e++) {
+        const int i = i0 + kRowStep * e;
+        const bool up = j >= i, iu = up && j < nb, low = j < nb && j < i;  // (j < nb: i <= j too)
+        Tout[i * kNB + j] = make_float2(iu ? (float)t[e].x : 0.f, iu ? (float)t[e].y : 0.f);
+        Y[i * kNB + j] = make_double2(iu ? wx[e] : 0.0, iu ? wy[e] : 0.0);
+        if (i < Mp) {
+            const double2 rh = zmul(s_sign[i], R[e]);
+            if (j < nb)
+                A[(size_t)(j0 + j) * lda + j0 + i] =
+                    make_float2((float)(up ? rh.x : L[e].x), (float)(up ? rh.y : L[e].y));
+            Vd[(size_t)j * ldv + i] = make_float2(low ? (float)L[e].x : iu && j == i ? 1.f : 0.f,
+                                                  low ? (float)L[e].y : 0.f);
         }
-#pragma unroll
-        for (int i = 0; i < kNB; i++) Tout[i * kNB + j] = t[i];
     }
 }
 
-// Tall FP32 panels (more rows than the register panel holds): one launch per
-// column, the rows split over workgroups (one row per thread).  Launch jj
-// applies the reflector of column jj to the workgroup's rows and then forms
-// the partials of column jj + 1 from the updated rows: |x|^2 below its
-// diagonal and sum conj(x_r) a_c(r) for the later columns c, x being the
-// column below the diagonal before scaling.  With v = x / (alpha - beta) below
-// the diagonal and v_j = 1,
-//   v^H a_c = a_c(j) + conj(scale) sum_{r > j} conj(x_r) a_c(r),
-// so the reflector's products need no pass of their own after its norm.  The
-// partials are summed in a fixed order by every workgroup of the next launch.
-// Row j of the panel (alpha and the a_c(j)) travels in its own buffer,
-// written by the workgroup holding the row, because that workgroup overwrites
-// the row during the launch that reads it.  jj = -1 only forms the partials of
-// column 0.  Column indices are runtime values here, so the row is walked with
-// compile-time column loops and compares, never by a runtime register index.
-// Leaves the reflectors and R in place and tau_jj on Tout's diagonal.
-template <int NT>
-__global__ __launch_bounds__(NT) void qr_panel_col(float2 *A, long lda, int M, int j0, int jj, const float *zin,
-                                                   const float2 *rin, float *zout, float2 *rout, int nblk,
-                                                   float2 *Tout) {
-    __shared__ float s_red[NT / 64][2 * kNB];
-    __shared__ float s_z[2 * kNB];
-    __shared__ float2 s_d[kNB];
-    const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
-    const int i = j0 + blockIdx.x * NT + tid;
-    const bool live = i < M;
-    const int ic = min(i, M - 1);
-    float2 a[kNB];
+// Rows 32.. of V = P_2 U^-1 to the panel and to Vd, on FP64 MFMA in the
+// three-product form: 64 rows a workgroup, 16 a wave; U^-1 is the operand of the
+// result's rows, so that 16 lanes store 16 consecutive rows of a column.  With
+// *bad, Vd from the panel's reflectors, all rows.
+__global__ __launch_bounds__(256) void qr_form_v(const float2 *__restrict__ Pc, const double2 *__restrict__ Y,
+                                                 const int *__restrict__ bad, float2 *__restrict__ A, long lda, int M,
+                                                 int j0, int nb, float2 *__restrict__ Vd, long ldv) {
+    typedef double v4d __attribute__((ext_vector_type(4)));
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int m = lane & 15, kk = lane >> 4;
+    const int i = blockIdx.x * 64 + 16 * wave + m, ic = min(i, M - j0 - 1);
+    float2 p[kNB / 4];
+    double2 y[kNB / 4][2];
 #pragma unroll
-    for (int c = 0; c < kNB; c++) a[c] = A[(size_t)(j0 + c) * lda + ic];
-    if (jj >= 0) {
-        const int j = j0 + jj;
-        if (tid < 2 * kNB) {
-            float t = 0.f;
-            for (int q = 0; q < nblk; q++) t += zin[(size_t)q * 2 * kNB + tid];
-            s_z[tid] = t;
-        }
-        __syncthreads();
-        const float tot = s_z[2 * jj];
-        const float2 alpha = rin[jj];
-        const float aa = sqrtf(alpha.x * alpha.x + alpha.y * alpha.y);
-        const float xnorm = sqrtf(aa * aa + tot);
-        float tau = 0.f;
-        float2 scale = make_float2(0.f, 0.f), beta = alpha;
-        if (tot > 0 || (xnorm > 0 && alpha.y != 0)) {
-            const float phr = aa > 0 ? alpha.x / aa : 1.f, phi = aa > 0 ? alpha.y / aa : 0.f;
-            beta = make_float2(-phr * xnorm, -phi * xnorm);
-            const float dr = alpha.x - beta.x, di = alpha.y - beta.y;
-            const float dd = dr * dr + di * di;
-            scale = make_float2(dr / dd, -di / dd);
-            tau = 2.f / (1.f + tot / dd);
-        }
-        if (tid < kNB) {
-            const int c = tid;
-            float2 d = make_float2(0.f, 0.f);
-            if (c > jj) {
-                // tau (a_c(j) + conj(scale) S_c)
-                const float sx = s_z[2 * c], sy = s_z[2 * c + 1];
-                const float2 ac = rin[c];
-                d.x = tau * (ac.x + scale.x * sx + scale.y * sy);
-                d.y = tau * (ac.y + scale.x * sy - scale.y * sx);
-            }
-            s_d[c] = d;
-        }
-        if (blockIdx.x == 0 && tid == 0) Tout[jj * kNB + jj] = make_float2(tau, 0.f);
-        __syncthreads();
-        if (live && i >= j) {
-            float2 x = make_float2(0.f, 0.f);
+    for (int u = 0; u < kNB / 4; u++) {
+        p[u] = Pc[(size_t)(4 * u + kk) * ldv + ic];
 #pragma unroll
-            for (int c = 0; c < kNB; c++)
-                if (c == jj) x = a[c];
-            const bool below = i > j;
-            const float2 v = below ? make_float2(x.x * scale.x - x.y * scale.y, x.x * scale.y + x.y * scale.x)
-                                   : make_float2(1.f, 0.f);
+        for (int g = 0; g < 2; g++) y[u][g] = Y[(4 * u + kk) * kNB + 16 * g + m];
+    }
+    if (*bad) {
+        if (j0 + i < M)
+            for (int c = kk; c < kNB; c += 4)
+                Vd[(size_t)c * ldv + i] =
+                    c < nb ? vget((const float2 *)A, lda, j0, c, j0 + i) : make_float2(0.f, 0.f);
+        return;
+    }
+    v4d acc[2][3];
 #pragma unroll
-            for (int c = 0; c < kNB; c++) {
-                if (c == jj) {
-                    a[c] = below ? v : beta;
-                } else if (c > jj) {
-                    const float2 d = s_d[c];
-                    a[c].x -= d.x * v.x - d.y * v.y;
-                    a[c].y -= d.x * v.y + d.y * v.x;
-                }
-                if (c >= jj) A[(size_t)(j0 + c) * lda + i] = a[c];
-            }
+    for (int g = 0; g < 2; g++)
+#pragma unroll
+        for (int q = 0; q < 3; q++) acc[g][q] = (v4d){0, 0, 0, 0};
+#pragma unroll
+    for (int u = 0; u < kNB / 4; u++) {
+        const double pr = p[u].x, pi = p[u].y;
+#pragma unroll
+        for (int g = 0; g < 2; g++) {
+            const double yr = y[u][g].x, yi = y[u][g].y;
+            acc[g][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(yr, pr + pi, acc[g][0], 0, 0, 0);
+            acc[g][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(yr + yi, pi, acc[g][1], 0, 0, 0);
+            acc[g][2] = __builtin_amdgcn_mfma_f64_16x16x4f64(yi - yr, pr, acc[g][2], 0, 0, 0);
         }
     }
-    if (jj + 1 < kNB) {
-        const int k = jj + 1, j1 = j0 + k;
-        float2 x = make_float2(0.f, 0.f);
+    if (i < kNB || j0 + i >= M) return;
 #pragma unroll
-        for (int c = 0; c < kNB; c++)
-            if (c == k) x = a[c];
-        const bool below = live && i > j1;
-        float z[2 * kNB];
+    for (int g = 0; g < 2; g++)
 #pragma unroll
-        for (int c = 0; c < kNB; c++) {
-            float pr = 0.f, pi = 0.f;
-            if (below) {
-                if (c == k) {
-                    pr = x.x * x.x + x.y * x.y;
-                } else if (c > k) {
-                    pr = x.x * a[c].x + x.y * a[c].y;
-                    pi = x.x * a[c].y - x.y * a[c].x;
-                }
-            }
-            z[2 * c] = pr;
-            z[2 * c + 1] = pi;
+        for (int q = 0; q < 4; q++) {
+            const int c = 16 * g + kk + 4 * q;
+            const float2 v = make_float2((float)(acc[g][0][q] - acc[g][1][q]), (float)(acc[g][0][q] + acc[g][2][q]));
+            if (c < nb) A[(size_t)(j0 + c) * lda + j0 + i] = v;
+            Vd[(size_t)c * ldv + i] = v;  // (zero past nb)
         }
-        if (live && i == j1) {
-#pragma unroll
-            for (int c = 0; c < kNB; c++)
-                if (c >= k) rout[c] = a[c];
-        }
-        wave_reduce_scatter64(z, lane);
-        s_red[wid][lane] = z[0];
-        __syncthreads();
-        if (tid < 2 * kNB) {
-            float t = 0.f;
-#pragma unroll
-            for (int w = 0; w < NT / 64; w++) t += s_red[w][tid];
-            zout[(size_t)blockIdx.x * 2 * kNB + tid] = t;
-        }
-    }
 }
 
 // T of the compact WY form from the taus (on Tout's diagonal) and
@@ -741,29 +815,6 @@ __global__ void k_build_v(const typename QT<T>::c2 *A, long lda, int M, int j0, 
         z.y = 0;
     }
     Vd[(size_t)l * ldvd + (i - j0)] = z;
-}
-
-// W[c][l] = (T^H V^H C)[l][c] = conj(sum_q T[q][l] Z[q][c]) with Z[q][c] =
-// (C^H V)[c][q] (the adjoint product's output); rows l >= nb zero
-template <typename T>
-__global__ void k_qr_w(const typename QT<T>::c2 *Tm, int nb, const typename QT<T>::c2 *Z, long ldz, int nc,
-                       typename QT<T>::c2 *W) {
-    using C2 = typename QT<T>::c2;
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    const int l = blockIdx.y;
-    if (c >= nc) return;
-    T sr = 0, si = 0;
-    if (l < nb) {
-        for (int q = 0; q <= l; q++) {  // T upper triangular
-            const C2 t = Tm[q * kNB + l], z = Z[(size_t)q * ldz + c];
-            sr += t.x * z.x - t.y * z.y;
-            si += t.x * z.y + t.y * z.x;
-        }
-    }
-    C2 o;
-    o.x = sr;
-    o.y = -si;
-    W[(size_t)c * kNB + l] = o;
 }
 
 // R x = b (upper, non-unit), one workgroup per right-hand side, in place in B.
@@ -1147,24 +1198,25 @@ struct QRFactor {
     C2 *W = nullptr;   // workspace nb x max(ncols)
     int wcols = 0;
     C2 *Vd = nullptr;  // explicit panel V (FP32 MFMA trailing update)
-    C2 *Z = nullptr;   // (C^H V) of the trailing columns
     C2 *Yz = nullptr;  // V^H V of the panel (kNB x kNB)
     char *gws = nullptr;
     long ldv = 0;
-    // partials and panel rows of the one-launch-per-column tall panel
-    float *zcol = nullptr;
-    long zcol_stride = 0;
-    float2 *rcol = nullptr;
+    // panels by Householder reconstruction: copy of the panel, partials of its
+    // Gram matrix, U^-1, and whether it took the column-wise algorithm
+    float2 *Pc = nullptr;
+    double2 *gram = nullptr, *Y = nullptr;
+    int *bad = nullptr;
     hipStream_t st = nullptr;
     ~QRFactor() {
         sfree(Tb, st);
         sfree(W, st);
         sfree(Vd, st);
-        sfree(Z, st);
         sfree(Yz, st);
         sfree(gws, st);
-        sfree(zcol, st);
-        sfree(rcol, st);
+        sfree(Pc, st);
+        sfree(gram, st);
+        sfree(Y, st);
+        sfree(bad, st);
     }
 };
 
@@ -1193,15 +1245,14 @@ static int qr_factor(QRFactor<T> &f, int extra_cols, hipStream_t s) {
     HOST_CALL(salloc(&f.Tb, (size_t)np * kNB * kNB, s));
     f.wcols = std::max(f.N, extra_cols);
     HOST_CALL(salloc(&f.W, (size_t)kNB * f.wcols, s));
-    // FP32: trailing updates on MFMA (Z = C^H V with the adjoint product, then
-    // C -= V W with the rank-32 update); FP64 keeps the VALU kernels
+    // FP32: trailing updates on MFMA (C^H V with the adjoint product, then
+    // C -= V W with the rank-32 update, which also forms W); FP64 keeps the
+    // VALU kernels
     const bool mfma = sizeof(T) == 4 && !getenv("BEM_QR_VALU");
     const bool global_panel = getenv("BEM_QR_GPANEL") != nullptr;
-    const bool one_wg_panel = getenv("BEM_QR_ONE_WG_PANEL") != nullptr;
     if (mfma) {
         f.ldv = (f.lda + 63) / 64 * 64;
         HOST_CALL(salloc(&f.Vd, (size_t)f.ldv * kNB, s));
-        HOST_CALL(salloc(&f.Z, (size_t)kNB * f.N, s));
         HOST_CALL(salloc(&f.Yz, (size_t)kNB * kNB, s));
         size_t wsz = 0;
         for (int p = 0; p < np; p++) {
@@ -1210,9 +1261,12 @@ static int qr_factor(QRFactor<T> &f, int extra_cols, hipStream_t s) {
             if (f.N - (j0 + nb) > 0) wsz = std::max(wsz, ws_gemm_h_f32(f.M - j0, f.N - (j0 + nb), kNB));
         }
         HOST_CALL(salloc(&f.gws, std::max<size_t>(wsz, 1), s));
-        f.zcol_stride = (long)((f.M + kColThreads - 1) / kColThreads) * 2 * kNB;
-        HOST_CALL(salloc(&f.zcol, (size_t)2 * f.zcol_stride, s));
-        HOST_CALL(salloc(&f.rcol, (size_t)2 * kNB, s));
+        if (!global_panel) {
+            HOST_CALL(salloc(&f.Pc, (size_t)f.ldv * kNB, s));
+            HOST_CALL(salloc(&f.gram, (size_t)kGramParts * kNN, s));
+            HOST_CALL(salloc(&f.Y, (size_t)kNN, s));
+            HOST_CALL(salloc(&f.bad, 1, s));
+        }
     }
     for (int p = 0; p < np; p++) {
         const int j0 = p * kNB, nb = std::min(kNB, f.N - j0);
@@ -1220,34 +1274,18 @@ static int qr_factor(QRFactor<T> &f, int extra_cols, hipStream_t s) {
         timing_begin(tr, sizeof(T) == 4 ? "qr_panel_f32" : "qr_panel_f64", s);
         C2 *Tp = f.Tb + (size_t)p * kNB * kNB;
         const int Mp = f.M - j0;
-        // panels of up to 1024 rows: the register kernel also forms T and the
-        // explicit V; taller ones (and a narrow last panel) run the global
-        // panel kernel, then V, V^H V on MFMA and T from it
-        const bool fit = mfma && nb == kNB && !global_panel;
-        const int reg = !fit ? 0 : Mp <= 256 ? 1 : Mp <= 512 ? 2 : Mp <= 1024 ? 3 : 0;
-        float2 *Tf = (float2 *)Tp, *Vf = (float2 *)f.Vd;
-        if (reg == 1) {
-            qr_panel_reg<256, 1><<<1, 256, 0, s>>>((float2 *)f.A, f.lda, f.M, j0, Tf, Vf, f.ldv);
-        } else if (reg == 2) {
-            qr_panel_reg<512, 1><<<1, 512, 0, s>>>((float2 *)f.A, f.lda, f.M, j0, Tf, Vf, f.ldv);
-        } else if (reg == 3) {
-            qr_panel_reg<512, 2><<<1, 512, 0, s>>>((float2 *)f.A, f.lda, f.M, j0, Tf, Vf, f.ldv);
-        } else if (fit && !one_wg_panel) {
-            // tall panel: one launch per column over kColThreads-row workgroups
-            const int nblk = (Mp + kColThreads - 1) / kColThreads;
-            for (int jj = -1; jj < kNB; jj++) {
-                const int bi = jj & 1, bo = (jj + 1) & 1;
-                qr_panel_col<kColThreads><<<nblk, kColThreads, 0, s>>>(
-                    (float2 *)f.A, f.lda, f.M, j0, jj, f.zcol + (size_t)bi * f.zcol_stride,
-                    (const float2 *)f.rcol + (size_t)bi * kNB, f.zcol + (size_t)bo * f.zcol_stride,
-                    (float2 *)f.rcol + (size_t)bo * kNB, nblk, Tf);
-                HIP_CALL(hipGetLastError());
-            }
+        if (mfma && !global_panel) {
+            const int rpb = kGramChunk * ((Mp + kGramChunk * kGramParts - 1) / (kGramChunk * kGramParts));
+            const int nblk = (Mp + rpb - 1) / rpb;
+            float2 *Af = (float2 *)f.A, *Vf = (float2 *)f.Vd;
+            qr_gram<<<nblk, 256, 0, s>>>(Af, f.lda, f.M, j0, nb, rpb, f.gram, f.Pc, f.ldv);
+            qr_recon<<<1, kRecThreads, 0, s>>>(f.gram, nblk, Af, f.lda, f.M, j0, nb, (float2 *)Tp, Vf, f.ldv, f.Y, f.bad);
+            qr_form_v<<<(Mp + 63) / 64, 256, 0, s>>>(f.Pc, f.Y, f.bad, Af, f.lda, f.M, j0, nb, Vf, f.ldv);
         } else {
             qr_panel<T><<<1, 1024, 0, s>>>(f.A, f.lda, f.M, j0, nb, Tp, mfma ? 0 : 1);
         }
         HIP_CALL(hipGetLastError());
-        if (mfma && !reg) {
+        if (mfma && global_panel) {
             dim3 gv((unsigned)((Mp + 255) / 256), kNB);
             k_build_v<T><<<gv, 256, 0, s>>>(f.A, f.lda, f.M, j0, nb, f.Vd, f.ldv);
             HIP_CALL(hipGetLastError());
@@ -1264,13 +1302,12 @@ static int qr_factor(QRFactor<T> &f, int extra_cols, hipStream_t s) {
             timing_begin(tu, sizeof(T) == 4 ? "qr_trailing_f32" : "qr_trailing_f64", s);
             if (mfma) {
                 float2 *Cb = (float2 *)(Ct + j0);  // rows j0.., columns j0+nb..
-                HOST_CALL(gemm_h_f32(Cb, f.lda, Mp, nc, (const float2 *)f.Vd, f.ldv, (float2 *)f.Z, f.N, kNB, f.gws,
-                                     s));
-                dim3 gw((unsigned)((nc + 255) / 256), kNB);
-                k_qr_w<T><<<gw, 256, 0, s>>>(f.Tb + (size_t)p * kNB * kNB, nb, f.Z, f.N, nc, f.W);
-                HIP_CALL(hipGetLastError());
-                HOST_CALL(rank_update_f32((const float2 *)f.Vd, f.ldv, Mp, (const float2 *)f.W, kNB, nc, Cb, f.lda,
-                                          s));
+                const bool direct = Mp <= kTrailRows;
+                ProdParts zp;
+                HOST_CALL(gemm_h_f32(Cb, f.lda, Mp, nc, (const float2 *)f.Vd, f.ldv, (float2 *)f.W, f.N, kNB, f.gws, s,
+                                     false, direct ? &zp : nullptr));
+                if (!direct) zp = {(const float2 *)f.W, f.N, 1};
+                HOST_CALL(qr_trail_f32((const float2 *)f.Vd, f.ldv, Mp, (const float2 *)Tp, nb, zp, nc, Cb, f.lda, s));
             } else {
                 qr_vhc<T><<<nc, 256, 0, s>>>(f.A, f.lda, f.M, j0, nb, f.Tb + (size_t)p * kNB * kNB, Ct, f.lda,
                                              f.W, 1);
