@@ -1011,179 +1011,399 @@ __global__ __launch_bounds__(NT) void qr_solve_small(const typename QT<T>::c2 *A
     for (int i = tid; i < N; i += NT) b[i] = sb[i];
 }
 
-// Q^H B for systems past the one-workgroup solve: one launch per panel, the
-// rows split over workgroups of NT threads (one row per thread, one
-// right-hand side per blockIdx.y).  Launch p finishes panel p on the block's
-// rows (z = sum of the partials of V_p^H b in a fixed order, w = T_p^H z,
-// b -= V_p w) and then forms the block's partial of V_{p+1}^H b over the same
-// rows, whose values are final for panel p+1.  p = -1 only forms the partials
-// of panel 0.  Partials alternate between two buffers by panel parity.
-template <typename T, int NT>
-__global__ __launch_bounds__(NT) void qr_apply_step(const typename QT<T>::c2 *A, long lda, int M, int N,
-                                                    const typename QT<T>::c2 *Tb, typename QT<T>::c2 *B, long ldb,
-                                                    int p, const T *zin, T *zout, int nblk) {
+// Solves with a factored system, by groups of kGB panels (kGW columns).  A group's
+// reflectors act as one block, I - V T V^H with V the kGB panels side by side,
+// and its diagonal block of R is used through its inverse, so Q^H b takes one
+// launch per group and the back substitution another, instead of one per
+// panel; the launches are bound by latency (each a few loads deep), so their
+// number is what counts.  The two kGW x kGW triangles of every group are formed
+// once after the factorisation (qr_cross, qr_group, 70 us), in FP64.  A solve of
+// 642 unknowns takes 13 launches of 7 to 12 us, where a launch per panel took 43
+// of 8 to 10.  QR solve with refinement: 642 nodes 2.8 -> 2.3 ms, 1962: 9.1 ->
+// 6.9, 10242: 150 -> 128.
+constexpr int kGB = 4, kGW = kGB * kNB, kGG = kGW * kGW;
+constexpr int kPairs = kGB * (kGB - 1) / 2;  // panels s < t of a group
+
+__device__ __forceinline__ double2 to_d2(float2 v) { return make_double2(v.x, v.y); }
+__device__ __forceinline__ double2 to_d2(double2 v) { return v; }
+
+// V's entry of row i and column c (unit diagonal, zero above it), from the
+// matrix's
+template <typename C2>
+__device__ __forceinline__ C2 v_entry(C2 raw, int i, int c) {
+    C2 z;
+    z.x = i > c ? raw.x : i == c ? 1 : 0;
+    z.y = i > c ? raw.y : 0;
+    return z;
+}
+
+// Workgroups of the pairs: cross[((g kPairs + q) nsplit + split)][i][j] = the
+// split's part of V_s^H V_t, q the pair (s, t) of group g, on FP64 MFMA (as
+// qr_gram).  Workgroups past them (one per panel): Rinv[p], the inverse of the
+// panel's diagonal block of R, lane j of one wave its column j by back
+// substitution.  Both zero past N.
+template <typename T>
+__global__ __launch_bounds__(256) void qr_cross(const typename QT<T>::c2 *__restrict__ A, long lda, int M, int N,
+                                                int npair, int nsplit, double2 *__restrict__ cross,
+                                                double2 *__restrict__ Rinv) {
     using C2 = typename QT<T>::c2;
-    __shared__ T s_red[NT / 64][2 * kNB];
-    __shared__ C2 s_z[kNB], s_w[kNB];
-    const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6, col = blockIdx.y;
-    const int i = blockIdx.x * NT + tid;
-    const bool live = i < M;
-    C2 *b = B + (size_t)col * ldb;
-    C2 bi;
-    bi.x = 0;
-    bi.y = 0;
-    if (live) bi = b[i];
-    const int ic = min(i, M - 1);
+    typedef double v4d __attribute__((ext_vector_type(4)));
+    constexpr int kRows = 32;
+    __shared__ double2 s_v[2][kNB][kRows + 1];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int np = (N + kNB - 1) / kNB;
-    if (p >= 0) {
-        const int j0 = p * kNB, nb = min(kNB, N - j0);
-        if (tid < 2 * kNB) {
-            T t = 0;
-            for (int q = 0; q < nblk; q++) t += zin[((size_t)col * nblk + q) * 2 * kNB + tid];
-            ((T *)s_z)[tid] = t;
+    if ((int)blockIdx.x >= npair * nsplit) {
+        const int c0 = (blockIdx.x - npair * nsplit) * kNB, nb = min(kNB, N - c0);
+        double2(*s_r)[kRows + 1] = s_v[0];
+        for (int e = tid; e < kNN; e += 256) {
+            const int i = e % kNB, k = e / kNB;
+            double2 v = make_double2(i == k ? 1.0 : 0.0, 0.0);
+            if (i <= k && k < nb) v = to_d2(A[(size_t)(c0 + k) * lda + c0 + i]);
+            s_r[i][k] = v;
         }
         __syncthreads();
-        if (tid < nb) {
-            // w = T^H z; T upper triangular
-            const C2 *Tm = Tb + (size_t)p * kNB * kNB;
-            T wr = 0, wi = 0;
-            for (int q = 0; q <= tid; q++) {
-                const C2 t = Tm[q * kNB + tid];
-                wr += t.x * s_z[q].x + t.y * s_z[q].y;
-                wi += t.x * s_z[q].y - t.y * s_z[q].x;
+        if (tid < kNB) {
+            const int j = tid;
+            double tx[kNB], ty[kNB];
+#pragma unroll
+            for (int i = kNB - 1; i >= 0; i--) {
+                double sr = i == j ? 1.0 : 0.0, si = 0;
+#pragma unroll
+                for (int k = i + 1; k < kNB; k++) {
+                    const double2 r = s_r[i][k];
+                    sr = fma(-r.x, tx[k], fma(r.y, ty[k], sr));
+                    si = fma(-r.x, ty[k], fma(-r.y, tx[k], si));
+                }
+                const double2 d = s_r[i][i];
+                const double q = 1.0 / fma(d.x, d.x, d.y * d.y);
+                tx[i] = fma(sr, d.x, si * d.y) * q;
+                ty[i] = fma(si, d.x, -sr * d.y) * q;
             }
-            s_w[tid].x = wr;
-            s_w[tid].y = wi;
-        } else if (tid < kNB) {
-            // a narrow last panel: these meet zeros below, which shared
-            // memory's old contents (infinities, NaNs) would not survive
-            s_w[tid].x = 0;
-            s_w[tid].y = 0;
-        }
-        __syncthreads();
-        T sr = 0, si = 0;
+            double2 *out = Rinv + (size_t)(c0 / kNB) * kNN;
 #pragma unroll
-        for (int l0 = 0; l0 < kNB; l0 += kCG) {
-            C2 raw[kCG];
-#pragma unroll
-            for (int u = 0; u < kCG; u++) raw[u] = A[(size_t)min(j0 + l0 + u, N - 1) * lda + ic];
-#pragma unroll
-            for (int u = 0; u < kCG; u++) {
-                const int l = l0 + u;
-                const bool below = i > j0 + l && l < nb, diag = i == j0 + l && l < nb;
-                const T vx = below ? raw[u].x : (diag ? (T)1 : (T)0), vy = below ? raw[u].y : (T)0;
-                sr += vx * s_w[l].x - vy * s_w[l].y;
-                si += vx * s_w[l].y + vy * s_w[l].x;
+            for (int i = 0; i < kNB; i++) {
+                const bool in = i <= j && j < nb;
+                out[i * kNB + j] = make_double2(in ? tx[i] : 0.0, in ? ty[i] : 0.0);
             }
         }
-        if (live && i >= j0) {
-            bi.x -= sr;
-            bi.y -= si;
-            b[i] = bi;
+        return;
+    }
+    const int pair = blockIdx.x / nsplit, split = blockIdx.x % nsplit;
+    const int g = pair / kPairs, q = pair % kPairs;
+    const int t = q >= 3 ? 3 : q >= 1 ? 2 : 1, sp = q - t * (t - 1) / 2;  // (0,1) (0,2) (1,2) (0,3) (1,3) (2,3)
+    const int ps = g * kGB + sp, pt = g * kGB + t;
+    const int m = lane & 15, kk = lane >> 4, a0 = 16 * (wave & 1), b0 = 16 * (wave >> 1);
+    v4d acc[3];
+#pragma unroll
+    for (int c = 0; c < 3; c++) acc[c] = (v4d){0, 0, 0, 0};
+    if (pt < np) {
+        // rows from panel t's first on (V_t is zero above), in chunks
+        const int r0 = pt * kNB, nch = (M - r0 + kRows - 1) / kRows;
+        const int per = (nch + nsplit - 1) / nsplit, ch1 = min(nch, (split + 1) * per);
+        for (int ch = split * per; ch < ch1; ch++) {
+            const int i = r0 + ch * kRows + (tid & 31), ic = min(i, M - 1);
+            double2 v[2][kNB / 8];
+#pragma unroll
+            for (int h = 0; h < 2; h++)
+#pragma unroll
+                for (int u = 0; u < kNB / 8; u++) {
+                    const int c = (h ? pt : ps) * kNB + (tid >> 5) + 8 * u;
+                    const C2 raw = A[(size_t)min(c, N - 1) * lda + ic];
+                    v[h][u] = i < M && c < N ? to_d2(v_entry(raw, i, c)) : make_double2(0.0, 0.0);
+                }
+            __syncthreads();  // the previous rows are read
+#pragma unroll
+            for (int h = 0; h < 2; h++)
+#pragma unroll
+                for (int u = 0; u < kNB / 8; u++) s_v[h][(tid >> 5) + 8 * u][tid & 31] = v[h][u];
+            __syncthreads();
+#pragma unroll
+            for (int r = 0; r < kRows; r += 4) {
+                const double2 x = s_v[0][a0 + m][r + kk], y = s_v[1][b0 + m][r + kk];
+                const double ur = x.x, ui = -x.y, vr = y.x, vi = y.y;
+                acc[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(ur, vr + vi, acc[0], 0, 0, 0);
+                acc[1] = __builtin_amdgcn_mfma_f64_16x16x4f64(ur + ui, vi, acc[1], 0, 0, 0);
+                acc[2] = __builtin_amdgcn_mfma_f64_16x16x4f64(ui - ur, vr, acc[2], 0, 0, 0);
+            }
         }
     }
-    if (p + 1 < np) {
-        const int j0 = (p + 1) * kNB, nb = min(kNB, N - j0);
-        T x[2 * kNB];
+    double2 *out = cross + (size_t)blockIdx.x * kNN;
 #pragma unroll
-        for (int l = 0; l < 2 * kNB; l++) x[l] = 0;
-#pragma unroll
-        for (int l0 = 0; l0 < kNB; l0 += kCG) {
-            C2 raw[kCG];
-#pragma unroll
-            for (int u = 0; u < kCG; u++) raw[u] = A[(size_t)min(j0 + l0 + u, N - 1) * lda + ic];
-#pragma unroll
-            for (int u = 0; u < kCG; u++) {
-                const int l = l0 + u;
-                const bool below = live && i > j0 + l && l < nb, diag = i == j0 + l && l < nb;
-                const T vx = below ? raw[u].x : (diag ? (T)1 : (T)0), vy = below ? raw[u].y : (T)0;
-                x[2 * l] = vx * bi.x + vy * bi.y;
-                x[2 * l + 1] = vx * bi.y - vy * bi.x;
-            }
+    for (int v = 0; v < 4; v++)
+        out[(a0 + kk + 4 * v) * kNB + b0 + m] = make_double2(acc[0][v] - acc[1][v], acc[0][v] + acc[2][v]);
+}
+
+// The triangles of a group: G = T (GT[g][k kGW + l] = T_kl), whose inverse has
+// the panels' T^-1 on its diagonal and V_s^H V_t above it, and G = R_gg^-1
+// (GR[g][k kGW + l] = (R_gg^-1)_lk, so that both are read with l across the
+// lanes).  Blocks of column t from the diagonal up,
+//   G_tt = D_t,  G_st = -D_s sum_{u = s+1..t} O_su G_ut,
+// D the panels' T or Rinv, O the cross products or R.  One workgroup per column
+// t (blockIdx.y) and triangle (blockIdx.z), thread (i, j) one entry of a block,
+// FP64; the finished blocks of the column stay in shared memory.
+template <typename T>
+__global__ __launch_bounds__(1024) void qr_group(const typename QT<T>::c2 *__restrict__ A, long lda, int N,
+                                                 const typename QT<T>::c2 *__restrict__ Tb,
+                                                 const double2 *__restrict__ cross, int nsplit,
+                                                 const double2 *__restrict__ Rinv, double2 *__restrict__ GT,
+                                                 double2 *__restrict__ GR) {
+    __shared__ double2 s_o[kNB][kNB + 1], s_g[kNB][kNB];
+    const int i = threadIdx.x >> 5, j = threadIdx.x & 31;
+    const int g = blockIdx.x, t = blockIdx.y;
+    const bool tri_r = blockIdx.z;
+    const int np = (N + kNB - 1) / kNB;
+    double2 *out = (tri_r ? GR : GT) + (size_t)g * kGG;
+    auto diag = [&](int sp) {  // entry (i, j) of D_sp
+        const int p = g * kGB + sp;
+        if (p >= np) return make_double2(0.0, 0.0);
+        return tri_r ? Rinv[(size_t)p * kNN + threadIdx.x] : to_d2(Tb[(size_t)p * kNN + threadIdx.x]);
+    };
+    auto off = [&](int sp, int u) {  // entry (i, j) of O_su, sp < u
+        const int ps = g * kGB + sp, pu = g * kGB + u;
+        double2 v = make_double2(0.0, 0.0);
+        if (pu >= np) return v;
+        if (tri_r) {
+            const int c = pu * kNB + j;
+            return c < N ? to_d2(A[(size_t)c * lda + ps * kNB + i]) : v;
         }
-        wave_reduce_scatter64(x, lane);
-        s_red[wid][lane] = x[0];
+        const double2 *x = cross + (size_t)(g * kPairs + u * (u - 1) / 2 + sp) * nsplit * kNN + threadIdx.x;
+        for (int k = 0; k < nsplit; k++) {
+            const double2 w = x[(size_t)k * kNN];
+            v.x += w.x;
+            v.y += w.y;
+        }
+        return v;
+    };
+    auto store = [&](int sp, double2 v) {
+        const int k = sp * kNB + i, l = t * kNB + j;
+        out[tri_r ? l * kGW + k : k * kGW + l] = v;
+    };
+    double2 own[kGB];  // this thread's entries of G_tt, G_{t-1,t}, ..
+    own[0] = diag(t);
+    store(t, own[0]);
+    for (int sp = t + 1; sp < kGB; sp++) store(sp, make_double2(0.0, 0.0));
+#pragma unroll
+    for (int d = 1; d < kGB; d++) {
+        const int sp = t - d;
+        if (sp < 0) break;
+        double2 acc = make_double2(0.0, 0.0);
+        const double2 dd = diag(sp);
+#pragma unroll
+        for (int e = 0; e < d; e++) {  // u = t - e
+            const double2 o = off(sp, t - e);
+            __syncthreads();
+            s_o[i][j] = o;
+            s_g[i][j] = own[e];
+            __syncthreads();
+#pragma unroll 8
+            for (int k = 0; k < kNB; k++) acc = zfms(acc, s_o[i][k], s_g[k][j]);
+        }
         __syncthreads();
-        if (tid < 2 * kNB) {
-            T t = 0;
-#pragma unroll
-            for (int w = 0; w < NT / 64; w++) t += s_red[w][tid];
-            zout[((size_t)col * nblk + blockIdx.x) * 2 * kNB + tid] = t;
-        }
+        s_o[i][j] = dd;
+        s_g[i][j] = make_double2(-acc.x, -acc.y);
+        __syncthreads();
+        acc = make_double2(0.0, 0.0);
+#pragma unroll 8
+        for (int k = 0; k < kNB; k++) acc = zfms(acc, s_o[i][k], s_g[k][j]);
+        own[d] = acc;
+        store(sp, acc);
     }
 }
 
-// One block column of R x = b for systems past the one-workgroup solve: every
-// workgroup solves the nb x nb diagonal block at c0 redundantly (one wave,
-// the block's rows of R in registers; b[c0..c0+nb) is not written in this
-// step), workgroup 0 stores the unknowns in X, and every workgroup removes
-// them from its rows below c0 of the working right-hand side B.
-template <typename T, int NT>
-__global__ __launch_bounds__(NT) void trsv_block_step(const typename QT<T>::c2 *A, long lda, int N,
-                                                      typename QT<T>::c2 *B, long ldb, typename QT<T>::c2 *X,
-                                                      long ldx, int c0, int nb) {
+// s_w[h][l] = part h of sum_k f(G[k][l], s_z[k]) over the kGW / 2 entries k of
+// half h = tid / kGW, l = tid % kGW, f = conj(g) z (CONJ) or g z; the sum of the
+// two parts is the product.  The first loads are independent of s_z: the
+// caller's barrier that completes s_z is between them and the products.
+template <bool CONJ>
+struct TriProduct {
+    static constexpr int kLoads = kGW / 8;  // in flight
+    const double2 *Gl;
+    double2 v[kLoads];
+    __device__ __forceinline__ TriProduct(const double2 *G) {
+        Gl = G + (size_t)(threadIdx.x / kGW) * (kGW / 2) * kGW + threadIdx.x % kGW;
+#pragma unroll
+        for (int k = 0; k < kLoads; k++) v[k] = Gl[(size_t)k * kGW];
+    }
+    __device__ __forceinline__ double2 apply(const double2 *s_z) {
+        const double2 *z = s_z + (threadIdx.x / kGW) * (kGW / 2);
+        double sr = 0, si = 0;
+#pragma unroll
+        for (int k0 = 0; k0 < kGW / 2; k0 += kLoads) {
+            double2 n[kLoads];
+            if (k0 + kLoads < kGW / 2) {
+#pragma unroll
+                for (int k = 0; k < kLoads; k++) n[k] = Gl[(size_t)(k0 + kLoads + k) * kGW];
+            }
+#pragma unroll
+            for (int k = 0; k < kLoads; k++) {
+                const double2 x = z[k0 + k];
+                const double gy = CONJ ? -v[k].y : v[k].y;
+                sr = fma(v[k].x, x.x, fma(-gy, x.y, sr));
+                si = fma(v[k].x, x.y, fma(gy, x.x, si));
+            }
+            if (k0 + kLoads < kGW / 2) {
+#pragma unroll
+                for (int k = 0; k < kLoads; k++) v[k] = n[k];
+            }
+        }
+        return make_double2(sr, si);
+    }
+};
+
+// Launch g of Q^H B (g = -1, 0, ..): finishes group g on the workgroup's rows
+// (z = sum of the partials of V_g^H b in a fixed order, w = T_g^H z, b -= V_g w),
+// then forms their partial of V_{g+1}^H b, b being final for group g + 1.
+// g = -1 only forms the partials of group 0.  A workgroup takes rpb rows (a
+// multiple of 64), 64 at a time, wave w the panel w of either group, one
+// right-hand side per blockIdx.y.  The partials (kGW values a workgroup)
+// alternate between two buffers.  Triangles and sums are FP64 for either type:
+// FP32 solves of 252 to 1962 unknowns are off by 1.8e-7, one panel at a time in
+// FP32 by 4.5e-7, and by 5.1e-7 with FP32 triangles (which saved 1 to 2 us a
+// launch).
+template <typename T>
+__global__ __launch_bounds__(256) void qr_apply_group(const typename QT<T>::c2 *__restrict__ A, long lda, int M, int N,
+                                                      const double2 *__restrict__ GT, typename QT<T>::c2 *B, long ldb,
+                                                      int g, int ng, int rpb, const double *__restrict__ zin,
+                                                      double *__restrict__ zout, int nblk) {
     using C2 = typename QT<T>::c2;
-    __shared__ C2 s_x[kNB];
-    const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6, col = blockIdx.y;
+    __shared__ double2 s_z[kGW], s_w[2][kGW], s_part[2][4][64];
+    const int tid = threadIdx.x, lane = tid & 63, col = blockIdx.y;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int ca = (g * kGB + wave) * kNB, cb = ca + kGW;  // first columns of the wave's panels
+    const bool next = g + 1 < ng;
     C2 *b = B + (size_t)col * ldb;
-    if (wid == 0) {
-        const int r = c0 + lane, rc = min(r, N - 1);
-        C2 rr[kNB];
+    const int row0 = blockIdx.x * rpb;
+    C2 va[kNB], vb[kNB], braw;
+    // columns past N read the last one: they meet zeros of T
+    auto load = [&](int i) {
+        const int ic = min(i, M - 1);
+        braw = b[ic];
+        const C2 *pa = A + ic;
+        if (g >= 0) {
 #pragma unroll
-        for (int m = 0; m < kNB; m++) rr[m] = A[(size_t)min(c0 + m, N - 1) * lda + rc];
+            for (int l = 0; l < kNB; l++) va[l] = pa[(unsigned)min(ca + l, N - 1) * (size_t)lda];
+        }
+        if (next) {
 #pragma unroll
-        for (int m = 0; m < kNB; m++) {
-            if (!(lane < nb && m < nb && m >= lane)) {
-                rr[m].x = 0;
-                rr[m].y = 0;
+            for (int l = 0; l < kNB; l++) vb[l] = pa[(unsigned)min(cb + l, N - 1) * (size_t)lda];
+        }
+    };
+    if (sizeof(T) == 4) load(row0 + lane);
+    if (g >= 0) {
+        TriProduct<true> tp(GT + (size_t)g * kGG);
+        double t = 0;
+        const double *zp = zin + (size_t)col * nblk * 2 * kGW + tid;
+        for (int q0 = 0; q0 < nblk; q0 += 8) {
+            double z[8];
+#pragma unroll
+            for (int u = 0; u < 8; u++) z[u] = zp[(size_t)min(q0 + u, nblk - 1) * 2 * kGW];
+#pragma unroll
+            for (int u = 0; u < 8; u++) t += q0 + u < nblk ? z[u] : 0;
+        }
+        ((double *)s_z)[tid] = t;
+        __syncthreads();
+        s_w[tid / kGW][tid % kGW] = tp.apply(s_z);
+        __syncthreads();
+    }
+    double x[2 * kNB];
+#pragma unroll
+    for (int l = 0; l < 2 * kNB; l++) x[l] = 0;
+    for (int r = 0; r < rpb; r += 64) {
+        const int i = row0 + r + lane;
+        if (r || sizeof(T) != 4) load(i);
+        const int il = i - ca, in = i - cb;  // rows of the panels
+        double2 bi = to_d2(braw);
+        if (g >= 0) {
+            double2 sum = make_double2(0.0, 0.0);
+#pragma unroll
+            for (int l = 0; l < kNB; l++) {
+                const double2 v = to_d2(v_entry(va[l], il, l));
+                const double2 w0 = s_w[0][wave * kNB + l], w1 = s_w[1][wave * kNB + l];
+                const double wx = w0.x + w1.x, wy = w0.y + w1.y;
+                sum.x = fma(v.x, wx, fma(-v.y, wy, sum.x));
+                sum.y = fma(v.x, wy, fma(v.y, wx, sum.y));
             }
-        }
-        C2 bl = b[rc];
-        if (lane >= nb) {
-            bl.x = 0;
-            bl.y = 0;
-        }
+            const int h = (r >> 6) & 1;
+            s_part[h][wave][lane] = sum;
+            __syncthreads();
 #pragma unroll
-        for (int m = kNB - 1; m >= 0; m--) {
-            if (m < nb) {
-                C2 xm;
-                const T d = rr[m].x * rr[m].x + rr[m].y * rr[m].y;
-                xm.x = lane == m ? (bl.x * rr[m].x + bl.y * rr[m].y) / d : 0;
-                xm.y = lane == m ? (bl.y * rr[m].x - bl.x * rr[m].y) / d : 0;
-                xm.x = __shfl(xm.x, m, 64);
-                xm.y = __shfl(xm.y, m, 64);
-                if (lane < m) {
-                    bl.x -= rr[m].x * xm.x - rr[m].y * xm.y;
-                    bl.y -= rr[m].x * xm.y + rr[m].y * xm.x;
-                } else if (lane == m) {
-                    bl = xm;
-                }
+            for (int w = 0; w < 4; w++) {
+                bi.x -= s_part[h][w][lane].x;
+                bi.y -= s_part[h][w][lane].y;
             }
+            C2 o;
+            o.x = (T)bi.x;
+            o.y = (T)bi.y;
+            if (wave == 0 && i < M) b[i] = o;
+            bi = to_d2(o);  // (what later launches read)
         }
-        if (lane < nb) {
-            s_x[lane] = bl;
-            if (blockIdx.x == 0) X[(size_t)col * ldx + r] = bl;
+        if (next) {
+            if (i >= M) bi.x = bi.y = 0;
+#pragma unroll
+            for (int l = 0; l < kNB; l++) {
+                const C2 v = v_entry(vb[l], in, l);
+                x[2 * l] = fma((double)v.x, bi.x, fma((double)v.y, bi.y, x[2 * l]));
+                x[2 * l + 1] = fma((double)v.x, bi.y, fma(-(double)v.y, bi.x, x[2 * l + 1]));
+            }
         }
     }
+    if (next) {
+        wave_reduce_scatter64(x, lane);
+        zout[((size_t)col * nblk + blockIdx.x) * 2 * kGW + wave * 2 * kNB + lane] = x[0];
+    }
+}
+
+// One group of R x = b from the bottom: every workgroup forms the group's
+// unknowns R_gg^-1 b_g (b_g is not written in this step), workgroup 0 stores
+// them in X, and every workgroup removes them from its 64 rows above the group,
+// wave w the columns of panel w.  Sums in FP64.
+template <typename T>
+__global__ __launch_bounds__(256) void trsv_group(const typename QT<T>::c2 *__restrict__ A, long lda, int N,
+                                                  const double2 *__restrict__ GR, typename QT<T>::c2 *B, long ldb,
+                                                  typename QT<T>::c2 *__restrict__ X, long ldx, int g) {
+    using C2 = typename QT<T>::c2;
+    __shared__ double2 s_b[kGW], s_x[2][kGW], s_part[4][64];
+    const int tid = threadIdx.x, lane = tid & 63, col = blockIdx.y;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int c0 = g * kGW, i = blockIdx.x * 64 + lane, ic = min(i, c0 > 0 ? c0 - 1 : 0);
+    C2 *b = B + (size_t)col * ldb;
+    C2 v[kNB];
+    const C2 braw = b[ic];
+#pragma unroll
+    for (int l = 0; l < kNB; l++) v[l] = A[(size_t)min(c0 + wave * kNB + l, N - 1) * lda + ic];
+    TriProduct<false> tp(GR + (size_t)g * kGG);
+    if (tid < kGW) s_b[tid] = c0 + tid < N ? to_d2(b[c0 + tid]) : make_double2(0.0, 0.0);
     __syncthreads();
-    const int i = blockIdx.x * NT + tid;
-    if (i < c0) {
-        T sr = 0, si = 0;
+    s_x[tid / kGW][tid % kGW] = tp.apply(s_b);
+    __syncthreads();
+    if (blockIdx.x == 0 && tid < kGW && c0 + tid < N) {
+        C2 x;
+        x.x = (T)(s_x[0][tid].x + s_x[1][tid].x);
+        x.y = (T)(s_x[0][tid].y + s_x[1][tid].y);
+        X[(size_t)col * ldx + c0 + tid] = x;
+    }
+    double2 sum = make_double2(0.0, 0.0);
 #pragma unroll
-        for (int m0 = 0; m0 < kNB; m0 += kCG) {
-            C2 raw[kCG];
+    for (int l = 0; l < kNB; l++) {
+        const double2 x0 = s_x[0][wave * kNB + l], x1 = s_x[1][wave * kNB + l], a = to_d2(v[l]);
+        const bool in = c0 + wave * kNB + l < N;
+        const double xx = in ? x0.x + x1.x : 0, xy = in ? x0.y + x1.y : 0;
+        sum.x = fma(a.x, xx, fma(-a.y, xy, sum.x));
+        sum.y = fma(a.x, xy, fma(a.y, xx, sum.y));
+    }
+    s_part[wave][lane] = sum;
+    __syncthreads();
+    if (wave == 0 && i < c0) {
+        double2 bi = to_d2(braw);
 #pragma unroll
-            for (int u = 0; u < kCG; u++) raw[u] = A[(size_t)min(c0 + m0 + u, N - 1) * lda + i];
-#pragma unroll
-            for (int u = 0; u < kCG; u++) {
-                if (m0 + u < nb) {
-                    sr += raw[u].x * s_x[m0 + u].x - raw[u].y * s_x[m0 + u].y;
-                    si += raw[u].x * s_x[m0 + u].y + raw[u].y * s_x[m0 + u].x;
-                }
-            }
+        for (int w = 0; w < 4; w++) {
+            bi.x -= s_part[w][lane].x;
+            bi.y -= s_part[w][lane].y;
         }
-        b[i].x -= sr;
-        b[i].y -= si;
+        C2 o;
+        o.x = (T)bi.x;
+        o.y = (T)bi.y;
+        b[i] = o;
     }
 }
 
@@ -1206,6 +1426,8 @@ struct QRFactor {
     float2 *Pc = nullptr;
     double2 *gram = nullptr, *Y = nullptr;
     int *bad = nullptr;
+    // triangles of the groups of panels, for the solves
+    double2 *GT = nullptr, *GR = nullptr;
     hipStream_t st = nullptr;
     ~QRFactor() {
         sfree(Tb, st);
@@ -1217,6 +1439,8 @@ struct QRFactor {
         sfree(gram, st);
         sfree(Y, st);
         sfree(bad, st);
+        sfree(GT, st);
+        sfree(GR, st);
     }
 };
 
@@ -1322,17 +1546,40 @@ static int qr_factor(QRFactor<T> &f, int extra_cols, hipStream_t s) {
     return EXIT_SUCCESS;
 }
 
+// The triangles of the groups of panels (qr_cross, qr_group), once per
+// factorisation.  The cross products split their rows over up to 16 workgroups
+// while there are few groups.
+template <typename T>
+static int qr_groups(QRFactor<T> &f, hipStream_t s) {
+    if (f.GT) return EXIT_SUCCESS;
+    const int np = (f.N + kNB - 1) / kNB, ng = (np + kGB - 1) / kGB;
+    const int npair = ng * kPairs, nsplit = std::max(1, std::min(16, 1024 / npair));
+    double2 *cross = nullptr, *rinv = nullptr;
+    HOST_CALL(salloc(&f.GT, (size_t)ng * kGG, s));
+    HOST_CALL(salloc(&f.GR, (size_t)ng * kGG, s));
+    HOST_CALL(salloc(&cross, (size_t)npair * nsplit * kNN, s));
+    int rc = salloc(&rinv, (size_t)np * kNN, s);
+    if (rc == EXIT_SUCCESS) {
+        qr_cross<T><<<npair * nsplit + np, 256, 0, s>>>(f.A, f.lda, f.M, f.N, npair, nsplit, cross, rinv);
+        qr_group<T><<<dim3(ng, kGB, 2), 1024, 0, s>>>(f.A, f.lda, f.N, f.Tb, cross, nsplit, rinv, f.GT, f.GR);
+        if (hipGetLastError() != hipSuccess) rc = EXIT_FAILURE;
+    }
+    sfree(cross, s);
+    sfree(rinv, s);
+    if (rc != EXIT_SUCCESS) BEM_FAIL("QR solve launches failed");
+    return EXIT_SUCCESS;
+}
+
 // Least squares solve with a factored A: B (M x R, ldb) <- solution in B[0:N].
 constexpr size_t kSmallSolveLds = 48 * 1024;  // b of up to 6144 FP32 / 3072 FP64 rows
 constexpr int kSmallSolveRhs = 64;
 
 template <typename T>
-static int qr_solve_factored(const QRFactor<T> &f, typename QT<T>::c2 *B, long ldb, int R, hipStream_t s) {
+static int qr_solve_factored(QRFactor<T> &f, typename QT<T>::c2 *B, long ldb, int R, hipStream_t s) {
     using C2 = typename QT<T>::c2;
     if (R <= 0) return EXIT_SUCCESS;
     // the whole solve in one workgroup per right-hand side, b in shared memory
-    // (on request; the row-split launches below measured faster at every size
-    // from 129 to 4096 rows)
+    // (on request; the row-split launches below are faster at every size)
     const size_t lds = sizeof(C2) * (size_t)f.M;
     if (lds <= kSmallSolveLds && R <= kSmallSolveRhs && getenv("BEM_QR_ONE_WG_SOLVE")) {
         // 2 kNB partial sums per thread plus a chunk of 8 loads: the register
@@ -1348,26 +1595,24 @@ static int qr_solve_factored(const QRFactor<T> &f, typename QT<T>::c2 *B, long l
         HIP_CALL(hipGetLastError());
         return EXIT_SUCCESS;
     }
-    // one launch per panel for Q^H B and one per block column for the back
-    // substitution, the rows spread over workgroups
-    constexpr int nt = 256;
-    const int np = (f.N + kNB - 1) / kNB;
-    const int nblk = (f.M + nt - 1) / nt;
-    T *zb = nullptr;
+    // one launch per group of panels for Q^H B and one for the back
+    // substitution, the rows spread over at most 64 workgroups
+    HOST_CALL(qr_groups<T>(f, s));
+    const int ng = ((f.N + kNB - 1) / kNB + kGB - 1) / kGB;
+    const int rpb = 64 * ((f.M + 64 * 64 - 1) / (64 * 64)), nblk = (f.M + rpb - 1) / rpb;
+    const size_t zn = (size_t)R * nblk * 2 * kGW;
+    double *zb = nullptr;
     C2 *X = nullptr;
-    HOST_CALL(salloc(&zb, (size_t)2 * R * nblk * 2 * kNB, s));
-    HOST_CALL(salloc(&X, (size_t)f.N * R, s));
-    int rc = EXIT_SUCCESS;
-    for (int p = -1; p < np && rc == EXIT_SUCCESS; p++) {
-        const T *zin = zb + (size_t)((p + 2) & 1) * R * nblk * 2 * kNB;
-        T *zout = zb + (size_t)((p + 1) & 1) * R * nblk * 2 * kNB;
-        qr_apply_step<T, nt><<<dim3(nblk, R), nt, 0, s>>>(f.A, f.lda, f.M, f.N, f.Tb, B, ldb, p, zin, zout, nblk);
+    HOST_CALL(salloc(&zb, 2 * zn, s));
+    int rc = salloc(&X, (size_t)f.N * R, s);
+    for (int g = -1; g < ng && rc == EXIT_SUCCESS; g++) {
+        qr_apply_group<T><<<dim3(nblk, R), 256, 0, s>>>(f.A, f.lda, f.M, f.N, f.GT, B, ldb, g, ng, rpb,
+                                                        zb + (g & 1) * zn, zb + ((g + 1) & 1) * zn, nblk);
         if (hipGetLastError() != hipSuccess) rc = EXIT_FAILURE;
     }
-    for (int p = np - 1; p >= 0 && rc == EXIT_SUCCESS; p--) {
-        const int c0 = p * kNB, nb = std::min(kNB, f.N - c0);
-        const int g = std::max(1, (c0 + nt - 1) / nt);
-        trsv_block_step<T, nt><<<dim3(g, R), nt, 0, s>>>(f.A, f.lda, f.N, B, ldb, X, f.N, c0, nb);
+    for (int g = ng - 1; g >= 0 && rc == EXIT_SUCCESS; g--) {
+        const unsigned rows = std::max(1, g * kGW / 64);
+        trsv_group<T><<<dim3(rows, R), 256, 0, s>>>(f.A, f.lda, f.N, f.GR, B, ldb, X, f.N, g);
         if (hipGetLastError() != hipSuccess) rc = EXIT_FAILURE;
     }
     if (rc == EXIT_SUCCESS &&
