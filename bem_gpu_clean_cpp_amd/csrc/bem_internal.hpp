@@ -351,6 +351,7 @@ int gemm_n_f32z_batched(const float2 *A, long lda, long astride, int nmat, long 
                         ProdParts *parts = nullptr);
 int mres_f32a_batched(const float2 *A, long lda, long astride, int nmat, long M, long N, const double2 *X, long ldx,
                       const double2 *b, long ldb, double2 *out, long ldo, int R, void *ws, hipStream_t s);
+size_t qr_work_bytes(int M, int N, bool fp64);
 // C -= V (T^H (V^H C)) from the partials of C^H V (QR trailing update, V with 32
 // columns)
 int qr_trail_f32(const float2 *V, long ldv, int M, const float2 *T, int nb, const ProdParts &zp, int nc, float2 *C,

@@ -1546,6 +1546,19 @@ static int qr_factor(QRFactor<T> &f, int extra_cols, hipStream_t s) {
     return EXIT_SUCCESS;
 }
 
+static int group_splits(int npair) { return std::max(1, std::min(16, 1024 / npair)); }
+
+// device bytes of a factorisation beyond the matrix, and of the largest solve's
+// scratch that does not grow with the right-hand sides
+size_t qr_work_bytes(int M, int N, bool fp64) {
+    const size_t np = ((size_t)N + kNB - 1) / kNB, ng = (np + kGB - 1) / kGB, ld = ((size_t)M + 63) / 64 * 64;
+    const size_t splits = group_splits((int)(ng * kPairs));
+    size_t b = (fp64 ? sizeof(double2) : sizeof(float2)) * kNB * (np * kNB + N);   // T factors, W
+    b += sizeof(double2) * (2 * ng * kGG + (ng * kPairs * splits + np) * kNN);       // triangles and what forms them
+    if (!fp64) b += sizeof(float2) * 2 * kNB * ld + sizeof(double2) * (kGramParts + 1) * kNN;  // V, panel, Gram
+    return b;
+}
+
 // The triangles of the groups of panels (qr_cross, qr_group), once per
 // factorisation.  The cross products split their rows over up to 16 workgroups
 // while there are few groups.
@@ -1553,7 +1566,7 @@ template <typename T>
 static int qr_groups(QRFactor<T> &f, hipStream_t s) {
     if (f.GT) return EXIT_SUCCESS;
     const int np = (f.N + kNB - 1) / kNB, ng = (np + kGB - 1) / kGB;
-    const int npair = ng * kPairs, nsplit = std::max(1, std::min(16, 1024 / npair));
+    const int npair = ng * kPairs, nsplit = group_splits(npair);
     double2 *cross = nullptr, *rinv = nullptr;
     HOST_CALL(salloc(&f.GT, (size_t)ng * kGG, s));
     HOST_CALL(salloc(&f.GR, (size_t)ng * kGG, s));

@@ -180,7 +180,7 @@ double bem_request_footprint(int M, int N, int E, int nrhs, int precision, int m
     b += (2 * sizeof(double2) + sizeof(float2)) * ld * R;           // B, X (FP64), X (FP32)
     if (method == BEM_SOLVE_QR) {
         b += ea * ld * N;                                           // factored copy of A
-        b += sizeof(float2) * 32 * (ld + 32 * ((N + 31) / 32));     // block reflectors, T factors
+        b += qr_work_bytes(M, N, precision == BEM_PREC_FP64);       // panels, T factors, triangles of the solves
         b += 2 * sizeof(double2) * ld + ws_gemv_n(M, N, 1);
     } else {
         const size_t K = (size_t)std::max(1, std::min(restart, N));
