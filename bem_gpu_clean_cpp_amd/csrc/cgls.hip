@@ -268,7 +268,21 @@ __global__ void kc_act_init(int R, const double *__restrict__ g0, const int *__r
 
 // ------------------------------------------------------------ block CG ---
 constexpr int kMaxBlock = 64;    // right-hand sides of one block (Rb <= 64)
-constexpr double kBlockMinWork = 4e8;  // M N R below which block CG takes the lockstep iteration
+// Whether the block iteration repays its steps' fixed cost (three dozen small
+// launches, a host wait and the R x R algebra on the host: 0.08 ms up to 4
+// right-hand sides, 0.1 at 16, 0.3 at 32) against lockstep CG steps of
+// 20 us + 3 us per 1e6 of M N.  Solves of 16 CHIEF points to 1e-8, lockstep over
+// block time at an easy and a hard frequency (ka 5 and 16 at 4002 nodes):
+//   up to 16 right-hand sides, by the reads of the matrix they save:
+//     4002 nodes, R = 8: 1.03, 1.77; R = 16: 1.07, 2.5; 4842, R = 6: 1.35, 1.6;
+//     6252, R = 4: 1.10, 1.6; R = 16: 1.75, 4.2; 7842, R = 2: 1.07, 1.04;
+//     but 3242, R = 16: 0.83, 1.7; 4002, R = 6: 0.9, 1.5; 6252, R = 2: 0.8, 0.95;
+//   more than 16, where the host algebra grows: 2562, R = 32: 0.6, 1.05;
+//     3242, R = 32: 0.65, 1.25; 4002, R = 32: 0.7, 1.8; 10242, R = 32: 1.5.
+static bool block_pays(double M, double N, double R) {
+    const double mn = M * N;
+    return mn * R >= 4e8 || (R <= 16 && mn >= 1.5e7 && mn * R >= 1.2e8);
+}
 constexpr int kGramRows = 64;    // rows of one Gram partial
 constexpr int kGramSub = 32;     // rows staged in LDS at a time
 constexpr int kGramSegs = 16;    // first-level groups of partials in the sum
@@ -633,14 +647,8 @@ int cgls_device(const float2 *A32, const double2 *A64, long lda, int M, int N, c
     HOST_CALL(salloc(&w.act, 2 * (size_t)R, s));
     HOST_CALL(salloc(&w.done, R, s));
     HOST_CALL(salloc(&w.gws, std::max(std::max(ws_gemv_n(M, N, 1), ws_gemm(M, N, R)), ws_mres(M, N, R)), s));
-    // Block steps pay three dozen small launches, a host wait and the R x R
-    // algebra on the host (about 0.1 ms at R = 16, 0.3 ms at R = 32); below
-    // about 4e8 of M N R a lockstep CG step is that cheap that the block's
-    // 2x fewer steps do not repay it (s4 with 16 right-hand sides: 7.9 ms
-    // against 4.8 ms; s5 with 32: 33.5 ms against 51.3 ms).  BEM_BLOCK_CG_ALWAYS
-    // takes the block at every size.
-    bool block_on = block && R > 1 &&
-                    ((double)M * (double)N * (double)R >= kBlockMinWork || getenv("BEM_BLOCK_CG_ALWAYS"));
+    // (BEM_BLOCK_CG_ALWAYS takes the block at every size)
+    bool block_on = block && R > 1 && (block_pays(M, N, R) || getenv("BEM_BLOCK_CG_ALWAYS"));
     // FP16-split block products: A and the block vectors read as FP16 hi/lo
     // pairs on FP16 MFMA; the adjoint product reads the conjugate-transposed
     // copy, which also leaves the bound amax on |Re A|, |Im A| (per-tile

@@ -54,3 +54,21 @@ def test_cg_stops_at_the_limit(maxit):
     X = s.solution()
     s.close()
     assert st["iterations"] == maxit and np.isfinite(X).all()
+
+
+# more than 1.2e8 of M N nrhs and 1.5e7 of M N at 16 or fewer right-hand sides: the
+# block iteration, whose steps are fewer; one system less: the lockstep one
+@pytest.mark.parametrize("R,block", [(1, False), (2, True)])
+def test_block_size_policy_few_right_hand_sides(R, block):
+    m, k, s, dirs = _problem(5, 16, R)
+    st = s.solve(bem.SOLVE_BLOCK_CG, tol=1e-6, maxit=6000, refine_tol=1e-10, max_refine=50)
+    X = s.solution()
+    sl = s.solve(bem.SOLVE_CGLS, tol=1e-6, maxit=6000, refine_tol=1e-10, max_refine=50)
+    Xl = s.solution()
+    s.close()
+    print("case:", st, sl, flush=True)
+    assert st["converged"] == 1 and sl["converged"] == 1
+    assert (st["iterations"] < sl["iterations"]) == block
+    assert block or np.array_equal(X, Xl)
+    # both to 1e-10 on the normal equations (condition numbers as above)
+    assert np.linalg.norm(X - Xl) <= 1e-5 * np.linalg.norm(Xl)
