@@ -330,7 +330,7 @@ __device__ __forceinline__ void wave_reduce_scatter64<float>(float (&x)[2 * kNB]
 // not finite) and those with a column that needs no reflection take the
 // column-wise algorithm inside qr_recon instead.
 //
-// 5 + 36 + 5 us a panel of up to 2000 rows.  The column-wise panels that this
+// 5 + 32 + 5 us a panel of up to 2000 rows.  The column-wise panels that this
 // replaces were bound by their 32 serial steps: 69 us (256 rows), 98 (512) and
 // 135 (1024) with the panel in one workgroup's registers, 330 + 40 us with a
 // launch per column above.  With qr_trail, a QR solve of 642 nodes went from
@@ -407,27 +407,6 @@ __device__ __forceinline__ double2 zfms(double2 c, double2 a, double2 b) {  // c
     return make_double2(fma(-a.x, b.x, fma(a.y, b.y, c.x)), fma(-a.x, b.y, fma(-a.y, b.x, c.y)));
 }
 
-// The reflectors of a panel from the partials of its Gram matrix: R (above and
-// on the diagonal) and L (below it) to the top rows of the panel, T to Tout,
-// the top rows of V to Vd, U^-1 to Y (row-major), *bad = 0.  Panels that the
-// reconstruction does not take (above) are factored column by column instead,
-// with T, and *bad = 1.
-//
-// One workgroup; thread t holds the entries (i, j), i = t / 32 + kRowStep e,
-// j = t % 32, of two matrices that are eliminated in place and in step: G and
-// P_1 - S R.  Step k needs row k of R only, which is row k of G's elimination
-// scaled, so both take one barrier a step: the rows and columns k of both as
-// they stand go through shared memory, and every thread finishes the pivots for
-// itself.  The update is one multiply-add per entry without a condition: the
-// pivot entry of a published row is 1 and that of a column -1, and the
-// publishing threads clear the entries that start anew (inverse of row and
-// column k).  Afterwards G holds U0^-1 (j >= i), and P_1 - S R holds U^-1
-// (j >= i) and L^-1 (j < i); U0, U and L follow from the published rows and
-// columns.  36 us, bound by the 32 steps (0.8 us each: the FP64 chain of the
-// pivots, two rounds through shared memory, a barrier); 256 threads 41 us, 1024
-// 37; the two eliminations one after the other 45.  (Entries are separate
-// doubles: branches on whole entries, or a select of their addresses, put them
-// in scratch memory: 93 us.)
 // R_kk = d rd from the pivot d of G, and for the pivot p of the top rows
 // s = -phase(p) and 1 / (p - s R_kk) = -conj(s) / (|p| + R_kk)
 struct PanelPivot {
@@ -441,101 +420,128 @@ struct PanelPivot {
         inv = make_double2(-s.x * q, s.y * q);
     }
 };
-constexpr int kRecThreads = 512;
-constexpr int kRowStep = kRecThreads / kNB, kEnt = kNN / kRecThreads;
+
+// The reflectors of a panel from the partials of its Gram matrix: R (above and
+// on the diagonal) and L (below it) to the top rows of the panel, T to Tout,
+// the top rows of V to Vd, U^-1 to Y (row-major), *bad = 0.  Panels that the
+// reconstruction does not take (above) are factored column by column instead,
+// with T, and *bad = 1.
+//
+// One workgroup eliminates two matrices in place and in step: G and P_1 - S R.
+// Step k needs row k of R only, which is row k of G's elimination scaled, so
+// both take one barrier a step: the rows and columns k of both as they stand go
+// through shared memory, and every thread finishes the pivots for itself.  Wave
+// w holds the rows w + 8 e (e < 4), lanes 0..31 the columns of G, lanes 32..63
+// those of P_1 - S R, so that what depends on the row is known to the wave.  The
+// update is one multiply-add per entry: the pivot entry of a published row is 1
+// and that of a column -1, and the publishing threads clear the entries that
+// start anew (inverse of row and column k).  Afterwards G holds U0^-1 (j >= i),
+// and P_1 - S R holds U^-1 (j >= i) and L^-1 (j < i); U0, U and L follow from the
+// published rows and columns.
+// 32 us, 21 of them the 32 steps (the FP64 chain of the pivots, a round through
+// shared memory and a barrier each).  Both matrices in every thread, the row
+// conditions per lane: 36 us; 256 or 1024 threads 37 to 41; the two eliminations
+// one after the other 45.  (Entries are separate doubles: branches on whole
+// entries, or a select of their addresses, put them in scratch memory: 93 us.)
+constexpr int kRecThreads = 512, kRecWaves = kRecThreads / 64, kEnt = kNB / kRecWaves;
 __global__ __launch_bounds__(kRecThreads) void qr_recon(const double2 *__restrict__ part, int nblk, float2 *A, long lda,
                                                         int M, int j0, int nb, float2 *__restrict__ Tout,
                                                         float2 *__restrict__ Vd, long ldv, double2 *__restrict__ Y,
                                                         int *__restrict__ bad) {
-    __shared__ double2 s_ra[kNB][kNB + 1], s_rb[kNB][kNB + 1], s_cb[kNB][kNB + 1];  // published rows, columns
-    __shared__ double2 s_ca[2][kNB];
-    __shared__ double2 s_pb[kNB], s_sign[kNB], s_u[kNB], s_inv[kNB];
-    __shared__ double s_pa[kNB], s_g[kNB], s_w[kRecThreads / 64];
+    __shared__ double2 s_row[2][kNB][kNB];   // published rows of G and P_1 - S R
+    __shared__ double2 s_cw[kNB][kNB + 1];   // published columns of P_1 - S R
+    __shared__ double2 s_cg[2][kNB];         // and of G (two buffers)
+    __shared__ double2 s_piv[2][kNB], s_sign[kNB], s_u[kNB], s_inv[kNB];
+    __shared__ double s_g[kNB], s_w[kRecWaves];
     __shared__ int s_flat;
-    const int tid = threadIdx.x, i0 = tid >> 5, j = tid & 31;
+    const int tid = threadIdx.x, lane = tid & 63, j = tid & 31;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const bool top = lane >= kNB;  // this lane's matrix is P_1 - S R
     const int Mp = M - j0;
-    double gx[kEnt], gy[kEnt], wx[kEnt], wy[kEnt];  // entries of G and of P_1 - S R
+    double x[kEnt], y[kEnt];
     {
-        double2 v[kEnt][kGramParts];
+        // the lanes of either matrix sum half of the partials of G
+        constexpr int kHalf = kGramParts / 2;
+        double2 v[kEnt][kHalf];
+        const int b0 = top ? kHalf : 0;
 #pragma unroll
         for (int e = 0; e < kEnt; e++)
 #pragma unroll
-            for (int b = 0; b < kGramParts; b++)
-                v[e][b] = part[(size_t)min(b, nblk - 1) * kNN + tid + kRecThreads * e];
+            for (int b = 0; b < kHalf; b++)
+                v[e][b] = part[(size_t)min(b0 + b, nblk - 1) * kNN + (w + kRecWaves * e) * kNB + j];
 #pragma unroll
         for (int e = 0; e < kEnt; e++) {
-            const int i = i0 + kRowStep * e;
-            float2 top = make_float2(0.f, 0.f);
-            if (i < Mp && j < nb) top = A[(size_t)(j0 + j) * lda + j0 + i];
-            wx[e] = top.x;
-            wy[e] = top.y;
-            double x = 0, y = 0;
+            const int i = w + kRecWaves * e;
+            float2 t = make_float2(0.f, 0.f);
+            if (i < Mp && j < nb) t = A[(size_t)(j0 + j) * lda + j0 + i];
+            double gx = 0, gy = 0;
 #pragma unroll
-            for (int b = 0; b < kGramParts; b++) {
-                x += b < nblk ? v[e][b].x : 0.0;
-                y += b < nblk ? v[e][b].y : 0.0;
+            for (int b = 0; b < kHalf; b++) {
+                gx += b0 + b < nblk ? v[e][b].x : 0.0;
+                gy += b0 + b < nblk ? v[e][b].y : 0.0;
             }
+            gx += __shfl_xor(gx, 32, 64);
+            gy += __shfl_xor(gy, 32, 64);
             const bool in = i < nb && j < nb;
-            gx[e] = in ? x : i == j ? 1.0 : 0.0;
-            gy[e] = in ? y : 0.0;
-            if (i == j) s_g[i] = gx[e];  // |P_i|^2
+            gx = in ? gx : i == j ? 1.0 : 0.0;
+            gy = in ? gy : 0.0;
+            if (i == j) s_g[i] = gx;  // |P_i|^2
+            x[e] = top ? (double)t.x : gx;
+            y[e] = top ? (double)t.y : gy;
         }
     }
     if (tid == 0) s_flat = 0;
-    for (int k = 0; k < kNB; k++) {
-        const int b = k & 1;
+    double2 *const myrow = &s_row[top][0][0];
 #pragma unroll
-        for (int e = 0; e < kEnt; e++) {
-            const int i = i0 + kRowStep * e;
+    for (int ek = 0; ek < kEnt; ek++) {  // k = kRecWaves ek + kw: row k is entry ek of wave kw
+        for (int kw = 0; kw < kRecWaves; kw++) {
+            const int k = kRecWaves * ek + kw;
             const bool at = j == k;
-            if (i == k) {
-                s_ra[k][j] = make_double2(at ? 1.0 : j > k ? gx[e] : 0.0, j > k ? gy[e] : 0.0);
-                s_rb[k][j] = make_double2(at ? 1.0 : wx[e], at ? 0.0 : wy[e]);
-            }
-            if (at) {
-                s_ca[b][i] = make_double2(i == k ? -1.0 : gx[e], i == k ? 0.0 : gy[e]);
-                s_cb[k][i] = make_double2(i == k ? -1.0 : wx[e], i == k ? 0.0 : wy[e]);
-                if (i == k) {
-                    s_pa[k] = gx[e];
-                    s_pb[k] = make_double2(wx[e], wy[e]);
+            double2 *const col = top ? s_cw[k] : s_cg[k & 1];
+            if (w == kw) {
+                const bool none = !top && j < k;
+                myrow[k * kNB + j] = make_double2(at ? 1.0 : none ? 0.0 : x[ek], at || none ? 0.0 : y[ek]);
+                if (at) s_piv[top][k] = make_double2(x[ek], y[ek]);
+                if (j >= k) {
+                    x[ek] = at ? -1.0 : 0.0;
+                    y[ek] = 0.0;
                 }
             }
-            const bool fresh = at || (i == k && j > k);
-            gx[e] = fresh ? 0.0 : gx[e];
-            gy[e] = fresh ? 0.0 : gy[e];
-            wx[e] = fresh ? 0.0 : wx[e];
-            wy[e] = fresh ? 0.0 : wy[e];
-        }
-        __syncthreads();
-        const double d = s_pa[k];
-        const double2 p = s_pb[k], ra = s_ra[k][j], rw = s_rb[k][j];
-        double2 ca[kEnt], cb[kEnt];
+            if (at) {
 #pragma unroll
-        for (int e = 0; e < kEnt; e++) {
-            ca[e] = s_ca[b][i0 + kRowStep * e];
-            cb[e] = s_cb[k][i0 + kRowStep * e];
-        }
-        const PanelPivot pv(d, p);
-        const double di = pv.rd * pv.rd;
-        const double tx = j > k ? ra.x * pv.rd : 0.0, ty = j > k ? ra.y * pv.rd : 0.0;  // R_kj
-        const double2 rb = zfms(rw, pv.s, make_double2(tx, ty));
+                for (int e = 0; e < kEnt; e++) {
+                    col[w + kRecWaves * e] = make_double2(x[e], y[e]);
+                    x[e] = 0.0;
+                    y[e] = 0.0;
+                }
+            }
+            __syncthreads();
+            const double2 ra = s_row[0][k][j], rw = s_row[1][k][j];
+            double2 c[kEnt];
 #pragma unroll
-        for (int e = 0; e < kEnt; e++) {
-            const double ax = ca[e].x * di, ay = ca[e].y * di;
-            gx[e] = fma(-ax, ra.x, fma(ay, ra.y, gx[e]));
-            gy[e] = fma(-ax, ra.y, fma(-ay, ra.x, gy[e]));
+            for (int e = 0; e < kEnt; e++) c[e] = col[w + kRecWaves * e];
+            const PanelPivot pv(s_piv[0][k].x, s_piv[1][k]);
+            const double tx = j > k ? ra.x * pv.rd : 0.0, ty = j > k ? ra.y * pv.rd : 0.0;  // R_kj
+            const double2 rb = zfms(rw, pv.s, make_double2(tx, ty));
+            const double rx = top ? rb.x : ra.x, ry = top ? rb.y : ra.y;
+            const double ix = top ? pv.inv.x : pv.rd * pv.rd, iy = top ? pv.inv.y : 0.0;
             // rows up to k keep their entries left of column k
-            const bool old = j < k && i0 + kRowStep * e <= k;
-            const double2 f = zmul(cb[e], pv.inv);
-            const double bx = old ? 0.0 : f.x, by = old ? 0.0 : f.y;
-            wx[e] = fma(-bx, rb.x, fma(by, rb.y, wx[e]));
-            wy[e] = fma(-bx, rb.y, fma(-by, rb.x, wy[e]));
+            const double mx = j < k ? 0.0 : rx, my = j < k ? 0.0 : ry;
+            const bool below = w > kw;
+            const double ex = below ? rx : mx, ey = below ? ry : my;
+#pragma unroll
+            for (int e = 0; e < kEnt; e++) {
+                const double fx = fma(c[e].x, ix, -c[e].y * iy), fy = fma(c[e].x, iy, c[e].y * ix);
+                const double qx = e > ek ? rx : e < ek ? mx : ex, qy = e > ek ? ry : e < ek ? my : ey;
+                x[e] = fma(-fx, qx, fma(fy, qy, x[e]));
+                y[e] = fma(-fx, qy, fma(-fy, qx, y[e]));
+            }
         }
     }
     __syncthreads();
     if (tid < kNB) {
-        const double d = s_pa[tid];
-        const double2 p = s_pb[tid];
+        const double d = s_piv[0][tid].x;
+        const double2 p = s_piv[1][tid];
         const PanelPivot pv(d, p);
         s_sign[tid] = pv.s;
         s_inv[tid] = pv.inv;
@@ -545,82 +551,86 @@ __global__ __launch_bounds__(kRecThreads) void qr_recon(const double2 *__restric
     }
     __syncthreads();
     // G = U0^H D^-1 U0, D = diag(U0): R = D^-1/2 U0, R^-1 = U0^-1 D^1/2; the
-    // condition number of the panel with its columns scaled to norm 1
-    double2 R[kEnt], U[kEnt], L[kEnt], Ri[kEnt];
-    const double2 sgn = s_sign[j], inv = s_inv[j];
+    // condition number of the panel with its columns scaled to norm 1.  The lanes
+    // of G form Ri = R^-1 S^H and R_h = S R, those of P_1 - S R form -U and L.
+    double2 first[kEnt], second[kEnt];
     double k2 = 0;
-    const double dj = s_pa[j], rj = dj * rsq_step(dj);
+    {
+        const double2 sgn = s_sign[j], inv = s_inv[j];
+        const double dj = s_piv[0][j].x, rj = dj * rsq_step(dj);
 #pragma unroll
-    for (int e = 0; e < kEnt; e++) {
-        const int i = i0 + kRowStep * e;
-        const bool up = j >= i, off = j > i;
-        const double ri = rsq_step(s_pa[i]);
-        const double2 ra = s_ra[i][j], rb = s_rb[i][j], cb = s_cb[j][i], ui = s_u[i];
-        const double2 r = make_double2(off ? ra.x * ri : 0.0, off ? ra.y * ri : 0.0);
-        const double2 u = zfms(rb, s_sign[i], r), l = zmul(cb, inv);
-        R[e] = make_double2(j == i ? rj : r.x, r.y);
-        U[e] = make_double2(off ? u.x : j == i ? ui.x : 0.0, off ? u.y : j == i ? ui.y : 0.0);
-        L[e] = make_double2(up ? (j == i ? 1.0 : 0.0) : l.x, up ? 0.0 : l.y);
-        Ri[e] = make_double2(up ? gx[e] * rj : 0.0, up ? gy[e] * rj : 0.0);
-        k2 = fma(kNB * s_g[i], fma(Ri[e].x, Ri[e].x, Ri[e].y * Ri[e].y), k2);
+        for (int e = 0; e < kEnt; e++) {
+            const int i = w + kRecWaves * e;
+            const bool up = j >= i, off = j > i;
+            const double ri = rsq_step(s_piv[0][i].x);
+            const double2 ra = s_row[0][i][j], si = s_sign[i], ui = s_u[i];
+            const double2 r = make_double2(off ? ra.x * ri : 0.0, off ? ra.y * ri : 0.0);
+            const double2 Rh = zmul(si, make_double2(j == i ? rj : r.x, r.y));
+            const double2 Ri = make_double2(up ? x[e] * rj : 0.0, up ? y[e] * rj : 0.0);
+            const double2 Ris = zmul(Ri, make_double2(sgn.x, -sgn.y));
+            const double2 u = zfms(s_row[1][i][j], si, r), l = zmul(s_cw[j][i], inv);
+            k2 = top ? 0.0 : fma(kNB * s_g[i], fma(Ri.x, Ri.x, Ri.y * Ri.y), k2);
+            first[e].x = !top ? Ris.x : off ? -u.x : j == i ? -ui.x : 0.0;
+            first[e].y = !top ? Ris.y : off ? -u.y : j == i ? -ui.y : 0.0;
+            second[e].x = !top ? Rh.x : up ? (j == i ? 1.0 : 0.0) : l.x;
+            second[e].y = !top ? Rh.y : up ? 0.0 : l.y;
+        }
     }
 #pragma unroll
     for (int m = 32; m >= 1; m >>= 1) k2 += __shfl_xor(k2, m, 64);
-    if ((tid & 63) == 0) s_w[tid >> 6] = k2;
+    if (lane == 0) s_w[w] = k2;
     __syncthreads();
     k2 = 0;
 #pragma unroll
-    for (int w = 0; w < kRecThreads / 64; w++) k2 += s_w[w];
+    for (int q = 0; q < kRecWaves; q++) k2 += s_w[q];
     if (!(k2 <= kPanelCond2) || s_flat) {  // (also NaN)
         __syncthreads();
-        panel_one_wg<float>(A, lda, M, j0, nb, Tout, 1, (float2(*)[kNB])&s_ra[0][0], (float2(*)[kNB])&s_rb[0][0]);
+        panel_one_wg<float>(A, lda, M, j0, nb, Tout, 1, (float2(*)[kNB])&s_row[0][0][0],
+                            (float2(*)[kNB])&s_row[1][0][0]);
         if (tid == 0) *bad = 1;
         return;
     }
     if (tid == 0) *bad = 0;
-    // T = -U (R^-1 S^H) L^-H
-    double2 t[kEnt];
+    // T = -U (R^-1 S^H) L^-H: rows of entries 2 top, 2 top + 1 of the wave
 #pragma unroll
     for (int e = 0; e < kEnt; e++) {
-        const int i = i0 + kRowStep * e;
-        s_ra[i][j] = zmul(Ri[e], make_double2(sgn.x, -sgn.y));
-        s_rb[j][i] = make_double2(i == j ? 1.0 : j > i ? 0.0 : wx[e], j >= i ? 0.0 : -wy[e]);  // L^-H
-        s_cb[i][j] = make_double2(-U[e].x, -U[e].y);
-        t[e] = make_double2(0.0, 0.0);
+        const int i = w + kRecWaves * e;
+        s_row[top][i][j] = first[e];
+        if (top) s_cw[j][i] = make_double2(i == j ? 1.0 : j > i ? 0.0 : x[e], j >= i ? 0.0 : -y[e]);  // L^-H
     }
-    __syncthreads();
+    const int e0 = top ? kEnt / 2 : 0;
+    double2 t[kEnt / 2];
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+        __syncthreads();
+#pragma unroll
+        for (int e = 0; e < kEnt / 2; e++) t[e] = make_double2(0.0, 0.0);
 #pragma unroll 4
-    for (int k = 0; k < kNB; k++) {
-        const double2 y = s_rb[k][j];
+        for (int k = 0; k < kNB; k++) {
+            const double2 v = s_cw[k][j];
 #pragma unroll
-        for (int e = 0; e < kEnt; e++) t[e] = zfms(t[e], s_ra[i0 + kRowStep * e][k], y);
-    }
-    __syncthreads();
+            for (int e = 0; e < kEnt / 2; e++) t[e] = zfms(t[e], s_row[h][w + kRecWaves * (e0 + e)][k], v);
+        }
+        __syncthreads();
 #pragma unroll
-    for (int e = 0; e < kEnt; e++) {
-        s_rb[i0 + kRowStep * e][j] = t[e];
-        t[e] = make_double2(0.0, 0.0);
-    }
-    __syncthreads();
-#pragma unroll 4
-    for (int k = 0; k < kNB; k++) {
-        const double2 y = s_rb[k][j];
-#pragma unroll
-        for (int e = 0; e < kEnt; e++) t[e] = zfms(t[e], s_cb[i0 + kRowStep * e][k], y);
+        for (int e = 0; e < kEnt / 2; e++) {
+            const int i = w + kRecWaves * (e0 + e);
+            if (h == 0) s_cw[i][j] = t[e];
+            else {
+                const bool iu = j >= i && j < nb;
+                Tout[i * kNB + j] = make_float2(iu ? (float)t[e].x : 0.f, iu ? (float)t[e].y : 0.f);
+            }
+        }
     }
 #pragma unroll
     for (int e = 0; e < kEnt; e++) {
-        const int i = i0 + kRowStep * e;
-        const bool up = j >= i, iu = up && j < nb, low = j < nb && j < i;  // (j < nb: i <= j too)
-        Tout[i * kNB + j] = make_float2(iu ? (float)t[e].x : 0.f, iu ? (float)t[e].y : 0.f);
-        Y[i * kNB + j] = make_double2(iu ? wx[e] : 0.0, iu ? wy[e] : 0.0);
+        const int i = w + kRecWaves * e;
+        const bool iu = j >= i && j < nb, low = j < nb && j < i;
+        const float2 v = make_float2((float)second[e].x, (float)second[e].y);
+        if (top) Y[i * kNB + j] = make_double2(iu ? x[e] : 0.0, iu ? y[e] : 0.0);
         if (i < Mp) {
-            const double2 rh = zmul(s_sign[i], R[e]);
-            if (j < nb)
-                A[(size_t)(j0 + j) * lda + j0 + i] =
-                    make_float2((float)(up ? rh.x : L[e].x), (float)(up ? rh.y : L[e].y));
-            Vd[(size_t)j * ldv + i] = make_float2(low ? (float)L[e].x : iu && j == i ? 1.f : 0.f,
-                                                  low ? (float)L[e].y : 0.f);
+            if (top ? low : iu) A[(size_t)(j0 + j) * lda + j0 + i] = v;
+            if (top) Vd[(size_t)j * ldv + i] = j < nb ? v : make_float2(0.f, 0.f);
         }
     }
 }
