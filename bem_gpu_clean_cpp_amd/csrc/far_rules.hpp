@@ -23,8 +23,8 @@
 // equations in FP64 (largest moment residual 1e-14).
 //
 // What bounds it: the vector ALU (large meshes run at 100 % VALU issue).  A
-// pair costs about 1000 VALU instructions with 36 points; 222 with 7, 370 with
-// 12.  10242 nodes at 2 kHz: 5.16 -> 1.92 ms; 40962 nodes at 12 kHz: 81 -> 32 ms.
+// pair costs about 1000 VALU instructions with 36 points; 250 with 7, 420 with
+// 12.  10242 nodes at 2 kHz: 5.16 -> 2.0 ms; 40962 nodes at 12 kHz: 81 -> 36 ms.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -155,14 +155,22 @@ struct FarSums {
     float hr[3], hi[3], gr[3], gi[3], c;
 };
 
-// one point: t = (r / r0)^2 - 1, phi / (2 pi) = (k r0 / 2 pi) t / (1 + sqrt(1 + t)).
-// Nothing cancels, so a point's phase carries no rounding of r itself (the
-// 36-point path's phase k r is rounded at every point).
+// one point: t = (r / r0)^2 - 1, phi / (2 pi) = (k r0 / 2 pi) d, d = r / r0 - 1 =
+// sqrt(1 + t) - 1.  d is first 1 + t times its reciprocal square root, less 1, which
+// carries the rounding of both (6e-8 and a bias of about 8e-9, times k r0: at 40
+// radians the phases were off by 4e-7, and the solution at 40962 nodes and 12 kHz
+// by 7.7e-7 where 36 points a pair give 5.5e-7); one Newton step on
+// (1 + d)^2 = 1 + t removes it (entries past 20 node spacings: 4.2e-7 -> 1.2e-7 of
+// their size, 36 points 7.8e-7; the solution 4.8e-7) for 4 more instructions, 5 %
+// of the assembly.  A division t / (1 + sqrt(1 + t)) took up to 8 %.
 template <bool G>
-__device__ __forceinline__ void far_point(float op, float kr0, float kr0rev, float &hr, float &hi, float &p, float &gr,
+__device__ __forceinline__ void far_point(float t, float kr0, float kr0rev, float &hr, float &hi, float &p, float &gr,
                                           float &gi) {
+    const float op = t + 1.0f;
     const float w = __builtin_amdgcn_rsqf(op);
-    const float u = kr0rev * __builtin_fmaf(op, w, -1.0f);
+    float d = __builtin_fmaf(op, w, -1.0f);
+    d = __builtin_fmaf(0.5f, __builtin_fmaf(-d, d, __builtin_fmaf(-2.0f, d, t)), d);
+    const float u = kr0rev * d;
     const float sn = __builtin_amdgcn_sinf(u), cs = __builtin_amdgcn_cosf(u);
     const float w2 = w * w, q = w2 * kr0;
     p = w2 * w;
@@ -202,7 +210,7 @@ __device__ __forceinline__ void far_sums(CFloat *uu, CFloat *dd, float T1, float
             float hr[3], hi[3], p[3], gr[3], gi[3];
 #pragma unroll
             for (int j = 0; j < 3; j++) {
-                const float t = __builtin_fmaf((float)(l * l), D[j], __builtin_fmaf((float)l, T[j], 1.0f));
+                const float t = __builtin_fmaf((float)(l * l), D[j], (float)l * T[j]);
                 far_point<G>(t, kr0, kr0rev, hr[j], hi[j], p[j], gr[j], gi[j]);
                 s.hr[j] = __builtin_fmaf((float)(W * l), hr[j], s.hr[j]);
                 s.hi[j] = __builtin_fmaf((float)(W * l), hi[j], s.hi[j]);
@@ -233,7 +241,7 @@ __device__ __forceinline__ void far_sums(CFloat *uu, CFloat *dd, float T1, float
 #pragma unroll
     for (int q = 0; q < R::ng; q++) {
         const double N[3] = {R::g1[q], R::g2[q], 1.0 - R::g1[q] - R::g2[q]}, W = R::wg[q];
-        const float t = __builtin_fmaf((float)(N[0] - N[2]), T1, __builtin_fmaf((float)(N[1] - N[2]), T2, __builtin_fmaf(dd[q], i02, 1.0f)));
+        const float t = __builtin_fmaf((float)(N[0] - N[2]), T1, __builtin_fmaf((float)(N[1] - N[2]), T2, dd[q] * i02));
         float hr, hi, p, gr, gi;
         far_point<G>(t, kr0, kr0rev, hr, hi, p, gr, gi);
 #pragma unroll
