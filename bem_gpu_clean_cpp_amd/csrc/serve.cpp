@@ -187,7 +187,9 @@ double bem_request_footprint(int M, int N, int E, int nrhs, int precision, int m
         b += sizeof(double2) * ldv * (K + 1) * R;                   // Krylov basis
         b += (3 * sizeof(double2) + 3 * sizeof(float2)) * ldv * R;  // work vectors
         b += std::max(std::max(ws_gemv_n(M, N, 1), ws_gemm(M, N, nrhs)), ws_mres(M, N, nrhs));
-        b += sizeof(double2) * (K + 2) * (2 + ((size_t)std::max(M, N) + 1023) / 1024) * R;
+        // Hessenberg columns, and the dots' partials of up to 256, 512 or 1024 rows
+        const size_t rows = (size_t)std::max(M, N);
+        b += sizeof(double2) * (K + 2) * (10 + std::max((rows + 1023) / 1024, std::min<size_t>(32, (rows + 255) / 256))) * R;
         if (method == BEM_SOLVE_GMRES && precision != BEM_PREC_FP64 && nrhs == 1 && M > N && ne_fused_fits(M, N))
             b += sizeof(float2) * (size_t)M * ne_ldr(N) + std::max(ws_ne_resid(M, N), ws_ne_rhs(M, N));  // row-major copy of A
         // conjugate-transposed copy of A (block CG makes it for its FP16-split
