@@ -56,7 +56,7 @@ long round64(long m) { return (m + 63) / 64 * 64; }
 // took 18 ms each way, where one contiguous copy takes 2-3 ms.  So contiguous
 // host columns are packed (unpacked) on the device, at most kPackBytes at a
 // time; host columns with gaps keep the pitched copy, which leaves the gaps
-// untouched.
+// untouched, and so does a device with no room for the packed columns.
 constexpr size_t kPackBytes = size_t(64) << 20;
 
 __global__ void k_copy_cols(const float2 *__restrict__ src, long lds, float2 *__restrict__ dst, long ldd, int n) {
@@ -75,11 +75,21 @@ int pack_columns(int n, int cols) {
     return (int)std::min<size_t>({(size_t)cols, std::max<size_t>(1, kPackBytes / (8 * (size_t)n)), 32768});
 }
 
+// room for n units, or null where the device has none left
+float2 *pack_alloc(size_t n, hipStream_t s) {
+    void *p = nullptr;
+    if (hipMallocAsync(&p, n * sizeof(float2), s) == hipSuccess) return (float2 *)p;
+    (void)hipGetLastError();
+    return nullptr;
+}
+
 // host (ldh >= n units) <- device; the stream is waited for
 int copy_out(void *host, long ldh, const float2 *dev, long ldd, int n, int cols, hipStream_t s) {
     if (n <= 0 || cols <= 0) return EXIT_SUCCESS;
     hipError_t e = hipSuccess;
-    if (ldh != n || ldd == n || cols == 1) {
+    const int per = pack_columns(n, cols);
+    float2 *pk = ldh == n && ldd != n && cols > 1 ? pack_alloc((size_t)n * per, s) : nullptr;
+    if (!pk) {
         if (ldh == n && ldd == n)
             e = hipMemcpyAsync(host, dev, (size_t)8 * n * cols, hipMemcpyDeviceToHost, s);
         else
@@ -88,9 +98,6 @@ int copy_out(void *host, long ldh, const float2 *dev, long ldd, int n, int cols,
         HIP_CALL(e);
         return EXIT_SUCCESS;
     }
-    const int per = pack_columns(n, cols);
-    float2 *pk = nullptr;
-    HOST_CALL(salloc(&pk, (size_t)n * per, s));
     for (int c = 0; c < cols && e == hipSuccess; c += per) {
         const int nc = std::min(per, cols - c);
         k_copy_cols<<<dim3((n + 255) / 256, nc), 256, 0, s>>>(dev + (size_t)c * ldd, ldd, pk, n, n);
@@ -107,13 +114,12 @@ int copy_out(void *host, long ldh, const float2 *dev, long ldd, int n, int cols,
 // device <- host; the host buffer may go once the stream has been waited for
 int copy_in(float2 *dev, long ldd, const void *host, long ldh, int n, int cols, hipStream_t s) {
     if (n <= 0 || cols <= 0) return EXIT_SUCCESS;
-    if (ldh != n || ldd == n || cols == 1) {
+    const int per = pack_columns(n, cols);
+    float2 *pk = ldh == n && ldd != n && cols > 1 ? pack_alloc((size_t)n * per, s) : nullptr;
+    if (!pk) {
         HIP_CALL(hipMemcpy2DAsync(dev, 8 * ldd, host, 8 * ldh, (size_t)8 * n, cols, hipMemcpyHostToDevice, s));
         return EXIT_SUCCESS;
     }
-    const int per = pack_columns(n, cols);
-    float2 *pk = nullptr;
-    HOST_CALL(salloc(&pk, (size_t)n * per, s));
     hipError_t e = hipSuccess;
     for (int c = 0; c < cols && e == hipSuccess; c += per) {
         const int nc = std::min(per, cols - c);
@@ -718,8 +724,17 @@ int bem_solver_get_solution(const bem_solver *sv, bem_complex *x, int ldx) {
     hipStream_t s = sv->stream;
     // narrowed on the device: half the bytes to copy, no pass over them here
     const int N = sv->dp.N, R = sv->rhs.nrhs;
-    float2 *xd = nullptr;
-    HOST_CALL(salloc(&xd, (size_t)N * R, s));
+    float2 *xd = R <= 32768 ? pack_alloc((size_t)N * R, s) : nullptr;  // grid.y
+    if (!xd) {
+        std::vector<double2> z((size_t)N * R);
+        HOST_CALL(copy_out(z.data(), 2L * N, (const float2 *)sv->X64, 2 * sv->dp.ldA, 2 * N, R, s));
+        for (int r = 0; r < R; r++)
+            for (int i = 0; i < N; i++) {
+                const double2 v = z[(size_t)r * N + i];
+                x[(size_t)r * ldx + i] = {(float)v.x, (float)v.y};
+            }
+        return EXIT_SUCCESS;
+    }
     k_narrow_cols<<<dim3((N + 255) / 256, R), 256, 0, s>>>(sv->X64, sv->dp.ldA, xd, N, N);
     int rc = hipGetLastError() == hipSuccess ? EXIT_SUCCESS : EXIT_FAILURE;
     if (rc != EXIT_SUCCESS) set_error(__FILE__, __LINE__, "launch failed");
