@@ -863,7 +863,8 @@ __global__ __launch_bounds__(256) void asm_tile_fast64(AsmArgs<double> a) {
         CElemRec64 &rec = ((CElemRec64 *)a.recs)[e];
         const double cx = fr.c[0] - x0, cy = fr.c[1] - x1, cz = fr.c[2] - x2;
         const double r02 = fma(cx, cx, fma(cy, cy, cz * cz));
-        const double kr0 = k * (r02 * rsq_f64(r02));
+        // (a row on the centroid: rsq_f64(0) is NaN, the distance is zero)
+        const double kr0 = r02 > 0 ? k * (r02 * rsq_f64(r02)) : 0.0;
         const double ax = rec.p3[0] - x0, ay = rec.p3[1] - x1, az = rec.p3[2] - x2;
         const double dn = rec.n[0] * ax + rec.n[1] * ay + rec.n[2] * az;
         const double aa = fma(ax, ax, fma(ay, ay, az * az));
