@@ -478,13 +478,17 @@ __global__ __launch_bounds__(256) void asm_tile(AsmArgs<R> a) {
 // the one r already carries: at 8 kHz on icosphere s5 the relative Frobenius
 // error of A against FP64 goes from 1.060e-7 to 1.063e-7, and the kernel
 // runs 5 % faster (two fewer dependent instructions per point).
-// The squared distance is expanded per theta row,
+// The squared distance of a point is formed from its coordinates' differences
+// a + rho_m v_n where a row is near the element (closer than the far rules
+// allow).  For the other rows on 36 points, those of elements that the
+// wavelength does not resolve, it is expanded per theta row,
 //   r^2 = |a|^2 + rho_m (2 a.v_n + rho_m |v_n|^2),
-// two FMAs per point instead of six.  Its rounding error grows as
-// (|a| / r)^2 where the point is much closer to the element than to the
-// vertex p3; the rows where r -> 0 (x a vertex of e) take the FP64 singular
-// rule, and on icosphere s5 at 2 and 8 kHz the entries are as close to FP64
-// as with the direct form (relative Frobenius error 9.3e-8 and 1.06e-7).
+// two FMAs per point instead of six.  Its rounding error grows as (|a| / r)^2,
+// that of the differences as |a| / r: on a 2562-node body, the entries of the
+// nearest nodes for rows 0.01 edge lengths off the surface were off by 1.2e-4
+// (median; at most 2e-3), with the differences by 8e-7 (7e-6); FP64 2e-13
+// (2e-12) and 1.5e-15 (1e-14).  It costs 0.08 of 2.0 ms at 10242 nodes, 5 of 43
+// us at 642.
 __device__ __forceinline__ constexpr float gl_theta(int n) { return (float)(0.5 + 0.5 * GL6::eta[n]); }
 __device__ __forceinline__ constexpr float gl_rho(int m) { return (float)(0.5 + 0.5 * GL6::eta[m]); }
 // theta_n - theta_{n+1} for n < 5, theta_5 for n = 5
@@ -501,6 +505,149 @@ __device__ __forceinline__ constexpr float gl_Wrho(int n, int m) {
 typedef __attribute__((address_space(4))) const ElemRec<float> CElemRec;
 
 __device__ __forceinline__ bool wave_all(bool p) { return __builtin_amdgcn_ballot_w64(!p) == 0; }
+
+// sums over the 36 points: S = sum W rho H~ and ht = sum W H~; the theta moment
+// h2 = sum_n theta_n A_n of the per-row sums A_n comes from the running totals
+// S_n of S after each row,
+//   h2 = sum_{n<5} (theta_n - theta_{n+1}) S_n + theta_5 S_5,
+// and h1 = S - h2 (likewise g1, g2 from SC = sum W rho G~)
+struct Sums36 {
+    float Sr = 0, Si = 0, h2r = 0, h2i = 0, htr = 0, hti = 0, gr = 0, gi = 0, cc = 0;
+    float SCr = 0, SCi = 0, g2r = 0, g2i = 0;
+};
+// one point: 4 pi r dG/dn / (-dn) = (cos kr - i sin kr)(1/r^3 + i k/r^2) and
+// 4 pi G = (cos kr - i sin kr) / r
+struct Point36 {
+    float Hr, Hi, Gr, Gi, q3;
+};
+template <bool RAW>
+__device__ __forceinline__ Point36 point36(float r2, float k, float krev) {
+    const float MAGIC = 12582912.0f;  // 1.5 * 2^23
+    const float rinv = __builtin_amdgcn_rsqf(r2);
+    const float r = r2 * rinv;
+    float u;
+    if (RAW) {
+        u = r * krev;
+    } else {
+        const float t2 = __builtin_fmaf(r, krev, MAGIC);
+        const float jf = t2 - MAGIC;
+        u = __builtin_fmaf(r, krev, -jf);
+    }
+    const float sn = __builtin_amdgcn_sinf(u), cs = __builtin_amdgcn_cosf(u);
+    const float rinv2 = rinv * rinv;
+    const float q2k = k * rinv2;  // k/r^2
+    Point36 p;
+    p.q3 = rinv2 * rinv;  // 1/r^3
+    p.Hr = __builtin_fmaf(cs, p.q3, sn * q2k);
+    p.Hi = __builtin_fmaf(cs, q2k, -sn * p.q3);
+    p.Gr = cs * rinv;
+    p.Gi = -sn * rinv;
+    return p;
+}
+template <bool IMP, bool RAW, bool SRC>
+__device__ __forceinline__ void sums36(CElemRec &rec, float ax, float ay, float az, float k, float krev, Sums36 &s) {
+    const float aa = __builtin_fmaf(ax, ax, __builtin_fmaf(ay, ay, az * az));
+    // 2 a.v_n = 2 a.e1 + 2 theta_n a.f
+    const float ae1 = __builtin_fmaf(ax, rec.e1[0], __builtin_fmaf(ay, rec.e1[1], az * rec.e1[2]));
+    const float af = __builtin_fmaf(ax, rec.f[0], __builtin_fmaf(ay, rec.f[1], az * rec.f[2]));
+    const float ae1x2 = ae1 + ae1;
+#pragma unroll
+    for (int n = 0; n < 6; n++) {
+        const float th = gl_theta(n);
+        const float tav = __builtin_fmaf(2.0f * th, af, ae1x2);
+        const float vv = rec.vv[n];
+#pragma unroll
+        for (int m = 0; m < 6; m++) {
+            const float rho = gl_rho(m), W = gl_W(n, m), Wr = gl_Wrho(n, m);
+            const Point36 p = point36<RAW>(__builtin_fmaf(rho, __builtin_fmaf(rho, vv, tav), aa), k, krev);
+            s.Sr = __builtin_fmaf(Wr, p.Hr, s.Sr);
+            s.Si = __builtin_fmaf(Wr, p.Hi, s.Si);
+            s.htr = __builtin_fmaf(W, p.Hr, s.htr);
+            s.hti = __builtin_fmaf(W, p.Hi, s.hti);
+            if (IMP || SRC) {
+                s.gr = __builtin_fmaf(W, p.Gr, s.gr);
+                s.gi = __builtin_fmaf(W, p.Gi, s.gi);
+            }
+            if (IMP) {
+                s.SCr = __builtin_fmaf(Wr, p.Gr, s.SCr);
+                s.SCi = __builtin_fmaf(Wr, p.Gi, s.SCi);
+            }
+            s.cc = __builtin_fmaf(W, p.q3, s.cc);
+        }
+        // theta moment of the rho-weighted sums from their running totals
+        const float dth = gl_dtheta(n);
+        s.h2r = __builtin_fmaf(dth, s.Sr, s.h2r);
+        s.h2i = __builtin_fmaf(dth, s.Si, s.h2i);
+        if (IMP) {
+            s.g2r = __builtin_fmaf(dth, s.SCr, s.g2r);
+            s.g2i = __builtin_fmaf(dth, s.SCi, s.g2i);
+        }
+    }
+}
+// theta and 0.25 w of a theta row
+struct ThetaRow32 {
+    float th, w;
+};
+__device__ constexpr ThetaRow32 kTheta32[6] = {
+#define BEM_TH(n) {(float)(0.5 + 0.5 * GL6::eta[n]), (float)(0.25 * GL6::w[n])}
+    BEM_TH(0), BEM_TH(1), BEM_TH(2), BEM_TH(3), BEM_TH(4), BEM_TH(5)
+#undef BEM_TH
+};
+// the same for a row near the element.  (The theta rows are a loop: unrolled,
+// both forms together take 111 to 185 registers instead of 72 to 91, and the
+// assembly of 10242 nodes 2.3 ms instead of 2.0.)
+template <bool IMP, bool RAW, bool SRC>
+__device__ __forceinline__ void sums36_near(CElemRec &rec, float ax, float ay, float az, float k, float krev,
+                                            Sums36 &s) {
+#pragma unroll 1
+    for (int n = 0; n < 6; n++) {
+        const ThetaRow32 t = kTheta32[n];
+        const float vx = __builtin_fmaf(t.th, rec.f[0], rec.e1[0]), vy = __builtin_fmaf(t.th, rec.f[1], rec.e1[1]),
+                    vz = __builtin_fmaf(t.th, rec.f[2], rec.e1[2]);
+        // sums over m with w_m rho_m and w_m rho_m^2
+        float br = 0, bi = 0, ar = 0, ai = 0, gbr = 0, gbi = 0, gar = 0, gai = 0, c = 0;
+#pragma unroll
+        for (int m = 0; m < 6; m++) {
+            const float rho = gl_rho(m), wr = (float)(GL6::w[m] * (0.5 + 0.5 * GL6::eta[m])),
+                        wr2 = (float)(GL6::w[m] * (0.5 + 0.5 * GL6::eta[m]) * (0.5 + 0.5 * GL6::eta[m]));
+            const float dx = __builtin_fmaf(rho, vx, ax), dy = __builtin_fmaf(rho, vy, ay),
+                        dz = __builtin_fmaf(rho, vz, az);
+            const Point36 p =
+                point36<RAW>(__builtin_fmaf(dx, dx, __builtin_fmaf(dy, dy, dz * dz)), k, krev);
+            br = __builtin_fmaf(wr, p.Hr, br);
+            bi = __builtin_fmaf(wr, p.Hi, bi);
+            ar = __builtin_fmaf(wr2, p.Hr, ar);
+            ai = __builtin_fmaf(wr2, p.Hi, ai);
+            if (IMP || SRC) {
+                gbr = __builtin_fmaf(wr, p.Gr, gbr);
+                gbi = __builtin_fmaf(wr, p.Gi, gbi);
+            }
+            if (IMP) {
+                gar = __builtin_fmaf(wr2, p.Gr, gar);
+                gai = __builtin_fmaf(wr2, p.Gi, gai);
+            }
+            c = __builtin_fmaf(wr, p.q3, c);
+        }
+        const float w2 = t.w * t.th;
+        s.htr = __builtin_fmaf(t.w, br, s.htr);
+        s.hti = __builtin_fmaf(t.w, bi, s.hti);
+        s.Sr = __builtin_fmaf(t.w, ar, s.Sr);
+        s.Si = __builtin_fmaf(t.w, ai, s.Si);
+        s.h2r = __builtin_fmaf(w2, ar, s.h2r);
+        s.h2i = __builtin_fmaf(w2, ai, s.h2i);
+        if (IMP || SRC) {
+            s.gr = __builtin_fmaf(t.w, gbr, s.gr);
+            s.gi = __builtin_fmaf(t.w, gbi, s.gi);
+        }
+        if (IMP) {
+            s.SCr = __builtin_fmaf(t.w, gar, s.SCr);
+            s.SCi = __builtin_fmaf(t.w, gai, s.SCi);
+            s.g2r = __builtin_fmaf(w2, gar, s.g2r);
+            s.g2i = __builtin_fmaf(w2, gai, s.g2i);
+        }
+        s.cc = __builtin_fmaf(t.w, c, s.cc);
+    }
+}
 
 // The rule is chosen per (wave, element): the fewest points that every row of
 // the wave may take.  Element records and tile lists are read as scalar loads
@@ -526,7 +673,6 @@ __global__ __launch_bounds__(256) void asm_tile_fast(AsmArgs<float> a) {
     const float k = a.k;
     const float krev = a.kf;  // k / (2 pi)
     const float inv4pi = (float)(1.0 / (4.0 * kPi));
-    const float MAGIC = 12582912.0f;  // 1.5 * 2^23
     float c_acc = 0, br_acc = 0, bi_acc = 0;
     CInt *entries = (CInt *)a.tile_entries, *slots = (CInt *)a.tile_slots;
     const int it0 = ((CInt *)a.tile_ptr)[tile], it1 = ((CInt *)a.tile_ptr)[tile + 1];
@@ -573,7 +719,8 @@ __global__ __launch_bounds__(256) void asm_tile_fast(AsmArgs<float> a) {
         const float r02f = fd.r02f;
         const int rho2 = cur.rho2;  // (positive floats compare as integers: scalar compares)
         float pr[3], pi[3], cval, btr = 0, bti = 0;
-        if (rho2 <= a.far_rho2 && wave_all(!active || r02f >= cur.far16)) {
+        const bool distant = wave_all(!active || r02f >= cur.far16);
+        if (distant && rho2 <= a.far_rho2) {
             const FarGeom g = far_geom(fr, fd, k, krev, a.kf64);
             FarSums s;
             if (rho2 <= a.far7_rho2 && wave_all(!active || r02f >= fr.far7))
@@ -587,90 +734,28 @@ __global__ __launch_bounds__(256) void asm_tile_fast(AsmArgs<float> a) {
             CElemRec &rec = ((CElemRec *)a.recs)[e];
             const float ax = rec.p3[0] - xp.x, ay = rec.p3[1] - xp.y, az = rec.p3[2] - xp.z;
             const float dn = rec.n[0] * ax + rec.n[1] * ay + rec.n[2] * az;
-            const float aa = __builtin_fmaf(ax, ax, __builtin_fmaf(ay, ay, az * az));
-            // 2 a.v_n = 2 a.e1 + 2 theta_n a.f
-            const float ae1 = __builtin_fmaf(ax, rec.e1[0], __builtin_fmaf(ay, rec.e1[1], az * rec.e1[2]));
-            const float af = __builtin_fmaf(ax, rec.f[0], __builtin_fmaf(ay, rec.f[1], az * rec.f[2]));
-            const float ae1x2 = ae1 + ae1;
-            // S = sum W rho H~ and ht = sum W H~ over all 36 points; the theta
-            // moment h2 = sum_n theta_n A_n of the per-row sums A_n comes from the
-            // running totals S_n of S after each row,
-            //   h2 = sum_{n<5} (theta_n - theta_{n+1}) S_n + theta_5 S_5,
-            // and h1 = S - h2 (likewise g1, g2 from SC = sum W rho G~)
-            float Sr = 0, Si = 0, h2r = 0, h2i = 0, htr = 0, hti = 0, gr = 0, gi = 0, cc = 0;
-            float SCr = 0, SCi = 0, g2r = 0, g2i = 0;
-    #pragma unroll
-            for (int n = 0; n < 6; n++) {
-                const float th = gl_theta(n);
-                const float tav = __builtin_fmaf(2.0f * th, af, ae1x2);
-                const float vv = rec.vv[n];
-    #pragma unroll
-                for (int m = 0; m < 6; m++) {
-                    const float rho = gl_rho(m), W = gl_W(n, m), Wr = gl_Wrho(n, m);
-                    const float r2 = __builtin_fmaf(rho, __builtin_fmaf(rho, vv, tav), aa);
-                    const float rinv = __builtin_amdgcn_rsqf(r2);
-                    const float r = r2 * rinv;
-                    float u;
-                    if (RAW) {
-                        u = r * krev;
-                    } else {
-                        const float t2 = __builtin_fmaf(r, krev, MAGIC);
-                        const float jf = t2 - MAGIC;
-                        u = __builtin_fmaf(r, krev, -jf);
-                    }
-                    const float sn = __builtin_amdgcn_sinf(u), cs = __builtin_amdgcn_cosf(u);
-                    const float rinv2 = rinv * rinv;
-                    const float q3 = rinv2 * rinv;  // 1/r^3
-                    const float q2k = k * rinv2;    // k/r^2
-                    // 4 pi r dG/dn / (-dn) = (cos kr - i sin kr)(1/r^3 + i k/r^2)
-                    const float Hr = __builtin_fmaf(cs, q3, sn * q2k);
-                    const float Hi = __builtin_fmaf(cs, q2k, -sn * q3);
-                    Sr = __builtin_fmaf(Wr, Hr, Sr);
-                    Si = __builtin_fmaf(Wr, Hi, Si);
-                    htr = __builtin_fmaf(W, Hr, htr);
-                    hti = __builtin_fmaf(W, Hi, hti);
-                    // 4 pi G = (cos kr - i sin kr) / r
-                    if (IMP) {
-                        const float Gr = cs * rinv, Gi = -sn * rinv;
-                        gr = __builtin_fmaf(W, Gr, gr);
-                        gi = __builtin_fmaf(W, Gi, gi);
-                        SCr = __builtin_fmaf(Wr, Gr, SCr);
-                        SCi = __builtin_fmaf(Wr, Gi, SCi);
-                    } else if (SRC) {
-                        const float Wg = W * rinv;
-                        gr = __builtin_fmaf(Wg, cs, gr);
-                        gi = __builtin_fmaf(-Wg, sn, gi);
-                    }
-                    cc = __builtin_fmaf(W, q3, cc);
-                }
-                // theta moment of the rho-weighted sums from their running totals
-                const float dth = gl_dtheta(n);
-                h2r = __builtin_fmaf(dth, Sr, h2r);
-                h2i = __builtin_fmaf(dth, Si, h2i);
-                if (IMP) {
-                    g2r = __builtin_fmaf(dth, SCr, g2r);
-                    g2i = __builtin_fmaf(dth, SCi, g2i);
-                }
-            }
-            const float h1r = Sr - h2r, h1i = Si - h2i;
-            const float g1r = SCr - g2r, g1i = SCi - g2i;
+            Sums36 q;
+            if (distant) sums36<IMP, RAW, SRC>(rec, ax, ay, az, k, krev, q);
+            else sums36_near<IMP, RAW, SRC>(rec, ax, ay, az, k, krev, q);
+            const float h1r = q.Sr - q.h2r, h1i = q.Si - q.h2i;
+            const float g1r = q.SCr - q.g2r, g1i = q.SCi - q.g2i;
             const float sJ = rec.J * inv4pi;
             const float sh = -dn * sJ;
             float p0r = sh * h1r, p0i = sh * h1i;
-            float p1r = sh * h2r, p1i = sh * h2i;
-            float p2r = sh * (htr - Sr), p2i = sh * (hti - Si);
+            float p1r = sh * q.h2r, p1i = sh * q.h2i;
+            float p2r = sh * (q.htr - q.Sr), p2i = sh * (q.hti - q.Si);
             const float sg = a.rw * sJ;
-            const float gsr = -sg * gi, gsi = sg * gr;
+            const float gsr = -sg * q.gi, gsi = sg * q.gr;
             if (IMP) {
                 const float br = rec.beta[0], bi = rec.beta[1];
                 const float G0r = -sg * g1i, G0i = sg * g1r;
-                const float G1r = -sg * g2i, G1i = sg * g2r;
+                const float G1r = -sg * q.g2i, G1i = sg * q.g2r;
                 const float G2r = gsr - G0r - G1r, G2i = gsi - G0i - G1i;
                 p0r -= br * G0r - bi * G0i; p0i -= br * G0i + bi * G0r;
                 p1r -= br * G1r - bi * G1i; p1i -= br * G1i + bi * G1r;
                 p2r -= br * G2r - bi * G2i; p2i -= br * G2i + bi * G2r;
             }
-            cval = -dn * sJ * cc;
+            cval = -dn * sJ * q.cc;
             if (IMP || SRC) {
                 btr = rec.gamma[0] * gsr - rec.gamma[1] * gsi;
                 bti = rec.gamma[0] * gsi + rec.gamma[1] * gsr;
@@ -761,28 +846,40 @@ __device__ constexpr ThetaRow kTheta[6] = {
 #undef BEM_TH
 };
 
+typedef __attribute__((address_space(4))) const ElemRec<double> CElemRec64;
+
 // Sums of the 36 points relative to the phase k r0 of the element's centroid;
 // SMALL: |k (r - r0)| <= 0.8 on the element, so its sine and cosine need no
-// quadrant.
+// quadrant.  NEAR: distances from the coordinates' differences, otherwise
+// expanded per theta row (as sums36).
 struct FastSums64 {
     double hr[3], hi[3], gr[3], gi[3], c;
 };
-template <bool IMP, bool SRC, bool SMALL>
-__device__ __forceinline__ void fast_sums64(double aa, double ae1x2, double af,
-                                            __attribute__((address_space(4))) const double *vv, double k, double kr0,
+template <bool IMP, bool SRC, bool SMALL, bool NEAR>
+__device__ __forceinline__ void fast_sums64(CElemRec64 &rec, double ax, double ay, double az, double k, double kr0,
                                             FastSums64 &s) {
+    const double aa = fma(ax, ax, fma(ay, ay, az * az));
+    const double ae1 = fma(ax, rec.e1[0], fma(ay, rec.e1[1], az * rec.e1[2]));
+    const double af = fma(ax, rec.f[0], fma(ay, rec.f[1], az * rec.f[2]));
     double htr = 0, hti = 0, gtr = 0, gti = 0;
     s.hr[0] = s.hr[1] = s.hi[0] = s.hi[1] = s.gr[0] = s.gr[1] = s.gi[0] = s.gi[1] = s.c = 0;
 #pragma unroll 1
     for (int n = 0; n < 6; n++) {
         const ThetaRow th = kTheta[n];
-        const double tav = fma(th.th2, af, ae1x2), v = vv[n];
+        const double tav = fma(th.th2, af, ae1 + ae1), v = rec.vv[n], t = 0.5 * th.th2;
+        const double vx = fma(t, rec.f[0], rec.e1[0]), vy = fma(t, rec.f[1], rec.e1[1]), vz = fma(t, rec.f[2], rec.e1[2]);
         // sums over m: B with w_m rho_m, A with w_m rho_m^2
         double ar = 0, ai = 0, br = 0, bi = 0, gbr = 0, gbi = 0, gar = 0, gai = 0, c = 0;
 #pragma unroll
         for (int m = 0; m < 6; m++) {
             const double rho = 0.5 + 0.5 * GL6::eta[m], wr = GL6::w[m] * rho, wr2 = wr * rho;
-            const double r2 = fma(rho, fma(rho, v, tav), aa);
+            double r2;
+            if (NEAR) {
+                const double dx = fma(rho, vx, ax), dy = fma(rho, vy, ay), dz = fma(rho, vz, az);
+                r2 = fma(dx, dx, fma(dy, dy, dz * dz));
+            } else {
+                r2 = fma(rho, fma(rho, v, tav), aa);
+            }
             const double y = rsq_f64(r2);
             const double d = fma(k, r2 * y, -kr0);
             double sn, cs;
@@ -830,8 +927,6 @@ __device__ __forceinline__ void fast_sums64(double aa, double ae1x2, double af,
     s.gi[2] = gti - s.gi[0] - s.gi[1];
 }
 
-typedef __attribute__((address_space(4))) const ElemRec<double> CElemRec64;
-
 // The FP64 form of asm_tile_fast: the separable 36-point rule on every pair, on
 // the element-once plan.  Bound by the vector ALU: the generic kernel spent
 // about 290 issue slots a point on the library's sincos, square root and
@@ -867,15 +962,15 @@ __global__ __launch_bounds__(256) void asm_tile_fast64(AsmArgs<double> a) {
         const double kr0 = r02 > 0 ? k * (r02 * rsq_f64(r02)) : 0.0;
         const double ax = rec.p3[0] - x0, ay = rec.p3[1] - x1, az = rec.p3[2] - x2;
         const double dn = rec.n[0] * ax + rec.n[1] * ay + rec.n[2] * az;
-        const double aa = fma(ax, ax, fma(ay, ay, az * az));
-        const double ae1 = fma(ax, rec.e1[0], fma(ay, rec.e1[1], az * rec.e1[2]));
-        const double af = fma(ax, rec.f[0], fma(ay, rec.f[1], az * rec.f[2]));
         FastSums64 s;
+        const bool distant = wave_all(!active || r02 >= (double)fr.far12);
         // (positive floats compare as integers)
-        if (__float_as_int(fr.rho2) <= a.far_rho2)
-            fast_sums64<IMP, SRC, true>(aa, ae1 + ae1, af, rec.vv, k, kr0, s);
+        if (__float_as_int(fr.rho2) > a.far_rho2)
+            fast_sums64<IMP, SRC, false, true>(rec, ax, ay, az, k, kr0, s);
+        else if (distant)
+            fast_sums64<IMP, SRC, true, false>(rec, ax, ay, az, k, kr0, s);
         else
-            fast_sums64<IMP, SRC, false>(aa, ae1 + ae1, af, rec.vv, k, kr0, s);
+            fast_sums64<IMP, SRC, true, true>(rec, ax, ay, az, k, kr0, s);
         double s0, c0;
         sincos_wide(kr0, s0, c0);
         const double sJ = rec.J * inv4pi, m = -dn * sJ;

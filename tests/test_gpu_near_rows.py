@@ -110,3 +110,57 @@ def test_row_at_a_centroid(prec, u, n, k):
     A = _matrix_rows(m, xs, k, prec)
     A0, tol = _rows(p, e, (0.5 + 0.25j, 1.0 - 0.5j), float(np.float32(k)), xs, u)
     assert np.all(np.abs(A - A0) <= tol)
+
+
+def _body(subdiv, bc):
+    m = bem.Mesh().ellipsoid(subdiv, (0.075, 0.09, 0.11), nbumps=8, lmax=6, amp=0.05, seed=70 + subdiv)
+    m.set_bc(*bc, 0.0)
+    return m
+
+
+def _above(p, elems, height, count):
+    """Points over quadrature points of some elements, `height` edges off, on
+    either side in turn."""
+    gp = np.polynomial.legendre.leggauss(6)[0]
+    sel = np.linspace(0, len(elems) - 1, count).astype(int)
+    t = p[elems[sel]].astype(np.float64)
+    th, rho = (1 + gp[np.arange(count) % 6]) / 2, (1 + gp[np.arange(count) // 2 % 6]) / 2
+    y = t[:, 0] * (rho * (1 - th))[:, None] + t[:, 1] * (rho * th)[:, None] + t[:, 2] * (1 - rho)[:, None]
+    n = np.cross(t[:, 0] - t[:, 2], t[:, 1] - t[:, 2])
+    n /= np.linalg.norm(n, axis=1, keepdims=True)
+    edge = np.linalg.norm(t[:, 0] - t[:, 1], axis=1)[:, None]
+    side = np.where(np.arange(count) % 2, -1.0, 1.0)[:, None]
+    return (y + side * height * edge * n).astype(np.float32)
+
+
+# a mesh on the element-once plan of few rows, and one past 4e6 pairs; elements
+# within and past the phase limit of the FP64 kernel (k rho 0.79)
+@pytest.mark.gpu
+@pytest.mark.parametrize("prec,u", [(bem.PREC_FP32, 6e-8), (bem.PREC_FP64, 1.1e-16)], ids=["fp32", "fp64"])
+@pytest.mark.parametrize("bc", [(0, 1), (0.5 + 0.25j, 1.0 - 0.5j)], ids=["rigid", "impedance"])
+@pytest.mark.parametrize("subdiv,k", [(2, 9.0), (2, 90.0), (4, 30.0)])
+@pytest.mark.parametrize("height", [0.3, 0.1, 0.03, 0.01])
+def test_rows_next_to_the_surface(height, subdiv, k, bc, prec, u):
+    m = _body(subdiv, bc)
+    p, e, _ = C.mesh_arrays(m)
+    xs = _above(p, e, height, 12)
+    A = _matrix_rows(m, xs, k, prec)
+    A0, tol = _rows(p, e, bc, float(np.float32(k)), xs, u)
+    ratio = np.abs(A - A0) / tol
+    print("case: height %g: worst %.2g of the tolerance, median %.2g" % (height, ratio.max(), np.median(ratio)), flush=True)
+    assert ratio.max() <= 1
+
+
+# the rows of a radiation operator, on the small mesh's tiles
+@pytest.mark.gpu
+@pytest.mark.parametrize("height", [0.3, 0.1, 0.03, 0.01])
+def test_operator_rows_next_to_the_surface(height):
+    m = _body(2, (0, 1))
+    p, e, _ = C.mesh_arrays(m)
+    xs = _above(p, e, height, 70)
+    s = bem.Solver(m)
+    s.assemble(9.0, bem.PREC_FP32)
+    F = s.field_matrix(xs).get_field_matrix()
+    s.close()
+    F0, tol = _rows(p, e, (0, 1), 9.0, xs, 6e-8)
+    assert np.all(np.abs(F - F0) <= tol)
