@@ -268,20 +268,28 @@ __global__ void kc_act_init(int R, const double *__restrict__ g0, const int *__r
 
 // ------------------------------------------------------------ block CG ---
 constexpr int kMaxBlock = 64;    // right-hand sides of one block (Rb <= 64)
+// M N R from which the block iteration pays for any number of right-hand sides,
+// and from which its FP32 products run as FP16-split ones
+constexpr double kSplitMinWork = 4e8;
 // Whether the block iteration repays its steps' fixed cost (three dozen small
 // launches, a host wait and the R x R algebra on the host: 0.08 ms up to 4
 // right-hand sides, 0.1 at 16, 0.3 at 32) against lockstep CG steps of
 // 20 us + 3 us per 1e6 of M N.  Solves of 16 CHIEF points to 1e-8, lockstep over
-// block time at an easy and a hard frequency (ka 5 and 16 at 4002 nodes):
-//   up to 16 right-hand sides, by the reads of the matrix they save:
-//     4002 nodes, R = 8: 1.03, 1.77; R = 16: 1.07, 2.5; 4842, R = 6: 1.35, 1.6;
-//     6252, R = 4: 1.10, 1.6; R = 16: 1.75, 4.2; 7842, R = 2: 1.07, 1.04;
-//     but 3242, R = 16: 0.83, 1.7; 4002, R = 6: 0.9, 1.5; 6252, R = 2: 0.8, 0.95;
+// block time at an easy and a hard frequency (k a 5 and 16):
+//   up to 16 right-hand sides, by the reads of the matrix they save, on FP32
+//   products:
+//     4002 nodes, R = 8: 1.38, 1.56; R = 16: 1.24, 2.0; 4842, R = 6: 1.36, 1.49;
+//     6252, R = 4: 1.29, 1.33; R = 10: 1.60, 2.3; 7842, R = 2: 1.12, 1.13;
+//     10242, R = 2: 1.35, 1.25;
 //   more than 16, where the host algebra grows: 2562, R = 32: 0.6, 1.05;
 //     3242, R = 32: 0.65, 1.25; 4002, R = 32: 0.7, 1.8; 10242, R = 32: 1.5.
+// The FP16-split products are worth their passes over the block vectors on large
+// systems only: below kSplitMinWork the FP32 products are as fast or faster
+// (4002 nodes, R = 8: 2.71 against 3.22 ms; 6252, R = 8: 12.3 against 14.9; 10242,
+// R = 2: 12.8 against 13.7 and 55.2 against 54.3).
 static bool block_pays(double M, double N, double R) {
     const double mn = M * N;
-    return mn * R >= 4e8 || (R <= 16 && mn >= 1.5e7 && mn * R >= 1.2e8);
+    return mn * R >= kSplitMinWork || (R <= 16 && mn >= 1.5e7 && mn * R >= 1.2e8);
 }
 constexpr int kGramRows = 64;    // rows of one Gram partial
 constexpr int kGramSub = 32;     // rows staged in LDS at a time
@@ -654,8 +662,10 @@ int cgls_device(const float2 *A32, const double2 *A64, long lda, int M, int N, c
     // copy, which also leaves the bound amax on |Re A|, |Im A| (per-tile
     // maxima).  At M = N = 40962 with 32 right-hand sides: 2.6 ms a product
     // against 3.37 ms on the FP32 kernels, the same error against the FP64
-    // solve.  BEM_GEMM_NO_F16 keeps the FP32 products.
-    const bool want_f16s = block_on && f32 && R > 1 && getenv("BEM_GEMM_NO_F16") == nullptr;
+    // solve.  BEM_GEMM_NO_F16 keeps the FP32 products, BEM_BLOCK_CG_ALWAYS takes
+    // the split ones at every size.
+    const bool want_f16s = block_on && f32 && ((double)M * N * R >= kSplitMinWork || getenv("BEM_BLOCK_CG_ALWAYS")) &&
+                           getenv("BEM_GEMM_NO_F16") == nullptr;
     if (want_f16s) HOST_CALL(salloc(&w.amaxws, ws_adjoint_absmax(M, N) / sizeof(float), s));
     if (f32 && R > 1) HOST_CALL(adjoint_copy_make(A32, lda, M, N, R, &w.AH, s, w.amaxws, want_f16s));
     const int gblk = (N + kGramRows - 1) / kGramRows;

@@ -242,9 +242,12 @@ int bem_solver_set_rhs(bem_solver *s, int kind, const float *params, int nrhs, f
  * conjugate gradients over all right-hand sides at once (one shared block
  * Krylov space, orthonormalised residual block), with the same refinement;
  * falls back to BEM_SOLVE_CGLS's iteration when the block breaks down (e.g.
- * two equal right-hand sides), and takes that iteration from the start when
- * M * N * nrhs < 4e8, where a block step's fixed cost outweighs its fewer
- * steps (environment BEM_BLOCK_CG_ALWAYS: the block at every size).
+ * two equal right-hand sides), and takes that iteration from the start on
+ * small systems, where a block step's fixed cost outweighs its fewer steps: for
+ * more than 16 right-hand sides below M * N * nrhs = 4e8, for up to 16 below
+ * M * N * nrhs = 1.2e8 or M * N = 1.5e7.  Its FP32 products read the operands as
+ * FP16 hi/lo pairs from M * N * nrhs = 4e8 on (environment BEM_BLOCK_CG_ALWAYS:
+ * the block, on such products, at every size; BEM_GEMM_NO_F16: FP32 products).
  * iterations counts block steps. */
 int bem_solver_solve(bem_solver *s, int method, int restart, float tol, int maxit, double refine_tol,
                      int max_refine, bem_solve_stats *stats);
