@@ -1921,10 +1921,12 @@ struct TileShape {
 std::mutex g_tune_mu;
 std::map<std::pair<int, int>, TileShape> g_tune;
 thread_local const TileShape *t_force = nullptr;  // candidate under test
+thread_local bool t_untuned = false;              // no shape asked for, whatever the table holds
 
 int half_octave(long v) { return (int)std::lround(2.0 * std::log2((double)std::max(1L, v))); }
 
 bool tuned_shape(int M, int E, TileShape &out) {
+    if (t_untuned) return false;
     if (t_force) {
         out = *t_force;
         return true;
@@ -1997,7 +1999,17 @@ int autotune_assembly(const Mesh &m, double k, int precision, int *best_qg, int 
     std::vector<TileShape> cand;
     for (int qg : {1, 4})
         for (int w : {4096, 8192, 16384, 32768}) cand.push_back(TileShape{qg, w});
-    TileShape def{(precision == BEM_PREC_FP64 && (long)M * E < 4000000L) ? 4 : 1, kDefaultWaves};
+    // the shape of an untuned build
+    TileShape def{1, kDefaultWaves};
+    {
+        DeviceProblem dp;
+        t_untuned = true;
+        const int rc = device_problem_build(m, dp, s);
+        t_untuned = false;
+        if (!dp.use_ghost) def.qg = dp.qg;
+        device_problem_free(dp);
+        HOST_CALL(rc);
+    }
     double bms = 1e300, dms = -1;
     TileShape best = def;
     hipEvent_t e0, e1;
@@ -2168,7 +2180,7 @@ int halo_plan(DeviceProblem &dp, hipStream_t s) {
     for (int e = 0; e < dp.E; e++)
         for (int j = 0; j < 3; j++) m.elems[e].nodes[j] = dp.helems[3 * e + j];
     TilePlan plan;
-    build_tile_plan(m, choose_tiles(dp.M, dp.N, dp.E, 64 / dp.qg), plan);
+    build_tile_plan(m, dp.hP, plan);
     Pack pk;
     pk.add(&dp.tile_ptr, (const int *)plan.ptr.data(), plan.ptr.size());
     pk.add(&dp.tile_entries, (const int *)plan.entries.data(), plan.entries.size());
@@ -2245,6 +2257,7 @@ int device_problem_build(const Mesh &m, DeviceProblem &dp, hipStream_t s) {
     dp.n_isolated = (int)isolated.size();
     const int qg = choose_qg(dp.M, dp.E);
     dp.qg = qg;
+    dp.hP = choose_tiles(dp.M, dp.N, dp.E, 64 / qg);
     // element-once plan for the FP32 fast kernel: taken when the halo plan
     // integrates at least 5 % of the elements twice and the side columns stay
     // within ghost_slot_bound (device_problem_bytes counts that bound).  It
@@ -2338,6 +2351,7 @@ int device_problem_rows(const DeviceProblem &base, const float *xs, int P, Devic
             }
     }
     dp.diam = diagonal(dp.lo, dp.hi);
+    if (dp.P == 0) dp.hP = choose_tiles(dp.M, dp.N, dp.E, 64 / dp.qg);
     Pack pk;
     pk.add(&dp.pts, (const float4 *)p4.data(), p4.size());
     pk.add(&dp.pts64, (const double *)dp.hpts.data(), dp.hpts.size());

@@ -179,8 +179,9 @@ struct DeviceProblem {
     int source = 0;               // some element has cc != 0
     double lo[3] = {0, 0, 0}, hi[3] = {0, 0, 0};  // bounding box of the M points
     double diam = 0;              // its diagonal: bounds every |x - y|
-    // halo plan (TilePlan): P column tiles, 0 until a kernel that walks them runs
-    int P = 0;
+    // halo plan (TilePlan): hP column tiles asked for when the problem is built,
+    // P of them made, 0 until a kernel that walks them runs
+    int hP = 0, P = 0;
     int *tile_ptr = nullptr;
     int *tile_entries = nullptr;
     int n_isolated = 0;
