@@ -2098,30 +2098,28 @@ void tune_clear() {
     product_tune_clear();
 }
 
-// Upper bound of the HBM bytes device_problem_build allocates for a mesh of
-// M rows (nodes + CHIEF), N nodes and E elements.
-size_t device_problem_bytes(int M, int N, int E) {
-    const size_t Mp = ((size_t)M + 63) / 64 * 64;
+// Upper bound of the HBM bytes that the problem of a mesh of M rows (nodes +
+// CHIEF), N nodes and E elements and its assemblies in one precision allocate.
+size_t device_problem_bytes(int M, int N, int E, bool fp64) {
+    const size_t Mp = ((size_t)M + 63) / 64 * 64, real = fp64 ? sizeof(double) : sizeof(float);
     const int qg = choose_qg(M, E);
     const size_t P = (size_t)choose_tiles(M, N, E, 64 / qg);
     size_t b = 0;
     b += sizeof(float4) * M + sizeof(double) * 3 * M + sizeof(double2) * M;        // points, bterm
     b += (sizeof(int) + sizeof(float2)) * 3 * (size_t)E;                            // elements, bc
     b += (sizeof(ElemRec<float>) + sizeof(ElemRec<double>) + sizeof(FarRec)) * (size_t)E;  // element records
-    b += (sizeof(float) + sizeof(double)) * 48 * (size_t)E;                          // singular terms
+    b += real * 48 * (size_t)E;                                                      // singular terms
     b += sizeof(int) * (P + 1 + 3 * (size_t)E + N);                                  // tile CSR, isolated
     b += 40 * 256;                                                                   // the packed arrays' alignment
-    b += (sizeof(float) + sizeof(float2) + sizeof(double) + sizeof(double2)) * P * Mp;  // tile partials
+    size_t tiles = P, sides = 0;
     if (asked_qg(M, E) != 4) {
         // element-once plan: its side columns and index arrays
         const int gP = choose_tiles(M, N, E, 64, 2);
-        const size_t gs = (size_t)ghost_slot_bound(N, gP);
-        b += (sizeof(float2) + sizeof(double2)) * gs * Mp;
-        if ((size_t)gP > P)  // its tile partials
-            b += (sizeof(float) + sizeof(float2) + sizeof(double) + sizeof(double2)) * ((size_t)gP - P) * Mp;
-        b += sizeof(int) * (gP + 1 + 4 * (size_t)E + 2 * (size_t)N + 2 * gs);
+        sides = (size_t)ghost_slot_bound(N, gP);
+        tiles = std::max(P, (size_t)gP);
+        b += sizeof(int) * (gP + 1 + 4 * (size_t)E + 2 * (size_t)N + 2 * sides);
     }
-    return b;
+    return b + real * (3 * tiles + 2 * sides) * Mp;  // tile partials, side columns
 }
 
 namespace {

@@ -213,7 +213,7 @@ int device_problem_build(const Mesh &m, DeviceProblem &dp, hipStream_t s);
 // rows for the P points xs over base's elements and tiles (base outlives dp)
 int device_problem_rows(const DeviceProblem &base, const float *xs, int P, DeviceProblem &dp, hipStream_t s);
 void device_problem_free(DeviceProblem &dp);
-size_t device_problem_bytes(int M, int N, int E);
+size_t device_problem_bytes(int M, int N, int E, bool fp64);
 // assembly launch-shape tuning (assembly.hip)
 int autotune_assembly(const Mesh &m, double k, int precision, int *best_qg, int *best_waves, double *best_ms,
                       double *default_ms, hipStream_t s);
@@ -352,7 +352,7 @@ int gemm_n_f32z_batched(const float2 *A, long lda, long astride, int nmat, long 
                         ProdParts *parts = nullptr);
 int mres_f32a_batched(const float2 *A, long lda, long astride, int nmat, long M, long N, const double2 *X, long ldx,
                       const double2 *b, long ldb, double2 *out, long ldo, int R, void *ws, hipStream_t s);
-size_t qr_work_bytes(int M, int N, bool fp64);
+size_t qr_work_bytes(int M, int N, int R, bool fp64);
 // C -= V (T^H (V^H C)) from the partials of C^H V (QR trailing update, V with 32
 // columns)
 int qr_trail_f32(const float2 *V, long ldv, int M, const float2 *T, int nb, const ProdParts &zp, int nc, float2 *C,

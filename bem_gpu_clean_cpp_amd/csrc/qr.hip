@@ -1558,14 +1558,19 @@ static int qr_factor(QRFactor<T> &f, int extra_cols, hipStream_t s) {
 
 static int group_splits(int npair) { return std::max(1, std::min(16, 1024 / npair)); }
 
-// device bytes of a factorisation beyond the matrix, and of the largest solve's
-// scratch that does not grow with the right-hand sides
-size_t qr_work_bytes(int M, int N, bool fp64) {
+// rows of a workgroup of a solve's launches: at most 64 workgroups
+static int solve_rows(int M) { return 64 * ((M + 64 * 64 - 1) / (64 * 64)); }
+
+// device bytes of a factorisation beyond the matrix and of its solves (FP64: R
+// right-hand sides at once, FP32: one after the other)
+size_t qr_work_bytes(int M, int N, int R, bool fp64) {
     const size_t np = ((size_t)N + kNB - 1) / kNB, ng = (np + kGB - 1) / kGB, ld = ((size_t)M + 63) / 64 * 64;
     const size_t splits = group_splits((int)(ng * kPairs));
     size_t b = (fp64 ? sizeof(double2) : sizeof(float2)) * kNB * (np * kNB + N);   // T factors, W
     b += sizeof(double2) * (2 * ng * kGG + (ng * kPairs * splits + np) * kNN);       // triangles and what forms them
     if (!fp64) b += sizeof(float2) * 2 * kNB * ld + sizeof(double2) * (kGramParts + 1) * kNN;  // V, panel, Gram
+    const size_t nblk = ((size_t)M + solve_rows(M) - 1) / solve_rows(M);
+    b += (fp64 ? (size_t)R : 1) * (2 * nblk * 2 * kGW * sizeof(double) + (fp64 ? sizeof(double2) : sizeof(float2)) * N);
     return b;
 }
 
@@ -1622,7 +1627,7 @@ static int qr_solve_factored(QRFactor<T> &f, typename QT<T>::c2 *B, long ldb, in
     // substitution, the rows spread over at most 64 workgroups
     HOST_CALL(qr_groups<T>(f, s));
     const int ng = ((f.N + kNB - 1) / kNB + kGB - 1) / kGB;
-    const int rpb = 64 * ((f.M + 64 * 64 - 1) / (64 * 64)), nblk = (f.M + rpb - 1) / rpb;
+    const int rpb = solve_rows(f.M), nblk = (f.M + rpb - 1) / rpb;
     const size_t zn = (size_t)R * nblk * 2 * kGW;
     double *zb = nullptr;
     C2 *X = nullptr;

@@ -175,12 +175,13 @@ double bem_request_footprint(int M, int N, int E, int nrhs, int precision, int m
     const size_t ldv = ((size_t)std::max(M, N) + 63) / 64 * 64;
     const size_t R = (size_t)nrhs;
     const size_t ea = precision == BEM_PREC_FP64 ? sizeof(double2) : sizeof(float2);
-    size_t b = device_problem_bytes(M, N, E);
+    const bool fp64 = precision == BEM_PREC_FP64;
+    size_t b = device_problem_bytes(M, N, E, fp64);
     b += ea * ld * N;                                               // A
     b += (2 * sizeof(double2) + sizeof(float2)) * ld * R;           // B, X (FP64), X (FP32)
     if (method == BEM_SOLVE_QR) {
         b += ea * ld * N;                                           // factored copy of A
-        b += qr_work_bytes(M, N, precision == BEM_PREC_FP64);       // panels, T factors, triangles of the solves
+        b += qr_work_bytes(M, N, nrhs, fp64);                       // panels, T factors, triangles and sums of the solves
         b += 2 * sizeof(double2) * ld + ws_gemv_n(M, N, 1);
     } else {
         const size_t K = (size_t)std::max(1, std::min(restart, N));
