@@ -2189,13 +2189,15 @@ int halo_plan(DeviceProblem &dp, hipStream_t s) {
 
 // The arrays an assembly in R writes besides the matrix, one allocation per
 // precision, grown when a plan of more tiles asks for it: the singular terms,
-// the tile partials of c and the BC sums (P tiles), the side columns.
+// the tile partials of c and the BC sums (P tiles), the side columns, for Mp
+// rows at a time.
 template <typename R>
-int asm_scratch(DeviceProblem &dp, int P, long nside, R **sing, R **cpart, R **bpart, R **side, hipStream_t s) {
+int asm_scratch(DeviceProblem &dp, int P, long nside, long Mp, R **sing, R **cpart, R **bpart, R **side,
+                hipStream_t s) {
     const size_t pad = 256 / sizeof(R);
     auto up = [&](size_t n) { return (n + pad - 1) / pad * pad; };
-    const size_t ns = up((size_t)dp.E * 48), nc = up((size_t)P * dp.Mp), nb = up((size_t)2 * P * dp.Mp);
-    const size_t n = ns + nc + nb + (size_t)2 * nside * dp.Mp;
+    const size_t ns = up((size_t)dp.E * 48), nc = up((size_t)P * Mp), nb = up((size_t)2 * P * Mp);
+    const size_t n = ns + nc + nb + (size_t)2 * nside * Mp;
     char *&mem = sizeof(R) == 4 ? dp.scratch32 : dp.scratch64;
     size_t &cap = sizeof(R) == 4 ? dp.cap32 : dp.cap64;
     if (cap < n * sizeof(R)) {
@@ -2393,80 +2395,16 @@ static void sing_tab(SingTab &t) {
     }
 }
 
-// Rows r0..M-1 of the system into A (ld ldA, row r0 first) and their
-// boundary-condition sums into bterm; r0 = 0 is the whole collocation system.
+// Rows a.r0..a.M-1 into a.A and their boundary-condition sums into bterm.
 template <typename R, typename C2>
-static int assemble_impl(DeviceProblem &dp, R k, C2 *A, long ldA, int r0, double2 *bterm, hipStream_t s) {
-    HOST_CALL(ensure_quad());
-    if (dp.M == 0) BEM_FAIL("device problem not built");
-    const Config &cfg = config();
-    const double kd = (double)k;
-    const double rw = (double)cfg.density * (double)(k * (R)cfg.speed);  // rho * omega, omega = k c
-    QuadTables qt;
-    quad_tables(qt);
-    SingTab st;
-    sing_tab(st);
-    // the plan this call walks, and the arrays it writes
-    // (FP64: the fast kernel's phases hold up to 2^30 quadrants)
-    const bool ghost = dp.use_ghost && !getenv("BEM_ASM_HALO") && !getenv("BEM_GENERIC_TILE") &&
-                       (sizeof(R) == 4 || std::fabs(kd) * dp.diam < 1e8);
-    if (!ghost) HOST_CALL(halo_plan(dp, s));
-    const int P = ghost ? dp.gP : dp.P;
-    R *sing = nullptr, *cpart = nullptr, *bpart = nullptr, *side = nullptr;
-    HOST_CALL(asm_scratch<R>(dp, P, ghost ? dp.nslots : 0, &sing, &cpart, &bpart, &side, s));
-    {
-        TimedRegion tr;
-        timing_begin(tr, "sing_elems", s);
-        const int n = 3 * dp.E, bs = 128;
-        sing_elems<R><<<(n + bs - 1) / bs, bs, 0, s>>>(dp.pts64, dp.elems, dp.bc, dp.E, kd, rw, st, sing);
-        HIP_CALL(hipGetLastError());
-        timing_end(tr, s);
-    }
-    AsmArgs<R> a;
-    a.pts = dp.pts;
-    a.recs = (const ElemRec<R> *)(sizeof(R) == 4 ? (void *)dp.rec32 : (void *)dp.rec64);
-    a.far = dp.far32;
-    a.sing = sing;
-    a.tile_ptr = dp.tile_ptr;
-    a.tile_entries = dp.tile_entries;
-    a.A = A;
-    a.cpart = cpart;
-    a.bpart = (C2 *)bpart;
-    a.ldA = ldA;
-    a.Mp = dp.Mp;
-    a.M = dp.M;
-    a.N = dp.N;
-    a.r0 = r0;
-    const int rpw = 64 / dp.qg;
-    const int nrb = (dp.M - r0 + rpw - 1) / rpw;
-    a.nrbg = (nrb + 3) / 4;
+static int assemble_rows(const DeviceProblem &dp, AsmArgs<R> a, bool ghost, int P, double2 *bterm, hipStream_t s) {
+    const int nrows = a.M - a.r0, rpw = ghost ? 64 : 64 / dp.qg;
+    a.nrbg = ((nrows + rpw - 1) / rpw + 3) / 4;
     a.nwg = a.nrbg * P;
-    a.k = k;
-    a.kf = (R)(kd / (2.0 * kPi));
-    a.kf64 = kd / (2.0 * kPi);
-    a.rw = (R)rw;
-    far_limits(kd, sizeof(R) == 4 ? kFarK2 : kSmallPhase64, a.far_rho2, a.far7_rho2);
-    a.impedance = dp.impedance;
-    for (int q = 0; q < kNQ; q++) {
-        a.q.xi1[q] = sizeof(R) == 4 ? (R)qt.xi1[q] : (R)qt.dxi1[q];
-        a.q.xi2[q] = sizeof(R) == 4 ? (R)qt.xi2[q] : (R)qt.dxi2[q];
-        a.q.w[q] = sizeof(R) == 4 ? (R)qt.w[q] : (R)qt.dw[q];
-    }
-    a.tile_slots = nullptr;
-    a.side = nullptr;
-    const int nrows = dp.M - r0;
     {
         TimedRegion tr;
         timing_begin(tr, sizeof(R) == 4 ? "asm_tile_f32" : "asm_tile_f64", s);
-        if (ghost) {
-            a.nrbg = ((nrows + 63) / 64 + 3) / 4;
-            a.nwg = a.nrbg * P;
-            a.tile_ptr = dp.gtile_ptr;
-            a.tile_entries = dp.gtile_entries;
-            a.tile_slots = dp.gtile_slots;
-            a.side = (C2 *)side;
-        }
-        dim3 grid(a.nwg), block(256);
+        const dim3 grid(a.nwg), block(256);
         if (sizeof(R) == 8 && ghost) {
             AsmArgs<double> &ad = *(AsmArgs<double> *)&a;
             if (dp.impedance) asm_tile_fast64<true, true><<<grid, block, 0, s>>>(ad);
@@ -2480,7 +2418,7 @@ static int assemble_impl(DeviceProblem &dp, R k, C2 *A, long ldA, int r0, double
             // the phase k r / (2 pi) goes to them unreduced while every
             // distance (at most the bounding-box diagonal of the points) keeps
             // it below that
-            const bool raw = kd / (2.0 * kPi) * dp.diam < 250.0;
+            const bool raw = a.kf64 * dp.diam < 250.0;
             AsmArgs<float> &af = *(AsmArgs<float> *)&a;
 #define BEM_FAST(IMP_, SRC_)                                                                     \
     do {                                                                                         \
@@ -2501,29 +2439,113 @@ static int assemble_impl(DeviceProblem &dp, R k, C2 *A, long ldA, int r0, double
         timing_end(tr, s);
     }
     if (ghost && dp.ngnodes > 0) {
-        if (ldA % 2 || dp.Mp % 2) BEM_FAIL("ghost_reduce needs even leading dimensions (ldA %ld, Mp %ld)", ldA, dp.Mp);
+        if (a.ldA % 2 || a.Mp % 2) BEM_FAIL("ghost_reduce needs even leading dimensions (ldA %ld, Mp %ld)", a.ldA, a.Mp);
         TimedRegion tr;
         timing_begin(tr, "ghost_reduce", s);
         constexpr int W = sizeof(R) == 4 ? 2 : 1;
         using V4 = typename std::conditional<sizeof(R) == 4, float4, double2>::type;
         dim3 grid(((nrows + W - 1) / W + 255) / 256, dp.ngnodes);
-        ghost_reduce<V4, W><<<grid, 256, 0, s>>>((V4 *)A, ldA, nrows, (const V4 *)side, dp.Mp, dp.gred_ptr,
+        ghost_reduce<V4, W><<<grid, 256, 0, s>>>((V4 *)a.A, a.ldA, nrows, (const V4 *)a.side, a.Mp, dp.gred_ptr,
                                                  dp.gred_node, dp.gred_own, dp.gred_slot);
         HIP_CALL(hipGetLastError());
         timing_end(tr, s);
     }
     if (dp.n_isolated > 0) {
         dim3 grid((nrows + 255) / 256, dp.n_isolated);
-        zero_columns<C2><<<grid, 256, 0, s>>>(A, ldA, nrows, dp.isolated, dp.n_isolated);
+        zero_columns<C2><<<grid, 256, 0, s>>>(a.A, a.ldA, nrows, dp.isolated, dp.n_isolated);
         HIP_CALL(hipGetLastError());
     }
     {
         TimedRegion tr;
         timing_begin(tr, "asm_finalize", s);
         asm_finalize<R, C2><<<(nrows + 63) / 64, 64 * kFinRuns, 0, s>>>(
-            A, ldA, dp.M, dp.N, P, dp.Mp, r0, a.cpart, a.bpart, bterm, dp.impedance || dp.source);
+            a.A, a.ldA, a.M, dp.N, P, a.Mp, a.r0, a.cpart, a.bpart, bterm, dp.impedance || dp.source);
         HIP_CALL(hipGetLastError());
         timing_end(tr, s);
+    }
+    return EXIT_SUCCESS;
+}
+
+// Rows of a radiation operator of n rows that are assembled at a time in P tiles:
+// blocks of equal height (a multiple of a workgroup's 256 rows) of at most 8192
+// workgroups.  The tiles are the mesh's, however many points there are, so the
+// partials and side columns of all of them at once would take up to twice the
+// operator's own bytes: 642 nodes, 200000 points: 2.0 GB beside 1.03 GB; in blocks
+// 0.15.  (4096 workgroups leave the 6001 points of a 2562-node map in two blocks:
+// 0.55 ms instead of 0.39.)
+static int operator_rows(int n, int P) {
+    const int most = 256 * ((8192 + P - 1) / P), blocks = (n + most - 1) / most;
+    return ((n + blocks - 1) / blocks + 255) / 256 * 256;
+}
+
+// Rows r0..M-1 of the system into A (ld ldA, row r0 first) and their
+// boundary-condition sums into bterm; r0 = 0 is the whole collocation system,
+// r0 = N the operator of a field's points.
+template <typename R, typename C2>
+static int assemble_impl(DeviceProblem &dp, R k, C2 *A, long ldA, int r0, double2 *bterm, hipStream_t s) {
+    HOST_CALL(ensure_quad());
+    if (dp.M == 0) BEM_FAIL("device problem not built");
+    const Config &cfg = config();
+    const double kd = (double)k;
+    const double rw = (double)cfg.density * (double)(k * (R)cfg.speed);  // rho * omega, omega = k c
+    QuadTables qt;
+    quad_tables(qt);
+    SingTab st;
+    sing_tab(st);
+    // the plan this call walks, and the arrays it writes
+    // (FP64: the fast kernel's phases hold up to 2^30 quadrants)
+    const bool ghost = dp.use_ghost && !getenv("BEM_ASM_HALO") && !getenv("BEM_GENERIC_TILE") &&
+                       (sizeof(R) == 4 || std::fabs(kd) * dp.diam < 1e8);
+    if (!ghost) HOST_CALL(halo_plan(dp, s));
+    const int P = ghost ? dp.gP : dp.P;
+    R *sing = nullptr, *cpart = nullptr, *bpart = nullptr, *side = nullptr;
+    const int block = r0 < dp.N ? dp.M - r0 : std::min(dp.M - r0, operator_rows(dp.M - r0, P));
+    const long Mp = ((long)block + 63) / 64 * 64;
+    HOST_CALL(asm_scratch<R>(dp, P, ghost ? dp.nslots : 0, Mp, &sing, &cpart, &bpart, &side, s));
+    if (r0 < dp.N) {  // (rows that are no nodes meet no singular pair)
+        TimedRegion tr;
+        timing_begin(tr, "sing_elems", s);
+        const int n = 3 * dp.E, bs = 128;
+        sing_elems<R><<<(n + bs - 1) / bs, bs, 0, s>>>(dp.pts64, dp.elems, dp.bc, dp.E, kd, rw, st, sing);
+        HIP_CALL(hipGetLastError());
+        timing_end(tr, s);
+    }
+    AsmArgs<R> a;
+    a.pts = dp.pts;
+    a.recs = (const ElemRec<R> *)(sizeof(R) == 4 ? (void *)dp.rec32 : (void *)dp.rec64);
+    a.far = dp.far32;
+    a.sing = sing;
+    a.tile_ptr = dp.tile_ptr;
+    a.tile_entries = dp.tile_entries;
+    a.cpart = cpart;
+    a.bpart = (C2 *)bpart;
+    a.ldA = ldA;
+    a.Mp = Mp;
+    a.N = dp.N;
+    a.k = k;
+    a.kf = (R)(kd / (2.0 * kPi));
+    a.kf64 = kd / (2.0 * kPi);
+    a.rw = (R)rw;
+    far_limits(kd, sizeof(R) == 4 ? kFarK2 : kSmallPhase64, a.far_rho2, a.far7_rho2);
+    a.impedance = dp.impedance;
+    for (int q = 0; q < kNQ; q++) {
+        a.q.xi1[q] = sizeof(R) == 4 ? (R)qt.xi1[q] : (R)qt.dxi1[q];
+        a.q.xi2[q] = sizeof(R) == 4 ? (R)qt.xi2[q] : (R)qt.dxi2[q];
+        a.q.w[q] = sizeof(R) == 4 ? (R)qt.w[q] : (R)qt.dw[q];
+    }
+    a.tile_slots = nullptr;
+    a.side = nullptr;
+    if (ghost) {
+        a.tile_ptr = dp.gtile_ptr;
+        a.tile_entries = dp.gtile_entries;
+        a.tile_slots = dp.gtile_slots;
+        a.side = (C2 *)side;
+    }
+    for (int b0 = r0; b0 < dp.M; b0 += block) {
+        a.r0 = b0;
+        a.M = std::min(dp.M, b0 + block);
+        a.A = A + (b0 - r0);
+        HOST_CALL((assemble_rows<R, C2>(dp, a, ghost, P, bterm + (b0 - r0), s)));
     }
     // opt-in FP64 near-singular corrections, after every row is complete
     if (cfg.near_factor > 0 || dp.near_factor > 0) HOST_CALL((near_correct<R, C2>(dp, kd, rw, A, ldA, r0, bterm, s)));
