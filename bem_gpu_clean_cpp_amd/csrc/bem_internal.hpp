@@ -5,6 +5,7 @@
 #include <cstdint>
 #include <cstdio>
 #include <cstdlib>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -440,5 +441,41 @@ void sfree(T *&p, hipStream_t s) {
     if (p) (void)hipFreeAsync((void *)p, s);
     p = nullptr;
 }
+
+// Pinned host blocks (block CG's R x R transfers, the flags of QR panels), reused
+// across solves and threads: hipHostFree waits for the whole device, which would
+// stall the other solvers of a batch or server at every solve's end.  The blocks
+// live until the process ends (one per solve running at once).
+class PinnedPool {
+public:
+    static constexpr size_t kBytes = sizeof(double2) * (4 + 4 + 6) * 64 * 64;
+    static int acquire(double2 **p) {
+        {
+            std::lock_guard<std::mutex> lk(mu());
+            if (!free_list().empty()) {
+                *p = free_list().back();
+                free_list().pop_back();
+                return EXIT_SUCCESS;
+            }
+        }
+        HIP_CALL(hipHostMalloc((void **)p, kBytes, hipHostMallocDefault));
+        return EXIT_SUCCESS;
+    }
+    static void release(double2 *p) {
+        if (!p) return;
+        std::lock_guard<std::mutex> lk(mu());
+        free_list().push_back(p);
+    }
+
+private:
+    static std::mutex &mu() {
+        static std::mutex m;
+        return m;
+    }
+    static std::vector<double2 *> &free_list() {
+        static std::vector<double2 *> v;
+        return v;
+    }
+};
 
 }  // namespace bem

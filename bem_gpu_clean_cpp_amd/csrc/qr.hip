@@ -19,7 +19,9 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <chrono>
 #include <cstdlib>
+#include <thread>
 #include <vector>
 
 #include "bem_internal.hpp"
@@ -39,6 +41,7 @@ struct QT<double> {
 
 constexpr int kNB = 32;  // panel width
 constexpr int kCG = 8;   // panel columns updated together
+constexpr int kColThreads = 256;  // rows per workgroup of the column launches
 
 template <typename T>
 __device__ __forceinline__ T wsum(T v) {
@@ -328,7 +331,9 @@ __device__ __forceinline__ void wave_reduce_scatter64<float>(float (&x)[2 * kNB]
 // scaled to norm 1), so panels of kappa^2 > 1e9, those whose Gram matrix is not
 // numerically positive definite (dependent or zero columns, numbers that are
 // not finite) and those with a column that needs no reflection take the
-// column-wise algorithm inside qr_recon instead.
+// column-wise algorithm inside qr_recon instead, in one workgroup; where the panels
+// of a matrix do so again and again, PanelRoute sends the next ones to a launch per
+// column.
 //
 // 5 + 32 + 5 us a panel of up to 2000 rows.  The column-wise panels that this
 // replaces were bound by their 32 serial steps: 69 us (256 rows), 98 (512) and
@@ -425,7 +430,7 @@ struct PanelPivot {
 // on the diagonal) and L (below it) to the top rows of the panel, T to Tout,
 // the top rows of V to Vd, U^-1 to Y (row-major), *bad = 0.  Panels that the
 // reconstruction does not take (above) are factored column by column instead,
-// with T, and *bad = 1.
+// with T, and *bad = 1.  The host learns it from seen (pinned memory, or null).
 //
 // One workgroup eliminates two matrices in place and in step: G and P_1 - S R.
 // Step k needs row k of R only, which is row k of G's elimination scaled, so
@@ -447,7 +452,7 @@ constexpr int kRecThreads = 512, kRecWaves = kRecThreads / 64, kEnt = kNB / kRec
 __global__ __launch_bounds__(kRecThreads) void qr_recon(const double2 *__restrict__ part, int nblk, float2 *A, long lda,
                                                         int M, int j0, int nb, float2 *__restrict__ Tout,
                                                         float2 *__restrict__ Vd, long ldv, double2 *__restrict__ Y,
-                                                        int *__restrict__ bad) {
+                                                        int *__restrict__ bad, int *seen) {
     __shared__ double2 s_row[2][kNB][kNB];   // published rows of G and P_1 - S R
     __shared__ double2 s_cw[kNB][kNB + 1];   // published columns of P_1 - S R
     __shared__ double2 s_cg[2][kNB];         // and of G (two buffers)
@@ -583,7 +588,9 @@ __global__ __launch_bounds__(kRecThreads) void qr_recon(const double2 *__restric
     k2 = 0;
 #pragma unroll
     for (int q = 0; q < kRecWaves; q++) k2 += s_w[q];
-    if (!(k2 <= kPanelCond2) || s_flat) {  // (also NaN)
+    const bool take = k2 <= kPanelCond2 && !s_flat;  // (not a NaN)
+    if (tid == 0 && seen) __hip_atomic_store(seen, take ? 0 : 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    if (!take) {
         __syncthreads();
         panel_one_wg<float>(A, lda, M, j0, nb, Tout, 1, (float2(*)[kNB])&s_row[0][0][0],
                             (float2(*)[kNB])&s_row[1][0][0]);
@@ -687,6 +694,132 @@ __global__ __launch_bounds__(256) void qr_form_v(const float2 *__restrict__ Pc, 
             if (c < nb) A[(size_t)(j0 + c) * lda + j0 + i] = v;
             Vd[(size_t)c * ldv + i] = v;  // (zero past nb)
         }
+}
+
+// FP32 panels of a matrix whose panels the Gram matrix does not take (PanelRoute):
+// one launch per column, the rows split over workgroups (one row per thread).
+// Launch jj applies the reflector of column jj to the workgroup's rows and then forms
+// the partials of column jj + 1 from the updated rows: |x|^2 below its
+// diagonal and sum conj(x_r) a_c(r) for the later columns c, x being the
+// column below the diagonal before scaling.  With v = x / (alpha - beta) below
+// the diagonal and v_j = 1,
+//   v^H a_c = a_c(j) + conj(scale) sum_{r > j} conj(x_r) a_c(r),
+// so the reflector's products need no pass of their own after its norm.  The
+// partials are summed in a fixed order by every workgroup of the next launch.
+// Row j of the panel (alpha and the a_c(j)) travels in its own buffer,
+// written by the workgroup holding the row, because that workgroup overwrites
+// the row during the launch that reads it.  jj = -1 only forms the partials of
+// column 0.  Column indices are runtime values here, so the row is walked with
+// compile-time column loops and compares, never by a runtime register index.
+// Leaves the reflectors and R in place and tau_jj on Tout's diagonal.
+template <int NT>
+__global__ __launch_bounds__(NT) void qr_panel_col(float2 *A, long lda, int M, int j0, int jj, const float *zin,
+                                                   const float2 *rin, float *zout, float2 *rout, int nblk,
+                                                   float2 *Tout) {
+    __shared__ float s_red[NT / 64][2 * kNB];
+    __shared__ float s_z[2 * kNB];
+    __shared__ float2 s_d[kNB];
+    const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+    const int i = j0 + blockIdx.x * NT + tid;
+    const bool live = i < M;
+    const int ic = min(i, M - 1);
+    float2 a[kNB];
+#pragma unroll
+    for (int c = 0; c < kNB; c++) a[c] = A[(size_t)(j0 + c) * lda + ic];
+    if (jj >= 0) {
+        const int j = j0 + jj;
+        if (tid < 2 * kNB) {
+            float t = 0.f;
+            for (int q = 0; q < nblk; q++) t += zin[(size_t)q * 2 * kNB + tid];
+            s_z[tid] = t;
+        }
+        __syncthreads();
+        const float tot = s_z[2 * jj];
+        const float2 alpha = rin[jj];
+        const float aa = sqrtf(alpha.x * alpha.x + alpha.y * alpha.y);
+        const float xnorm = sqrtf(aa * aa + tot);
+        float tau = 0.f;
+        float2 scale = make_float2(0.f, 0.f), beta = alpha;
+        if (tot > 0 || (xnorm > 0 && alpha.y != 0)) {
+            const float phr = aa > 0 ? alpha.x / aa : 1.f, phi = aa > 0 ? alpha.y / aa : 0.f;
+            beta = make_float2(-phr * xnorm, -phi * xnorm);
+            const float dr = alpha.x - beta.x, di = alpha.y - beta.y;
+            const float dd = dr * dr + di * di;
+            scale = make_float2(dr / dd, -di / dd);
+            tau = 2.f / (1.f + tot / dd);
+        }
+        if (tid < kNB) {
+            const int c = tid;
+            float2 d = make_float2(0.f, 0.f);
+            if (c > jj) {
+                // tau (a_c(j) + conj(scale) S_c)
+                const float sx = s_z[2 * c], sy = s_z[2 * c + 1];
+                const float2 ac = rin[c];
+                d.x = tau * (ac.x + scale.x * sx + scale.y * sy);
+                d.y = tau * (ac.y + scale.x * sy - scale.y * sx);
+            }
+            s_d[c] = d;
+        }
+        if (blockIdx.x == 0 && tid == 0) Tout[jj * kNB + jj] = make_float2(tau, 0.f);
+        __syncthreads();
+        if (live && i >= j) {
+            float2 x = make_float2(0.f, 0.f);
+#pragma unroll
+            for (int c = 0; c < kNB; c++)
+                if (c == jj) x = a[c];
+            const bool below = i > j;
+            const float2 v = below ? make_float2(x.x * scale.x - x.y * scale.y, x.x * scale.y + x.y * scale.x)
+                                   : make_float2(1.f, 0.f);
+#pragma unroll
+            for (int c = 0; c < kNB; c++) {
+                if (c == jj) {
+                    a[c] = below ? v : beta;
+                } else if (c > jj) {
+                    const float2 d = s_d[c];
+                    a[c].x -= d.x * v.x - d.y * v.y;
+                    a[c].y -= d.x * v.y + d.y * v.x;
+                }
+                if (c >= jj) A[(size_t)(j0 + c) * lda + i] = a[c];
+            }
+        }
+    }
+    if (jj + 1 < kNB) {
+        const int k = jj + 1, j1 = j0 + k;
+        float2 x = make_float2(0.f, 0.f);
+#pragma unroll
+        for (int c = 0; c < kNB; c++)
+            if (c == k) x = a[c];
+        const bool below = live && i > j1;
+        float z[2 * kNB];
+#pragma unroll
+        for (int c = 0; c < kNB; c++) {
+            float pr = 0.f, pi = 0.f;
+            if (below) {
+                if (c == k) {
+                    pr = x.x * x.x + x.y * x.y;
+                } else if (c > k) {
+                    pr = x.x * a[c].x + x.y * a[c].y;
+                    pi = x.x * a[c].y - x.y * a[c].x;
+                }
+            }
+            z[2 * c] = pr;
+            z[2 * c + 1] = pi;
+        }
+        if (live && i == j1) {
+#pragma unroll
+            for (int c = 0; c < kNB; c++)
+                if (c >= k) rout[c] = a[c];
+        }
+        wave_reduce_scatter64(z, lane);
+        s_red[wid][lane] = z[0];
+        __syncthreads();
+        if (tid < 2 * kNB) {
+            float t = 0.f;
+#pragma unroll
+            for (int w = 0; w < NT / 64; w++) t += s_red[w][tid];
+            zout[(size_t)blockIdx.x * 2 * kNB + tid] = t;
+        }
+    }
 }
 
 // T of the compact WY form from the taus (on Tout's diagonal) and
@@ -1436,10 +1569,21 @@ struct QRFactor {
     float2 *Pc = nullptr;
     double2 *gram = nullptr, *Y = nullptr;
     int *bad = nullptr;
+    double2 *pinned = nullptr;  // PinnedPool block: which panels took it
+    // partials and panel rows of the column launches
+    float *zcol = nullptr;
+    long zcol_stride = 0;
+    float2 *rcol = nullptr;
     // triangles of the groups of panels, for the solves
     double2 *GT = nullptr, *GR = nullptr;
     hipStream_t st = nullptr;
     ~QRFactor() {
+        if (pinned) {
+            (void)hipStreamSynchronize(st);  // (a panel may still write its flag)
+            PinnedPool::release(pinned);
+        }
+        sfree(zcol, st);
+        sfree(rcol, st);
         sfree(Tb, st);
         sfree(W, st);
         sfree(Vd, st);
@@ -1470,6 +1614,89 @@ static int qr_apply(const QRFactor<T> &f, typename QT<T>::c2 *C, long ldc, int n
     }
     return EXIT_SUCCESS;
 }
+
+// A panel of kNB columns column by column, one launch each
+template <typename T>
+static int panel_columns(QRFactor<T> &f, int j0, float2 *Tp, hipStream_t s) {
+    if (!f.zcol) {
+        f.zcol_stride = (long)((f.M + kColThreads - 1) / kColThreads) * 2 * kNB;
+        HOST_CALL(salloc(&f.rcol, (size_t)2 * kNB, s));
+        HOST_CALL(salloc(&f.zcol, (size_t)2 * f.zcol_stride, s));
+    }
+    const int nblk = (f.M - j0 + kColThreads - 1) / kColThreads;
+    for (int jj = -1; jj < kNB; jj++) {
+        const int bi = jj & 1, bo = (jj + 1) & 1;
+        qr_panel_col<kColThreads><<<nblk, kColThreads, 0, s>>>(
+            (float2 *)f.A, f.lda, f.M, j0, jj, f.zcol + (size_t)bi * f.zcol_stride,
+            (const float2 *)f.rcol + (size_t)bi * kNB, f.zcol + (size_t)bo * f.zcol_stride,
+            (float2 *)f.rcol + (size_t)bo * kNB, nblk, Tp);
+        HIP_CALL(hipGetLastError());
+    }
+    return EXIT_SUCCESS;
+}
+
+// Whether a panel is tried by way of its Gram matrix or goes column by column at
+// once.  After one that was tried and not taken, the next 4 go column by column,
+// then one is tried, and so on: with each one not taken the wait doubles, up to 64
+// panels, and with each one taken it halves.  A panel's outcome is asked for two
+// panels later, by when qr_recon has written it and the device has the panel
+// between to work on.  The rule depends on the outcomes only, not on when they
+// arrive.
+//
+// A panel that is not taken costs qr_recon's one workgroup 0.5 ms at 700 rows, 1.7
+// at 4000, 5.7 at 10000; the column launches 0.3 to 0.6.  QR solves of matrices
+// with no panel that is taken, all of them tried before: 700 x 642 14.1 -> 9.2 ms
+// (3.2 with all taken), 4200 x 4000 228 -> 77 (22), 10300 x 2000 380 -> 78 (19).
+class PanelRoute {
+public:
+    int start(int np, double2 **pinned) {
+        if ((size_t)np * sizeof(int) > PinnedPool::kBytes) return EXIT_SUCCESS;  // (no flags: all are tried)
+        HOST_CALL(PinnedPool::acquire(pinned));
+        flag_ = (int *)*pinned;
+        for (int p = 0; p < np; p++) flag_[p] = -1;
+        return EXIT_SUCCESS;
+    }
+    int *seen(int p) const { return flag_ ? flag_ + p : nullptr; }
+    int decide(int p, hipStream_t s, bool *gram) {
+        if (flag_ && p >= 2 && tried_[p & 1]) {
+            int bad = 0;
+            HOST_CALL(outcome(flag_ + p - 2, s, &bad));
+            hold_ = bad ? std::min(64, std::max(4, 2 * hold_)) : hold_ / 2;
+            until_ = bad ? p + hold_ : std::min(until_, p + hold_);
+        }
+        // (one panel at a time while there is a wait)
+        *gram = !hold_ || (p >= until_ && !tried_[(p + 1) & 1]);
+        tried_[p & 1] = *gram;
+        return EXIT_SUCCESS;
+    }
+
+private:
+    // waits for a panel's outcome; an error of the stream, asked for every 20 ms
+    // (a query itself goes through the stream: at every turn it took 3 us a panel),
+    // ends the wait
+    static int outcome(int *flag, hipStream_t s, int *bad) {
+        using clock = std::chrono::steady_clock;
+        auto next = clock::now() + std::chrono::milliseconds(20);
+        for (;;) {
+            for (int n = 0; n < 64; n++) {
+                const int v = __atomic_load_n(flag, __ATOMIC_ACQUIRE);
+                if (v >= 0) {
+                    *bad = v;
+                    return EXIT_SUCCESS;
+                }
+            }
+            std::this_thread::yield();
+            if (clock::now() < next) continue;
+            const hipError_t e = hipStreamQuery(s);
+            if (e != hipErrorNotReady && __atomic_load_n(flag, __ATOMIC_ACQUIRE) < 0)
+                BEM_FAIL("a QR panel did not run: %s", hipGetErrorString(e));
+            next = clock::now() + std::chrono::milliseconds(20);
+        }
+    }
+    int *flag_ = nullptr;
+    bool tried_[2] = {false, false};  // of the last two panels, by parity
+    int hold_ = 0, until_ = 0;
+};
 
 template <typename T>
 static int qr_factor(QRFactor<T> &f, int extra_cols, hipStream_t s) {
@@ -1502,24 +1729,32 @@ static int qr_factor(QRFactor<T> &f, int extra_cols, hipStream_t s) {
             HOST_CALL(salloc(&f.bad, 1, s));
         }
     }
+    PanelRoute route;
+    if (mfma && !global_panel) HOST_CALL(route.start(np, &f.pinned));
     for (int p = 0; p < np; p++) {
         const int j0 = p * kNB, nb = std::min(kNB, f.N - j0);
         TimedRegion tr;
         timing_begin(tr, sizeof(T) == 4 ? "qr_panel_f32" : "qr_panel_f64", s);
         C2 *Tp = f.Tb + (size_t)p * kNB * kNB;
         const int Mp = f.M - j0;
-        if (mfma && !global_panel) {
+        bool gram = mfma && !global_panel;
+        if (gram) HOST_CALL(route.decide(p, s, &gram));
+        if (mfma && !global_panel && !gram && nb == kNB) {
+            HOST_CALL(panel_columns(f, j0, (float2 *)Tp, s));
+        } else if (mfma && !global_panel) {
+            gram = true;  // (also a narrow last panel, which the column launches do not take)
             const int rpb = kGramChunk * ((Mp + kGramChunk * kGramParts - 1) / (kGramChunk * kGramParts));
             const int nblk = (Mp + rpb - 1) / rpb;
             float2 *Af = (float2 *)f.A, *Vf = (float2 *)f.Vd;
             qr_gram<<<nblk, 256, 0, s>>>(Af, f.lda, f.M, j0, nb, rpb, f.gram, f.Pc, f.ldv);
-            qr_recon<<<1, kRecThreads, 0, s>>>(f.gram, nblk, Af, f.lda, f.M, j0, nb, (float2 *)Tp, Vf, f.ldv, f.Y, f.bad);
+            qr_recon<<<1, kRecThreads, 0, s>>>(f.gram, nblk, Af, f.lda, f.M, j0, nb, (float2 *)Tp, Vf, f.ldv, f.Y, f.bad,
+                                              route.seen(p));
             qr_form_v<<<(Mp + 63) / 64, 256, 0, s>>>(f.Pc, f.Y, f.bad, Af, f.lda, f.M, j0, nb, Vf, f.ldv);
         } else {
             qr_panel<T><<<1, 1024, 0, s>>>(f.A, f.lda, f.M, j0, nb, Tp, mfma ? 0 : 1);
         }
         HIP_CALL(hipGetLastError());
-        if (mfma && global_panel) {
+        if (mfma && !gram) {
             dim3 gv((unsigned)((Mp + 255) / 256), kNB);
             k_build_v<T><<<gv, 256, 0, s>>>(f.A, f.lda, f.M, j0, nb, f.Vd, f.ldv);
             HIP_CALL(hipGetLastError());
@@ -1569,6 +1804,7 @@ size_t qr_work_bytes(int M, int N, int R, bool fp64) {
     size_t b = (fp64 ? sizeof(double2) : sizeof(float2)) * kNB * (np * kNB + N);   // T factors, W
     b += sizeof(double2) * (2 * ng * kGG + (ng * kPairs * splits + np) * kNN);       // triangles and what forms them
     if (!fp64) b += sizeof(float2) * 2 * kNB * ld + sizeof(double2) * (kGramParts + 1) * kNN;  // V, panel, Gram
+    if (!fp64) b += 2 * kNB * (sizeof(float2) + 2 * sizeof(float) * (((size_t)M + kColThreads - 1) / kColThreads));  // column launches
     const size_t nblk = ((size_t)M + solve_rows(M) - 1) / solve_rows(M);
     b += (fp64 ? (size_t)R : 1) * (2 * nblk * 2 * kGW * sizeof(double) + (fp64 ? sizeof(double2) : sizeof(float2)) * N);
     return b;
