@@ -57,7 +57,17 @@ long round64(long m) { return (m + 63) / 64 * 64; }
 // host columns are packed (unpacked) on the device, at most kPackBytes at a
 // time; host columns with gaps keep the pitched copy, which leaves the gaps
 // untouched, and so does a device with no room for the packed columns.
-constexpr size_t kPackBytes = size_t(64) << 20;
+//
+// Columns that lie within kSpanBytes on the device come in one copy, padding and
+// all, and are put in place here: a kernel and its buffer take 35 us, a pitched
+// column 7 (solutions of 642 nodes: 2 columns 23 us pitched, 48 packed, 17 this way).
+// Few wide columns are not packed: into a buffer already in use, 16 columns of 164
+// kB take 0.23 ms pitched and 0.42 packed, 8 of 655 kB 0.28 and 0.86; but a matrix
+// of 642 columns of 480 kB takes 20.8 and 17.0.
+constexpr size_t kPackBytes = size_t(64) << 20, kSpanBytes = size_t(128) << 10;
+bool packs(long ldh, long ldd, int n, int cols) {
+    return ldh == n && ldd != n && cols > 1 && (n < (128 << 10) / 8 || cols > 64);
+}
 
 __global__ void k_copy_cols(const float2 *__restrict__ src, long lds, float2 *__restrict__ dst, long ldd, int n) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -83,12 +93,33 @@ float2 *pack_alloc(size_t n, hipStream_t s) {
     return nullptr;
 }
 
+// bytes from the first column's start to the last one's end
+size_t span_bytes(long ldd, int n, int cols) { return 8 * ((size_t)ldd * (cols - 1) + n); }
+
+// n units of dev in this thread's buffer (of one copy of a few 100 kB at most)
+int span_out(const void *dev, size_t bytes, hipStream_t s, const char **host) {
+    static thread_local std::vector<char> buf;
+    if (buf.size() < bytes) buf.resize(bytes);
+    // (as a pitched copy of one row: 13 us with its wait, a linear one 23)
+    HIP_CALL(hipMemcpy2DAsync(buf.data(), bytes, dev, bytes, bytes, 1, hipMemcpyDeviceToHost, s));
+    HIP_CALL(hipStreamSynchronize(s));
+    *host = buf.data();
+    return EXIT_SUCCESS;
+}
+
 // host (ldh >= n units) <- device; the stream is waited for
 int copy_out(void *host, long ldh, const float2 *dev, long ldd, int n, int cols, hipStream_t s) {
     if (n <= 0 || cols <= 0) return EXIT_SUCCESS;
+    if (cols > 1 && !(ldh == n && ldd == n) && span_bytes(ldd, n, cols) <= kSpanBytes) {
+        const char *span = nullptr;
+        HOST_CALL(span_out(dev, span_bytes(ldd, n, cols), s, &span));
+        for (int c = 0; c < cols; c++)
+            memcpy((char *)host + 8 * (size_t)ldh * c, span + 8 * (size_t)ldd * c, 8 * (size_t)n);
+        return EXIT_SUCCESS;
+    }
     hipError_t e = hipSuccess;
     const int per = pack_columns(n, cols);
-    float2 *pk = ldh == n && ldd != n && cols > 1 ? pack_alloc((size_t)n * per, s) : nullptr;
+    float2 *pk = packs(ldh, ldd, n, cols) ? pack_alloc((size_t)n * per, s) : nullptr;
     if (!pk) {
         if (ldh == n && ldd == n)
             e = hipMemcpyAsync(host, dev, (size_t)8 * n * cols, hipMemcpyDeviceToHost, s);
@@ -115,7 +146,7 @@ int copy_out(void *host, long ldh, const float2 *dev, long ldd, int n, int cols,
 int copy_in(float2 *dev, long ldd, const void *host, long ldh, int n, int cols, hipStream_t s) {
     if (n <= 0 || cols <= 0) return EXIT_SUCCESS;
     const int per = pack_columns(n, cols);
-    float2 *pk = ldh == n && ldd != n && cols > 1 ? pack_alloc((size_t)n * per, s) : nullptr;
+    float2 *pk = packs(ldh, ldd, n, cols) ? pack_alloc((size_t)n * per, s) : nullptr;
     if (!pk) {
         HIP_CALL(hipMemcpy2DAsync(dev, 8 * ldd, host, 8 * ldh, (size_t)8 * n, cols, hipMemcpyHostToDevice, s));
         return EXIT_SUCCESS;
@@ -722,8 +753,20 @@ int bem_solver_get_solution(const bem_solver *sv, bem_complex *x, int ldx) {
     if (sv->xr <= 0) BEM_FAIL("no solution");
     std::lock_guard<std::mutex> lk(sv->mu);
     hipStream_t s = sv->stream;
-    // narrowed on the device: half the bytes to copy, no pass over them here
+    // narrowed on the device: half the bytes to copy, no pass over them here; small
+    // ones here (642 nodes, 1 column: 15 against 47 us; 10242: 25 and 54)
     const int N = sv->dp.N, R = sv->rhs.nrhs;
+    const size_t span = span_bytes(2 * sv->dp.ldA, 2 * N, R);
+    if (span <= kSpanBytes + kSpanBytes / 2) {
+        const char *z = nullptr;
+        HOST_CALL(span_out(sv->X64, span, s, &z));
+        for (int r = 0; r < R; r++)
+            for (int i = 0; i < N; i++) {
+                const double2 v = ((const double2 *)z)[(size_t)r * sv->dp.ldA + i];
+                x[(size_t)r * ldx + i] = {(float)v.x, (float)v.y};
+            }
+        return EXIT_SUCCESS;
+    }
     float2 *xd = R <= 32768 ? pack_alloc((size_t)N * R, s) : nullptr;  // grid.y
     if (!xd) {
         std::vector<double2> z((size_t)N * R);
