@@ -1184,7 +1184,7 @@ constexpr int kFieldWaves = 16;
 constexpr int kFieldR = 16;
 
 struct FieldArgs {
-    const float4 *__restrict__ xs;
+    const float4 *__restrict__ xs;  // w: the point's place in the result (int)
     const ElemRec<double> *__restrict__ recs;
     const FarRec *__restrict__ far;
     const float2 *__restrict__ X;  // N x R, ldx
@@ -1335,8 +1335,8 @@ __global__ __launch_bounds__(64 * kFieldWaves) void field_part(FieldArgs a) {
     }
 }
 
-// out[p, r] = inc_r(x_p) - sum_chunks part, in FP64: 16 runs of every 16th
-// chunk per point, then the runs in order
+// out[w, r] = inc_r(x_p) - sum_chunks part, w the place that x_p names, in FP64: 16
+// runs of every 16th chunk per point, then the runs in order
 constexpr int kFieldRuns = 16;
 __global__ __launch_bounds__(256) void field_finalize(const float4 *__restrict__ xs, int P, int R, int nchunks,
                                                       const float2 *__restrict__ part, double k, int kind, double amp,
@@ -1359,7 +1359,8 @@ __global__ __launch_bounds__(256) void field_finalize(const float4 *__restrict__
         sr += red[q][lp].x;
         si += red[q][lp].y;
     }
-    const double x = xs[p].x, y = xs[p].y, z = xs[p].z;
+    const float4 xp = xs[p];
+    const double x = xp.x, y = xp.y, z = xp.z;
     double ir = 0, ii = 0;
     if (params) {
         const double px = params[3 * r], py = params[3 * r + 1], pz = params[3 * r + 2];
@@ -1376,7 +1377,7 @@ __global__ __launch_bounds__(256) void field_finalize(const float4 *__restrict__
             ii = -amp * sn / (4.0 * kPi * rr);
         }
     }
-    out[(size_t)r * ldo + p] = make_float2((float)(ir - sr), (float)(ii - si));
+    out[(size_t)r * ldo + __float_as_int(xp.w)] = make_float2((float)(ir - sr), (float)(ii - si));
 }
 
 size_t field_part_bytes(int E, int P, int R) {
@@ -1420,12 +1421,114 @@ int field_run(const DeviceProblem &dp, float k, const float4 *xs, int P, const f
     return EXIT_SUCCESS;
 }
 
-int field_fp32(DeviceProblem &dp, float k, const float4 *xs, int P, const float2 *X, long ldx, int R,
-               const RhsSpec &rhs, float2 *out, long ldo, hipStream_t s) {
+// Points in the order of a Z-curve through 32^3 cells of a box (lo, and cells per
+// length inv); points outside go to its outer cells, and so does a NaN.  Each point
+// takes the rule that its own distance to an element asks for, so a wave of points
+// from all over the body runs every rule on most elements; a point's value is the
+// same in any order.
+constexpr int kCells = 1 << 15;
+struct CellBox {
+    float lo[3], inv[3];
+};
+__global__ void k_cell_count(const float4 *__restrict__ xs, int P, CellBox b, int *__restrict__ cell,
+                             int *__restrict__ count) {
+    const int p = blockIdx.x * blockDim.x + threadIdx.x;
+    if (p >= P) return;
+    const float x[3] = {xs[p].x, xs[p].y, xs[p].z};
+    int z = 0;
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+        const float t = (x[d] - b.lo[d]) * b.inv[d];
+        const int c = t >= 31.f ? 31 : t > 0.f ? (int)t : 0;
+#pragma unroll
+        for (int q = 0; q < 5; q++) z |= ((c >> q) & 1) << (3 * q + d);
+    }
+    cell[p] = z;
+    atomicAdd(&count[z], 1);
+}
+// counts to first places, one workgroup
+__global__ __launch_bounds__(1024) void k_cell_scan(int *count) {
+    __shared__ int s[1024];
+    const int t = threadIdx.x;
+    int c[kCells / 1024], sum = 0;
+#pragma unroll
+    for (int i = 0; i < kCells / 1024; i++) {
+        c[i] = count[t * (kCells / 1024) + i];
+        sum += c[i];
+    }
+    s[t] = sum;
+    __syncthreads();
+    for (int d = 1; d < 1024; d *= 2) {
+        const int v = t >= d ? s[t - d] : 0;
+        __syncthreads();
+        s[t] += v;
+        __syncthreads();
+    }
+    int at = s[t] - sum;
+#pragma unroll
+    for (int i = 0; i < kCells / 1024; i++) {
+        count[t * (kCells / 1024) + i] = at;
+        at += c[i];
+    }
+}
+__global__ void k_cell_place(const float4 *__restrict__ xs, int P, const int *__restrict__ cell,
+                             int *__restrict__ at, float4 *__restrict__ out) {
+    const int p = blockIdx.x * blockDim.x + threadIdx.x;
+    if (p < P) out[atomicAdd(&at[cell[p]], 1)] = xs[p];
+}
+__global__ void k_zero_int(int *v, int n) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) v[i] = 0;
+}
+
+// Whether the points are sorted: from 4e6 pairs on (30 us of launches) and 256
+// elements (of fewer, most are near to most points in any order), with one point at
+// least within the 12-point rule's distance (8 rho) of the body's box.  Points at
+// 1.05 radii in random order, in the order given and sorted: 2562 nodes, 1030: 0.43 and
+// 0.35 ms, 30000: 8.4 and 2.7 (6.6 with 36 points everywhere); 642 nodes, 3200: 0.40
+// and 0.29; 162, 13000: 0.41 and 0.33; 42, 60000: 0.47 and 0.56.
+static bool field_sorts(const DeviceProblem &dp, const bem_cart_coord *pts, int P) {
+    if (dp.E < 256 || (double)dp.E * P < 4e6) return false;
+    const double m = std::sqrt((double)kFar12D2) * dp.rho;
+    float lo[3], hi[3];
+    for (int d = 0; d < 3; d++) {
+        lo[d] = (float)(dp.nlo[d] - m);
+        hi[d] = (float)(dp.nhi[d] + m);
+    }
+    for (int p = 0; p < P; p++) {
+        const float *x = pts[p].coords;
+        if (x[0] > lo[0] && x[0] < hi[0] && x[1] > lo[1] && x[1] < hi[1] && x[2] > lo[2] && x[2] < hi[2]) return true;
+    }
+    return false;
+}
+
+int field_fp32(DeviceProblem &dp, float k, const float4 *xs, const bem_cart_coord *pts, int P, const float2 *X,
+               long ldx, int R, const RhsSpec &rhs, float2 *out, long ldo, hipStream_t s) {
     if (P <= 0 || R <= 0) return EXIT_SUCCESS;
-    float2 *part = nullptr;
+    // (one allocation: smaller ones beside it may be cut out of the block that its
+    // last use left, which then has to be mapped anew, 1 ms for 77 MB)
+    const bool sort = field_sorts(dp, pts, P);
+    const size_t pbytes = (field_part_bytes(dp.E, P, R) + 255) / 256 * 256;
+    char *mem = nullptr;
     float *params = nullptr;
-    HOST_CALL(salloc(&part, field_part_bytes(dp.E, P, R) / sizeof(float2), s));
+    HOST_CALL(salloc(&mem, pbytes + (sort ? sizeof(float4) * P + sizeof(int) * ((size_t)P + kCells) : 0), s));
+    float2 *part = (float2 *)mem;
+    if (sort) {
+        float4 *sorted = (float4 *)(mem + pbytes);
+        int *cell = (int *)(sorted + P);
+        CellBox b;
+        for (int d = 0; d < 3; d++) {
+            const double m = std::sqrt((double)kFar7D2) * dp.rho, w = dp.nhi[d] - dp.nlo[d] + 2 * m;
+            b.lo[d] = (float)(dp.nlo[d] - m);
+            b.inv[d] = w > 0 ? (float)(32.0 / w) : 0.f;
+        }
+        int *count = cell + P;
+        k_zero_int<<<kCells / 1024, 1024, 0, s>>>(count, kCells);
+        k_cell_count<<<(P + 255) / 256, 256, 0, s>>>(xs, P, b, cell, count);
+        k_cell_scan<<<1, 1024, 0, s>>>(count);
+        k_cell_place<<<(P + 255) / 256, 256, 0, s>>>(xs, P, cell, count, sorted);
+        xs = sorted;
+    }
     if (!rhs.params.empty()) {
         HOST_CALL(salloc(&params, rhs.params.size(), s));
         HIP_CALL(hipMemcpyAsync(params, rhs.params.data(), rhs.params.size() * sizeof(float), hipMemcpyHostToDevice, s));
@@ -1433,7 +1536,7 @@ int field_fp32(DeviceProblem &dp, float k, const float4 *xs, int P, const float2
     const int rc = field_run(dp, k, xs, P, X, ldx, R, rhs.kind, (double)rhs.amp, rhs.nrhs >= R ? params : nullptr, part,
                              out, ldo, s);
     (void)hipStreamSynchronize(s);
-    sfree(part, s);
+    sfree(mem, s);
     sfree(params, s);
     return rc;
 }
@@ -1871,7 +1974,7 @@ size_t round256(size_t b) { return (b + 255) / 256 * 256; }
 __global__ void k_pack_field_points(const float *__restrict__ xs, int P, float4 *__restrict__ xs4, float sx, float sy,
                                     float sz, float *__restrict__ params) {
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p < P) xs4[p] = make_float4(xs[3 * p], xs[3 * p + 1], xs[3 * p + 2], 0.f);
+    if (p < P) xs4[p] = make_float4(xs[3 * p], xs[3 * p + 1], xs[3 * p + 2], __int_as_float(p));
     if (p == 0) {
         params[0] = sx;
         params[1] = sy;
@@ -2237,6 +2340,13 @@ int device_problem_build(const Mesh &m, DeviceProblem &dp, hipStream_t s) {
         }
     }
     dp.diam = diagonal(dp.lo, dp.hi);
+    for (int i = 0; i < dp.N; i++)
+        for (int d = 0; d < 3; d++) {
+            const double x = dp.hpts[3 * (size_t)i + d];
+            dp.nlo[d] = i ? std::min(dp.nlo[d], x) : x;
+            dp.nhi[d] = i ? std::max(dp.nhi[d], x) : x;
+        }
+    dp.rho = 0;
     dp.helems.resize(3 * (size_t)dp.E);
     std::vector<float2> bc(3 * (size_t)dp.E);
     std::vector<char> used(dp.N, 0);
@@ -2247,6 +2357,20 @@ int device_problem_build(const Mesh &m, DeviceProblem &dp, hipStream_t s) {
             used[m.elems[e].nodes[j]] = 1;
             bc[3 * e + j] = make_float2(m.elems[e].bc[j].x, m.elems[e].bc[j].y);
         }
+        double c[3], q = 0;
+        for (int d = 0; d < 3; d++) {
+            c[d] = 0;
+            for (int j = 0; j < 3; j++) c[d] += dp.hpts[3 * (size_t)dp.helems[3 * e + j] + d] / 3.0;
+        }
+        for (int j = 0; j < 3; j++) {
+            double r2 = 0;
+            for (int d = 0; d < 3; d++) {
+                const double y = dp.hpts[3 * (size_t)dp.helems[3 * e + j] + d] - c[d];
+                r2 += y * y;
+            }
+            q = std::max(q, r2);
+        }
+        dp.rho = std::max(dp.rho, std::sqrt(q));
         // (a NaN counts as set)
         if (!(bc[3 * e].x == 0.f && bc[3 * e].y == 0.f)) dp.impedance = 1;
         if (!(bc[3 * e + 2].x == 0.f && bc[3 * e + 2].y == 0.f)) dp.source = 1;

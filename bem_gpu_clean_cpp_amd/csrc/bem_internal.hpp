@@ -180,6 +180,8 @@ struct DeviceProblem {
     int source = 0;               // some element has cc != 0
     double lo[3] = {0, 0, 0}, hi[3] = {0, 0, 0};  // bounding box of the M points
     double diam = 0;              // its diagonal: bounds every |x - y|
+    double nlo[3] = {0, 0, 0}, nhi[3] = {0, 0, 0};  // bounding box of the nodes
+    double rho = 0;               // the largest centroid-vertex distance of an element
     // halo plan (TilePlan): hP column tiles asked for when the problem is built,
     // P of them made, 0 until a kernel that walks them runs
     int hP = 0, P = 0;
@@ -241,9 +243,11 @@ int assemble_fp64(DeviceProblem &dp, double k, double2 *A, hipStream_t s);
 int rhs_fp32(DeviceProblem &dp, double k, float2 *B, long ldB, const RhsSpec &rhs, hipStream_t s);
 int rhs_fp64(DeviceProblem &dp, double k, double2 *B, long ldB, const RhsSpec &rhs, hipStream_t s);
 // Exterior field: out[P x R] = inc - sum_e (...) for nodal solutions X (N x R).
-int field_fp32(DeviceProblem &dp, float k, const float4 *xs, int P, const float2 *X, long ldx, int R,
-               const RhsSpec &rhs, float2 *out, long ldo, hipStream_t s);
+// (pts: the points on the host)
+int field_fp32(DeviceProblem &dp, float k, const float4 *xs, const bem_cart_coord *pts, int P, const float2 *X,
+               long ldx, int R, const RhsSpec &rhs, float2 *out, long ldo, hipStream_t s);
 
+// (xs of field_fp32 and field_run: the point and, as an int in w, its place in out)
 // queued on s without allocations: params (3 R or null) and part
 // (field_part_bytes) in device memory
 size_t field_part_bytes(int E, int P, int R);

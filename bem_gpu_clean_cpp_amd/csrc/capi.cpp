@@ -865,13 +865,16 @@ int bem_solver_field(bem_solver *sv, const bem_cart_coord *pts, int P, bem_compl
     k_z2c_copy<<<(unsigned)((n + 255) / 256), 256, 0, s>>>(sv->X64, sv->X32, n);
     HIP_CALL(hipGetLastError());
     std::vector<float4> xh(P);
-    for (int p = 0; p < P; p++) xh[p] = make_float4(pts[p].coords[0], pts[p].coords[1], pts[p].coords[2], 0.f);
+    for (int p = 0; p < P; p++) {
+        xh[p] = make_float4(pts[p].coords[0], pts[p].coords[1], pts[p].coords[2], 0.f);
+        memcpy(&xh[p].w, &p, sizeof p);
+    }
     float4 *xd = nullptr;
     float2 *od = nullptr;
     HOST_CALL(salloc(&xd, P, s));
     HOST_CALL(salloc(&od, (size_t)P * R, s));
     HIP_CALL(hipMemcpyAsync(xd, xh.data(), sizeof(float4) * P, hipMemcpyHostToDevice, s));
-    int rc = field_fp32(dp, sv->k, xd, P, sv->X32, dp.ldA, R, sv->rhs, od, P, s);
+    int rc = field_fp32(dp, sv->k, xd, pts, P, sv->X32, dp.ldA, R, sv->rhs, od, P, s);
     hipError_t e = hipMemcpy2DAsync(out, sizeof(bem_complex) * ldo, od, sizeof(float2) * P, sizeof(float2) * P, R,
                                     hipMemcpyDeviceToHost, s);
     (void)hipStreamSynchronize(s);
