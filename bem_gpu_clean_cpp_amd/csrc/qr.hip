@@ -1842,10 +1842,15 @@ template <typename T>
 static int qr_solve_factored(QRFactor<T> &f, typename QT<T>::c2 *B, long ldb, int R, hipStream_t s) {
     using C2 = typename QT<T>::c2;
     if (R <= 0) return EXIT_SUCCESS;
-    // the whole solve in one workgroup per right-hand side, b in shared memory
-    // (on request; the row-split launches below are faster at every size)
+    // the whole solve in one workgroup per right-hand side, b in shared memory: on
+    // request, and for small FP64 systems, whose factorisation serves one solve, so
+    // that the triangles of the row-split launches below (70 us) do not pay (14
+    // unknowns: 0.33 against 0.45 ms for factorisation and solve; 194: 6.12 and 6.19;
+    // 642: 21.96 and 21.57).  FP32 systems of that size are solved several times, or
+    // with FP64 sums that this kernel does not have.
     const size_t lds = sizeof(C2) * (size_t)f.M;
-    if (lds <= kSmallSolveLds && R <= kSmallSolveRhs && getenv("BEM_QR_ONE_WG_SOLVE")) {
+    const bool small = sizeof(T) == 8 && f.N <= 256 && !getenv("BEM_QR_PER_COLUMN_SOLVE");
+    if (lds <= kSmallSolveLds && R <= kSmallSolveRhs && (small || getenv("BEM_QR_ONE_WG_SOLVE"))) {
         // 2 kNB partial sums per thread plus a chunk of 8 loads: the register
         // room of 512 (FP32) or 256 (FP64) threads
         constexpr int nt = sizeof(T) == 4 ? 512 : 256;
