@@ -22,9 +22,11 @@
 // (Gatermann 1988), their points and weights found by solving the moment
 // equations in FP64 (largest moment residual 1e-14).
 //
-// What bounds it: the vector ALU (large meshes run at 100 % VALU issue).  A
-// pair costs about 1000 VALU instructions with 36 points; 250 with 7, 420 with
-// 12.  10242 nodes at 2 kHz: 5.16 -> 2.0 ms; 40962 nodes at 12 kHz: 81 -> 36 ms.
+// What bounds it: the vector ALU.  At 10242 nodes and 2 kHz the kernel issues
+// 305 VALU instructions a pair (915 with 36 points for every pair), 0.195 per
+// SIMD-cycle of the 0.25 that a SIMD of 16 lanes can, with 4 waves per SIMD.
+// There it takes 2.08 ms (5.16 with 36 points everywhere), and for 40962 nodes
+// at 12 kHz 36.4 ms alone, 38.5 to 40 within a solve (81).
 #pragma once
 
 #include <hip/hip_runtime.h>

@@ -1820,7 +1820,10 @@ __global__ __launch_bounds__(NT) void mh_kernel(const double2 *__restrict__ A, l
 }
 
 // about 768 workgroups of 256 rows (5778 x 5762, 4 right-hand sides: 110 us
-// with 2048, 93 us with 700, 111 us with 350)
+// with 2048, 93 us with 700, 111 us with 350).  Whole FP64 solves with these
+// products, against one product per right-hand side: 162 nodes 1.2 (2 right-hand
+// sides) to 2.8 times faster (33), 642 1.3 to 3.6, 2562 1.8 to 5.3, 10242 2.0 (2)
+// and 3.7 (4); none of 42 to 10242 nodes with 1 to 33 right-hand sides slower.
 static void mres_shape(long M, long N, int &nch, int &kc) {
     const long tiles = (M + 255) / 256;
     long target = std::max(1L, 768 / std::max(1L, tiles));

@@ -56,7 +56,7 @@ READ_CEILING_GBS = 6200.0
 FLOP_PER_EVAL = 80.0       # nominal FP32 flops per (row, quadrature point) evaluation
 # measured VALU issue rate of the FP32 assembly kernel (wave-instructions per
 # SIMD-cycle, SQ counters of profiles/precision_s5_asm_valu_counters.txt)
-ASM_VALU_ISSUE = 0.198
+ASM_VALU_ISSUE = 0.195
 
 PRECISION = dict(subdiv=5, radius=0.1, freq=2000.0, nchief=16, seed=102)
 
