@@ -1507,11 +1507,17 @@ int field_fp32(DeviceProblem &dp, float k, const float4 *xs, const bem_cart_coor
     if (P <= 0 || R <= 0) return EXIT_SUCCESS;
     // (one allocation: smaller ones beside it may be cut out of the block that its
     // last use left, which then has to be mapped anew, 1 ms for 77 MB)
-    const bool sort = field_sorts(dp, pts, P);
+    bool sort = field_sorts(dp, pts, P);
     const size_t pbytes = (field_part_bytes(dp.E, P, R) + 255) / 256 * 256;
     char *mem = nullptr;
     float *params = nullptr;
-    HOST_CALL(salloc(&mem, pbytes + (sort ? sizeof(float4) * P + sizeof(int) * ((size_t)P + kCells) : 0), s));
+    if (sort && hipMallocAsync((void **)&mem, pbytes + sizeof(float4) * P + sizeof(int) * ((size_t)P + kCells), s) !=
+                    hipSuccess) {
+        (void)hipGetLastError();
+        mem = nullptr;
+        sort = false;  // (no room: the order given)
+    }
+    if (!mem) HOST_CALL(salloc(&mem, pbytes, s));
     float2 *part = (float2 *)mem;
     if (sort) {
         float4 *sorted = (float4 *)(mem + pbytes);
